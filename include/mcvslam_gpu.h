@@ -132,11 +132,12 @@ int mcv_match_filter_orientation(mcv_ctx* ctx, const int32_t* matches, int n, co
 int mcv_distinctive_descriptors(mcv_ctx* ctx, const uint8_t* desc, const int32_t* ptr, int n, int32_t* best,
                                 uint8_t* out_desc);
 /* Launch variant of the top-2 kernel used by mcv_match_knn2* on this context
- * (0 .. 11: 0-3, 5-7 popcount kernels with scalar-loaded trains, 4 LDS-tiled,
- * 8-9 distances on the int8 matrix cores, 10-11 on the fp4 ones (train sets
- * of 65536 or more rows run variant 8); no counterpart in the reference: the
- * autotuner's choice, also settable for testing).  Every variant returns the
- * same rows. */
+ * (0 .. 11: 0, the default, the library's choice (currently 10); 1-3, 5-7
+ * popcount kernels with scalar-loaded trains, 4 LDS-tiled, 8-9 distances on
+ * the int8 matrix cores, 10-11 on the fp4 ones, which cut large train sets
+ * into segments when there are few queries; no counterpart in the reference:
+ * the autotuner's choice, also settable for testing).  Every variant returns
+ * the same rows. */
 int mcv_match_set_variant(mcv_ctx* ctx, int variant);
 int mcv_match_knn2_dev(mcv_ctx* ctx, const uint8_t* d_q, int nq, const uint8_t* d_t, int nt, int32_t* d_out);
 /* Replaces MatchResKnn::FilterRatio(ratio).FilterThreshold(th)

@@ -401,7 +401,7 @@ enum EnqPart {
 constexpr int kFastSplitLevel = 3;
 
 struct Tuning {
-    int knn = 0;   // launch_knn2 variant
+    int knn = 0;   // launch_knn2 variant (0: its rule)
     int blur = 0;  // 0: k_blur<false>, 1: k_blur<true>
     int kp = 2;    // keypoints per wave: 0: one (k_keypoints), 1: 8, 2: 16, 3: 32 (k_keypoints_k<K>)
     int heap = 1;  // 0: k_octree_heap_r (register top), 1: k_octree_heap (LDS), the faster one measured
@@ -862,7 +862,7 @@ struct mcv_ctx {
     int single_key_w = -1, single_key_h = -1;
     std::vector<int> single_key_seeds;
     DevBuf in_img, out_kps, out_desc, out_cnt;
-    DevBuf m_q, m_t, m_out, m_pairs, f_knn, f_out, f_cnt, f_scr, f_jobs;
+    DevBuf m_q, m_t, m_out, m_part, f_knn, f_out, f_cnt, f_scr, f_jobs;
     DevBuf d_desc_in, d_ptr, d_best, d_desc_out;
     DevBuf o_m, o_a1, o_a2, o_out, o_cnt, o_jobs;
     DevBuf w_pts, w_pdesc, w_plev, w_kxy, w_kdesc, w_cs, w_ci, w_out, w_view, w_cams;
@@ -906,7 +906,7 @@ struct mcv_rig {
     std::unique_ptr<OrbPlan> batch;                 // all 3n images
     std::vector<std::unique_ptr<OrbPlan>> single;   // per camera, one image
     int cap = 0;
-    DevBuf kps, desc, counts, knn, matches, mcounts, pairs, jobs, scratch, porder;
+    DevBuf kps, desc, counts, knn, matches, mcounts, pairs, jobs, scratch, porder, part;
     std::vector<MatchPair> hp;
     std::vector<FilterJob> hj;
     // Captured graphs of the batched run, one set per launch-variant set used
@@ -1405,12 +1405,21 @@ int mcv_orb_batch_pyramid_dev(mcv_ctx* c, int image, int level, int blurred, con
 }
 
 // ---- matching ---------------------------------------------------------------
-static void launch_knn(hipStream_t s, DevBuf& pbuf, const std::vector<MatchPair>& pairs, int max_nq, int variant) {
-    if (pairs.empty() || max_nq <= 0) return;
-    upload(pbuf, pairs, s);
-    int max_nt = 0;
-    for (const MatchPair& p : pairs) max_nt = std::max(max_nt, p.nt);
-    launch_knn2(variant, pbuf.as<MatchPair>(), (int)pairs.size(), max_nq, s, max_nt);
+// one pair of host-known sizes (the pair travels as a kernel argument), at
+// most kKnnChunk queries a launch: the segment keys stay below 64 MiB
+constexpr int kKnnChunk = 1 << 17;
+static void launch_knn(mcv_ctx* c, const MatchPair& pair) {
+    for (int q0 = 0; q0 < pair.nq; q0 += kKnnChunk) {
+        KnnLaunch K;
+        K.one = pair;
+        K.one.q += (size_t)q0 * 32;
+        K.one.out += (size_t)q0 * 4;
+        K.one.nq = K.max_nq = std::min(kKnnChunk, pair.nq - q0);
+        K.max_nt = pair.nt;
+        c->m_part.ensure(knn_part_bytes(c->knn_variant, 1, K.max_nq, pair.nt));
+        K.part = c->m_part.as<uint2>();
+        launch_knn2(c->knn_variant, K, c->stream);
+    }
     HIP_OK(hipGetLastError());
 }
 
@@ -1418,8 +1427,7 @@ int mcv_match_knn2_dev(mcv_ctx* c, const uint8_t* d_q, int nq, const uint8_t* d_
     API_BEGIN(c)
     REQUIRE(c && nq >= 0 && nt >= 0 && nt < (1 << 22), MCV_ERR_INVALID, "bad sizes");
     c->set_device();
-    MatchPair p{d_q, d_t, nullptr, nullptr, nq, nt, d_out};
-    launch_knn(c->stream, c->m_pairs, {p}, nq, c->knn_variant);
+    launch_knn(c, MatchPair{d_q, d_t, nullptr, nullptr, nq, nt, d_out});
     API_END
 }
 
@@ -1507,8 +1515,8 @@ int mcv_match_knn2(mcv_ctx* c, const uint8_t* q, int nq, const uint8_t* t, int n
     c->m_out.ensure((size_t)nq * 16);
     HIP_OK(hipMemcpyAsync(c->m_q.p, q, (size_t)nq * 32, hipMemcpyHostToDevice, c->stream));
     if (nt) HIP_OK(hipMemcpyAsync(c->m_t.p, t, (size_t)nt * 32, hipMemcpyHostToDevice, c->stream));
-    MatchPair p{c->m_q.as<uint8_t>(), c->m_t.as<uint8_t>(), nullptr, nullptr, nq, nt, c->m_out.as<int32_t>()};
-    launch_knn(c->stream, c->m_pairs, {p}, nq, c->knn_variant);
+    launch_knn(c, MatchPair{c->m_q.as<uint8_t>(), c->m_t.as<uint8_t>(), nullptr, nullptr, nq, nt,
+                            c->m_out.as<int32_t>()});
     HIP_OK(hipMemcpyAsync(out, c->m_out.p, (size_t)nq * 16, hipMemcpyDeviceToHost, c->stream));
     HIP_OK(hipStreamSynchronize(c->stream));
     API_END
@@ -1608,6 +1616,8 @@ int mcv_rig_create(mcv_ctx* c, int n_frames, const int32_t* w3, const int32_t* h
     r->mcounts.ensure((size_t)n * 4);
     r->scratch.ensure((size_t)n * r->cap * 8);
     r->porder.ensure((size_t)(2 * n + 1) * sizeof(int));
+    // segment keys of the fp4 top-2: the batched launch's or one pair's
+    r->part.ensure(std::max(knn_part_bytes(0, n, r->cap, r->cap), knn_part_bytes(0, 1, r->cap, r->cap)));
     // pairs per frame: L-R (query L), W-L (query W), W-R (query W)
     const int qa[3] = {0, 2, 2}, ta[3] = {1, 0, 1};
     for (int f = 0; f < n_frames; f++)
@@ -1642,17 +1652,25 @@ int mcv_rig_create(mcv_ctx* c, int n_frames, const int32_t* w3, const int32_t* h
 
 void mcv_rig_destroy(mcv_rig* r) { delete r; }
 
+// top-2 launch of np pairs of the rig's table from pair p0 on
+static KnnLaunch rig_knn_launch(mcv_rig* r, int p0, int np) {
+    KnnLaunch K;
+    K.pairs = r->pairs.as<MatchPair>() + p0;
+    K.npairs = np;
+    K.max_nq = K.max_nt = r->cap;
+    K.part = r->part.as<uint2>();
+    return K;
+}
+
 // the rig's top-2 launch: the pairs ordered by train count first (the
 // counts are on the device), then the chosen variant
 static void rig_knn(mcv_rig* r, hipStream_t s) {
-    const int np = (int)r->hp.size();
-    const int* order = nullptr;
-    if (np <= kPairOrderMax) {
-        hipLaunchKernelGGL(k_pair_order, dim3(1), dim3(256), 0, s, r->pairs.as<MatchPair>(), np,
-                           r->porder.as<int>());
-        order = r->porder.as<int>();
+    KnnLaunch K = rig_knn_launch(r, 0, (int)r->hp.size());
+    if (K.npairs <= kPairOrderMax) {
+        hipLaunchKernelGGL(k_pair_order, dim3(1), dim3(256), 0, s, K.pairs, K.npairs, r->porder.as<int>());
+        K.order = r->porder.as<int>();
     }
-    launch_knn2(r->tune.knn, r->pairs.as<MatchPair>(), np, r->cap, s, -1, order);
+    launch_knn2(r->tune.knn, K, s);
 }
 
 static void rig_enqueue_batched(mcv_rig* r, const SinCosTables& tb, hipStream_t s, KernelTimer* rec = nullptr,
@@ -1999,7 +2017,7 @@ int mcv_rig_run(mcv_rig* r, const uint8_t* const* d_images, int flags) {
             }
             for (int k = 0; k < 3; k++) {
                 const int p = 3 * f + k;
-                launch_knn2(r->tune.knn, r->pairs.as<MatchPair>() + p, 1, r->cap, s);
+                launch_knn2(r->tune.knn, rig_knn_launch(r, p, 1), s);
                 hipLaunchKernelGGL(k_filter, dim3(1), dim3(1024), 0, s, r->jobs.as<FilterJob>() + p);
             }
             // the single-image plans are reused by the next frame

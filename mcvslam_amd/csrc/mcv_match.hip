@@ -60,9 +60,9 @@ __device__ __forceinline__ void top2_insert2(uint32_t& k0, uint32_t& k1, uint32_
 // wave-uniform and come through scalar loads (SGPR operands of the XORs),
 // UNR rows per iteration; the four waves' top-2 keys merge through LDS.
 template <int QPL, int UNR>
-__global__ __launch_bounds__(256) void k_knn2_s(const MatchPair* pairs) {
+__global__ __launch_bounds__(256) void k_knn2_s(const MatchPair* pairs, MatchPair one) {
     __shared__ uint32_t sk[2][4][64 * QPL];
-    const MatchPair P = pairs[blockIdx.y];
+    const MatchPair P = pairs ? pairs[blockIdx.y] : one;
     const int nq = P.nq_dev ? min(*P.nq_dev, P.nq) : P.nq;
     const int nt = P.nt_dev ? min(*P.nt_dev, P.nt) : P.nt;
     const int lane = threadIdx.x & 63;
@@ -151,9 +151,9 @@ __global__ __launch_bounds__(256) void k_knn2_s(const MatchPair* pairs) {
 constexpr int kKnnTile = 128;
 constexpr int kKnnQ = 256;  // queries per workgroup
 
-__global__ __launch_bounds__(256) void k_knn2_lds(const MatchPair* pairs) {
+__global__ __launch_bounds__(256) void k_knn2_lds(const MatchPair* pairs, MatchPair one) {
     __shared__ uint4 s_t[2][2 * kKnnTile];
-    const MatchPair P = pairs[blockIdx.y];
+    const MatchPair P = pairs ? pairs[blockIdx.y] : one;
     const int nq = P.nq_dev ? min(*P.nq_dev, P.nq) : P.nq;
     const int nt = P.nt_dev ? min(*P.nt_dev, P.nt) : P.nt;
     const int q0 = blockIdx.x * kKnnQ;
@@ -285,9 +285,9 @@ __device__ __forceinline__ void knn_m_tile(const mcv_v4i (&a)[QT][9], const mcv_
 constexpr int kMSub = 4;  // 32-train sub-tiles per 128-train super-tile
 
 template <int QT>
-__global__ __launch_bounds__(256) void k_knn2_m(const MatchPair* pairs) {
+__global__ __launch_bounds__(256) void k_knn2_m(const MatchPair* pairs, MatchPair one) {
     __shared__ mcv_v4i s_b[kMSub][9][64];  // a super-tile as B operands, [sub-tile][step][lane]
-    const MatchPair P = pairs[blockIdx.y];
+    const MatchPair P = pairs ? pairs[blockIdx.y] : one;
     const int nq = P.nq_dev ? min(*P.nq_dev, P.nq) : P.nq;
     const int nt = P.nt_dev ? min(*P.nt_dev, P.nt) : P.nt;
     const int q0 = blockIdx.x * 128 * QT;
@@ -407,7 +407,7 @@ __global__ __launch_bounds__(256) void k_knn2_m(const MatchPair* pairs) {
 // |t| the same way), so the f32 accumulators hold the distances exactly
 // (integers <= 256).  Such a float's top 16 bits order it like the integer
 // and keep it exactly, so a key is (bits & 0xFFFF0000) | j: one and-or per
-// distance, then the med3/min top-2 update; j < 65536 (the launcher checks).
+// distance, then the med3/min top-2 update; j < 65536 (knn_segments).
 typedef int mcv_v8i __attribute__((ext_vector_type(8)));
 typedef float mcv_v16f __attribute__((ext_vector_type(16)));
 
@@ -463,12 +463,46 @@ __device__ __forceinline__ void knn_f4_tile(const mcv_v4i (&a)[5], mcv_v4i ones,
     }
 }
 
+// A fp4 key as a (distance << 22) | train index key; base: the train its
+// indices count from
+__device__ __forceinline__ uint32_t f4_key(uint32_t k, int base) {
+    if (k == kF4Sentinel) return kSentinel;
+    return ((uint32_t)__builtin_bit_cast(float, k & 0xFFFF0000u) << kIdxBits) | (uint32_t)(base + (int)(k & 0xFFFFu));
+}
+
+__device__ __forceinline__ int4 knn_row(uint32_t a0, uint32_t a1) {
+    // the sentinel keeps index 0 and distance 999, as the reference's d_idx init does
+    return make_int4((int)(a0 & kIdxMask), (int)(a0 >> kIdxBits), (int)(a1 & kIdxMask), (int)(a1 >> kIdxBits));
+}
+
+// Halves the rows of a lane's top-2 keys: keeps rows [0, N) or, with hi,
+// [N, 2N) and merges in the keys the DPP partner holds of those rows.
+template <int kCtrl, int N>
+__device__ __forceinline__ void f4_merge_step(uint32_t (&k0)[16], uint32_t (&k1)[16], int hi) {
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+        const uint32_t s0 = hi ? k0[r] : k0[r + N], s1 = hi ? k1[r] : k1[r + N];  // the partner's rows
+        const uint32_t a0 = hi ? k0[r + N] : k0[r], a1 = hi ? k1[r + N] : k1[r];
+        const uint32_t b0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)s0, kCtrl, 0xF, 0xF, false);
+        const uint32_t b1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)s1, kCtrl, 0xF, 0xF, false);
+        k1[r] = min(max(a0, b0), min(a1, b1));
+        k0[r] = min(a0, b0);
+    }
+}
+
 // kDb: two super-tiles as B operands (4 bit steps, then |t|), the next one
 // expanded between the current one's first and second blocks, one barrier
 // per super-tile (40 KB of LDS); else one super-tile expanded between two
 // barriers (20 KB).  kWaves: waves per SIMD the registers are cut for.
+// pairs: the pair table, or null: the single pair `one`.
+// part: null when one workgroup walks a tile's whole train set; else the
+// train set is cut into gridDim.z segments of whole super-tiles, and segment
+// z leaves its top-2 keys of query qi in part[(pair * cap + qi) * gridDim.z + z]
+// for k_knn2_merge.  Train indices are kept relative to the segment, so they fit
+// 16 bits as long as a segment holds at most 512 super-tiles.
 template <bool kDb, int kWaves>
-__global__ __launch_bounds__(256, kWaves) void k_knn2_f4(const MatchPair* pairs, const int* order, int np) {
+__global__ __launch_bounds__(256, kWaves) void k_knn2_f4(const MatchPair* pairs, MatchPair one, const int* order,
+                                                         int np, uint2* part, int cap) {
     __shared__ mcv_v4i s_b[kDb ? 2 : 1][kMSub][5][64];
     // with an order: a 1-D grid over the real 128-query tiles of the pairs
     // in that order (largest train sets first), the spare workgroups last;
@@ -485,7 +519,7 @@ __global__ __launch_bounds__(256, kWaves) void k_knn2_f4(const MatchPair* pairs,
         pi = order[lo];
         tile = b - order[np + lo];
     }
-    const MatchPair P = pairs[pi];
+    const MatchPair P = pairs ? pairs[pi] : one;
     const int nq = P.nq_dev ? min(*P.nq_dev, P.nq) : P.nq;
     const int nt = P.nt_dev ? min(*P.nt_dev, P.nt) : P.nt;
     const int q0 = tile * 128;
@@ -525,7 +559,13 @@ __global__ __launch_bounds__(256, kWaves) void k_knn2_f4(const MatchPair* pairs,
         const int j = st * 32 * kMSub + (threadIdx.x >> 1);
         return j < nt ? tv[2ll * j + (threadIdx.x & 1)] : make_uint4(0u, 0u, 0u, 0u);
     };
-    const int nsuper = (nt + 32 * kMSub - 1) / (32 * kMSub);
+    int st0 = 0, nsuper = (nt + 32 * kMSub - 1) / (32 * kMSub);  // this workgroup's super-tiles: [st0, nsuper)
+    if (part) {
+        const int per = (nsuper + (int)gridDim.z - 1) / (int)gridDim.z;
+        st0 = (int)blockIdx.z * per;
+        nsuper = min(nsuper, st0 + per);
+    }
+    const int jbase = st0 * 32 * kMSub;
     const int jl = threadIdx.x >> 1, sub = jl >> 5, col = jl & 31, th = threadIdx.x & 1;
     auto expand = [&](const uint4 raw, int buf) {
         const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
@@ -544,70 +584,89 @@ __global__ __launch_bounds__(256, kWaves) void k_knn2_f4(const MatchPair* pairs,
         s_b[buf][sub][4][32 * th + col] = count_nibbles(pc, th);
     };
     uint4 raw = make_uint4(0u, 0u, 0u, 0u);
-    if (nsuper > 0) {
-        expand(fetch(0), 0);
-        if (nsuper > 1) raw = fetch(1);
+    if (st0 < nsuper) {
+        expand(fetch(st0), 0);
+        if (st0 + 1 < nsuper) raw = fetch(st0 + 1);
     }
-    for (int st = 0; st < nsuper; st++) {
+    for (int st = st0; st < nsuper; st++) {
         if constexpr (!kDb) {
-            if (st > 0) {
+            if (st > st0) {
                 __syncthreads();  // the previous super-tile's operands are read
                 expand(raw, 0);
                 if (st + 1 < nsuper) raw = fetch(st + 1);
             }
         }
-        // (two buffers) super-tile st is in buffer st & 1; the other buffer
-        // was last read in iteration st - 1, which every wave has finished here
+        // (two buffers) super-tile st is in buffer (st - st0) & 1; the other
+        // buffer was last read in iteration st - 1, which every wave has finished here
         __syncthreads();
-        const int cb = kDb ? (st & 1) : 0;
+        const int cb = kDb ? ((st - st0) & 1) : 0;
         const int tj = st * 32 * kMSub;
+        const uint32_t jr = (uint32_t)(tj - jbase + (lane & 31));  // relative to the segment
         if (tj + 32 * kMSub <= nt) {
-            knn_f4_tile<false>(a, ones, &s_b[cb][0][0][lane], (uint32_t)(tj + (lane & 31)), true, k0, k1);
+            knn_f4_tile<false>(a, ones, &s_b[cb][0][0][lane], jr, true, k0, k1);
             if (kDb && st + 1 < nsuper) {
                 expand(raw, cb ^ 1);
                 if (st + 2 < nsuper) raw = fetch(st + 2);
             }
 #pragma unroll 1
             for (int sb = 1; sb < kMSub; sb++)
-                knn_f4_tile<false>(a, ones, &s_b[cb][sb][0][lane], (uint32_t)(tj + 32 * sb + (lane & 31)), true, k0,
-                                   k1);
+                knn_f4_tile<false>(a, ones, &s_b[cb][sb][0][lane], jr + 32u * (uint32_t)sb, true, k0, k1);
         } else {
             // a partial super-tile is the last one: nothing left to expand
 #pragma unroll
             for (int sb = 0; sb < kMSub; sb++) {
                 const int tj0 = tj + 32 * sb;
-                if (tj0 < nt) {
-                    const uint32_t j = (uint32_t)(tj0 + (lane & 31));
-                    knn_f4_tile<true>(a, ones, &s_b[cb][sb][0][lane], j, (int)j < nt, k0, k1);
-                }
+                if (tj0 < nt)
+                    knn_f4_tile<true>(a, ones, &s_b[cb][sb][0][lane], jr + 32u * (uint32_t)sb,
+                                      tj0 + (lane & 31) < nt, k0, k1);
             }
         }
     }
-    // the 32 lanes of a half hold the same rows: merge their top-2 keys
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-        uint32_t a0 = k0[r], a1 = k1[r];
-#pragma unroll
-        for (int o = 1; o < 32; o <<= 1) {
-            const uint32_t b0 = (uint32_t)__shfl_xor((int)a0, o, 64), b1 = (uint32_t)__shfl_xor((int)a1, o, 64);
-            const uint32_t n1 = min(max(a0, b0), min(a1, b1));
-            a0 = min(a0, b0);
-            a1 = n1;
-        }
-        const int qi = wq0 + 8 * (r >> 2) + 4 * half + (r & 3);
-        if ((lane & 31) == 0 && qi < nq) {
-            // the sentinel keeps index 0 and distance 999, as the reference's d_idx init does
-            auto dist = [](uint32_t k) {
-                return k == kF4Sentinel ? 999 : (int)__builtin_bit_cast(float, k & 0xFFFF0000u);
-            };
-            int4 o;
-            o.x = (int)(a0 & 0xFFFFu);
-            o.y = dist(a0);
-            o.z = (int)(a1 & 0xFFFFu);
-            o.w = dist(a1);
-            reinterpret_cast<int4*>(P.out)[qi] = o;
+    // The 32 lanes of a half hold the same 16 rows: merge their top-2 keys.
+    // Each step halves the rows a lane keeps (by one bit of its number) and
+    // takes the partner's keys of those rows, so 15 row exchanges by DPP move
+    // do what 16 rows x 4 butterfly steps of LDS shuffles did; lane l ends
+    // with row l % 16, and one shuffle adds the other 16 lanes.
+    f4_merge_step<0x140, 8>(k0, k1, lane & 8);  // row mirror: lane ^ 15
+    f4_merge_step<0x141, 4>(k0, k1, lane & 4);  // half-row mirror: lane ^ 7
+    f4_merge_step<0x1B, 2>(k0, k1, lane & 2);   // quad reversal: lane ^ 3
+    f4_merge_step<0xB1, 1>(k0, k1, lane & 1);   // lane ^ 1
+    const uint32_t b0 = (uint32_t)__shfl_xor((int)k0[0], 16, 64), b1 = (uint32_t)__shfl_xor((int)k1[0], 16, 64);
+    const uint32_t a1 = f4_key(min(max(k0[0], b0), min(k1[0], b1)), jbase), a0 = f4_key(min(k0[0], b0), jbase);
+    const int qi = wq0 + 8 * ((lane & 15) >> 2) + 4 * half + (lane & 3);
+    if ((lane & 16) == 0 && qi < nq) {
+        if (part)
+            part[((long long)pi * cap + qi) * gridDim.z + blockIdx.z] = make_uint2(a0, a1);
+        else
+            reinterpret_cast<int4*>(P.out)[qi] = knn_row(a0, a1);
+    }
+}
+
+// The rows of a launch whose train sets were cut into nseg segments: per
+// query the two smallest of the segments' keys, which are the keys of the
+// whole train set (a key holds its train index, so keys are distinct and the
+// order of the segments does not matter).  16 lanes per query.
+__global__ __launch_bounds__(256) void k_knn2_merge(const MatchPair* pairs, MatchPair one, const uint2* part, int cap,
+                                                    int nseg) {
+    const int pi = blockIdx.y;
+    const MatchPair P = pairs ? pairs[pi] : one;
+    const int nq = P.nq_dev ? min(*P.nq_dev, P.nq) : P.nq;
+    const int qi = blockIdx.x * 16 + (threadIdx.x >> 4), sl = threadIdx.x & 15;
+    uint32_t k0 = kSentinel, k1 = kSentinel;
+    if (qi < nq) {
+        const uint2* p = part + ((long long)pi * cap + qi) * nseg;
+        for (int z = sl; z < nseg; z += 16) {
+            const uint2 k = p[z];
+            top2_insert2(k0, k1, k.x, k.y);
         }
     }
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) {
+        const uint32_t b0 = (uint32_t)__shfl_xor((int)k0, o, 64), b1 = (uint32_t)__shfl_xor((int)k1, o, 64);
+        k1 = min(max(k0, b0), min(k1, b1));
+        k0 = min(k0, b0);
+    }
+    if (qi < nq && sl == 0) reinterpret_cast<int4*>(P.out)[qi] = knn_row(k0, k1);
 }
 
 // Dispatch order of the pairs for the top-2 kernels: a workgroup's work is
@@ -650,42 +709,82 @@ __global__ __launch_bounds__(256) void k_pair_order(const MatchPair* pairs, int 
 }
 
 // Variants of the same exact computation; the autotuner picks one per
-// workload (kKnnVariants of them).
+// workload (kKnnVariants of them).  Variant 0 is the choice without tuning:
+// F4, the fastest or within 1 us of it at every size measured (us, best
+// popcount form / F4: 100 x 100 3.8 / 4.5, 500 x 500 9.7 / 7.5, 2000 x 2000
+// 31 / 7.7, 4000 x 100 4.1 / 5.0, 100 x 48000 672 / 15.6, 4000 x 48000
+// 679 / 57).
 constexpr int kKnnVariants = 12;
 inline const char* knn_variant_name(int v) {
-    static const char* names[kKnnVariants] = {"S<1,2>", "S<1,4>", "S<2,2>", "S<2,4>", "L",   "S<2,8>",
-                                              "S<1,8>", "S<4,2>", "M<1>",  "M<2>",  "F4",    "F4s5"};
+    static const char* names[kKnnVariants] = {"rule",   "S<1,4>", "S<2,2>", "S<2,4>", "L",   "S<2,8>",
+                                              "S<1,8>", "S<4,2>", "M<1>",   "M<2>",   "F4",  "F4s5"};
     return (v >= 0 && v < kKnnVariants) ? names[v] : "?";
 }
 
-// max_nt: the largest train count of the pairs (the fp4 variant keys train
-// indices in 16 bits and hands larger sets to M<1>); order: the output of
-// k_pair_order (2 npairs + 1 ints), or null (used by the fp4 variant)
-inline void launch_knn2(int variant, const MatchPair* pairs, int npairs, int max_nq, hipStream_t s, int max_nt = -1,
-                        const int* order = nullptr) {
-    if (max_nt < 0) max_nt = max_nq;
-    if ((variant == 10 || variant == 11) && max_nt >= 65536) variant = 8;
+// Segments the fp4 variants cut the train sets into.  One workgroup per
+// 128-query tile leaves most of the 256 CUs idle below a few thousand
+// queries (4000 queries are 32 workgroups: 250 us for 48000 trains), so the
+// trains are cut until about three workgroups per CU are launched, down to
+// one 128-train super-tile each (2000 x 2000, us: 7.7 with one super-tile per
+// segment, 9.2 with two; 4000 x 48000: 79, 61, 57, 55 for 256, 512, 768, 1024
+// workgroups; 100 x 48000: 14.1, 15.6, 15.6, 15.7).  The rig's batches have
+// enough tiles of their own and are not cut.
+inline int knn_segments(int npairs, int max_nq, int max_nt) {
+    const long long tiles = (long long)((max_nq + 127) / 128) * npairs;
+    const int nsuper = (max_nt + 127) / 128;
+    long long seg = std::min<long long>(768 / std::max<long long>(tiles, 1), nsuper);
+    seg = std::max<long long>(seg, (nsuper + 511) / 512);  // 16-bit train indices
+    return (int)std::max<long long>(seg, 1);
+}
+
+// bytes of segment keys a launch_knn2 of these sizes needs (0: none)
+inline size_t knn_part_bytes(int variant, int npairs, int max_nq, int max_nt) {
+    if (variant != 0 && variant != 10 && variant != 11) return 0;
+    const int seg = knn_segments(npairs, max_nq, max_nt);
+    return seg > 1 ? (size_t)seg * npairs * max_nq * sizeof(uint2) : 0;
+}
+
+// One top-2 launch over npairs pairs of at most max_nq queries and max_nt
+// trains.  pairs: device table, or null with npairs == 1: `one`; order: the
+// output of k_pair_order (2 npairs + 1 ints) or null, used by the fp4
+// variants; part: knn_part_bytes() bytes of workspace.
+struct KnnLaunch {
+    const MatchPair* pairs = nullptr;
+    MatchPair one{};
+    int npairs = 1, max_nq = 0, max_nt = 0;
+    const int* order = nullptr;
+    uint2* part = nullptr;
+};
+
+inline void launch_knn2(int variant, const KnnLaunch& K, hipStream_t s) {
+    const int np = K.npairs, nq = K.max_nq;
+    auto grid = [&](int per) { return dim3((nq + per - 1) / per, np); };
+    if (variant == 0) variant = 10;
     switch (variant) {
     case 10:
     case 11: {
+        const int seg = knn_segments(np, nq, K.max_nt);
+        const int tiles = (nq + 127) / 128;
         // with an order, a 1-D grid of the real tiles first
-        const dim3 grid = order ? dim3((max_nq + 127) / 128 * npairs) : dim3((max_nq + 127) / 128, npairs);
+        const dim3 g = K.order ? dim3(tiles * np, 1, seg) : dim3(tiles, np, seg);
+        uint2* part = seg > 1 ? K.part : nullptr;
         if (variant == 10)
-            hipLaunchKernelGGL((k_knn2_f4<true, 4>), grid, dim3(256), 0, s, pairs, order, npairs);
+            hipLaunchKernelGGL((k_knn2_f4<true, 4>), g, dim3(256), 0, s, K.pairs, K.one, K.order, np, part, nq);
         else
-            hipLaunchKernelGGL((k_knn2_f4<false, 5>), grid, dim3(256), 0, s, pairs, order, npairs);
+            hipLaunchKernelGGL((k_knn2_f4<false, 5>), g, dim3(256), 0, s, K.pairs, K.one, K.order, np, part, nq);
+        if (seg > 1)
+            hipLaunchKernelGGL(k_knn2_merge, grid(16), dim3(256), 0, s, K.pairs, K.one, part, nq, seg);
         break;
     }
-    case 1: hipLaunchKernelGGL((k_knn2_s<1, 4>), dim3((max_nq + 63) / 64, npairs), dim3(256), 0, s, pairs); break;
-    case 2: hipLaunchKernelGGL((k_knn2_s<2, 2>), dim3((max_nq + 127) / 128, npairs), dim3(256), 0, s, pairs); break;
-    case 3: hipLaunchKernelGGL((k_knn2_s<2, 4>), dim3((max_nq + 127) / 128, npairs), dim3(256), 0, s, pairs); break;
-    case 4: hipLaunchKernelGGL(k_knn2_lds, dim3((max_nq + kKnnQ - 1) / kKnnQ, npairs), dim3(256), 0, s, pairs); break;
-    case 5: hipLaunchKernelGGL((k_knn2_s<2, 8>), dim3((max_nq + 127) / 128, npairs), dim3(256), 0, s, pairs); break;
-    case 6: hipLaunchKernelGGL((k_knn2_s<1, 8>), dim3((max_nq + 63) / 64, npairs), dim3(256), 0, s, pairs); break;
-    case 7: hipLaunchKernelGGL((k_knn2_s<4, 2>), dim3((max_nq + 255) / 256, npairs), dim3(256), 0, s, pairs); break;
-    case 8: hipLaunchKernelGGL((k_knn2_m<1>), dim3((max_nq + 127) / 128, npairs), dim3(256), 0, s, pairs); break;
-    case 9: hipLaunchKernelGGL((k_knn2_m<2>), dim3((max_nq + 255) / 256, npairs), dim3(256), 0, s, pairs); break;
-    default: hipLaunchKernelGGL((k_knn2_s<1, 2>), dim3((max_nq + 63) / 64, npairs), dim3(256), 0, s, pairs); break;
+    case 1: hipLaunchKernelGGL((k_knn2_s<1, 4>), grid(64), dim3(256), 0, s, K.pairs, K.one); break;
+    case 2: hipLaunchKernelGGL((k_knn2_s<2, 2>), grid(128), dim3(256), 0, s, K.pairs, K.one); break;
+    case 3: hipLaunchKernelGGL((k_knn2_s<2, 4>), grid(128), dim3(256), 0, s, K.pairs, K.one); break;
+    case 4: hipLaunchKernelGGL(k_knn2_lds, grid(kKnnQ), dim3(256), 0, s, K.pairs, K.one); break;
+    case 5: hipLaunchKernelGGL((k_knn2_s<2, 8>), grid(128), dim3(256), 0, s, K.pairs, K.one); break;
+    case 6: hipLaunchKernelGGL((k_knn2_s<1, 8>), grid(64), dim3(256), 0, s, K.pairs, K.one); break;
+    case 7: hipLaunchKernelGGL((k_knn2_s<4, 2>), grid(256), dim3(256), 0, s, K.pairs, K.one); break;
+    case 8: hipLaunchKernelGGL((k_knn2_m<1>), grid(128), dim3(256), 0, s, K.pairs, K.one); break;
+    default: hipLaunchKernelGGL((k_knn2_m<2>), grid(256), dim3(256), 0, s, K.pairs, K.one); break;
     }
 }
 

@@ -55,6 +55,21 @@ def test_knn2_fp4_variant_large_train_sets(gpu_ctx):
     assert (want[: nq // 2, 0] == np.arange(69000, 69000 + nq // 2)).all()
 
 
+@pytest.mark.parametrize("nq,nt", [(1, 127), (128, 128), (129, 129), (33, 5 * 128 + 1), (200, 97 * 128),
+                                   (2, 769 * 128 + 3), (131073, 130)])
+def test_knn2_train_segments(gpu_ctx, nq, nt):
+    """The default launch cuts the trains into segments of 128-row tiles (as
+    many as there are tiles, fewer, more than 512 tiles in all) and more than
+    131072 queries into several launches; duplicated trains in different
+    segments keep the scan order."""
+    rng = np.random.default_rng(nq + nt)
+    q, t = _desc(rng, nq), _desc(rng, nt)
+    t[nt - nt // 3:] = t[: nt // 3]
+    m = min(nq, nt) // 2
+    q[:m] = t[nt - m:]
+    np.testing.assert_array_equal(Matcher.KnnMatch(q, t, ctx=gpu_ctx).rows, oracle.knn2(q, t))
+
+
 def test_knn2_ties_keep_scan_order(gpu_ctx):
     """Duplicated trains: the first occurrence wins (strict '<' in order)."""
     rng = np.random.default_rng(3)
