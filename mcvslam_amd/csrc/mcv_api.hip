@@ -24,6 +24,7 @@
 #include <unistd.h>
 
 #include "../../include/mcvslam_gpu.h"
+#include "mcv_device.hpp"
 #include "mcv_ba.hip"
 #include "mcv_bow.hip"
 #include "mcv_match.hip"
@@ -1000,9 +1001,10 @@ struct mcv_ba {
     bool schur_ready = false, schur_done = false;
     int npf = 0, Fp = 0, nblk = 0;
     bool free_points_with_edges = true;
-    DevBuf pe_ptr, pe, pf_ptr, pf_obs_ptr, pf_obs, pf_point, pf_frame, sfptr, sfobs, fpf_ptr, fpf, blk_ptr, blk_items,
+    int nechunk = 0, esub = 1, nichunk = 0;
+    DevBuf pe_ptr, pe, pf_ptr, pf_obs_ptr, pf_obs, pf_frame, pf_row, echunk, eptr, elist, ichunk, blk_chunk, blk_items,
         blk_ij;
-    DevBuf Dinv, bl, db, Hll, Hpl, Hpp, bs, bp, Sout;
+    DevBuf prec, hd, Z, epart, ipart, Hpp, bs, bp, Sout;
 };
 
 // Launch shapes of k_ba_linearize (same arithmetic per observation; the
@@ -2970,25 +2972,36 @@ static void ba_build_schur(mcv_ba* b, hipStream_t s) {
         pf_ptr[p + 1] = (int)pf_point.size();
     }
     const int npf = (int)pf_point.size();
-    // free frame -> active edges, free frame -> pf entries
-    std::vector<int> sfptr(Fp + 1, 0), fpf_ptr(Fp + 1, 0);
-    for (int i = 0; i < M; i++)
-        if (act_m(i) && fidx[b->h_fr[i]] >= 0) sfptr[fidx[b->h_fr[i]] + 1]++;
-    for (int j = 0; j < Ms; j++)
-        if (act_s(j) && fidx[b->h_sfr[j]] >= 0) sfptr[fidx[b->h_sfr[j]] + 1]++;
+    // rows of the pf entries: by free frame, then by point
+    std::vector<int> fpf_ptr(Fp + 1, 0), pf_row(std::max(npf, 1));
     for (int q = 0; q < npf; q++) fpf_ptr[pf_free[q] + 1]++;
-    for (int f = 0; f < Fp; f++) {
-        sfptr[f + 1] += sfptr[f];
-        fpf_ptr[f + 1] += fpf_ptr[f];
-    }
-    std::vector<int> sfobs(std::max(sfptr[Fp], 1)), fpf(std::max(npf, 1));
+    for (int f = 0; f < Fp; f++) fpf_ptr[f + 1] += fpf_ptr[f];
     {
-        std::vector<int> a(sfptr.begin(), sfptr.end() - 1), c(fpf_ptr.begin(), fpf_ptr.end() - 1);
-        for (int i = 0; i < M; i++)
-            if (act_m(i) && fidx[b->h_fr[i]] >= 0) sfobs[a[fidx[b->h_fr[i]]]++] = i;
-        for (int j = 0; j < Ms; j++)
-            if (act_s(j) && fidx[b->h_sfr[j]] >= 0) sfobs[a[fidx[b->h_sfr[j]]]++] = M + j;
-        for (int q = 0; q < npf; q++) fpf[c[pf_free[q]]++] = q;
+        std::vector<int> c(fpf_ptr.begin(), fpf_ptr.end() - 1);
+        for (int q = 0; q < npf; q++) pf_row[q] = c[pf_free[q]]++;
+    }
+    // chunks of kEdgeChunk consecutive edges, each with the local numbers of
+    // its active edges of free frames, sorted by frame
+    std::vector<EdgeChunk> echunk;
+    std::vector<uint16_t> eptr, elist;
+    for (int st = 0; st < 2; st++) {
+        const int n = st ? Ms : M;
+        const int* fr = st ? b->h_sfr.data() : b->h_fr.data();
+        std::vector<int> cnt(Fp + 1);
+        for (int e0 = 0; e0 < n && Fp > 0; e0 += kEdgeChunk) {
+            const int m = std::min(kEdgeChunk, n - e0);
+            std::fill(cnt.begin(), cnt.end(), 0);
+            auto use = [&](int k) { return (st ? act_s(e0 + k) : act_m(e0 + k)) && fidx[fr[e0 + k]] >= 0; };
+            for (int k = 0; k < m; k++)
+                if (use(k)) cnt[fidx[fr[e0 + k]] + 1]++;
+            for (int f = 0; f < Fp; f++) cnt[f + 1] += cnt[f];
+            const size_t l0 = elist.size();
+            echunk.push_back(EdgeChunk{e0, m, (int)l0, st});
+            for (int f = 0; f <= Fp; f++) eptr.push_back((uint16_t)cnt[f]);
+            elist.resize(l0 + cnt[Fp]);
+            for (int k = 0; k < m; k++)
+                if (use(k)) elist[l0 + cnt[fidx[fr[e0 + k]]]++] = (uint16_t)k;
+        }
     }
     // pair blocks, upper triangle row-major
     const int nblk = Fp * (Fp + 1) / 2;
@@ -2999,34 +3012,60 @@ static void ba_build_schur(mcv_ba* b, hipStream_t s) {
             for (int qb = qa; qb < pf_ptr[p + 1]; qb++) blk_ptr[bidx(pf_free[qa], pf_free[qb]) + 1]++;
     for (int k = 0; k < nblk; k++) blk_ptr[k + 1] += blk_ptr[k];
     std::vector<int2> items(std::max(blk_ptr[nblk], 1)), ij(std::max(nblk, 1));
+    std::vector<int> item_point(std::max(blk_ptr[nblk], 1));
     {
         std::vector<int> a(blk_ptr.begin(), blk_ptr.end() - 1);
         for (int p = 0; p < P; p++)
             for (int qa = pf_ptr[p]; qa < pf_ptr[p + 1]; qa++)
-                for (int qb = qa; qb < pf_ptr[p + 1]; qb++)
-                    items[a[bidx(pf_free[qa], pf_free[qb])]++] = make_int2(qa, qb);
+                for (int qb = qa; qb < pf_ptr[p + 1]; qb++) {
+                    const int t = a[bidx(pf_free[qa], pf_free[qb])]++;
+                    items[t] = make_int2(pf_row[qa], pf_row[qb]);
+                    item_point[t] = p;
+                }
         for (int i = 0; i < Fp; i++)
             for (int j = i; j < Fp; j++) ij[bidx(i, j)] = make_int2(i, j);
     }
+    // Chunks of a block's items, one wave each: at most csz items (about
+    // 16384 waves) and, from 128 items on, at most 1/32 of the points,
+    // launched in the order of their first point (see k_schur_items).
+    const int csz = std::min(2048, std::max(256, (blk_ptr[nblk] / 16384 + 63) / 64 * 64)), span = std::max(P / 32, 1);
+    std::vector<int> blk_chunk(nblk + 1, 0);
+    std::vector<ItemChunk> ichunk;
+    for (int k = 0; k < nblk; k++) {
+        for (int i0 = blk_ptr[k], i1; i0 < blk_ptr[k + 1]; i0 = i1) {
+            const int p0 = item_point[i0], end = std::min(i0 + csz, blk_ptr[k + 1]);
+            i1 = std::min(i0 + 128, end);
+            while (i1 < end && item_point[i1] - p0 < span) i1++;
+            ichunk.push_back(ItemChunk{i0, i1, (int)ichunk.size(), ij[k].x == ij[k].y ? 1 : 0});
+        }
+        blk_chunk[k + 1] = (int)ichunk.size();
+    }
+    std::stable_sort(ichunk.begin(), ichunk.end(),
+                     [&](const ItemChunk& x, const ItemChunk& y) { return item_point[x.i0] < item_point[y.i0]; });
     upload(b->pe_ptr, pe_ptr, s);
     upload(b->pe, pe, s);
     upload(b->pf_ptr, pf_ptr, s);
     upload(b->pf_obs_ptr, pf_obs_ptr, s);
     upload(b->pf_obs, pf_obs, s);
-    upload(b->pf_point, pf_point, s);
     upload(b->pf_frame, pf_free, s);
-    upload(b->sfptr, sfptr, s);
-    upload(b->sfobs, sfobs, s);
-    upload(b->fpf_ptr, fpf_ptr, s);
-    upload(b->fpf, fpf, s);
-    upload(b->blk_ptr, blk_ptr, s);
+    upload(b->pf_row, pf_row, s);
+    upload(b->echunk, echunk, s);
+    upload(b->eptr, eptr, s);
+    upload(b->elist, elist, s);
+    upload(b->ichunk, ichunk, s);
+    upload(b->blk_chunk, blk_chunk, s);
     upload(b->blk_items, items, s);
     upload(b->blk_ij, ij, s);
-    b->Dinv.ensure((size_t)P * 36);
-    b->bl.ensure((size_t)P * 12);
-    b->db.ensure((size_t)P * 12);
-    b->Hll.ensure((size_t)P * 36);
-    b->Hpl.ensure((size_t)std::max(npf, 1) * 72);
+    b->nechunk = (int)echunk.size();
+    b->nichunk = (int)ichunk.size();
+    // threads that share a frame sum in k_schur_edges: its 512 threads cover
+    // the 27 Fp sums once
+    b->esub = Fp > 0 ? std::max(1, 512 / (kFrameSums * Fp)) : 1;
+    b->prec.ensure((size_t)P * kPointRec * 4);
+    b->hd.ensure((size_t)P * 12);
+    b->Z.ensure((size_t)std::max(npf, 1) * kZRow * 4);
+    b->epart.ensure((size_t)std::max(b->nechunk * b->esub, 1) * kFrameSums * std::max(Fp, 1) * 4);
+    b->ipart.ensure((size_t)std::max(b->nichunk, 1) * kItemSums * 4);
     b->Hpp.ensure((size_t)std::max(Fp, 1) * 144);
     b->bs.ensure((size_t)std::max(Fp, 1) * 24);
     b->bp.ensure((size_t)std::max(Fp, 1) * 24);
@@ -3053,24 +3092,27 @@ static SchurArgs ba_schur_args(mcv_ba* b, float lambda) {
     a.pf_ptr = b->pf_ptr.as<int>();
     a.pf_obs_ptr = b->pf_obs_ptr.as<int>();
     a.pf_obs = b->pf_obs.as<int>();
-    a.pf_point = b->pf_point.as<int>();
     a.pf_frame = b->pf_frame.as<int>();
-    a.fptr = b->sfptr.as<int>();
-    a.fobs = b->sfobs.as<int>();
-    a.fpf_ptr = b->fpf_ptr.as<int>();
-    a.fpf = b->fpf.as<int>();
-    a.blk_ptr = b->blk_ptr.as<int>();
-    a.blk_items = b->blk_items.as<int2>();
+    a.pf_row = b->pf_row.as<int>();
+    a.echunk = b->echunk.as<EdgeChunk>();
+    a.eptr = b->eptr.as<uint16_t>();
+    a.elist = b->elist.as<uint16_t>();
+    a.ichunk = b->ichunk.as<ItemChunk>();
+    a.blk_chunk = b->blk_chunk.as<int>();
+    a.items = b->blk_items.as<int2>();
     a.blk_ij = b->blk_ij.as<int2>();
     a.P = b->P;
     a.Fp = b->Fp;
     a.nblk = b->nblk;
+    a.nechunk = b->nechunk;
+    a.esub = b->esub;
+    a.nichunk = b->nichunk;
     a.lambda = lambda;
-    a.Dinv = b->Dinv.as<float>();
-    a.bl = b->bl.as<float>();
-    a.db = b->db.as<float>();
-    a.Hll = b->Hll.as<float>();
-    a.Hpl = b->Hpl.as<float>();
+    a.prec = b->prec.as<float>();
+    a.hd = b->hd.as<float>();
+    a.Z = b->Z.as<float>();
+    a.epart = b->epart.as<float>();
+    a.ipart = b->ipart.as<float>();
     a.Hpp = b->Hpp.as<float>();
     a.bs = b->bs.as<float>();
     a.bp = b->bp.as<float>();
@@ -3078,14 +3120,18 @@ static SchurArgs ba_schur_args(mcv_ba* b, float lambda) {
     return a;
 }
 
-// the Schur launches (structure ready); with blocks = false only H_ll, H_pl,
-// H_pp, b_p (what the largest-diagonal search needs)
+// the Schur launches (structure ready); with blocks = false only the points'
+// and the frames' sums (what the largest-diagonal search needs)
 static void ba_enqueue_schur(mcv_ba* b, float lambda, hipStream_t s, bool blocks = true) {
     const SchurArgs a = ba_schur_args(b, lambda);
-    hipLaunchKernelGGL(k_schur_points, dim3((b->P + 255) / 256), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_schur_points, dim3(xcd_grid((b->P + 31) / 32)), dim3(256), 0, s, a);
     if (b->Fp > 0) {
-        hipLaunchKernelGGL(k_schur_frames, dim3(b->Fp), dim3(256), 0, s, a);
-        if (blocks) hipLaunchKernelGGL(k_schur_blocks, dim3(b->nblk), dim3(256), 0, s, a);
+        if (b->nechunk > 0) hipLaunchKernelGGL(k_schur_edges, dim3(b->nechunk), dim3(512), 0, s, a);
+        hipLaunchKernelGGL(k_schur_edge_sums, dim3((kFrameSums * b->Fp + 15) / 16), dim3(1024), 0, s, a);
+        if (blocks) {
+            if (b->nichunk > 0) hipLaunchKernelGGL(k_schur_items, dim3(xcd_grid((b->nichunk + 3) / 4)), dim3(256), 0, s, a);
+            hipLaunchKernelGGL(k_schur_assemble, dim3(b->nblk), dim3(8 * kItemSums), 0, s, a);
+        }
     }
     HIP_OK(hipGetLastError());
 }
@@ -3317,7 +3363,7 @@ static void ba_enqueue_rho(mcv_ba* b, hipStream_t s, int slot) {
     const int Ms = b->have_stereo ? b->Ms : 0;
     const int n = b->M + Ms;
     const int blocks = std::max((n + 255) / 256, 1);
-    b->partial.ensure((size_t)std::max(blocks, (b->P + 255) / 256 + 1) * 8);
+    b->partial.ensure((size_t)std::max(blocks, (b->P + 31) / 32 + 1) * 8);
     b->dsum.ensure(64);
     hipLaunchKernelGGL(k_ba_rho_sum, dim3(blocks), dim3(256), 0, s, b->planes.as<float>() + 2 * (size_t)b->M,
                        b->pair.as<uint32_t>(), b->pairs.as<BAPair>(),
@@ -3387,7 +3433,7 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
             const int mblocks = std::max(1, std::min(1024, (3 * std::max(P, 2 * Fp) + 255) / 256));
             b->partial.ensure((size_t)mblocks * 8);
             hipLaunchKernelGGL(k_ba_max_diag, dim3(mblocks), dim3(256), 0, s, b->Hpp.as<float>(), Fp,
-                               b->Hll.as<float>(), b->pe_ptr.as<int>(), P, reinterpret_cast<float*>(b->partial.p));
+                               b->hd.as<float>(), b->pe_ptr.as<int>(), P, reinterpret_cast<float*>(b->partial.p));
             hipLaunchKernelGGL(k_max_partials, dim3(1), dim3(256), 0, s, reinterpret_cast<const float*>(b->partial.p),
                                mblocks, b->fmax.as<float>());
             HIP_OK(hipGetLastError());
@@ -3422,9 +3468,10 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
                 }
                 if (n) HIP_OK(hipMemcpyAsync(b->xp.p, xpf.data(), (size_t)n * 4, hipMemcpyHostToDevice, s));
                 const SchurArgs a = ba_schur_args(b, (float)lambda);
-                hipLaunchKernelGGL(k_schur_backsub, dim3(std::max(pblocks, 1)), dim3(256), 0, s, a, b->xp.as<float>(),
+                const int bblocks = (P + 31) / 32;
+                hipLaunchKernelGGL(k_schur_backsub, dim3(bblocks), dim3(256), 0, s, a, b->xp.as<float>(),
                                    b->xl.as<float>(), b->partial.as<double>());
-                hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, s, b->partial.as<double>(), pblocks,
+                hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, s, b->partial.as<double>(), bblocks,
                                    b->dsum.as<double>() + 1);
                 // update: points on the device, frames on the host
                 hipLaunchKernelGGL(k_ba_points_apply, dim3(std::max(pblocks, 1)), dim3(256), 0, s,

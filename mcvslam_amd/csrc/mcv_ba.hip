@@ -445,15 +445,41 @@ namespace mcv {
 // k_ba_stereo_linearize planes) edges; edge index i < M is mono edge i,
 // i >= M stereo edge i - M.  Fixed points have no edge lists (their edges
 // still enter H_pp and b_p through the frame lists); fixed frames have no
-// pose block.
-//   S1  per point: H_ll = sum W J_x^T J_x, b_l = -sum W J_x^T e,
-//       D^-1 = (H_ll + lambda I)^-1, db = D^-1 b_l, and per (point, free
-//       frame) H_pl = sum W J_p^T J_x (6x3); W = Huber weight * inv sigma^2
-//   S3  per free frame: H_pp = sum W J_p^T J_p, b_p = -sum W J_p^T e,
-//       b_schur = b_p - sum H_pl db
-//   S2  per free-frame pair block (i <= j): S_ij = [i == j](H_pp + lambda I)
-//       - sum over shared points H_pl,i D^-1 H_pl,j^T
-//   back-substitution: x_l = D^-1 (b_l - sum H_pl^T x_p)
+// pose block.  W = Huber weight * inv sigma^2.
+//   k_schur_points  per point: H_ll = sum W J_x^T J_x, b_l = -sum W J_x^T e,
+//       the Cholesky factor C of D = H_ll + lambda I and y = C^-1 b_l; per
+//       (point, free frame) entry H_pl = sum W J_p^T J_x (6x3), kept as
+//       Z = H_pl C^-T, so that H_pl,i D^-1 H_pl,j^T = Z_i Z_j^T and
+//       H_pl D^-1 b_l = Z y
+//   k_schur_edges, k_schur_edge_sums  per free frame: H_pp = sum W J_p^T J_p,
+//       b_p = -sum W J_p^T e
+//   k_schur_items, k_schur_assemble  per free-frame pair block (i <= j):
+//       S_ij = [i == j](H_pp + lambda I) - sum over shared points Z_i Z_j^T,
+//       b_schur = b_p - sum Z y
+//   k_schur_backsub  x_l = C^-T (y - sum Z^T x_p)
+// What bounds them: the planes (88 B per mono edge) and the entry rows (96 B)
+// from memory; every plane is read in edge order, so that a wave's loads are
+// whole lines.  50 keyframes, 200k points, 1.5M edges, 1.2M entries, 5.4M
+// items: points 131, edges 47 + 9, items 139, assembly 6 us (one thread per
+// point, one workgroup per frame and per pair block: 391, 675 and 806 us).
+constexpr int kZRow = 24;          // floats per entry row: Z (6x3 row-major), Z y (6)
+constexpr int kPointRec = 12;      // floats per point: c10 c20 c21, 1/c00 1/c11 1/c22, y, b_l
+constexpr int kEdgeChunk = 512;    // edges per workgroup of k_schur_edges
+constexpr int kItemSums = 40;      // sums of an item chunk (36, or 27 on the diagonal)
+constexpr int kFrameSums = 27;     // per frame: H_pp upper triangle by rows, each row followed by b_p's entry
+
+struct EdgeChunk {
+    int e0, n;     // edges [e0, e0 + n) of the mono (or, stereo != 0, stereo) planes
+    int list0;     // first entry of its frame-sorted list of local edge numbers
+    int stereo;
+};
+
+struct ItemChunk {
+    int i0, i1;  // items [i0, i1) of one frame-pair block
+    int out;     // row of ipart: the chunks of a block in order, blocks in order
+    int diag;
+};
+
 struct SchurArgs {
     const float* planes;    // mono planes (22 of stride S)
     long long S;
@@ -467,22 +493,22 @@ struct SchurArgs {
     const int* pf_ptr;      // per point: first pf entry (P + 1)
     const int* pf_obs_ptr;  // per pf entry: range in pf_obs (npf + 1)
     const int* pf_obs;      // edge indices grouped by pf
-    const int* pf_point;    // point of each pf entry
     const int* pf_frame;    // free frame of each pf entry
-    const int* fptr;        // free frame -> active edges (Fp + 1)
-    const int* fobs;
-    const int* fpf_ptr;     // free frame -> pf entries (Fp + 1)
-    const int* fpf;
-    const int* blk_ptr;     // block (i <= j, row-major upper) -> item range
-    const int2* blk_items;  // (pf_i, pf_j)
+    const int* pf_row;      // row of each pf entry: rows are ordered by (frame, point)
+    const EdgeChunk* echunk;
+    const uint16_t* eptr;   // per chunk, Fp + 1: the frames' ranges in its list
+    const uint16_t* elist;
+    const ItemChunk* ichunk;
+    const int* blk_chunk;   // per block: its first item chunk (nblk + 1)
+    const int2* items;      // (row_i, row_j), by block, then by point
     const int2* blk_ij;     // block -> (i, j)
-    int P, Fp, nblk;
+    int P, Fp, nblk, nechunk, esub, nichunk;
     float lambda;
-    float* Dinv;            // P x 9
-    float* bl;              // P x 3
-    float* db;              // P x 3
-    float* Hll;             // P x 9 (without lambda)
-    float* Hpl;             // npf x 18 (6x3 row-major)
+    float* prec;            // P x kPointRec
+    float* hd;              // P x 3: diagonal of H_ll
+    float* Z;               // npf x kZRow
+    float* epart;           // (nechunk * esub) x (kFrameSums * Fp)
+    float* ipart;           // nichunk x kItemSums
     float* Hpp;             // Fp x 36 (without lambda)
     float* bs;              // Fp x 6 (b_schur)
     float* bp;              // Fp x 6 (b_p)
@@ -507,160 +533,382 @@ __device__ __forceinline__ EdgeRef edge_ref(const SchurArgs& a, int i) {
     return EdgeRef{a.splanes + j, a.SS, 3, 5, 23, a.splanes[4 * a.SS + j] * a.sisig[j]};
 }
 
+template <int R>
+struct RowCount {
+    static constexpr int value = R;
+};
+
+// f(row count, edge) for edge i
+template <typename F>
+__device__ __forceinline__ void with_edge(const SchurArgs& a, int i, F f) {
+    const EdgeRef E = edge_ref(a, i);
+    if (i < a.M) f(RowCount<2>{}, E);
+    else f(RowCount<3>{}, E);
+}
+
+template <int kCtrl>
+__device__ __forceinline__ float dpp_f(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xF, 0xF, false));
+}
+
+// sum over aligned groups of 8 lanes, in every lane of the group
+__device__ __forceinline__ float sum8(float v) {
+    v += dpp_f<0xB1>(v);   // lane ^ 1
+    v += dpp_f<0x4E>(v);   // lane ^ 2
+    v += dpp_f<0x141>(v);  // the other quad of the half row
+    return v;
+}
+
+// 8 lanes per point: they take its edges in turn (a wave's loads of a plane
+// then cover the edges of 8 neighbouring points, a few whole lines, where one
+// thread per point read the same lines once per edge of a point), and after
+// the sums and the factorization its entries in turn.
 __global__ __launch_bounds__(256) void k_schur_points(SchurArgs a) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const int xb = xcd_block((a.P + 31) / 32);
+    if (xb < 0) return;
+    const int p = xb * 32 + (threadIdx.x >> 3), g = threadIdx.x & 7;
+    float h00 = 0.f, h01 = 0.f, h02 = 0.f, h11 = 0.f, h12 = 0.f, h22 = 0.f, b0 = 0.f, b1 = 0.f, b2 = 0.f;
+    int e0 = 0, e1 = 0;
+    if (p < a.P) {
+        e0 = a.pe_ptr[p];
+        e1 = a.pe_ptr[p + 1];
+    }
+    for (int t = e0 + g; t < e1; t += 8)
+        with_edge(a, a.pe[t], [&](auto rows, const EdgeRef& E) {
+            // all of the edge's loads before the sums
+            constexpr int R = decltype(rows)::value;
+            float er[R], x[R], y[R], z[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                er[r] = E.e(r);
+                x[r] = E.Jx(r, 0);
+                y[r] = E.Jx(r, 1);
+                z[r] = E.Jx(r, 2);
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                b0 -= E.W * (x[r] * er[r]);
+                b1 -= E.W * (y[r] * er[r]);
+                b2 -= E.W * (z[r] * er[r]);
+                h00 += E.W * (x[r] * x[r]);
+                h01 += E.W * (x[r] * y[r]);
+                h02 += E.W * (x[r] * z[r]);
+                h11 += E.W * (y[r] * y[r]);
+                h12 += E.W * (y[r] * z[r]);
+                h22 += E.W * (z[r] * z[r]);
+            }
+        });
+    h00 = sum8(h00); h01 = sum8(h01); h02 = sum8(h02);
+    h11 = sum8(h11); h12 = sum8(h12); h22 = sum8(h22);
+    b0 = sum8(b0); b1 = sum8(b1); b2 = sum8(b2);
     if (p >= a.P) return;
-    float H[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, b[3] = {0, 0, 0};
-    const int e0 = a.pe_ptr[p], e1 = a.pe_ptr[p + 1];
-    for (int t = e0; t < e1; t++) {
-        const EdgeRef E = edge_ref(a, a.pe[t]);
-        for (int r = 0; r < E.rows; r++) {
-            const float er = E.e(r);
-            const float A[3] = {E.Jx(r, 0), E.Jx(r, 1), E.Jx(r, 2)};
-#pragma unroll
-            for (int i = 0; i < 3; i++) {
-                b[i] -= E.W * (A[i] * er);
-#pragma unroll
-                for (int c = 0; c < 3; c++) H[3 * i + c] += E.W * (A[i] * A[c]);
-            }
-        }
-    }
-    float Di[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    // D = H_ll + lambda I = C C^T; a pivot of D is at least lambda (H_ll is
+    // positive semidefinite), which also holds it against cancellation
+    float c10 = 0.f, c20 = 0.f, c21 = 0.f, i00 = 0.f, i11 = 0.f, i22 = 0.f;
     if (e1 > e0) {
-        float D[9];
-#pragma unroll
-        for (int k = 0; k < 9; k++) D[k] = H[k];
-        D[0] += a.lambda;
-        D[4] += a.lambda;
-        D[8] += a.lambda;
-        const float c00 = D[4] * D[8] - D[5] * D[7], c01 = D[5] * D[6] - D[3] * D[8], c02 = D[3] * D[7] - D[4] * D[6];
-        const float det = D[0] * c00 + D[1] * c01 + D[2] * c02;
-        const float id = 1.f / det;
-        Di[0] = c00 * id; Di[1] = (D[2] * D[7] - D[1] * D[8]) * id; Di[2] = (D[1] * D[5] - D[2] * D[4]) * id;
-        Di[3] = c01 * id; Di[4] = (D[0] * D[8] - D[2] * D[6]) * id; Di[5] = (D[2] * D[3] - D[0] * D[5]) * id;
-        Di[6] = c02 * id; Di[7] = (D[1] * D[6] - D[0] * D[7]) * id; Di[8] = (D[0] * D[4] - D[1] * D[3]) * id;
+        i00 = 1.f / sqrtf(h00 + a.lambda);
+        c10 = h01 * i00;
+        c20 = h02 * i00;
+        i11 = 1.f / sqrtf(fmaxf(h11 + a.lambda - c10 * c10, a.lambda));
+        c21 = (h12 - c20 * c10) * i11;
+        i22 = 1.f / sqrtf(fmaxf(h22 + a.lambda - c20 * c20 - c21 * c21, a.lambda));
     }
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        a.Hll[9 * p + k] = H[k];
-        a.Dinv[9 * p + k] = Di[k];
+    const float y0 = b0 * i00, y1 = (b1 - c10 * y0) * i11, y2 = (b2 - c20 * y0 - c21 * y1) * i22;
+    if (g == 0) {
+        float4* o = reinterpret_cast<float4*>(a.prec + (long long)kPointRec * p);
+        o[0] = make_float4(c10, c20, c21, i00);
+        o[1] = make_float4(i11, i22, y0, y1);
+        o[2] = make_float4(y2, b0, b1, b2);
+        a.hd[3 * p] = h00;
+        a.hd[3 * p + 1] = h11;
+        a.hd[3 * p + 2] = h22;
     }
+    const int q1 = a.pf_ptr[p + 1];
+    for (int q = a.pf_ptr[p] + g; q < q1; q += 8) {
+        float H[18];
 #pragma unroll
-    for (int r = 0; r < 3; r++) {
-        a.bl[3 * p + r] = b[r];
-        a.db[3 * p + r] = Di[3 * r] * b[0] + Di[3 * r + 1] * b[1] + Di[3 * r + 2] * b[2];
-    }
-    for (int q = a.pf_ptr[p]; q < a.pf_ptr[p + 1]; q++) {
-        float Hq[18];
+        for (int k = 0; k < 18; k++) H[k] = 0.f;
+        for (int t = a.pf_obs_ptr[q]; t < a.pf_obs_ptr[q + 1]; t++)
+            with_edge(a, a.pf_obs[t], [&](auto rows, const EdgeRef& E) {
+                constexpr int R = decltype(rows)::value;
+                float B[R][6], A[R][3];
 #pragma unroll
-        for (int k = 0; k < 18; k++) Hq[k] = 0.f;
-        for (int t = a.pf_obs_ptr[q]; t < a.pf_obs_ptr[q + 1]; t++) {
-            const EdgeRef E = edge_ref(a, a.pf_obs[t]);
-            for (int r = 0; r < E.rows; r++) {
-                float B[6], A[3];
+                for (int r = 0; r < R; r++) {
 #pragma unroll
-                for (int k = 0; k < 6; k++) B[k] = E.Jp(r, k);
+                    for (int k = 0; k < 6; k++) B[r][k] = E.Jp(r, k);
 #pragma unroll
-                for (int k = 0; k < 3; k++) A[k] = E.Jx(r, k);
+                    for (int k = 0; k < 3; k++) A[r][k] = E.Jx(r, k);
+                }
 #pragma unroll
-                for (int i = 0; i < 6; i++)
+                for (int r = 0; r < R; r++)
 #pragma unroll
-                    for (int c = 0; c < 3; c++) Hq[3 * i + c] += E.W * (B[i] * A[c]);
-            }
+                    for (int i = 0; i < 6; i++)
+#pragma unroll
+                        for (int c = 0; c < 3; c++) H[3 * i + c] += E.W * (B[r][i] * A[r][c]);
+            });
+        float zy[6];
+#pragma unroll
+        for (int i = 0; i < 6; i++) {
+            const float z0 = H[3 * i] * i00;
+            const float z1 = (H[3 * i + 1] - z0 * c10) * i11;
+            const float z2 = (H[3 * i + 2] - z0 * c20 - z1 * c21) * i22;
+            H[3 * i] = z0;
+            H[3 * i + 1] = z1;
+            H[3 * i + 2] = z2;
+            zy[i] = z0 * y0 + z1 * y1 + z2 * y2;
         }
-#pragma unroll
-        for (int k = 0; k < 18; k++) a.Hpl[18 * (long long)q + k] = Hq[k];
+        float4* o = reinterpret_cast<float4*>(a.Z + (long long)kZRow * a.pf_row[q]);
+        o[0] = make_float4(H[0], H[1], H[2], H[3]);
+        o[1] = make_float4(H[4], H[5], H[6], H[7]);
+        o[2] = make_float4(H[8], H[9], H[10], H[11]);
+        o[3] = make_float4(H[12], H[13], H[14], H[15]);
+        o[4] = make_float4(H[16], H[17], zy[0], zy[1]);
+        o[5] = make_float4(zy[2], zy[3], zy[4], zy[5]);
     }
 }
 
-// fixed-order tree reduction of 256 x n partial sums (n <= 36); red[0][k]
-// holds the sums
-__device__ __forceinline__ void block_sum(const float* acc, float (*red)[36], int n) {
-    for (int k = 0; k < n; k++) red[threadIdx.x][k] = acc[k];
+// Frame sums of one chunk of edges: the chunk's planes are read in edge order
+// into LDS (per edge W, then per row J_pose and e: an odd number of words, so
+// that different edges start in different banks), then a thread takes one of
+// a frame's 27 sums and walks the frame's edges of the chunk.  With few
+// frames, esub threads share a sum.  (A frame's edges gathered straight from
+// the planes put every 4-byte read in a line of its own.)
+__global__ __launch_bounds__(512) void k_schur_edges(SchurArgs a) {
+    constexpr int kWords = 23;  // 1 + 7 * 3 rows, and one to make it odd
+    __shared__ float s_e[kEdgeChunk * kWords];
+    __shared__ uint16_t s_list[kEdgeChunk];
+    const EdgeChunk C = a.echunk[blockIdx.x];
+    const int rows = C.stereo ? 3 : 2, words = C.stereo ? kWords : 15;
+    const uint16_t* ptr = a.eptr + (long long)blockIdx.x * (a.Fp + 1);
+    const int nl = ptr[a.Fp];
+    for (int i = threadIdx.x; i < nl; i += 512) s_list[i] = a.elist[C.list0 + i];
+    for (int i = threadIdx.x; i < C.n; i += 512) {
+        const EdgeRef E = edge_ref(a, C.stereo ? a.M + C.e0 + i : C.e0 + i);
+        float* o = s_e + i * words;
+        o[0] = E.W;
+        for (int r = 0; r < rows; r++) {
+#pragma unroll
+            for (int k = 0; k < 6; k++) o[1 + 7 * r + k] = E.Jp(r, k);
+            o[7 + 7 * r] = E.e(r);
+        }
+    }
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s)
-            for (int k = 0; k < n; k++) red[threadIdx.x][k] += red[threadIdx.x + s][k];
+    const int cols = kFrameSums * a.Fp;
+    for (int t = threadIdx.x; t < cols * a.esub; t += 512) {
+        const int sub = t / cols, col = t - sub * cols, f = col / kFrameSums;
+        // sum k of a frame is element (i, c) of the rows (i, i .. 6), i = 0..5
+        int i = 0, c = col - kFrameSums * f;
+        while (c >= 7 - i) {
+            c -= 7 - i;
+            i++;
+        }
+        c += i;
+        float acc = 0.f;
+        const int l1 = ptr[f + 1];
+        for (int l = ptr[f] + sub; l < l1; l += a.esub) {
+            const float* e = s_e + (int)s_list[l] * words;
+            const float W = e[0];
+            acc += W * (e[1 + i] * e[1 + c]);
+            acc += W * (e[8 + i] * e[8 + c]);
+            if (rows == 3) acc += W * (e[15 + i] * e[15 + c]);
+        }
+        a.epart[((long long)blockIdx.x * a.esub + sub) * cols + col] = c == 6 ? -acc : acc;
+    }
+}
+
+// H_pp and b_p from the chunks' sums: 16 sums per workgroup, 64 threads to a
+// sum, chunk order fixed
+__global__ __launch_bounds__(1024) void k_schur_edge_sums(SchurArgs a) {
+    __shared__ float red[64][17];
+    const int cols = kFrameSums * a.Fp, rows = a.nechunk * a.esub;
+    const int cl = threadIdx.x & 15, sl = threadIdx.x >> 4;
+    const int col = blockIdx.x * 16 + cl;
+    float acc = 0.f;
+    if (col < cols) {
+        int r = sl;
+        for (; r + 192 < rows; r += 256) {
+            const float v0 = a.epart[(long long)r * cols + col], v1 = a.epart[(long long)(r + 64) * cols + col],
+                        v2 = a.epart[(long long)(r + 128) * cols + col], v3 = a.epart[(long long)(r + 192) * cols + col];
+            acc += v0;
+            acc += v1;
+            acc += v2;
+            acc += v3;
+        }
+        for (; r < rows; r += 64) acc += a.epart[(long long)r * cols + col];
+    }
+    red[sl][cl] = acc;
+    __syncthreads();
+    for (int s = 32; s > 0; s >>= 1) {
+        if (sl < s) red[sl][cl] += red[sl + s][cl];
         __syncthreads();
     }
+    if (sl != 0 || col >= cols) return;
+    const int f = col / kFrameSums;
+    int i = 0, c = col - kFrameSums * f;
+    while (c >= 7 - i) {
+        c -= 7 - i;
+        i++;
+    }
+    c += i;
+    if (c == 6) {
+        a.bp[6 * f + i] = red[0][cl];
+    } else {
+        a.Hpp[36 * f + 6 * i + c] = red[0][cl];
+        a.Hpp[36 * f + 6 * c + i] = red[0][cl];
+    }
 }
 
-__global__ __launch_bounds__(256) void k_schur_frames(SchurArgs a) {
-    __shared__ float red[256][36];
-    const int f = blockIdx.x;
-    float acc[36];
-    float bp[12];  // b_p (0..5) and the Schur coupling sum H_pl db (6..11)
+// halves the sums a lane keeps: [0, N) or, with hi, [N, 2N), with the DPP
+// partner's share of them added
+template <int kCtrl, int N>
+__device__ __forceinline__ void sum_fold(float* v, int hi) {
 #pragma unroll
-    for (int k = 0; k < 36; k++) acc[k] = 0.f;
+    for (int k = 0; k < N; k++) {
+        const float send = hi ? v[k] : v[k + N], keep = hi ? v[k + N] : v[k];
+        v[k] = keep + dpp_f<kCtrl>(send);
+    }
+}
+
+// rows (one per lane, 16-byte pieces [0, Q) of each) into the wave's LDS, at
+// 16 Q bytes a row: consecutive lanes fetch consecutive pieces, so that a row
+// is fetched by one instruction
+typedef float mcv_f4 __attribute__((ext_vector_type(4)));
+
+template <int Q>
+__device__ __forceinline__ void rows_load(const mcv_f4* Z, int row, mcv_f4 (&v)[Q]) {
+    const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int k = 0; k < 12; k++) bp[k] = 0.f;
-    for (int t = a.fptr[f] + threadIdx.x; t < a.fptr[f + 1]; t += 256) {
-        const EdgeRef E = edge_ref(a, a.fobs[t]);
-        for (int r = 0; r < E.rows; r++) {
-            const float er = E.e(r);
-            float B[6];
+    for (int k = 0; k < Q; k++) {
+        const int e = 64 * k + lane, r = e / Q;
+        v[k] = Z[(long long)__shfl(row, r, 64) * (kZRow / 4) + (e - Q * r)];
+    }
+}
+
+template <bool kDiag>
+__device__ __forceinline__ void schur_items(const SchurArgs& a, const ItemChunk& C, mcv_f4* lds) {
+    constexpr int Q = kDiag ? 6 : 5;  // the diagonal also takes Z y
+    const int lane = threadIdx.x & 63;
+    const mcv_f4* Z = reinterpret_cast<const mcv_f4*>(a.Z);
+    // S_ij row-major, or on the diagonal its upper triangle by rows and Z y;
+    // padded to 8 n for the folds
+    constexpr int kN = kDiag ? 4 : 5;
+    float acc[8 * kN];
 #pragma unroll
-            for (int k = 0; k < 6; k++) B[k] = E.Jp(r, k);
+    for (int k = 0; k < 8 * kN; k++) acc[k] = 0.f;
+    int2 it = a.items[min(C.i0 + lane, C.i1 - 1)];
+    for (int t = C.i0; t < C.i1; t += 64) {
+        mcv_f4 vi[Q], vj[Q];
+        rows_load<Q>(Z, it.x, vi);
+        if constexpr (!kDiag) rows_load<Q>(Z, it.y, vj);
+        it = a.items[min(t + 64 + lane, C.i1 - 1)];
+        wave_lds_sync();  // the previous rows are read
 #pragma unroll
-            for (int i = 0; i < 6; i++) {
-                bp[i] -= E.W * (B[i] * er);
+        for (int k = 0; k < Q; k++) {
+            lds[64 * k + lane] = vi[k];
+            if constexpr (!kDiag) lds[64 * (Q + k) + lane] = vj[k];
+        }
+        wave_lds_sync();
+        // a lane past the end holds the last row again, with weight zero
+        const float on = t + lane < C.i1 ? 1.f : 0.f;
+        const float2* li = reinterpret_cast<const float2*>(lds + Q * lane);
+        const float2* lj = reinterpret_cast<const float2*>(lds + 64 * Q + Q * lane);
+        float A[18], B[18];
 #pragma unroll
-                for (int c = 0; c < 6; c++) acc[6 * i + c] += E.W * (B[i] * B[c]);
+        for (int k = 0; k < 18; k += 2) {
+            const float2 v = li[k >> 1];
+            A[k] = v.x * on;
+            A[k + 1] = v.y * on;
+            if constexpr (!kDiag) {
+                const float2 w = lj[k >> 1];
+                B[k] = w.x;
+                B[k + 1] = w.y;
             }
         }
-    }
-    for (int t = a.fpf_ptr[f] + threadIdx.x; t < a.fpf_ptr[f + 1]; t += 256) {
-        const int q = a.fpf[t];
-        const int p = a.pf_point[q];
-        const float* Hq = a.Hpl + 18 * (long long)q;
-        const float d0 = a.db[3 * p], d1 = a.db[3 * p + 1], d2 = a.db[3 * p + 2];
+        if constexpr (kDiag) {
 #pragma unroll
-        for (int r = 0; r < 6; r++) bp[6 + r] += Hq[3 * r] * d0 + Hq[3 * r + 1] * d1 + Hq[3 * r + 2] * d2;
-    }
-    block_sum(acc, red, 36);
-    if (threadIdx.x < 36) a.Hpp[36 * f + threadIdx.x] = red[0][threadIdx.x];
-    __syncthreads();
-    block_sum(bp, red, 12);
-    if (threadIdx.x < 6) {
-        a.bp[6 * f + threadIdx.x] = red[0][threadIdx.x];
-        a.bs[6 * f + threadIdx.x] = red[0][threadIdx.x] - red[0][6 + threadIdx.x];
-    }
-}
-
-__global__ __launch_bounds__(256) void k_schur_blocks(SchurArgs a) {
-    __shared__ float red[256][36];
-    const int blk = blockIdx.x;
-    const int2 ij = a.blk_ij[blk];
-    float acc[36];
-#pragma unroll
-    for (int k = 0; k < 36; k++) acc[k] = 0.f;
-    for (int t = a.blk_ptr[blk] + threadIdx.x; t < a.blk_ptr[blk + 1]; t += 256) {
-        const int2 it = a.blk_items[t];
-        const int p = a.pf_point[it.x];
-        const float* Hi = a.Hpl + 18 * (long long)it.x;
-        const float* Hj = a.Hpl + 18 * (long long)it.y;
-        const float* Di = a.Dinv + 9 * p;
-        // Y = D^-1 H_j^T (3 x 6)
-        float Y[18];
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-#pragma unroll
-            for (int c = 0; c < 6; c++)
-                Y[6 * r + c] = Di[3 * r] * Hj[3 * c] + Di[3 * r + 1] * Hj[3 * c + 1] + Di[3 * r + 2] * Hj[3 * c + 2];
+            for (int k = 0; k < 6; k += 2) {
+                const float2 v = li[9 + (k >> 1)];
+                acc[21 + k] += v.x * on;
+                acc[22 + k] += v.y * on;
+            }
+        }
+        int o = 0;
 #pragma unroll
         for (int r = 0; r < 6; r++)
 #pragma unroll
-            for (int c = 0; c < 6; c++)
-                acc[6 * r + c] += Hi[3 * r] * Y[c] + Hi[3 * r + 1] * Y[6 + c] + Hi[3 * r + 2] * Y[12 + c];
+            for (int c = kDiag ? r : 0; c < 6; c++, o++) {
+                const float* b = kDiag ? A + 3 * c : B + 3 * c;
+                acc[o] = fmaf(A[3 * r], b[0], fmaf(A[3 * r + 1], b[1], fmaf(A[3 * r + 2], b[2], acc[o])));
+            }
     }
-    block_sum(acc, red, 36);
+    // the 64 lanes' sums: each fold halves the sums a lane keeps, by lane bits
+    // 3, 2 and 1 (a third of the instructions of one butterfly per sum), and
+    // lanes 0, 2, .. 14 end with kN sums each
+    sum_fold<0x140, 4 * kN>(acc, lane & 8);
+    sum_fold<0x141, 2 * kN>(acc, lane & 4);
+    sum_fold<0x1B, kN>(acc, lane & 2);
+#pragma unroll
+    for (int k = 0; k < kN; k++) {
+        float v = acc[k];
+        v += dpp_f<0xB1>(v);
+        v += __shfl_xor(v, 16, 64);
+        v += __shfl_xor(v, 32, 64);
+        acc[k] = v;
+    }
+    if (lane < 16 && (lane & 1) == 0) {
+        float* o = a.ipart + (long long)kItemSums * C.out + (lane & 8 ? 4 * kN : 0) + (lane & 4 ? 2 * kN : 0) +
+                   (lane & 2 ? kN : 0);
+#pragma unroll
+        for (int k = 0; k < kN; k++) o[k] = acc[k];
+    }
+}
+
+// sum of Z_i Z_j^T (and, on the diagonal, Z y) over one chunk of a block's
+// items, one wave per chunk and one item per lane.  Bound by the entry rows
+// from memory (1.1 GB asked for by 5.4M items, 0.11 GB of rows).  The chunks
+// run in the order of their first point, neighbours on one XCD, so that all
+// blocks read the same points' rows while its L2 holds them: 142 us, against
+// 290 us in block order and 806 us with one workgroup per block.
+__global__ __launch_bounds__(256) void k_schur_items(SchurArgs a) {
+    __shared__ mcv_f4 s_rows[4][640];
+    const int xb = xcd_block((a.nichunk + 3) / 4);
+    if (xb < 0) return;
+    const int chunk = xb * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (chunk >= a.nichunk) return;
+    const ItemChunk C = a.ichunk[chunk];
+    mcv_f4* lds = s_rows[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
+    if (C.diag) schur_items<true>(a, C, lds);
+    else schur_items<false>(a, C, lds);
+}
+
+// S and b_schur from the chunks' sums, one workgroup per block: 8 threads to
+// a sum, chunk order fixed
+__global__ __launch_bounds__(8 * kItemSums) void k_schur_assemble(SchurArgs a) {
+    __shared__ float red[8][kItemSums];
+    const int blk = blockIdx.x, t = threadIdx.x % kItemSums, sl = threadIdx.x / kItemSums;
+    const int2 ij = a.blk_ij[blk];
+    const bool diag = ij.x == ij.y;
+    float sum = 0.f;
+    if (t < (diag ? 27 : 36))
+        for (int c = a.blk_chunk[blk] + sl; c < a.blk_chunk[blk + 1]; c += 8) sum += a.ipart[(long long)kItemSums * c + t];
+    red[sl][t] = sum;
+    __syncthreads();
+    if (sl == 0) {
+#pragma unroll
+        for (int k = 1; k < 8; k++) sum += red[k][t];
+        red[0][t] = sum;
+    }
+    __syncthreads();
     if (threadIdx.x < 36) {
-        const int r = threadIdx.x / 6, c = threadIdx.x % 6;
+        const int r = threadIdx.x / 6, c = threadIdx.x % 6, lo = min(r, c), hi = max(r, c);
         const int n = 6 * a.Fp;
-        float v = -red[0][threadIdx.x];
-        if (ij.x == ij.y) v += a.Hpp[36 * ij.x + threadIdx.x] + (r == c ? a.lambda : 0.f);
+        float v = -red[0][diag ? lo * 6 - lo * (lo - 1) / 2 + hi - lo : (int)threadIdx.x];
+        if (diag) v += a.Hpp[36 * ij.x + threadIdx.x] + (r == c ? a.lambda : 0.f);
         a.Sout[(long long)(6 * ij.x + r) * n + 6 * ij.y + c] = v;
-        if (ij.x != ij.y) a.Sout[(long long)(6 * ij.y + c) * n + 6 * ij.x + r] = v;
+        if (!diag) a.Sout[(long long)(6 * ij.y + c) * n + 6 * ij.x + r] = v;
+    } else if (diag && threadIdx.x < 42) {
+        const int r = threadIdx.x - 36;
+        a.bs[6 * ij.x + r] = a.bp[6 * ij.x + r] - red[0][21 + r];
     }
 }
 
@@ -675,29 +923,47 @@ __device__ __forceinline__ double block_sum_d(double v, double* red) {
     return red[0];
 }
 
-// x_l = D^-1 (b_l - sum over the point's pf entries of H_pl^T x_p) per point
-// (0 for points without edges), and per workgroup the partial sum of
-// x_l . (lambda x_l + b_l) (the points' share of the LM scale).
+// x_l = C^-T (y - sum over the point's entries of Z^T x_p) per point (0 for
+// points without edges), 8 lanes per point, and per workgroup the partial sum
+// of x_l . (lambda x_l + b_l) (the points' share of the LM scale).
 __global__ __launch_bounds__(256) void k_schur_backsub(SchurArgs a, const float* xp, float* xl, double* partial) {
     __shared__ double red[256];
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const int p = blockIdx.x * 32 + (threadIdx.x >> 3), g = threadIdx.x & 7;
     double sc = 0.0;
+    float s0 = 0.f, s1 = 0.f, s2 = 0.f;
     if (p < a.P) {
-        float c[3] = {a.bl[3 * p], a.bl[3 * p + 1], a.bl[3 * p + 2]};
-        for (int q = a.pf_ptr[p]; q < a.pf_ptr[p + 1]; q++) {
-            const float* Hq = a.Hpl + 18 * (long long)q;
+        const int q1 = a.pf_ptr[p + 1];
+        for (int q = a.pf_ptr[p] + g; q < q1; q += 8) {
+            const float4* z = reinterpret_cast<const float4*>(a.Z + (long long)kZRow * a.pf_row[q]);
             const float* x = xp + 6 * a.pf_frame[q];
+            float A[20];
 #pragma unroll
-            for (int k = 0; k < 3; k++)
-                c[k] -= Hq[k] * x[0] + Hq[3 + k] * x[1] + Hq[6 + k] * x[2] + Hq[9 + k] * x[3] + Hq[12 + k] * x[4] +
-                        Hq[15 + k] * x[5];
+            for (int k = 0; k < 5; k++) {
+                const float4 v = z[k];
+                A[4 * k] = v.x; A[4 * k + 1] = v.y; A[4 * k + 2] = v.z; A[4 * k + 3] = v.w;
+            }
+#pragma unroll
+            for (int k = 0; k < 6; k++) {
+                s0 += A[3 * k] * x[k];
+                s1 += A[3 * k + 1] * x[k];
+                s2 += A[3 * k + 2] * x[k];
+            }
         }
-        const float* Di = a.Dinv + 9 * p;
+    }
+    s0 = sum8(s0);
+    s1 = sum8(s1);
+    s2 = sum8(s2);
+    if (p < a.P && g == 0) {
+        const float4* rec = reinterpret_cast<const float4*>(a.prec + (long long)kPointRec * p);
+        const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
+        const float c10 = r0.x, c20 = r0.y, c21 = r0.z, i00 = r0.w, i11 = r1.x, i22 = r1.y;
+        const float x2 = (r2.x - s2) * i22, x1 = (r1.w - s1 - c21 * x2) * i11,
+                    x0 = (r1.z - s0 - c10 * x1 - c20 * x2) * i00;
+        const float v[3] = {x0, x1, x2}, b[3] = {r2.y, r2.z, r2.w};
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            const float v = Di[3 * k] * c[0] + Di[3 * k + 1] * c[1] + Di[3 * k + 2] * c[2];
-            xl[3 * p + k] = v;
-            sc += (double)v * ((double)a.lambda * (double)v + (double)a.bl[3 * p + k]);
+            xl[3 * p + k] = v[k];
+            sc += (double)v[k] * ((double)a.lambda * (double)v[k] + (double)b[k]);
         }
     }
     const double t = block_sum_d(sc, red);
@@ -741,7 +1007,7 @@ __global__ __launch_bounds__(256) void k_sum_partials(const double* partial, int
 // largest |diagonal entry| of H_pp (free frames) and H_ll (points with
 // edges), computeLambdaInit's maxDiagonal: per-workgroup maxima over a
 // grid-stride loop into partial[blockIdx.x], then k_max_partials
-__global__ __launch_bounds__(256) void k_ba_max_diag(const float* Hpp, int Fp, const float* Hll, const int* pe_ptr,
+__global__ __launch_bounds__(256) void k_ba_max_diag(const float* Hpp, int Fp, const float* hd, const int* pe_ptr,
                                                      int P, float* partial) {
     __shared__ float red[256];
     float m = 0.f;
@@ -750,7 +1016,7 @@ __global__ __launch_bounds__(256) void k_ba_max_diag(const float* Hpp, int Fp, c
         m = fmaxf(m, fabsf(Hpp[36 * (k / 6) + 7 * (k % 6)]));
     for (int k = blockIdx.x * 256 + threadIdx.x; k < 3 * P; k += stride) {
         const int p = k / 3;
-        if (pe_ptr[p + 1] > pe_ptr[p]) m = fmaxf(m, fabsf(Hll[9 * p + 4 * (k % 3)]));
+        if (pe_ptr[p + 1] > pe_ptr[p]) m = fmaxf(m, fabsf(hd[k]));
     }
     red[threadIdx.x] = m;
     __syncthreads();

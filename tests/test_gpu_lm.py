@@ -78,6 +78,30 @@ def test_schur_with_stereo_fixed_points_and_levels_vs_dense(gpu_ctx, robust):
     assert es < 1e-5 and eb < 1e-4
 
 
+@pytest.mark.parametrize("n_kf,n_points,obs,off", [(2, 20, 40, 0), (2, 260, 513, 0), (12, 150, 1030, 600),
+                                                   (21, 80, 1100, 0)])
+def test_schur_chunks_vs_dense(gpu_ctx, n_kf, n_points, obs, off):
+    """The Schur complement at the edges of its work division: 1, 11 and 20
+    free frames (18, 1 and 1 threads per frame sum), edge counts on both sides
+    of the 512-edge chunks, a chunk whose edges are all inactive, points with
+    more than 8 edges and frames.  Tolerances as the dense comparison above."""
+    lp = synth.local_ba_problem(seed=75, n_kf=n_kf, n_points=n_points, target_obs=obs, stereo_frac=0.6)
+    lin = _lin(lp, gpu_ctx)
+    am = np.ones(lin.M, np.uint8)
+    am[:off] = 0
+    lin.set_active(am)
+    lin.linearize()
+    lin.linearize_stereo()
+    H, b, _, free_f, _ = dense_system(lp, lp.mono.points, lp.mono.frames, active_m=am)
+    for lam in (1e2, 1e4):
+        S_ref, bs_ref = dense_schur(H, b, lam, 6 * len(free_f))
+        S, bs = lin.schur(lam)
+        assert np.linalg.norm(S - S_ref) < 1e-5 * np.linalg.norm(S_ref)
+        assert np.linalg.norm(bs - bs_ref) < 1e-4 * np.linalg.norm(bs_ref)
+    np.testing.assert_array_equal(lin.schur(1e4)[0], S)     # summation orders are fixed
+    lin.close()
+
+
 def test_robust_chi2_vs_oracle(gpu_ctx):
     lp = synth.local_ba_problem(seed=73, n_kf=6, n_points=3000, target_obs=30000, stereo_frac=0.8)
     lin = _lin(lp, gpu_ctx)
