@@ -91,6 +91,27 @@ struct DevBuf {
     ~DevBuf() { release(); }
 };
 
+// Parts of one allocation, at 256-byte offsets: first the sizes are summed
+// (base null), then, with a base, the parts are handed out.
+struct Carver {
+    char* base = nullptr;
+    size_t bytes = 0;
+    template <typename T>
+    void operator()(T*& p, size_t n) {
+        p = base ? reinterpret_cast<T*>(base + bytes) : nullptr;
+        bytes += (n * sizeof(T) + 255) / 256 * 256;
+    }
+};
+
+template <typename F>
+static void carve(DevBuf& d, F parts) {
+    Carver c;
+    parts(c);
+    d.ensure(std::max<size_t>(c.bytes, 256));
+    c = Carver{d.as<char>(), 0};
+    parts(c);
+}
+
 template <typename T>
 void upload(DevBuf& b, const std::vector<T>& v, hipStream_t s) {
     b.ensure(std::max<size_t>(v.size() * sizeof(T), 16));
@@ -868,6 +889,7 @@ struct mcv_ctx {
     DevBuf o_m, o_a1, o_a2, o_out, o_cnt, o_jobs;
     DevBuf w_pts, w_pdesc, w_plev, w_kxy, w_kdesc, w_cs, w_ci, w_out, w_view, w_cams;
     DevBuf b_d1, b_d2, b_f2, b_jobs, b_out;
+    DevBuf sb_work;  // ba_build_schur
     std::map<std::string, std::unique_ptr<OrbPlan>> plans;
 
     void set_device() { HIP_OK(hipSetDevice(device)); }
@@ -967,9 +989,8 @@ struct mcv_ba {
     int Ms = 0;
     StereoCam scam{};
     bool have_stereo = false, stereo_linearized = false;
-    DevBuf s_obs, s_pt, s_fr, s_isig, s_planes, fposes, flags;
+    DevBuf s_obs, s_pt, s_fr, s_isig, s_ptr, s_list, s_planes, fposes, flags;
     std::vector<int> h_gptr;  // observations of (frame, camera) group g: gobs[h_gptr[g] .. h_gptr[g + 1])
-    std::vector<int> h_pt, h_fr, h_pptr;
     std::vector<int> fixed;
     int variant = 0;  // k_ba_linearize launch shape (kBaVariant)
     bool have_obs = false, have_state = false, linearized = false;
@@ -991,7 +1012,6 @@ struct mcv_ba {
     // host, points on the device (p64) with the float pairs phi / plo
     std::vector<double> h_frames, h_cams;
     double h_scam[6] = {0, 0, 0, 0, 0, 0};
-    std::vector<int> h_spt, h_sfr;
     std::vector<int> point_fixed;                 // empty: no point fixed
     std::vector<uint8_t> active_m, active_s;      // empty: every edge active
     bool robust = true;                           // Huber kernels on
@@ -999,12 +1019,10 @@ struct mcv_ba {
     // Schur structure (depends on the edges, the active sets and the fixed
     // frames and points)
     bool schur_ready = false, schur_done = false;
-    int npf = 0, Fp = 0, nblk = 0;
+    int Fp = 0;
     bool free_points_with_edges = true;
-    int nechunk = 0, esub = 1, nichunk = 0;
-    DevBuf pe_ptr, pe, pf_ptr, pf_obs_ptr, pf_obs, pf_frame, pf_row, echunk, eptr, elist, ichunk, blk_chunk, blk_items,
-        blk_ij;
-    DevBuf prec, hd, Z, epart, ipart, Hpp, bs, bp, Sout;
+    SchurArgs sargs{};             // lists and work arrays in sb_lists and sb_items
+    DevBuf sb_lists, sb_items;
 };
 
 // Launch shapes of k_ba_linearize (same arithmetic per observation; the
@@ -1015,6 +1033,7 @@ struct BAVariantDesc {
     bool nt;
     const char* name;
 };
+constexpr int kMaxFreeFrames = 7700;  // (6 * 7700)^2 entries of S are the most 31 bits count
 constexpr int kBaVariants = 8;
 static const BAVariantDesc kBaVariant[kBaVariants] = {
     {256, 1024, 1, false, "256x1024 ilp1"},     {256, 1024, 2, false, "256x1024 ilp2"},
@@ -2623,9 +2642,6 @@ int mcv_ba_set_observations(mcv_ba* b, const float* uv, const int32_t* pt, const
     HIP_OK(hipStreamSynchronize(s));
     b->have_obs = sorted;
     REQUIRE(sorted, MCV_ERR_INVALID, "observations must be ordered by point");
-    b->h_pt.assign(pt, pt + M);
-    b->h_fr.assign(fr, fr + M);
-    b->h_pptr = pcount;
     b->schur_ready = false;
     b->touched(-1);
     API_END
@@ -2805,9 +2821,17 @@ int mcv_ba_set_stereo(mcv_ba* b, int Ms, const float* obs, const int32_t* pt, co
     for (int k = 0; k < 6; k++) b->h_scam[k] = cam[k];
     b->scam = StereoCam{(float)cam[0], (float)cam[1], (float)cam[2], (float)cam[3], (float)cam[4],
                         b->robust ? (float)cam[5] : INFINITY};
-    b->h_spt.assign(pt, pt + Ms);
-    b->h_sfr.assign(fr, fr + Ms);
     b->active_s.clear();
+    // CSR by point, edges of a point in index order
+    std::vector<int> sptr(b->P + 1, 0), slist(std::max(Ms, 1));
+    for (int i = 0; i < Ms; i++) sptr[pt[i] + 1]++;
+    for (int p = 0; p < b->P; p++) sptr[p + 1] += sptr[p];
+    {
+        std::vector<int> at(sptr.begin(), sptr.end() - 1);
+        for (int i = 0; i < Ms; i++) slist[at[pt[i]]++] = i;
+    }
+    upload(b->s_ptr, sptr, s);
+    upload(b->s_list, slist, s);
     b->schur_ready = false;
     const size_t m = (size_t)std::max(Ms, 1);
     b->s_obs.ensure(m * 12);
@@ -2915,208 +2939,184 @@ int mcv_ba_generation(mcv_ba* b, int64_t* gen) {
     return MCV_OK;
 }
 
-// Host side of the Schur structure: (point, free frame) groups of
-// observations, free-frame observation lists, and for every free-frame pair
-// block (i <= j) the list of (pf_i, pf_j) products, all in point order.
-// Edge lists of the Schur complement over the active mono and stereo edges
-// (index i < M mono, M + j stereo): per free point its edges, per (free
-// point, free frame) pair its edges, per free frame its edges (points fixed
-// or not) and its pairs, and the pair lists of every frame-pair block.
+// The edge lists of the Schur complement over the active edges, free points
+// and free frames (mcv_ba.hip, SchurBuild), and the division of the pair
+// blocks' items into chunks.  The work arrays are the context's; nothing
+// reads them after the final synchronization.
 static void ba_build_schur(mcv_ba* b, hipStream_t s) {
-    const int P = b->P, F = b->F, M = b->M;
-    const int Ms = b->have_stereo ? b->Ms : 0;
+    mcv_ctx* c = b->ctx;
+    const int P = b->P, F = b->F, M = b->M, Ms = b->have_stereo ? b->Ms : 0, E = M + Ms;
     if (b->fixed.empty()) b->fixed.assign(F, 0);
     std::vector<int> fidx(F, -1);
     int Fp = 0;
     for (int f = 0; f < F; f++)
         if (!b->fixed[f]) fidx[f] = Fp++;
-    auto act_m = [&](int i) { return b->active_m.empty() || b->active_m[i]; };
-    auto act_s = [&](int j) { return b->active_s.empty() || b->active_s[j]; };
-    auto pfree = [&](int p) { return b->point_fixed.empty() || !b->point_fixed[p]; };
-    // per point: active edges (mono in index order, then stereo)
-    std::vector<int> pe_ptr(P + 1, 0);
-    for (int i = 0; i < M; i++)
-        if (act_m(i) && pfree(b->h_pt[i])) pe_ptr[b->h_pt[i] + 1]++;
-    for (int j = 0; j < Ms; j++)
-        if (act_s(j) && pfree(b->h_spt[j])) pe_ptr[b->h_spt[j] + 1]++;
-    for (int p = 0; p < P; p++) pe_ptr[p + 1] += pe_ptr[p];
-    std::vector<int> pe(std::max(pe_ptr[P], 1));
-    {
-        std::vector<int> a(pe_ptr.begin(), pe_ptr.end() - 1);
-        for (int i = 0; i < M; i++)
-            if (act_m(i) && pfree(b->h_pt[i])) pe[a[b->h_pt[i]]++] = i;
-        for (int j = 0; j < Ms; j++)
-            if (act_s(j) && pfree(b->h_spt[j])) pe[a[b->h_spt[j]]++] = M + j;
-    }
-    auto frame_of = [&](int e) { return e < M ? b->h_fr[e] : b->h_sfr[e - M]; };
-    std::vector<int> pf_ptr(P + 1, 0), pf_obs_ptr(1, 0), pf_obs, pf_point, pf_free;
-    std::vector<std::pair<int, int>> tmp;
-    bool any_free_edges = false;
-    for (int p = 0; p < P; p++) {
-        tmp.clear();
-        if (pe_ptr[p + 1] > pe_ptr[p]) any_free_edges = true;
-        for (int t = pe_ptr[p]; t < pe_ptr[p + 1]; t++)
-            if (fidx[frame_of(pe[t])] >= 0) tmp.push_back({fidx[frame_of(pe[t])], pe[t]});
-        std::stable_sort(tmp.begin(), tmp.end(), [](const std::pair<int, int>& x, const std::pair<int, int>& y) {
-            return x.first < y.first;
-        });
-        for (size_t k = 0; k < tmp.size(); k++) {
-            if (k == 0 || tmp[k].first != tmp[k - 1].first) {
-                if (k) pf_obs_ptr.push_back((int)pf_obs.size());
-                pf_point.push_back(p);
-                pf_free.push_back(tmp[k].first);
-            }
-            pf_obs.push_back(tmp[k].second);
-        }
-        if (!tmp.empty()) pf_obs_ptr.push_back((int)pf_obs.size());
-        pf_ptr[p + 1] = (int)pf_point.size();
-    }
-    const int npf = (int)pf_point.size();
-    // rows of the pf entries: by free frame, then by point
-    std::vector<int> fpf_ptr(Fp + 1, 0), pf_row(std::max(npf, 1));
-    for (int q = 0; q < npf; q++) fpf_ptr[pf_free[q] + 1]++;
-    for (int f = 0; f < Fp; f++) fpf_ptr[f + 1] += fpf_ptr[f];
-    {
-        std::vector<int> c(fpf_ptr.begin(), fpf_ptr.end() - 1);
-        for (int q = 0; q < npf; q++) pf_row[q] = c[pf_free[q]]++;
-    }
-    // chunks of kEdgeChunk consecutive edges, each with the local numbers of
-    // its active edges of free frames, sorted by frame
-    std::vector<EdgeChunk> echunk;
-    std::vector<uint16_t> eptr, elist;
-    for (int st = 0; st < 2; st++) {
-        const int n = st ? Ms : M;
-        const int* fr = st ? b->h_sfr.data() : b->h_fr.data();
-        std::vector<int> cnt(Fp + 1);
-        for (int e0 = 0; e0 < n && Fp > 0; e0 += kEdgeChunk) {
-            const int m = std::min(kEdgeChunk, n - e0);
-            std::fill(cnt.begin(), cnt.end(), 0);
-            auto use = [&](int k) { return (st ? act_s(e0 + k) : act_m(e0 + k)) && fidx[fr[e0 + k]] >= 0; };
-            for (int k = 0; k < m; k++)
-                if (use(k)) cnt[fidx[fr[e0 + k]] + 1]++;
-            for (int f = 0; f < Fp; f++) cnt[f + 1] += cnt[f];
-            const size_t l0 = elist.size();
-            echunk.push_back(EdgeChunk{e0, m, (int)l0, st});
-            for (int f = 0; f <= Fp; f++) eptr.push_back((uint16_t)cnt[f]);
-            elist.resize(l0 + cnt[Fp]);
-            for (int k = 0; k < m; k++)
-                if (use(k)) elist[l0 + cnt[fidx[fr[e0 + k]]]++] = (uint16_t)k;
-        }
-    }
-    // pair blocks, upper triangle row-major
-    const int nblk = Fp * (Fp + 1) / 2;
-    auto bidx = [Fp](int i, int j) { return i * Fp - i * (i - 1) / 2 + (j - i); };
-    std::vector<int> blk_ptr(nblk + 1, 0);
-    for (int p = 0; p < P; p++)
-        for (int qa = pf_ptr[p]; qa < pf_ptr[p + 1]; qa++)
-            for (int qb = qa; qb < pf_ptr[p + 1]; qb++) blk_ptr[bidx(pf_free[qa], pf_free[qb]) + 1]++;
-    for (int k = 0; k < nblk; k++) blk_ptr[k + 1] += blk_ptr[k];
-    std::vector<int2> items(std::max(blk_ptr[nblk], 1)), ij(std::max(nblk, 1));
-    std::vector<int> item_point(std::max(blk_ptr[nblk], 1));
-    {
-        std::vector<int> a(blk_ptr.begin(), blk_ptr.end() - 1);
-        for (int p = 0; p < P; p++)
-            for (int qa = pf_ptr[p]; qa < pf_ptr[p + 1]; qa++)
-                for (int qb = qa; qb < pf_ptr[p + 1]; qb++) {
-                    const int t = a[bidx(pf_free[qa], pf_free[qb])]++;
-                    items[t] = make_int2(pf_row[qa], pf_row[qb]);
-                    item_point[t] = p;
-                }
-        for (int i = 0; i < Fp; i++)
-            for (int j = i; j < Fp; j++) ij[bidx(i, j)] = make_int2(i, j);
-    }
-    // Chunks of a block's items, one wave each: at most csz items (about
-    // 16384 waves) and, from 128 items on, at most 1/32 of the points,
-    // launched in the order of their first point (see k_schur_items).
-    const int csz = std::min(2048, std::max(256, (blk_ptr[nblk] / 16384 + 63) / 64 * 64)), span = std::max(P / 32, 1);
-    std::vector<int> blk_chunk(nblk + 1, 0);
-    std::vector<ItemChunk> ichunk;
-    for (int k = 0; k < nblk; k++) {
-        for (int i0 = blk_ptr[k], i1; i0 < blk_ptr[k + 1]; i0 = i1) {
-            const int p0 = item_point[i0], end = std::min(i0 + csz, blk_ptr[k + 1]);
-            i1 = std::min(i0 + 128, end);
-            while (i1 < end && item_point[i1] - p0 < span) i1++;
-            ichunk.push_back(ItemChunk{i0, i1, (int)ichunk.size(), ij[k].x == ij[k].y ? 1 : 0});
-        }
-        blk_chunk[k + 1] = (int)ichunk.size();
-    }
-    std::stable_sort(ichunk.begin(), ichunk.end(),
-                     [&](const ItemChunk& x, const ItemChunk& y) { return item_point[x.i0] < item_point[y.i0]; });
-    upload(b->pe_ptr, pe_ptr, s);
-    upload(b->pe, pe, s);
-    upload(b->pf_ptr, pf_ptr, s);
-    upload(b->pf_obs_ptr, pf_obs_ptr, s);
-    upload(b->pf_obs, pf_obs, s);
-    upload(b->pf_frame, pf_free, s);
-    upload(b->pf_row, pf_row, s);
-    upload(b->echunk, echunk, s);
-    upload(b->eptr, eptr, s);
-    upload(b->elist, elist, s);
-    upload(b->ichunk, ichunk, s);
-    upload(b->blk_chunk, blk_chunk, s);
-    upload(b->blk_items, items, s);
-    upload(b->blk_ij, ij, s);
-    b->nechunk = (int)echunk.size();
-    b->nichunk = (int)ichunk.size();
+    REQUIRE(Fp <= kMaxFreeFrames, MCV_ERR_INVALID, "too many free keyframes in one problem");
+    const int nb = (P + 255) / 256, etiles = std::max((E + 255) / 256, 1), rtiles = E / 64 + Fp + 1;
+    const int nblk = Fp * (Fp + 1) / 2, ncm = (M + kEdgeChunk - 1) / kEdgeChunk;
+    const int nec = Fp > 0 ? ncm + (Ms + kEdgeChunk - 1) / kEdgeChunk : 0;
+    // entries are at most the edges, so all lists but the items have a bound here
+    SchurBuild B{};
+    SchurArgs a{};
+    int* d_fidx = nullptr;
+    carve(c->sb_work, [&](Carver& t) {
+        t(d_fidx, F);
+        t(B.ef, E);
+        t(B.mask, (size_t)P * ((Fp + 63) / 64));
+        t(B.po_ptr, P + 1);
+        t(B.btot, (size_t)3 * (nb + 1));
+        t(B.pf_point, E);
+        t(B.row_q, E);
+        t(B.thist, (size_t)Fp * etiles);
+        t(B.fbase, Fp + 1);
+        t(B.tbase, Fp + 1);
+        t(B.tcount, (size_t)rtiles * Fp);
+        t(B.win, (size_t)nblk * (kWindows + 1));
+    });
     // threads that share a frame sum in k_schur_edges: its 512 threads cover
     // the 27 Fp sums once
-    b->esub = Fp > 0 ? std::max(1, 512 / (kFrameSums * Fp)) : 1;
-    b->prec.ensure((size_t)P * kPointRec * 4);
-    b->hd.ensure((size_t)P * 12);
-    b->Z.ensure((size_t)std::max(npf, 1) * kZRow * 4);
-    b->epart.ensure((size_t)std::max(b->nechunk * b->esub, 1) * kFrameSums * std::max(Fp, 1) * 4);
-    b->ipart.ensure((size_t)std::max(b->nichunk, 1) * kItemSums * 4);
-    b->Hpp.ensure((size_t)std::max(Fp, 1) * 144);
-    b->bs.ensure((size_t)std::max(Fp, 1) * 24);
-    b->bp.ensure((size_t)std::max(Fp, 1) * 24);
-    b->Sout.ensure((size_t)std::max(36 * Fp * Fp, 1) * 4);
+    a.esub = Fp > 0 ? std::max(1, 512 / (kFrameSums * Fp)) : 1;
+    const size_t np = P, fp = Fp;
+    carve(b->sb_lists, [&](Carver& t) {
+        t(B.pe_ptr, np + 1);
+        t(B.pf_ptr, np + 1);
+        t(B.pe, E);
+        t(B.pf_obs, E);
+        t(B.pf_obs_ptr, (size_t)E + 1);
+        t(B.pf_frame, E);
+        t(B.pf_row, E);
+        t(B.eptr, (size_t)nec * (fp + 1));
+        t(B.elist, (size_t)nec * kEdgeChunk);
+        t(a.prec, np * kPointRec);
+        t(a.hd, np * 3);
+        t(a.Z, (size_t)E * kZRow);
+        t(a.epart, (size_t)nec * a.esub * kFrameSums * fp);
+        t(a.Hpp, fp * 36);
+        t(a.bs, fp * 6);
+        t(a.bp, fp * 6);
+        t(a.Sout, 36 * fp * fp);
+    });
+    B.pptr = b->pptr.as<int>();
+    B.sptr = Ms ? b->s_ptr.as<int>() : nullptr;
+    B.slist = b->s_list.as<int>();
+    B.pair = b->pair.as<uint32_t>();
+    B.sfr = b->s_fr.as<uint32_t>();
+    B.act_m = b->active_m.empty() ? nullptr : b->act_m.as<uint8_t>();
+    B.act_s = b->active_s.empty() ? nullptr : b->act_s.as<uint8_t>();
+    B.pfix = b->point_fixed.empty() ? nullptr : b->pfix_d.as<uint8_t>();
+    B.fidx = d_fidx;
+    B.M = M;
+    B.Ms = Ms;
+    B.P = P;
+    B.C = b->C;
+    B.Fp = Fp;
+    B.words = (Fp + 63) / 64;
+    B.ntile = etiles;
+    B.nchunk_m = ncm;
+    HIP_OK(hipMemcpyAsync(d_fidx, fidx.data(), (size_t)F * 4, hipMemcpyHostToDevice, s));
+    if (E > 0) hipLaunchKernelGGL(k_sb_edges, dim3((E + 255) / 256), dim3(256), 0, s, B);
+    hipLaunchKernelGGL(k_sb_points, dim3(nb), dim3(256), 0, s, B);
+    hipLaunchKernelGGL(k_sb_offsets, dim3(1), dim3(1024), 0, s, B, nb);
+    hipLaunchKernelGGL(k_sb_fill, dim3(nb), dim3(256), 0, s, B, nb);
+    const size_t flds = (size_t)(Fp + 1) * 4;
+    if (Fp > 0) {
+        hipLaunchKernelGGL(k_sb_hist, dim3(etiles), dim3(256), flds, s, B, nb);
+        hipLaunchKernelGGL(k_sb_frames, dim3(Fp), dim3(1024), 0, s, B);
+        hipLaunchKernelGGL(k_sb_bases, dim3(1), dim3(1024), 0, s, B);
+        hipLaunchKernelGGL(k_sb_rows, dim3(etiles), dim3(256), 0, s, B, nb);
+        hipLaunchKernelGGL(k_sb_items<false>, dim3((rtiles + 3) / 4), dim3(256), 0, s, B);
+        hipLaunchKernelGGL(k_sb_blocks, dim3(Fp, Fp), dim3(64), 0, s, B);
+        if (nec > 0) hipLaunchKernelGGL(k_sb_chunks, dim3(nec), dim3(512), flds + kEdgeChunk * 4, s, B);
+    }
+    HIP_OK(hipGetLastError());
+    // the items' windows and the totals come back; the host cuts the chunks
+    std::vector<int> win((size_t)nblk * (kWindows + 1));
+    int tot[3] = {0, 0, 0};
+    if (nblk) HIP_OK(hipMemcpyAsync(win.data(), B.win, win.size() * 4, hipMemcpyDeviceToHost, s));
+    HIP_OK(hipMemcpyAsync(tot, B.btot + 3 * nb, 12, hipMemcpyDeviceToHost, s));
     HIP_OK(hipStreamSynchronize(s));
-    b->npf = npf;
+    // one upload: every block's first item, its first chunk, then the chunks
+    std::vector<int> up(2 * (size_t)(nblk + 1), 0);
+    int* blk_ptr = up.data();
+    int* blk_chunk = blk_ptr + nblk + 1;
+    for (int k = 0; k < nblk; k++) {
+        const long long n = (long long)blk_ptr[k] + win[(size_t)k * (kWindows + 1) + kWindows];
+        REQUIRE(n <= INT32_MAX, MCV_ERR_CAPACITY, "more than 2^31 frame-pair products");
+        blk_ptr[k + 1] = (int)n;
+    }
+    const int nitem = blk_ptr[nblk];
+    // Chunks of a block's items, one wave each: whole windows up to at least
+    // 128 items, at most csz items (about 16384 waves), launched in the order
+    // of their first window (see k_schur_items).
+    const int csz = std::min(2048, std::max(256, (nitem / 16384 + 63) / 64 * 64));
+    std::vector<ItemChunk> cut;
+    std::vector<int> first, cnt(kWindows + 1, 0);
+    for (int i = 0, k = 0; i < Fp; i++)
+        for (int j = i; j < Fp; j++, k++) {
+            const int* w = win.data() + (size_t)k * (kWindows + 1);
+            for (int x = 0, y = 0; x < kWindows && w[kWindows] > 0; x = y) {
+                for (y = x + 1; y < kWindows && w[y] - w[x] < 128; y++) {}
+                if (y < kWindows && w[kWindows] - w[y] < 64) y = kWindows;  // no remainder of its own
+                for (int i0 = w[x]; i0 < w[y]; i0 += csz) {
+                    cut.push_back(ItemChunk{blk_ptr[k] + i0, blk_ptr[k] + std::min(i0 + csz, w[y]), (int)cut.size(),
+                                            i == j ? 1 : 0});
+                    first.push_back(x);
+                    cnt[x + 1]++;
+                }
+            }
+            blk_chunk[k + 1] = (int)cut.size();
+        }
+    for (int x = 0; x < kWindows; x++) cnt[x + 1] += cnt[x];
+    a.nichunk = (int)cut.size();
+    static_assert(sizeof(ItemChunk) == 16, "chunks are uploaded behind ints");
+    const size_t head = (up.size() + 3) / 4 * 4;
+    up.resize(head + 4 * cut.size());
+    for (size_t k = 0; k < cut.size(); k++)
+        std::memcpy(up.data() + head + 4 * (size_t)cnt[first[k]]++, &cut[k], sizeof(ItemChunk));
+    int* d_up = nullptr;
+    carve(b->sb_items, [&](Carver& t) {
+        t(d_up, up.size());
+        t(B.items, nitem);
+        t(a.ipart, (size_t)a.nichunk * kItemSums);
+    });
+    HIP_OK(hipMemcpyAsync(d_up, up.data(), up.size() * 4, hipMemcpyHostToDevice, s));
+    B.blk_ptr = d_up;
+    if (nitem > 0) hipLaunchKernelGGL(k_sb_items<true>, dim3((rtiles + 3) / 4), dim3(256), 0, s, B);
+    HIP_OK(hipGetLastError());
+    HIP_OK(hipStreamSynchronize(s));  // the uploads' host arrays end here
+    a.M = M;
+    a.Ms = Ms;
+    a.S = M;
+    a.SS = b->Ms;
+    a.pe_ptr = B.pe_ptr;
+    a.pe = B.pe;
+    a.pf_ptr = B.pf_ptr;
+    a.pf_obs_ptr = B.pf_obs_ptr;
+    a.pf_obs = B.pf_obs;
+    a.pf_frame = B.pf_frame;
+    a.pf_row = B.pf_row;
+    a.eptr = B.eptr;
+    a.elist = B.elist;
+    a.nchunk_m = ncm;
+    a.nechunk = nec;
+    a.blk_chunk = d_up + nblk + 1;
+    a.ichunk = reinterpret_cast<const ItemChunk*>(d_up + head);
+    a.items = B.items;
+    a.P = P;
+    a.Fp = Fp;
+    b->sargs = a;
     b->Fp = Fp;
-    b->nblk = nblk;
-    b->free_points_with_edges = any_free_edges;
+    b->free_points_with_edges = tot[0] > 0;
     b->schur_ready = true;
 }
 
 static SchurArgs ba_schur_args(mcv_ba* b, float lambda) {
-    SchurArgs a{};
+    SchurArgs a = b->sargs;
     a.planes = b->planes.as<float>();
-    a.S = b->M;
     a.isig = b->isig.as<float>();
-    a.M = b->M;
     a.splanes = b->s_planes.as<float>();
-    a.SS = b->Ms;
     a.sisig = b->s_isig.as<float>();
-    a.pe_ptr = b->pe_ptr.as<int>();
-    a.pe = b->pe.as<int>();
-    a.pf_ptr = b->pf_ptr.as<int>();
-    a.pf_obs_ptr = b->pf_obs_ptr.as<int>();
-    a.pf_obs = b->pf_obs.as<int>();
-    a.pf_frame = b->pf_frame.as<int>();
-    a.pf_row = b->pf_row.as<int>();
-    a.echunk = b->echunk.as<EdgeChunk>();
-    a.eptr = b->eptr.as<uint16_t>();
-    a.elist = b->elist.as<uint16_t>();
-    a.ichunk = b->ichunk.as<ItemChunk>();
-    a.blk_chunk = b->blk_chunk.as<int>();
-    a.items = b->blk_items.as<int2>();
-    a.blk_ij = b->blk_ij.as<int2>();
-    a.P = b->P;
-    a.Fp = b->Fp;
-    a.nblk = b->nblk;
-    a.nechunk = b->nechunk;
-    a.esub = b->esub;
-    a.nichunk = b->nichunk;
     a.lambda = lambda;
-    a.prec = b->prec.as<float>();
-    a.hd = b->hd.as<float>();
-    a.Z = b->Z.as<float>();
-    a.epart = b->epart.as<float>();
-    a.ipart = b->ipart.as<float>();
-    a.Hpp = b->Hpp.as<float>();
-    a.bs = b->bs.as<float>();
-    a.bp = b->bp.as<float>();
-    a.Sout = b->Sout.as<float>();
     return a;
 }
 
@@ -3126,18 +3126,17 @@ static void ba_enqueue_schur(mcv_ba* b, float lambda, hipStream_t s, bool blocks
     const SchurArgs a = ba_schur_args(b, lambda);
     hipLaunchKernelGGL(k_schur_points, dim3(xcd_grid((b->P + 31) / 32)), dim3(256), 0, s, a);
     if (b->Fp > 0) {
-        if (b->nechunk > 0) hipLaunchKernelGGL(k_schur_edges, dim3(b->nechunk), dim3(512), 0, s, a);
+        if (a.nechunk > 0) hipLaunchKernelGGL(k_schur_edges, dim3(a.nechunk), dim3(512), 0, s, a);
         hipLaunchKernelGGL(k_schur_edge_sums, dim3((kFrameSums * b->Fp + 15) / 16), dim3(1024), 0, s, a);
         if (blocks) {
-            if (b->nichunk > 0) hipLaunchKernelGGL(k_schur_items, dim3(xcd_grid((b->nichunk + 3) / 4)), dim3(256), 0, s, a);
-            hipLaunchKernelGGL(k_schur_assemble, dim3(b->nblk), dim3(8 * kItemSums), 0, s, a);
+            if (a.nichunk > 0) hipLaunchKernelGGL(k_schur_items, dim3(xcd_grid((a.nichunk + 3) / 4)), dim3(256), 0, s, a);
+            hipLaunchKernelGGL(k_schur_assemble, dim3(b->Fp, b->Fp), dim3(8 * kItemSums), 0, s, a);
         }
     }
     HIP_OK(hipGetLastError());
 }
 
 static void ba_require_schur_inputs(mcv_ba* b) {
-    REQUIRE(b->pose_linearized, MCV_ERR_STATE, "linearize before the Schur complement");
     REQUIRE(b->linearized || !b->free_points_with_edges, MCV_ERR_STATE,
             "a pose-only linearization leaves no J_point for the free points");
     const bool stereo_edges = b->have_stereo && b->Ms > 0;
@@ -3205,6 +3204,7 @@ int mcv_ba_schur(mcv_ba* b, float lambda) {
     REQUIRE(b, MCV_ERR_INVALID, "null BA object");
     c->set_device();
     hipStream_t s = c->stream;
+    REQUIRE(b->pose_linearized, MCV_ERR_STATE, "linearize before the Schur complement");
     if (!b->schur_ready) ba_build_schur(b, s);
     ba_require_schur_inputs(b);
     ba_enqueue_schur(b, lambda, s);
@@ -3221,8 +3221,8 @@ int mcv_ba_read_schur(mcv_ba* b, double* S, double* bs, int32_t* n) {
     if (n) *n = m;
     std::vector<float> hs((size_t)m * m), hb(m);
     if (m) {
-        HIP_OK(hipMemcpyAsync(hs.data(), b->Sout.p, hs.size() * 4, hipMemcpyDeviceToHost, c->stream));
-        HIP_OK(hipMemcpyAsync(hb.data(), b->bs.p, hb.size() * 4, hipMemcpyDeviceToHost, c->stream));
+        HIP_OK(hipMemcpyAsync(hs.data(), b->sargs.Sout, hs.size() * 4, hipMemcpyDeviceToHost, c->stream));
+        HIP_OK(hipMemcpyAsync(hb.data(), b->sargs.bs, hb.size() * 4, hipMemcpyDeviceToHost, c->stream));
     }
     HIP_OK(hipStreamSynchronize(c->stream));
     if (S) for (size_t k = 0; k < hs.size(); k++) S[k] = hs[k];
@@ -3432,8 +3432,8 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
             ba_enqueue_schur(b, 1.f, s, false);
             const int mblocks = std::max(1, std::min(1024, (3 * std::max(P, 2 * Fp) + 255) / 256));
             b->partial.ensure((size_t)mblocks * 8);
-            hipLaunchKernelGGL(k_ba_max_diag, dim3(mblocks), dim3(256), 0, s, b->Hpp.as<float>(), Fp,
-                               b->hd.as<float>(), b->pe_ptr.as<int>(), P, reinterpret_cast<float*>(b->partial.p));
+            hipLaunchKernelGGL(k_ba_max_diag, dim3(mblocks), dim3(256), 0, s, b->sargs.Hpp, Fp,
+                               b->sargs.hd, b->sargs.pe_ptr, P, reinterpret_cast<float*>(b->partial.p));
             hipLaunchKernelGGL(k_max_partials, dim3(1), dim3(256), 0, s, reinterpret_cast<const float*>(b->partial.p),
                                mblocks, b->fmax.as<float>());
             HIP_OK(hipGetLastError());
@@ -3451,9 +3451,9 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
             HIP_OK(hipMemcpyAsync(b->p64_bak.p, b->p64.p, (size_t)P * 24, hipMemcpyDeviceToDevice, s));
             ba_enqueue_schur(b, (float)lambda, s);
             if (n) {
-                HIP_OK(hipMemcpyAsync(Sf.data(), b->Sout.p, Sf.size() * 4, hipMemcpyDeviceToHost, s));
-                HIP_OK(hipMemcpyAsync(bsf.data(), b->bs.p, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-                HIP_OK(hipMemcpyAsync(bpf.data(), b->bp.p, (size_t)n * 4, hipMemcpyDeviceToHost, s));
+                HIP_OK(hipMemcpyAsync(Sf.data(), b->sargs.Sout, Sf.size() * 4, hipMemcpyDeviceToHost, s));
+                HIP_OK(hipMemcpyAsync(bsf.data(), b->sargs.bs, (size_t)n * 4, hipMemcpyDeviceToHost, s));
+                HIP_OK(hipMemcpyAsync(bpf.data(), b->sargs.bp, (size_t)n * 4, hipMemcpyDeviceToHost, s));
             }
             HIP_OK(hipStreamSynchronize(s));
             for (size_t k = 0; k < Sf.size(); k++) S[k] = Sf[k];

@@ -468,17 +468,333 @@ constexpr int kEdgeChunk = 512;    // edges per workgroup of k_schur_edges
 constexpr int kItemSums = 40;      // sums of an item chunk (36, or 27 on the diagonal)
 constexpr int kFrameSums = 27;     // per frame: H_pp upper triangle by rows, each row followed by b_p's entry
 
-struct EdgeChunk {
-    int e0, n;     // edges [e0, e0 + n) of the mono (or, stereo != 0, stereo) planes
-    int list0;     // first entry of its frame-sorted list of local edge numbers
-    int stereo;
-};
-
 struct ItemChunk {
     int i0, i1;  // items [i0, i1) of one frame-pair block
     int out;     // row of ipart: the chunks of a block in order, blocks in order
     int diag;
 };
+
+// ---- edge lists of the Schur complement, built on the device ------------------
+// From the edges in point order (mono: CSR pptr; stereo: CSR sptr over slist)
+// and every edge's free frame: per free point its active edges and, by free
+// frame, its entries and their edges; the entries' rows by (frame, point); per
+// frame pair the items (row_i, row_j) in point order.  All orders are fixed.
+// Bound by the edge and entry arrays, read a few times; 1.5M edges, 1.2M
+// entries, 5.4M items: the host loops this replaces took 50 ms.
+constexpr int kWindows = 32;  // windows of a frame's rows, for the item chunks
+
+// frame-pair blocks (i <= j): the upper triangle by rows
+__host__ __device__ __forceinline__ int block_of(int i, int j, int Fp) { return i * Fp - i * (i - 1) / 2 + (j - i); }
+
+struct SchurBuild {
+    const int* pptr;
+    const int* sptr;          // null without stereo edges
+    const int* slist;
+    const uint32_t* pair;     // mono: frame * C + cam
+    const uint32_t* sfr;      // stereo: frame
+    const uint8_t* act_m;     // or null: every edge active
+    const uint8_t* act_s;
+    const uint8_t* pfix;      // or null: no point fixed
+    const int* fidx;          // frame -> free frame or -1
+    int M, Ms, P, C, Fp, words, ntile;  // words: u64 per frame mask; ntile: tiles of 256 entries (stride of thist)
+    int* ef;                  // M + Ms: the edge's free frame, -1 fixed frame, -2 inactive
+    unsigned long long* mask; // P x words: the free frames that see a point
+    int *pe_ptr, *po_ptr, *pf_ptr;      // P + 1 each
+    int* btot;                // per 256 points: (edges, edges of free frames, entries), then their totals
+    int *pe, *pf_obs, *pf_obs_ptr, *pf_frame, *pf_point, *pf_row, *row_q;
+    int* thist;               // Fp x ntile
+    int* fbase;               // Fp + 1: first row of a frame
+    int* tbase;               // Fp + 1: first 64-row tile of a frame
+    int* tcount;              // row tiles x Fp
+    int* win;                 // nblk x (kWindows + 1): items before each window
+    const int* blk_ptr;       // nblk
+    int2* items;
+    uint16_t *eptr, *elist;
+    int nchunk_m;             // chunks of the mono edges; the stereo edges' follow
+};
+
+__global__ __launch_bounds__(256) void k_sb_edges(SchurBuild b) {
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= b.M + b.Ms) return;
+    const bool mono = e < b.M;
+    const uint8_t* act = mono ? b.act_m : b.act_s;
+    const int k = mono ? e : e - b.M;
+    b.ef[e] = act && !act[k] ? -2 : b.fidx[mono ? b.pair[k] / (uint32_t)b.C : b.sfr[k]];
+}
+
+// f(edge, its free frame) for every active edge of point p, mono first
+template <typename F>
+__device__ __forceinline__ void point_edges(const SchurBuild& b, int p, F f) {
+    for (int e = b.pptr[p]; e < b.pptr[p + 1]; e++)
+        if (b.ef[e] != -2) f(e, b.ef[e]);
+    if (b.sptr)
+        for (int t = b.sptr[p]; t < b.sptr[p + 1]; t++) {
+            const int e = b.M + b.slist[t];
+            if (b.ef[e] != -2) f(e, b.ef[e]);
+        }
+}
+
+// exclusive scan of one int per thread over the workgroup; ws: 17 ints
+__device__ __forceinline__ int wg_excl(int v, int* ws, int& total) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    int x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) ws[w] = x;
+    __syncthreads();
+    int base = 0;
+    total = 0;
+    for (int k = 0; k < nw; k++) {
+        base += k < w ? ws[k] : 0;
+        total += ws[k];
+    }
+    __syncthreads();
+    return base + x - v;
+}
+
+// per point: counts (their scans within the 256 points), and the frame mask
+__global__ __launch_bounds__(256) void k_sb_points(SchurBuild b) {
+    __shared__ int ws[17];
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    int n = 0, nf = 0, nd = 0;
+    if (p < b.P) {
+        unsigned long long* m = b.mask + (long long)p * b.words;
+        for (int k = 0; k < b.words; k++) m[k] = 0;
+        if (!(b.pfix && b.pfix[p])) {
+            unsigned long long m0 = 0;
+            point_edges(b, p, [&](int, int f) {
+                n++;
+                if (f < 0) return;
+                nf++;
+                if (f < 64) m0 |= 1ull << f;
+                else m[f >> 6] |= 1ull << (f & 63);
+            });
+            if (b.words) m[0] = m0;
+            for (int k = 0; k < b.words; k++) nd += __popcll(m[k]);
+        }
+    }
+    int t0, t1, t2;
+    const int a0 = wg_excl(n, ws, t0), a1 = wg_excl(nf, ws, t1), a2 = wg_excl(nd, ws, t2);
+    if (p < b.P) {
+        b.pe_ptr[p] = a0;
+        b.po_ptr[p] = a1;
+        b.pf_ptr[p] = a2;
+    }
+    if (threadIdx.x == 0) {
+        b.btot[3 * blockIdx.x] = t0;
+        b.btot[3 * blockIdx.x + 1] = t1;
+        b.btot[3 * blockIdx.x + 2] = t2;
+    }
+}
+
+// the 256-point blocks' offsets, the totals after them (one workgroup)
+__global__ __launch_bounds__(1024) void k_sb_offsets(SchurBuild b, int nb) {
+    __shared__ int ws[17];
+    int run[3] = {0, 0, 0};
+    for (int k0 = 0; k0 < nb; k0 += 1024) {
+        const int k = k0 + threadIdx.x;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            int tot;
+            const int x = wg_excl(k < nb ? b.btot[3 * k + c] : 0, ws, tot);
+            if (k < nb) b.btot[3 * k + c] = run[c] + x;
+            run[c] += tot;
+        }
+    }
+    if (threadIdx.x == 0)
+        for (int c = 0; c < 3; c++) b.btot[3 * nb + c] = run[c];
+}
+
+// per point: final offsets, its edge list, its entries by frame and their edges
+__global__ __launch_bounds__(256) void k_sb_fill(SchurBuild b, int nb) {
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= b.P) return;
+    const int* bo = b.btot + 3 * blockIdx.x;
+    int n = b.pe_ptr[p] + bo[0], o = b.po_ptr[p] + bo[1], q = b.pf_ptr[p] + bo[2];
+    b.pe_ptr[p] = n;
+    b.pf_ptr[p] = q;
+    if (p == b.P - 1) {
+        b.pe_ptr[b.P] = b.btot[3 * nb];
+        b.pf_ptr[b.P] = b.btot[3 * nb + 2];
+        b.pf_obs_ptr[b.btot[3 * nb + 2]] = b.btot[3 * nb + 1];
+    }
+    if (b.pfix && b.pfix[p]) return;
+    point_edges(b, p, [&](int e, int) { b.pe[n++] = e; });
+    for (int k = 0; k < b.words; k++)
+        for (unsigned long long m = b.mask[(long long)p * b.words + k]; m; m &= m - 1, q++) {
+            const int f = 64 * k + __builtin_ctzll(m);
+            b.pf_obs_ptr[q] = o;
+            b.pf_frame[q] = f;
+            b.pf_point[q] = p;
+            point_edges(b, p, [&](int e, int fe) {
+                if (fe == f) b.pf_obs[o++] = e;
+            });
+        }
+}
+
+// entries per frame of 256 entries
+__global__ __launch_bounds__(256) void k_sb_hist(SchurBuild b, int nb) {
+    extern __shared__ int s_cnt[];  // Fp
+    const int npf = b.btot[3 * nb + 2], q = blockIdx.x * 256 + threadIdx.x;
+    for (int f = threadIdx.x; f < b.Fp; f += 256) s_cnt[f] = 0;
+    __syncthreads();
+    if (q < npf) atomicAdd(&s_cnt[b.pf_frame[q]], 1);
+    __syncthreads();
+    for (int f = threadIdx.x; f < b.Fp; f += 256) b.thist[(long long)f * b.ntile + blockIdx.x] = s_cnt[f];
+}
+
+// per frame: the tiles' offsets; the frame's entries to fbase[f + 1]
+__global__ __launch_bounds__(1024) void k_sb_frames(SchurBuild b) {
+    __shared__ int ws[17];
+    int* h = b.thist + (long long)blockIdx.x * b.ntile;
+    int run = 0;
+    for (int k0 = 0; k0 < b.ntile; k0 += 1024) {
+        const int k = k0 + threadIdx.x;
+        int tot;
+        const int x = wg_excl(k < b.ntile ? h[k] : 0, ws, tot);
+        if (k < b.ntile) h[k] = run + x;
+        run += tot;
+    }
+    if (threadIdx.x == 0) b.fbase[blockIdx.x + 1] = run;
+}
+
+__global__ __launch_bounds__(1024) void k_sb_bases(SchurBuild b) {
+    __shared__ int ws[17];
+    int r0 = 0, r1 = 0;
+    for (int k0 = 0; k0 < b.Fp; k0 += 1024) {
+        const int k = k0 + threadIdx.x;
+        const int n = k < b.Fp ? b.fbase[k + 1] : 0;
+        int t0, t1;
+        const int x0 = wg_excl(n, ws, t0), x1 = wg_excl((n + 63) / 64, ws, t1);
+        if (k < b.Fp) {
+            b.fbase[k + 1] = r0 + x0 + n;
+            b.tbase[k + 1] = r1 + x1 + (n + 63) / 64;
+        }
+        r0 += t0;
+        r1 += t1;
+    }
+    if (threadIdx.x == 0) b.fbase[0] = b.tbase[0] = 0;
+}
+
+// row of every entry: rank among the tile's earlier entries of its frame
+__global__ __launch_bounds__(256) void k_sb_rows(SchurBuild b, int nb) {
+    __shared__ int s_f[256];
+    const int npf = b.btot[3 * nb + 2], q = blockIdx.x * 256 + threadIdx.x;
+    const int f = q < npf ? b.pf_frame[q] : -1;
+    s_f[threadIdx.x] = f;
+    __syncthreads();
+    if (q >= npf) return;
+    int r = 0;
+    for (int k = 0; k < (int)threadIdx.x; k++) r += s_f[k] == f ? 1 : 0;
+    r += b.fbase[f] + b.thist[(long long)f * b.ntile + blockIdx.x];
+    b.pf_row[q] = r;
+    b.row_q[r] = q;
+}
+
+// Items of 64 rows of one frame i (one wave; rows are in point order): with
+// frame j, row l has an item when its point sees j, and its place among the
+// tile's items of (i, j) is the number of earlier rows that do.
+template <bool kFill>
+__global__ __launch_bounds__(256) void k_sb_items(SchurBuild b) {
+    const int tile = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (tile >= b.tbase[b.Fp]) return;
+    int lo = 0, hi = b.Fp - 1;  // the last frame whose first tile is <= tile (frames without rows have none)
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (b.tbase[mid] <= tile) lo = mid; else hi = mid - 1;
+    }
+    const int i = lo, r = b.fbase[i] + 64 * (tile - b.tbase[i]) + lane;
+    const bool on = r < b.fbase[i + 1];
+    int q = on ? b.row_q[r] : 0;
+    const unsigned long long* m = b.mask + (long long)(on ? b.pf_point[q] : 0) * b.words;
+    for (int w = i >> 6; w < b.words; w++) {
+        unsigned long long mw = on ? m[w] : 0;
+        if (w == i >> 6) mw &= ~0ull << (i & 63);
+        for (int j = max(i, 64 * w); j < min(b.Fp, 64 * w + 64); j++) {
+            const bool has = (mw >> (j & 63)) & 1ull;
+            const unsigned long long v = __ballot(has);
+            if constexpr (kFill) {
+                if (v == 0) continue;
+                const int at = b.blk_ptr[block_of(i, j, b.Fp)] + b.tcount[(long long)tile * b.Fp + j];
+                // q walks the point's entries from frame i on
+                if (has) b.items[at + (int)lanes_below(v)] = make_int2(r, b.pf_row[q++]);
+            } else if (lane == 0) {
+                b.tcount[(long long)tile * b.Fp + j] = __popcll(v);
+            }
+        }
+    }
+}
+
+// per block (i, j): the tiles' offsets, and the items before each window of
+// frame i's tiles (win[kWindows]: all of them).  One wave per block.
+__global__ __launch_bounds__(64) void k_sb_blocks(SchurBuild b) {
+    const int i = blockIdx.y, j = blockIdx.x;
+    if (j < i) return;
+    const int t0 = b.tbase[i], nt = b.tbase[i + 1] - t0, lane = threadIdx.x;
+    int* win = b.win + (long long)block_of(i, j, b.Fp) * (kWindows + 1);
+    int run = 0;
+    for (int k0 = 0; k0 < nt; k0 += 64) {
+        const int k = k0 + lane;
+        int* c = b.tcount + (long long)(t0 + k) * b.Fp + j;
+        const int v = k < nt ? *c : 0;
+        int x = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o, 64);
+            if (lane >= o) x += y;
+        }
+        if (k < nt) {
+            *c = run + x - v;
+            // windows whose first tile (w * nt / kWindows) is k
+            for (int w = (int)(((long long)k * kWindows + nt - 1) / nt);
+                 w < kWindows && (int)((long long)w * nt / kWindows) == k; w++)
+                win[w] = run + x - v;
+        }
+        run += __shfl(x, 63, 64);
+    }
+    if (nt == 0 && lane < kWindows) win[lane] = 0;
+    if (lane == 0) win[kWindows] = run;
+}
+
+// the frame-sorted edge lists of k_schur_edges' chunks
+__global__ __launch_bounds__(512) void k_sb_chunks(SchurBuild b) {
+    extern __shared__ int s_cnt[];  // Fp + 1, after it kEdgeChunk frames
+    int* s_f = s_cnt + b.Fp + 1;
+    const bool st = (int)blockIdx.x >= b.nchunk_m;
+    const int k = (int)(st ? blockIdx.x - b.nchunk_m : blockIdx.x) * kEdgeChunk + threadIdx.x;
+    int f = -1;
+    if (k < (st ? b.Ms : b.M)) f = max(b.ef[st ? b.M + k : k], -1);
+    for (int i = threadIdx.x; i <= b.Fp; i += 512) s_cnt[i] = 0;
+    s_f[threadIdx.x] = f;
+    __syncthreads();
+    if (f >= 0) atomicAdd(&s_cnt[f + 1], 1);
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        int run = 0;
+        for (int i0 = 0; i0 <= b.Fp; i0 += 64) {
+            const int i = i0 + threadIdx.x;
+            int x = i <= b.Fp ? s_cnt[i] : 0;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(x, o, 64);
+                if ((int)threadIdx.x >= o) x += y;
+            }
+            if (i <= b.Fp) s_cnt[i] = run + x;
+            run += __shfl(x, 63, 64);
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i <= b.Fp; i += 512)
+        b.eptr[(long long)blockIdx.x * (b.Fp + 1) + i] = (uint16_t)s_cnt[i];
+    if (f >= 0) {
+        int r = s_cnt[f];
+        for (int t = 0; t < (int)threadIdx.x; t++) r += s_f[t] == f ? 1 : 0;
+        b.elist[(long long)blockIdx.x * kEdgeChunk + r] = (uint16_t)threadIdx.x;
+    }
+}
 
 struct SchurArgs {
     const float* planes;    // mono planes (22 of stride S)
@@ -495,14 +811,15 @@ struct SchurArgs {
     const int* pf_obs;      // edge indices grouped by pf
     const int* pf_frame;    // free frame of each pf entry
     const int* pf_row;      // row of each pf entry: rows are ordered by (frame, point)
-    const EdgeChunk* echunk;
+    // chunks of kEdgeChunk consecutive edges, the mono edges' first: the local
+    // numbers of its active edges of free frames, by frame
     const uint16_t* eptr;   // per chunk, Fp + 1: the frames' ranges in its list
-    const uint16_t* elist;
+    const uint16_t* elist;  // per chunk, kEdgeChunk
+    int nchunk_m, Ms;
     const ItemChunk* ichunk;
     const int* blk_chunk;   // per block: its first item chunk (nblk + 1)
     const int2* items;      // (row_i, row_j), by block, then by point
-    const int2* blk_ij;     // block -> (i, j)
-    int P, Fp, nblk, nechunk, esub, nichunk;
+    int P, Fp, nechunk, esub, nichunk;
     float lambda;
     float* prec;            // P x kPointRec
     float* hd;              // P x 3: diagonal of H_ll
@@ -677,13 +994,14 @@ __global__ __launch_bounds__(512) void k_schur_edges(SchurArgs a) {
     constexpr int kWords = 23;  // 1 + 7 * 3 rows, and one to make it odd
     __shared__ float s_e[kEdgeChunk * kWords];
     __shared__ uint16_t s_list[kEdgeChunk];
-    const EdgeChunk C = a.echunk[blockIdx.x];
-    const int rows = C.stereo ? 3 : 2, words = C.stereo ? kWords : 15;
+    const bool st = (int)blockIdx.x >= a.nchunk_m;
+    const int rows = st ? 3 : 2, words = st ? kWords : 15;
+    const int e0 = (int)(st ? blockIdx.x - a.nchunk_m : blockIdx.x) * kEdgeChunk, n = min(kEdgeChunk, (st ? a.Ms : a.M) - e0);
     const uint16_t* ptr = a.eptr + (long long)blockIdx.x * (a.Fp + 1);
     const int nl = ptr[a.Fp];
-    for (int i = threadIdx.x; i < nl; i += 512) s_list[i] = a.elist[C.list0 + i];
-    for (int i = threadIdx.x; i < C.n; i += 512) {
-        const EdgeRef E = edge_ref(a, C.stereo ? a.M + C.e0 + i : C.e0 + i);
+    for (int i = threadIdx.x; i < nl; i += 512) s_list[i] = a.elist[(long long)blockIdx.x * kEdgeChunk + i];
+    for (int i = threadIdx.x; i < n; i += 512) {
+        const EdgeRef E = edge_ref(a, st ? a.M + e0 + i : e0 + i);
         float* o = s_e + i * words;
         o[0] = E.W;
         for (int r = 0; r < rows; r++) {
@@ -885,8 +1203,9 @@ __global__ __launch_bounds__(256) void k_schur_items(SchurArgs a) {
 // a sum, chunk order fixed
 __global__ __launch_bounds__(8 * kItemSums) void k_schur_assemble(SchurArgs a) {
     __shared__ float red[8][kItemSums];
-    const int blk = blockIdx.x, t = threadIdx.x % kItemSums, sl = threadIdx.x / kItemSums;
-    const int2 ij = a.blk_ij[blk];
+    const int2 ij = make_int2((int)blockIdx.y, (int)blockIdx.x);
+    if (ij.y < ij.x) return;
+    const int blk = block_of(ij.x, ij.y, a.Fp), t = threadIdx.x % kItemSums, sl = threadIdx.x / kItemSums;
     const bool diag = ij.x == ij.y;
     float sum = 0.f;
     if (t < (diag ? 27 : 36))
