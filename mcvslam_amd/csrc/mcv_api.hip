@@ -904,6 +904,16 @@ struct mcv_ctx {
         return side;
     }
 
+    // host memory the device writes k_pose_eval's sums to
+    double* sums = nullptr;
+    double* pose_sums() {
+        if (!sums) HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&sums), kPoseSums * sizeof(double), hipHostMallocDefault));
+        return sums;
+    }
+    ~mcv_ctx() {
+        if (sums) (void)hipHostFree(sums);
+    }
+
     const SinCosTables tables() {
         if (!sc.ready) {
             const SinCosHost& h = sincos_host();
@@ -1013,6 +1023,7 @@ struct mcv_ba {
     std::vector<double> h_frames, h_cams;
     double h_scam[6] = {0, 0, 0, 0, 0, 0};
     std::vector<int> point_fixed;                 // empty: no point fixed
+    bool all_points_fixed = false;
     std::vector<uint8_t> active_m, active_s;      // empty: every edge active
     bool robust = true;                           // Huber kernels on
     DevBuf p64, p64_bak, pfix_d, act_m, act_s, xl, xp, partial, dsum, fmax;
@@ -2664,52 +2675,53 @@ static void quat_to_R(const double* q, double R[9]) {
     R[6] = txz - twy; R[7] = tyz + twx; R[8] = 1 - (txx + tyy);
 }
 
-// The (frame, camera) table of the mono edges and the frame poses of the
-// stereo edges from the host FP64 frames and cameras; without the robust
-// kernel the Huber deltas are infinite (w = 1, rho = chi2).
-static void ba_upload_frames(mcv_ba* b, hipStream_t s) {
-    const double* frames = b->h_frames.data();
+// One frame's (frame, camera) records of the mono edges and its pose for the
+// stereo edges from its FP64 state; without the robust kernel the Huber
+// deltas are infinite (w = 1, rho = chi2).
+static void ba_frame_records(const mcv_ba* b, const double* fq, BAPair* pr, FramePose& fp) {
     const double* cams = b->h_cams.data();
+    double Rbw[9];
+    // g2o SE3Quat keeps a normalised quaternion with w >= 0 (se3quat.h:280-285)
+    double q[4] = {fq[0], fq[1], fq[2], fq[3]};
+    double qn = std::sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
+    for (double& v : q) v /= qn;
+    quat_to_R(q, Rbw);
+    const double* tbw = fq + 4;
+    for (int i = 0; i < 9; i++) split(Rbw[i], fp.Rh[i], fp.Rl[i]);
+    for (int i = 0; i < 3; i++) split(tbw[i], fp.th[i], fp.tl[i]);
+    for (int k = 0; k < b->C; k++) {
+        const double* cm = cams + 12 * k;
+        double Rcb[9];
+        double qc[4] = {cm[4], cm[5], cm[6], cm[7]};
+        double qcn = std::sqrt(qc[0] * qc[0] + qc[1] * qc[1] + qc[2] * qc[2] + qc[3] * qc[3]);
+        for (double& v : qc) v /= qcn;
+        quat_to_R(qc, Rcb);
+        const double* tcb = cm + 8;
+        BAPair& P = pr[k];
+        // Tcw = Tcb * Tbw
+        for (int r = 0; r < 3; r++) {
+            for (int cc = 0; cc < 3; cc++) {
+                double v = 0;
+                for (int m = 0; m < 3; m++) v += Rcb[3 * r + m] * Rbw[3 * m + cc];
+                split(v, P.Rh[3 * r + cc], P.Rl[3 * r + cc]);
+            }
+            double tv = tcb[r];
+            for (int m = 0; m < 3; m++) tv += Rcb[3 * r + m] * tbw[m];
+            split(tv, P.th[r], P.tl[r]);
+        }
+        for (int i = 0; i < 9; i++) { P.Rbw[i] = (float)Rbw[i]; P.Rcb[i] = (float)Rcb[i]; }
+        for (int i = 0; i < 3; i++) P.tbw[i] = (float)tbw[i];
+        P.fx = (float)cm[0]; P.fy = (float)cm[1]; P.cx = (float)cm[2]; P.cy = (float)cm[3];
+        P.delta = b->robust ? (float)cm[11] : INFINITY;
+        P.pad[0] = P.pad[1] = P.pad[2] = 0.f;
+    }
+}
+
+// every frame's records to the device
+static void ba_upload_frames(mcv_ba* b, hipStream_t s) {
     std::vector<BAPair> pr((size_t)b->F * b->C);
     std::vector<FramePose> fp(b->F);
-    for (int f = 0; f < b->F; f++) {
-        double Rbw[9];
-        const double* fq = frames + 7 * f;
-        // g2o SE3Quat keeps a normalised quaternion with w >= 0 (se3quat.h:280-285)
-        double q[4] = {fq[0], fq[1], fq[2], fq[3]};
-        double qn = std::sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
-        for (double& v : q) v /= qn;
-        quat_to_R(q, Rbw);
-        const double* tbw = fq + 4;
-        for (int i = 0; i < 9; i++) split(Rbw[i], fp[f].Rh[i], fp[f].Rl[i]);
-        for (int i = 0; i < 3; i++) split(tbw[i], fp[f].th[i], fp[f].tl[i]);
-        for (int k = 0; k < b->C; k++) {
-            const double* cm = cams + 12 * k;
-            double Rcb[9];
-            double qc[4] = {cm[4], cm[5], cm[6], cm[7]};
-            double qcn = std::sqrt(qc[0] * qc[0] + qc[1] * qc[1] + qc[2] * qc[2] + qc[3] * qc[3]);
-            for (double& v : qc) v /= qcn;
-            quat_to_R(qc, Rcb);
-            const double* tcb = cm + 8;
-            BAPair& P = pr[(size_t)f * b->C + k];
-            // Tcw = Tcb * Tbw
-            for (int r = 0; r < 3; r++) {
-                for (int cc = 0; cc < 3; cc++) {
-                    double v = 0;
-                    for (int m = 0; m < 3; m++) v += Rcb[3 * r + m] * Rbw[3 * m + cc];
-                    split(v, P.Rh[3 * r + cc], P.Rl[3 * r + cc]);
-                }
-                double tv = tcb[r];
-                for (int m = 0; m < 3; m++) tv += Rcb[3 * r + m] * tbw[m];
-                split(tv, P.th[r], P.tl[r]);
-            }
-            for (int i = 0; i < 9; i++) { P.Rbw[i] = (float)Rbw[i]; P.Rcb[i] = (float)Rcb[i]; }
-            for (int i = 0; i < 3; i++) P.tbw[i] = (float)tbw[i];
-            P.fx = (float)cm[0]; P.fy = (float)cm[1]; P.cx = (float)cm[2]; P.cy = (float)cm[3];
-            P.delta = b->robust ? (float)cm[11] : INFINITY;
-            P.pad[0] = P.pad[1] = P.pad[2] = 0.f;
-        }
-    }
+    for (int f = 0; f < b->F; f++) ba_frame_records(b, b->h_frames.data() + 7 * (size_t)f, &pr[(size_t)f * b->C], fp[f]);
     upload(b->pairs, pr, s);
     upload(b->fposes, fp, s);
     const double* sc = b->h_scam;
@@ -3164,6 +3176,7 @@ int mcv_ba_set_point_fixed(mcv_ba* b, const int32_t* point_fixed) {
     else b->point_fixed.clear();
     std::vector<uint8_t> f(b->P, 0);
     for (int p = 0; p < b->P && !b->point_fixed.empty(); p++) f[p] = b->point_fixed[p] ? 1 : 0;
+    b->all_points_fixed = std::find(f.begin(), f.end(), 0) == f.end();
     upload(b->pfix_d, f, c->stream);
     HIP_OK(hipStreamSynchronize(c->stream));
     b->schur_ready = false;
@@ -3397,6 +3410,119 @@ int mcv_ba_robust_chi2(mcv_ba* b, double* chi2) {
     API_END
 }
 
+}  // extern "C"
+
+// The frame of a problem whose only unknown is its pose and that fits
+// k_pose_eval, else -1.  (Points without edges would allow it too; the rule
+// asks for what PoseOptimization sets up, every point fixed.)
+static int ba_single_pose(const mcv_ba* b) {
+    const int E = b->M + (b->have_stereo ? b->Ms : 0);
+    if (E == 0 || E > kPoseMaxEdges || b->C > kPoseCams || !b->all_points_fixed) return -1;
+    int frame = -1;
+    for (int f = 0; f < b->F; f++)
+        if (b->fixed.empty() || !b->fixed[f]) {
+            if (frame >= 0) return -1;
+            frame = f;
+        }
+    return frame;
+}
+
+// The optimizer on a problem whose only unknown is one keyframe's pose: the
+// same iterations, trials and rules as mcv_ba_optimize, with one launch and
+// one wait per trial.  k_pose_eval gives chi2, H_pp and b_p of a state at
+// once, so a trial that is accepted has already linearized the next
+// iteration, and one that is rejected leaves the last H_pp and b_p in hand.
+static int ba_optimize_pose(mcv_ba* b, int frame, int iterations, double tau, int max_trials, double* stats,
+                            hipStream_t s) {
+    mcv_ctx* c = b->ctx;
+    const int Ms = b->have_stereo ? b->Ms : 0;
+    PoseArgs a{};
+    a.ob = BAObs{b->uv.as<float2>(), b->pt.as<uint32_t>(), b->pair.as<uint32_t>(), b->isig.as<float>(), b->M};
+    a.so = BAStereoObs{b->s_obs.as<float>(), b->s_pt.as<uint32_t>(), b->s_fr.as<uint32_t>(), b->s_isig.as<float>(), Ms};
+    a.hi = b->phi.as<float4>();
+    a.lo = b->plo.as<float4>();
+    a.pairs = b->pairs.as<BAPair>();
+    a.poses = b->fposes.as<FramePose>();
+    a.act_m = b->active_m.empty() ? nullptr : b->act_m.as<uint8_t>();
+    a.act_s = b->active_s.empty() ? nullptr : b->act_s.as<uint8_t>();
+    a.scam = b->scam;
+    a.frame = frame;
+    a.C = b->C;
+    double* sums = c->pose_sums();
+    a.out = sums;
+    double* fr = &b->h_frames[7 * (size_t)frame];
+    struct Eval {
+        double chi2, S[36], b[6];
+    };
+    auto eval = [&]() {
+        PoseState st{};
+        ba_frame_records(b, fr, st.pair, st.pose);
+        hipLaunchKernelGGL(k_pose_eval, dim3(1), dim3(kPoseThreads), 0, s, a, st);
+        HIP_OK(hipGetLastError());
+        HIP_OK(hipStreamSynchronize(s));
+        Eval e;
+        for (int r = 0, o = 0; r < 6; r++) {
+            for (int k = r; k < 6; k++, o++) e.S[6 * r + k] = e.S[6 * k + r] = sums[o];
+            e.b[r] = sums[o++];
+        }
+        e.chi2 = sums[27];
+        return e;
+    };
+    Eval cur = eval();
+    double lambda = 0, ni = 2;
+    int it_done = 0;
+    for (int it = 0; it < iterations; it++) {
+        if (stats) stats[4 * it] = cur.chi2;
+        if (it == 0) {
+            double mx = 0;
+            for (int k = 0; k < 6; k++) mx = std::max(mx, std::fabs(cur.S[7 * k]));
+            lambda = tau * mx;
+        }
+        double rho = 0;
+        int qmax = 0;
+        do {
+            double fr0[7], S[36], x[6];
+            std::memcpy(fr0, fr, sizeof fr0);
+            std::memcpy(S, cur.S, sizeof S);
+            for (int k = 0; k < 6; k++) S[7 * k] += lambda;
+            const bool ok = mcv_solve_llt(6, S, cur.b, x) == MCV_OK;
+            double scale = 1e-3;
+            Eval e = cur;
+            if (ok) {
+                for (int k = 0; k < 6; k++) scale += x[k] * (lambda * x[k] + cur.b[k]);
+                se3_oplus(fr, x);
+                e = eval();
+            } else {
+                e.chi2 = DBL_MAX;
+            }
+            rho = (cur.chi2 - e.chi2) / scale;
+            if (rho > 0 && std::isfinite(e.chi2)) {
+                lambda *= std::max(1. / 3., std::min(1. - std::pow(2 * rho - 1, 3), 2. / 3.));
+                ni = 2;
+                cur = e;
+            } else {
+                lambda *= ni;
+                ni *= 2;
+                std::memcpy(fr, fr0, sizeof fr0);
+                if (!std::isfinite(lambda)) break;
+            }
+            qmax++;
+        } while (rho < 0 && qmax < max_trials);
+        if (stats) {
+            stats[4 * it + 1] = cur.chi2;
+            stats[4 * it + 2] = lambda;
+            stats[4 * it + 3] = qmax;
+        }
+        it_done++;
+        if (qmax == max_trials || rho == 0 || !std::isfinite(lambda)) break;
+    }
+    ba_upload_frames(b, s);
+    HIP_OK(hipStreamSynchronize(s));
+    return it_done;
+}
+
+extern "C" {
+
 int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, double* stats, int32_t* done) {
     mcv_ctx* c = b ? b->ctx : nullptr;
     API_BEGIN(c)
@@ -3404,6 +3530,14 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
     REQUIRE(iterations >= 0 && max_trials >= 1 && tau >= 0, MCV_ERR_INVALID, "bad optimizer settings");
     c->set_device();
     hipStream_t s = c->stream;
+    const int pose = ba_single_pose(b);
+    if (pose >= 0) {
+        const int it_done = iterations > 0 ? ba_optimize_pose(b, pose, iterations, tau, max_trials, stats, s) : 0;
+        ba_lin_all(b, kBaResidual, s);
+        HIP_OK(hipStreamSynchronize(s));
+        if (done) *done = it_done;
+        return MCV_OK;
+    }
     if (!b->schur_ready) ba_build_schur(b, s);
     const int Fp = b->Fp, n = 6 * Fp, P = b->P;
     // free points without edges need no J_point: a pose-only linearization

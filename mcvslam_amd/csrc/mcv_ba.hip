@@ -147,8 +147,13 @@ __device__ __forceinline__ void ba_store(const BAOut& out, int k, uint32_t off, 
 // residual and J_pose, and a fixed point's J_point is never used).
 constexpr int kBaFull = 0, kBaResidual = 1, kBaPoseOnly = 2;
 
-template <bool kNt>
-__device__ __forceinline__ void ba_edge(int i, const BAIn& in, const BAPair& T, BAOut out, int mode) {
+// e, chi2 and the Huber weight of one edge, and the camera-frame point and
+// reciprocal depth its Jacobians start from
+struct BAEdge {
+    float e0, e1, chi2, w, x, y, iz;
+};
+
+__device__ __forceinline__ BAEdge ba_residual(const BAIn& in, const BAPair& T) {
     const float2 uv = in.uv;
     const float isig = in.isig;
     const float4 ph = in.ph, pl = in.pl;
@@ -172,24 +177,22 @@ __device__ __forceinline__ void ba_edge(int i, const BAIn& in, const BAPair& T, 
     const float chi2 = e0 * (isig * e0) + e1 * (isig * e1);
     const float d2 = T.delta * T.delta;
     const float w = chi2 <= d2 ? 1.f : T.delta * __builtin_amdgcn_rsqf(chi2);
-    const uint32_t off = (uint32_t)i * 4u;
-    ba_store<kNt>(out, 0, off, e0);
-    ba_store<kNt>(out, 1, off, e1);
-    ba_store<kNt>(out, 2, off, chi2);
-    ba_store<kNt>(out, 3, off, w);
-    if (mode == kBaResidual) return;
-    // Jacobians (FP32).  Jpi = [[fx/z, 0, -fx x/z^2], [0, fy/z, -fy y/z^2]]
-    const float x = C[0].hi, y = C[1].hi;
-    const float j00 = T.fx * iz, j02 = -T.fx * x * (iz * iz);
-    const float j11 = T.fy * iz, j12 = -T.fy * y * (iz * iz);
-    // J_point = -Jpi R_cw
-    if (mode != kBaPoseOnly) {
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            ba_store<kNt>(out, 16 + k, off, -(j00 * T.Rh[k] + j02 * T.Rh[6 + k]));
-            ba_store<kNt>(out, 19 + k, off, -(j11 * T.Rh[3 + k] + j12 * T.Rh[6 + k]));
-        }
-    }
+    return BAEdge{e0, e1, chi2, w, C[0].hi, C[1].hi, iz};
+}
+
+// J_pose (2x6) of one edge (FP32).  Jpi = [[fx/z, 0, -fx x/z^2], [0, fy/z, -fy y/z^2]]:
+// j00, j02, j11, j12
+__device__ __forceinline__ void ba_jpi(const BAEdge& E, const BAPair& T, float& j00, float& j02, float& j11, float& j12) {
+    j00 = T.fx * E.iz;
+    j02 = -T.fx * E.x * (E.iz * E.iz);
+    j11 = T.fy * E.iz;
+    j12 = -T.fy * E.y * (E.iz * E.iz);
+}
+
+__device__ __forceinline__ void ba_jpose(const BAIn& in, const BAEdge& E, const BAPair& T, float (&Jp)[12]) {
+    float j00, j02, j11, j12;
+    ba_jpi(E, T, j00, j02, j11, j12);
+    const float4 ph = in.ph;
     // P_b = R_bw P_w + t_bw; M = Jpi R_cb; J_pose = [M [P_b]x | -M]
     float pb[3];
 #pragma unroll
@@ -200,7 +203,6 @@ __device__ __forceinline__ void ba_edge(int i, const BAIn& in, const BAPair& T, 
         Mr[k] = j00 * T.Rcb[k] + j02 * T.Rcb[6 + k];
         Mr[3 + k] = j11 * T.Rcb[3 + k] + j12 * T.Rcb[6 + k];
     }
-    float Jp[12];
 #pragma unroll
     for (int r = 0; r < 2; r++) {
         const float m0 = Mr[3 * r], m1 = Mr[3 * r + 1], m2 = Mr[3 * r + 2];
@@ -212,6 +214,29 @@ __device__ __forceinline__ void ba_edge(int i, const BAIn& in, const BAPair& T, 
         Jp[6 * r + 4] = -m1;
         Jp[6 * r + 5] = -m2;
     }
+}
+
+template <bool kNt>
+__device__ __forceinline__ void ba_edge(int i, const BAIn& in, const BAPair& T, BAOut out, int mode) {
+    const BAEdge E = ba_residual(in, T);
+    const uint32_t off = (uint32_t)i * 4u;
+    ba_store<kNt>(out, 0, off, E.e0);
+    ba_store<kNt>(out, 1, off, E.e1);
+    ba_store<kNt>(out, 2, off, E.chi2);
+    ba_store<kNt>(out, 3, off, E.w);
+    if (mode == kBaResidual) return;
+    // J_point = -Jpi R_cw
+    if (mode != kBaPoseOnly) {
+        float j00, j02, j11, j12;
+        ba_jpi(E, T, j00, j02, j11, j12);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            ba_store<kNt>(out, 16 + k, off, -(j00 * T.Rh[k] + j02 * T.Rh[6 + k]));
+            ba_store<kNt>(out, 19 + k, off, -(j11 * T.Rh[3 + k] + j12 * T.Rh[6 + k]));
+        }
+    }
+    float Jp[12];
+    ba_jpose(in, E, T, Jp);
 #pragma unroll
     for (int k = 0; k < 12; k++) ba_store<kNt>(out, 4 + k, off, Jp[k]);
 }
@@ -303,15 +328,15 @@ struct BAStereoObs {
     int M;
 };
 
-__global__ __launch_bounds__(256) void k_ba_stereo_linearize(BAStereoObs ob, const float4* __restrict__ pts_hi,
-                                                             const float4* __restrict__ pts_lo,
-                                                             const FramePose* __restrict__ poses, StereoCam cam,
-                                                             BAOut out, int mode) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ob.M) return;
+struct StereoEdge {
+    float e[3], chi2, w, x, y, z;
+};
+
+__device__ __forceinline__ StereoEdge stereo_residual(const BAStereoObs& ob, int i, const float4* __restrict__ pts_hi,
+                                                      const float4* __restrict__ pts_lo, const FramePose& T,
+                                                      const StereoCam& cam) {
     const float ou = ob.obs[3 * i], ov = ob.obs[3 * i + 1], our = ob.obs[3 * i + 2];
     const float isig = ob.isig[i];
-    const FramePose& T = poses[ob.fr[i]];
     const uint32_t pi = ob.pt[i];
     const float4 ph = pts_hi[pi], pl = pts_lo[pi];
     const f2 P[3] = {{ph.x, pl.x}, {ph.y, pl.y}, {ph.z, pl.z}};
@@ -335,18 +360,15 @@ __global__ __launch_bounds__(256) void k_ba_stereo_linearize(BAStereoObs ob, con
     const float e0 = eu.hi + eu.lo, e1 = ev.hi + ev.lo, e2 = er.hi + er.lo;
     const float chi2 = isig * (e0 * e0 + e1 * e1 + e2 * e2);
     const float w = chi2 <= cam.delta * cam.delta ? 1.f : cam.delta * __builtin_amdgcn_rsqf(chi2);
-    const long long S = out.stride;
-    float* o = out.planes + i;
-    o[0] = e0;
-    o[S] = e1;
-    o[2 * S] = e2;
-    o[3 * S] = chi2;
-    o[4 * S] = w;
-    if (mode == kBaResidual) return;
-    const float x = C[0].hi, y = C[1].hi, z = C[2].hi;
-    const float iz = __builtin_amdgcn_rcpf(z), iz2 = iz * iz;
+    return StereoEdge{{e0, e1, e2}, chi2, w, C[0].hi, C[1].hi, C[2].hi};
+}
+
+// J_pose (3x6) of a stereo edge
+__device__ __forceinline__ void stereo_jpose(const StereoEdge& E, const StereoCam& cam, float (&J)[18]) {
+    const float x = E.x, y = E.y;
+    const float iz = __builtin_amdgcn_rcpf(E.z), iz2 = iz * iz;
     const float fx = cam.fx, fy = cam.fy, bf = cam.bf;
-    float J0[6], J1[6], J2[6];
+    float *J0 = J, *J1 = J + 6, *J2 = J + 12;
     J0[0] = x * y * iz2 * fx;
     J0[1] = -(1.f + x * x * iz2) * fx;
     J0[2] = y * iz * fx;
@@ -365,13 +387,32 @@ __global__ __launch_bounds__(256) void k_ba_stereo_linearize(BAStereoObs ob, con
     J2[3] = J0[3];
     J2[4] = 0.f;
     J2[5] = J0[5] - bf * iz2;
+}
+
+__global__ __launch_bounds__(256) void k_ba_stereo_linearize(BAStereoObs ob, const float4* __restrict__ pts_hi,
+                                                             const float4* __restrict__ pts_lo,
+                                                             const FramePose* __restrict__ poses, StereoCam cam,
+                                                             BAOut out, int mode) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= ob.M) return;
+    const FramePose& T = poses[ob.fr[i]];
+    const StereoEdge E = stereo_residual(ob, i, pts_hi, pts_lo, T, cam);
+    const long long S = out.stride;
+    float* o = out.planes + i;
+    o[0] = E.e[0];
+    o[S] = E.e[1];
+    o[2 * S] = E.e[2];
+    o[3 * S] = E.chi2;
+    o[4 * S] = E.w;
+    if (mode == kBaResidual) return;
+    float J[18];
+    stereo_jpose(E, cam, J);
 #pragma unroll
-    for (int k = 0; k < 6; k++) {
-        o[(5 + k) * S] = J0[k];
-        o[(11 + k) * S] = J1[k];
-        o[(17 + k) * S] = J2[k];
-    }
+    for (int k = 0; k < 18; k++) o[(5 + k) * S] = J[k];
     if (mode == kBaPoseOnly) return;
+    const float x = E.x, y = E.y;
+    const float iz = __builtin_amdgcn_rcpf(E.z), iz2 = iz * iz;
+    const float fx = cam.fx, fy = cam.fy, bf = cam.bf;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
         const float a = -fx * T.Rh[k] * iz + fx * x * T.Rh[6 + k] * iz2;
@@ -1312,6 +1353,122 @@ __global__ __launch_bounds__(256) void k_ba_rho_sum(const float* chi2, const uin
     }
     const double t = block_sum_d(v, red);
     if (threadIdx.x == 0) partial[blockIdx.x] = t;
+}
+
+// One evaluation of a problem whose only unknown is one keyframe's pose
+// (every point fixed, every other frame fixed): from the frame's state, sum of
+// rho(chi2), H_pp (upper triangle by rows, each row followed by b_p's entry)
+// in FP64 sums of the edges' FP32 terms, in a fixed order, written to host
+// memory.  Linearization, robust chi2 and normal equations in one launch of
+// one workgroup: a frame has at most a few thousand edges, so a trial of the
+// optimizer is bound by launches and by the host's wait (12 launches and 3
+// waits, 0.2 ms, before; see mcv_ba_optimize), not by the edges' arithmetic.
+constexpr int kPoseThreads = 1024;
+constexpr int kPoseCams = 8;       // cameras whose records fit the kernel arguments
+constexpr int kPoseMaxEdges = 16384;
+constexpr int kPoseSums = 28;
+
+struct PoseState {
+    BAPair pair[kPoseCams];  // (frame, camera) records of the free frame
+    FramePose pose;
+};
+
+struct PoseArgs {
+    BAObs ob;
+    BAStereoObs so;
+    const float4 *hi, *lo;
+    const BAPair* pairs;     // the other frames'
+    const FramePose* poses;
+    const uint8_t *act_m, *act_s;  // or null
+    StereoCam scam;
+    int frame, C;            // the free frame
+    double* out;             // kPoseSums
+};
+
+template <int kCtrl, int N>
+__device__ __forceinline__ void sum_fold_d(double* v, int hi) {
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const double send = hi ? v[k] : v[k + N], keep = hi ? v[k + N] : v[k];
+        const int lo32 = __builtin_amdgcn_update_dpp(0, __double2loint(send), kCtrl, 0xF, 0xF, false);
+        const int hi32 = __builtin_amdgcn_update_dpp(0, __double2hiint(send), kCtrl, 0xF, 0xF, false);
+        v[k] = keep + __hiloint2double(hi32, lo32);
+    }
+}
+
+__global__ __launch_bounds__(kPoseThreads) void k_pose_eval(PoseArgs a, PoseState st) {
+    __shared__ float s_state[sizeof(PoseState) / 4];
+    __shared__ double s_sum[kPoseThreads / 64][32];
+    for (int k = threadIdx.x; k < (int)(sizeof(PoseState) / 4); k += kPoseThreads)
+        s_state[k] = reinterpret_cast<const float*>(&st)[k];
+    __syncthreads();
+    const PoseState& S = *reinterpret_cast<const PoseState*>(s_state);
+    double acc[32];
+#pragma unroll
+    for (int k = 0; k < 32; k++) acc[k] = 0.0;
+    for (int i = threadIdx.x; i < a.ob.M; i += kPoseThreads) {
+        if (a.act_m && !a.act_m[i]) continue;
+        BAIn in;
+        ba_load_obs(i, a.ob, in);
+        ba_load_point(a.hi, a.lo, in);
+        const int f = (int)in.pair / a.C, c = (int)in.pair - f * a.C;
+        const BAPair& T = f == a.frame ? S.pair[c] : a.pairs[in.pair];
+        const BAEdge E = ba_residual(in, T);
+        acc[27] += huber_rho(E.chi2, T.delta);
+        if (f != a.frame) continue;
+        float J[12];
+        ba_jpose(in, E, T, J);
+        const float W = E.w * in.isig;
+        int o = 0;
+#pragma unroll
+        for (int r = 0; r < 6; r++) {
+#pragma unroll
+            for (int k = r; k < 6; k++, o++) acc[o] += (double)(W * (J[r] * J[k])) + (double)(W * (J[6 + r] * J[6 + k]));
+            acc[o++] -= (double)(W * (J[r] * E.e0)) + (double)(W * (J[6 + r] * E.e1));
+        }
+    }
+    for (int i = threadIdx.x; i < a.so.M; i += kPoseThreads) {
+        if (a.act_s && !a.act_s[i]) continue;
+        const int f = (int)a.so.fr[i];
+        const FramePose& T = f == a.frame ? S.pose : a.poses[f];
+        const StereoEdge E = stereo_residual(a.so, i, a.hi, a.lo, T, a.scam);
+        acc[27] += huber_rho(E.chi2, a.scam.delta);
+        if (f != a.frame) continue;
+        float J[18];
+        stereo_jpose(E, a.scam, J);
+        const float W = E.w * a.so.isig[i];
+        int o = 0;
+#pragma unroll
+        for (int r = 0; r < 6; r++) {
+#pragma unroll
+            for (int k = r; k < 6; k++, o++)
+                acc[o] += (double)(W * (J[r] * J[k])) + (double)(W * (J[6 + r] * J[6 + k])) +
+                          (double)(W * (J[12 + r] * J[12 + k]));
+            acc[o++] -= (double)(W * (J[r] * E.e[0])) + (double)(W * (J[6 + r] * E.e[1])) + (double)(W * (J[12 + r] * E.e[2]));
+        }
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    sum_fold_d<0x140, 16>(acc, lane & 8);
+    sum_fold_d<0x141, 8>(acc, lane & 4);
+    sum_fold_d<0x1B, 4>(acc, lane & 2);
+    sum_fold_d<0xB1, 2>(acc, lane & 1);
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        acc[k] += __shfl_xor(acc[k], 16, 64);
+        acc[k] += __shfl_xor(acc[k], 32, 64);
+    }
+    if (lane < 16) {
+        const int o = (lane & 8 ? 16 : 0) + (lane & 4 ? 8 : 0) + (lane & 2 ? 4 : 0) + (lane & 1 ? 2 : 0);
+        s_sum[wave][o] = acc[0];
+        s_sum[wave][o + 1] = acc[1];
+    }
+    __syncthreads();
+    if (threadIdx.x < kPoseSums) {
+        double v = 0.0;
+#pragma unroll
+        for (int w = 0; w < kPoseThreads / 64; w++) v += s_sum[w][threadIdx.x];
+        a.out[threadIdx.x] = v;
+    }
 }
 
 // out[0] = sum of partial[0 .. n) in a fixed order (one workgroup)

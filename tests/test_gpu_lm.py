@@ -207,3 +207,45 @@ def test_pose_optimization_rounds_vs_oracle(gpu_ctx):
     assert dt < 1e-5 and dq < 1e-6
     assert nd <= max(2, n_init // 1000)
     assert (am == 0).sum() > 0
+
+
+@pytest.mark.parametrize("n_kf,n_points,obs,stereo_frac", [(1, 40, 25, 0.9), (1, 1500, 1024, 0.0), (3, 900, 2049, 0.9),
+                                                           (1, 9000, 7000, 0.5)])
+@pytest.mark.parametrize("robust", [True, False])
+def test_single_pose_route_vs_oracle_and_general_route(gpu_ctx, n_kf, n_points, obs, stereo_frac, robust):
+    """One free keyframe, every point fixed: the one-launch trials against the
+    oracle LM and against the general route, which the same problem takes when
+    a point without edges is left free.  Edge counts around the workgroup's
+    1024 threads, other keyframes fixed, inactive edges.  Tolerances as
+    test_pose_optimization_rounds_vs_oracle, whose sums are as wide."""
+    lp = synth.local_ba_problem(seed=76, n_kf=n_kf, n_points=n_points, target_obs=obs, stereo_frac=stereo_frac,
+                                fixed_point_frac=1.0, perturb_pose=0.0)
+    mono, stereo = lp.mono, lp.stereo if len(lp.stereo.obs_pt) else None
+    free = n_kf - 1
+    mono.frame_fixed = np.ones(n_kf, np.int32)
+    mono.frame_fixed[free] = 0
+    f = oracle.se3_oplus(mono.frames[free], np.random.default_rng(5).normal(0, 0.01, 6))
+    mono.frames[free] = f
+    mono.points = np.concatenate([mono.points, [[0.0, 0.0, 5.0]]])       # seen by no edge
+    am = (np.random.default_rng(6).random(len(mono.obs_pt)) > 0.1).astype(np.uint8)
+    out = []
+    for last in (1, 0):
+        pfix = np.ones(len(mono.points), np.int32)
+        pfix[-1] = last
+        lin = local_ba_linearizer(mono, stereo, pfix, ctx=gpu_ctx)
+        lin.set_active(am)
+        lin.set_robust(robust)
+        stats, n = lin.optimize(6)
+        out.append((stats, lin.get_state()[1], lin.outliers(stereo=stereo is not None)))
+        lin.close()
+    _, frs, ost, _, _ = oracle.ba_lm(mono, stereo, iterations=6, point_fixed=np.ones(len(mono.points), np.int32),
+                                     active=am, robust=robust)
+    for stats, got, _ in out:
+        assert np.abs(got[free, 4:] - frs[free, 4:]).max() < 1e-5
+        assert np.abs(got[free, :4] - frs[free, :4]).max() < 1e-6
+        np.testing.assert_array_equal(np.delete(got, free, 0), np.delete(mono.frames, free, 0))
+        assert abs(stats[0, 0] - ost[0, 0]) < 1e-5 * ost[0, 0]
+        assert abs(stats[-1, 1] - ost[-1, 1]) < 1e-5 * ost[-1, 1]
+    for a, b in zip(out[0][2], out[1][2]):
+        if a is not None:
+            assert (a != b).sum() <= max(2, len(a) // 1000)
