@@ -76,6 +76,87 @@ __device__ void bitonic_sort(T* a, int n2) {
         }
     }
 }
+
+// the value of lane ^ M (64-bit), by DPP within rows of 16
+template <int kCtrl>
+__device__ __forceinline__ unsigned long long dpp_u64(unsigned long long v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, kCtrl, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), kCtrl, 0xF, 0xF, false);
+    return ((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo;
+}
+
+template <int M>
+__device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
+    if constexpr (M == 1) return dpp_u64<0xB1>(v);
+    else if constexpr (M == 2) return dpp_u64<0x4E>(v);
+    else if constexpr (M == 4) return dpp_u64<0x1B>(dpp_u64<0x141>(v));  // lane ^ 7, then ^ 3
+    else if constexpr (M == 8) return dpp_u64<0x128>(v);                 // row rotation by 8
+    else return (unsigned long long)__shfl_xor((long long)v, M, 64);
+}
+
+// One stage (k = K, distance J) of the bitonic network below: v[r] is element
+// threadIdx.x * R + r.
+template <int kThreads, int R, int K, int J>
+__device__ __forceinline__ void sort_stage(unsigned long long (&v)[R], unsigned long long* a) {
+    const int t = threadIdx.x;
+    if constexpr (J < R) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            if ((r & J) == 0) {
+                const bool up = K < R ? (r & K) == 0 : ((t * R) & K) == 0;
+                const bool swap = (v[r] > v[r | J]) == up;
+                const unsigned long long x = v[r], y = v[r | J];
+                v[r] = swap ? y : x;
+                v[r | J] = swap ? x : y;
+            }
+    } else {
+        constexpr int M = J / R;  // thread distance
+        const bool keep_min = (((t * R) & K) == 0) == ((t & M) == 0);
+        unsigned long long o[R];
+        if constexpr (M < 64) {
+#pragma unroll
+            for (int r = 0; r < R; r++) o[r] = lane_xor<M>(v[r]);
+        } else {
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < R; r++) a[t + r * kThreads] = v[r];
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < R; r++) o[r] = a[(t ^ M) + r * kThreads];
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r] = (v[r] < o[r]) == keep_min ? v[r] : o[r];
+    }
+}
+
+template <int kThreads, int R, int K, int J>
+__device__ __forceinline__ void sort_merge(unsigned long long (&v)[R], unsigned long long* a) {
+    sort_stage<kThreads, R, K, J>(v, a);
+    if constexpr (J > 1) sort_merge<kThreads, R, K, J / 2>(v, a);
+}
+
+template <int kThreads, int R, int K>
+__device__ __forceinline__ void sort_steps(unsigned long long (&v)[R], unsigned long long* a) {
+    if constexpr (K > 2) sort_steps<kThreads, R, K / 2>(v, a);
+    sort_merge<kThreads, R, K, K / 2>(v, a);
+}
+
+// Ascending sort of kThreads * R distinct-or-equal keys in LDS by the whole
+// workgroup, R keys of a thread in registers: of the network's stages only
+// those that pair keys of different waves go through LDS with barriers (10 of
+// 78 for 4096 keys on 1024 threads), the others are register or cross-lane
+// moves.  4096 keys: 69 us with every stage in LDS (bitonic_sort).
+template <int kThreads, int R>
+__device__ void block_sort(unsigned long long* a) {
+    unsigned long long v[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) v[r] = a[threadIdx.x + r * kThreads];  // any assignment: it is sorted next
+    sort_steps<kThreads, R, kThreads * R>(v, a);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; r++) a[threadIdx.x * R + r] = v[r];
+    __syncthreads();
+}
 #endif
 
 // ---------------------------------------------------------------------------

@@ -1018,7 +1018,9 @@ __global__ __launch_bounds__(kOctThreads) void k_octree_build(OrbGlobals g, cons
         __syncthreads();
     }
     // 2. keys = path << 24 | candidate index; sort
-    for (int i = threadIdx.x; i < n2; i += kOctThreads) {
+    // the LDS sort takes whole multiples of the workgroup
+    const int npad = n <= kCap ? max(n2, kOctThreads) : n2;
+    for (int i = threadIdx.x; i < npad; i += kOctThreads) {
         unsigned long long k = ~0ull;
         if (i < n) {
             const uint32_t r = g.lvl_cand[L.cand_base + i];
@@ -1028,7 +1030,17 @@ __global__ __launch_bounds__(kOctThreads) void k_octree_build(OrbGlobals g, cons
         keys[i] = k;
     }
     __syncthreads();
-    bitonic_sort<unsigned long long, (kCap / 2 + kOctThreads - 1) / kOctThreads>(keys, n2);
+    if (n > kCap) {
+        bitonic_sort<unsigned long long, (kCap / 2 + kOctThreads - 1) / kOctThreads>(keys, n2);
+    } else {
+        switch (npad / kOctThreads) {
+        case 1: block_sort<kOctThreads, 1>(s_keys); break;
+        case 2: block_sort<kOctThreads, 2>(s_keys); break;
+        case 4: block_sort<kOctThreads, 4>(s_keys); break;
+        default:
+            if constexpr (kCap / kOctThreads >= 8) block_sort<kOctThreads, 8>(s_keys);
+        }
+    }
     // 3. divergence depth of each sorted position
     for (int i = threadIdx.x; i < n; i += kOctThreads)
         dv[i] = (uint8_t)(i == 0 ? 0 : code_div(keys[i] >> 24, keys[i - 1] >> 24));

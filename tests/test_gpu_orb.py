@@ -173,3 +173,40 @@ def test_orb_batch_seeds(orb_default):
         out = orb_default.extract_batch_dev(dev, graph=graph, seeds=seeds)
         torch.cuda.synchronize()
         _check_batch(orb_default, imgs, *out, seeds=seeds)
+
+
+@pytest.fixture(scope="module")
+def own_ctx():
+    """A context whose extractor settings no other test shares."""
+    from mcvslam_amd import Context
+    ctx = Context(0)
+    yield ctx
+    ctx.close()
+
+
+def _check_distinct(orb, imgs, repeats):
+    """A batch of `imgs` repeated, each distinct image's first and last copy
+    against the oracle."""
+    import torch
+    dev = [torch.from_numpy(im).cuda() for im in imgs]
+    kps, desc, counts = orb.extract_batch_dev(dev * repeats, graph=False)
+    torch.cuda.synchronize()
+    n = len(imgs)
+    for lo in (0, n * (repeats - 1)):
+        _check_batch(orb, imgs, kps[lo:lo + n], desc[lo:lo + n], counts[lo:lo + n])
+
+
+@pytest.mark.parametrize("levels,repeats", [(8, 1), (8, 49)])
+def test_orb_octree_candidate_counts(own_ctx, levels, repeats):
+    """Octree builds over candidate counts from none to more than the sort
+    holds in LDS (a flat image, one with a single blob, noise), by the 1024-
+    and the 256-thread builds (2 and 98 images: 16 and 784 levels)."""
+    orb = ORB(2000, 1.2, levels, 20, 7, ctx=own_ctx)
+    rng = np.random.default_rng(5)
+    dot = np.full((250, 300), 90, np.uint8)
+    dot[80:84, 100:104] = 250
+    noise = rng.integers(0, 256, (240, 280), dtype=np.uint8)
+    _check_distinct(orb, [dot, noise], repeats)
+    if repeats == 1:
+        _check_distinct(orb, [np.full((250, 300), 128, np.uint8), synth.blob_image(8, 400, 300),
+                              rng.integers(0, 256, (720, 960), dtype=np.uint8)], 1)
