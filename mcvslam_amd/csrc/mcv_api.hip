@@ -438,11 +438,13 @@ struct ImageSpec {
 
 // A batch plan: geometry and work tables for a list of images.
 struct OrbPlan {
-    int n_images = 0, nlevels = 0, cap = 0, n_slots = 0;
+    int n_images = 0, nlevels = 0, cap = 0, n_slots = 0, strip_h = kStripH;
     std::vector<LevelDesc> lv;
     std::vector<CellDesc> cells;
     std::vector<Strip> strips;
     std::vector<int> strip_begin;  // per level index l: [strip_begin[l], strip_begin[l+1])
+    std::vector<Strip> rstrips;    // k_resize's strips
+    std::vector<int> rstrip_begin;
     std::vector<int2> coef;
     std::vector<int> slot_lvl;
     std::vector<float> seeds;
@@ -452,7 +454,7 @@ struct OrbPlan {
     std::vector<int> heap_order;  // levels by feature target, largest first
     std::vector<int> build_levels;  // large levels (1024-thread octree build) first, then the rest
     int n_build_large = 0;
-    DevBuf d_heap_order, d_build_levels, d_lv, d_cells, d_strips, d_coef, d_slot, d_seeds, d_pyr, d_blur, d_score, d_cell_cand, d_cell_n, d_lvl_cand, d_oct,
+    DevBuf d_heap_order, d_build_levels, d_lv, d_cells, d_strips, d_rstrips, d_coef, d_slot, d_seeds, d_pyr, d_blur, d_score, d_cell_cand, d_cell_n, d_lvl_cand, d_oct,
         d_pool, d_used, d_nodes, d_perm, d_src, d_stride;
     hipGraphExec_t graph = nullptr;
     // the captured graph bakes in every output pointer and the capacity
@@ -575,14 +577,17 @@ struct OrbPlan {
         cap = max_slots_img;
         heap_cap = 16;
         for (const LevelDesc& d : lv) heap_cap = std::max(heap_cap, std::max(d.nfeat, d.n_ini) + 16);
-        // levels of at least kOctLargePixels pixels (the most FAST
-        // candidates) get 1024-thread octree workgroups
+        // octree workgroups of 1024 threads: every level of a small batch, the
+        // large levels (the most FAST candidates) of a larger one
         build_levels.clear();
+        auto large = [&](const LevelDesc& d) {
+            return (int)lv.size() <= kOctWideLevels || (long long)d.w * d.h >= kOctLargePixels;
+        };
         for (size_t k = 0; k < lv.size(); k++)
-            if ((long long)lv[k].w * lv[k].h >= kOctLargePixels) build_levels.push_back((int)k);
+            if (large(lv[k])) build_levels.push_back((int)k);
         n_build_large = (int)build_levels.size();
         for (size_t k = 0; k < lv.size(); k++)
-            if ((long long)lv[k].w * lv[k].h < kOctLargePixels) build_levels.push_back((int)k);
+            if (!large(lv[k])) build_levels.push_back((int)k);
         // largest levels first in each launch: when a launch takes more than
         // one round of workgroups, the later rounds get the small levels
         auto by_area = [&](int a, int b) { return (long long)lv[a].w * lv[a].h > (long long)lv[b].w * lv[b].h; };
@@ -593,16 +598,25 @@ struct OrbPlan {
         std::stable_sort(heap_order.begin(), heap_order.end(),
                          [&](int a, int b) { return lv[a].nfeat > lv[b].nfeat; });
         // strips grouped by level index, then image
-        strip_begin.assign(nlevels + 1, 0);
-        for (int l = 0; l < nlevels; l++) {
-            strip_begin[l] = (int)strips.size();
-            for (int i = 0; i < n_images; i++) {
-                const LevelDesc& d = lv[lvl_of[i][l]];
-                for (int y = 0; y < d.h; y += kStripH)
-                    for (int x = 0; x < d.w; x += kStripW) strips.push_back(Strip{lvl_of[i][l], x, y});
+        long long tall = 0;
+        for (const LevelDesc& d : lv)
+            tall += (long long)((d.w + kStripW - 1) / kStripW) * ((d.h + kStripH - 1) / kStripH);
+        strip_h = tall < kStripMin ? kStripHLow : kStripH;
+        auto cut = [&](int sh, std::vector<Strip>& out, std::vector<int>& begin) {
+            out.clear();
+            begin.assign(nlevels + 1, 0);
+            for (int l = 0; l < nlevels; l++) {
+                begin[l] = (int)out.size();
+                for (int i = 0; i < n_images; i++) {
+                    const LevelDesc& d = lv[lvl_of[i][l]];
+                    for (int y = 0; y < d.h; y += sh)
+                        for (int x = 0; x < d.w; x += kStripW) out.push_back(Strip{lvl_of[i][l], x, y});
+                }
             }
-        }
-        strip_begin[nlevels] = (int)strips.size();
+            begin[nlevels] = (int)out.size();
+        };
+        cut(strip_h, strips, strip_begin);
+        cut(kResizeH, rstrips, rstrip_begin);
         // k_resize: the source bytes of 4 adjacent outputs (both taps)
         // lie in the 12 bytes from the first one's aligned word
         for (const LevelDesc& d : lv) {
@@ -624,6 +638,7 @@ struct OrbPlan {
         upload(d_lv, lv, s);
         upload(d_cells, cells, s);
         upload(d_strips, strips, s);
+        upload(d_rstrips, rstrips, s);
         upload(d_heap_order, heap_order, s);
         upload(d_build_levels, build_levels, s);
         upload(d_coef, coef, s);
@@ -730,10 +745,15 @@ void OrbPlan::enqueue(const OrbConfig& c, const SinCosTables& tb, hipStream_t s,
     taps.hi3 = (uint32_t)c.gauss[4] | (uint32_t)c.gauss[5] << 8 | (uint32_t)c.gauss[6] << 16;
     const int ns = (int)strips.size();
     auto blur = [&](hipStream_t bs) {
-        if (tune.blur & 1)
-            hipLaunchKernelGGL(k_blur<true>, strip_grid(ns), dim3(256), 0, bs, st, ns, g.lv, g.pyr, g.blur, taps);
+        if (strip_h == kStripHLow)
+            hipLaunchKernelGGL((k_blur<false, kStripHLow>), strip_grid(ns), dim3(256), 0, bs, st, ns, g.lv, g.pyr,
+                               g.blur, taps);
+        else if (tune.blur & 1)
+            hipLaunchKernelGGL((k_blur<true, kStripH>), strip_grid(ns), dim3(256), 0, bs, st, ns, g.lv, g.pyr, g.blur,
+                               taps);
         else
-            hipLaunchKernelGGL(k_blur<false>, strip_grid(ns), dim3(256), 0, bs, st, ns, g.lv, g.pyr, g.blur, taps);
+            hipLaunchKernelGGL((k_blur<false, kStripH>), strip_grid(ns), dim3(256), 0, bs, st, ns, g.lv, g.pyr, g.blur,
+                               taps);
         mark("k_blur");
     };
     // dynamic LDS: the heap (8 B per entry), then the node-table prefix (8 B per entry)
@@ -785,7 +805,7 @@ void OrbPlan::enqueue(const OrbConfig& c, const SinCosTables& tb, hipStream_t s,
         mark("k_zero_words");
         const int n0 = strip_begin[1] - strip_begin[0];
         if (n0 > 0) {
-            hipLaunchKernelGGL(k_copy_level0, strip_grid(n0), dim3(256), 0, s, st, n0, g.lv,
+            hipLaunchKernelGGL(k_copy_level0, strip_grid(n0), dim3(256), 0, s, st, n0, strip_h, g.lv,
                                d_src.as<const uint8_t*>(), d_stride.as<int>(), g.pyr);
             mark("k_copy_level0");
         }
@@ -793,10 +813,10 @@ void OrbPlan::enqueue(const OrbConfig& c, const SinCosTables& tb, hipStream_t s,
     // levels l0 .. l1 - 1, each from the one before
     auto resize_levels = [&](int l0, int l1) {
         for (int l = std::max(l0, 1); l < l1; l++) {
-            const int n = strip_begin[l + 1] - strip_begin[l];
+            const int n = rstrip_begin[l + 1] - rstrip_begin[l];
             if (n > 0) {
-                hipLaunchKernelGGL(k_resize, dim3(xcd_grid(n)), dim3(64), 0, s, st + strip_begin[l], n, g.lv,
-                                   d_coef.as<int2>(), g.pyr);
+                hipLaunchKernelGGL(k_resize, dim3(xcd_grid(n)), dim3(64), 0, s,
+                                   d_rstrips.as<Strip>() + rstrip_begin[l], n, g.lv, d_coef.as<int2>(), g.pyr);
                 mark("k_resize");
             }
         }
@@ -805,7 +825,7 @@ void OrbPlan::enqueue(const OrbConfig& c, const SinCosTables& tb, hipStream_t s,
     auto fast = [&](int l0, int l1) {
         const int b0 = strip_begin[l0], n = strip_begin[l1] - b0;
         if (n > 0) {
-            hipLaunchKernelGGL(k_fast_score, strip_grid(n), dim3(256), 0, s, st + b0, n, g.lv, g.pyr, g.score,
+            hipLaunchKernelGGL(k_fast_score, strip_grid(n), dim3(256), 0, s, st + b0, n, strip_h, g.lv, g.pyr, g.score,
                                std::min(g.ini_th, g.min_th));
             mark("k_fast_score");
         }

@@ -24,7 +24,7 @@ namespace mcv {
 
 struct Strip {
     int lvl;     // LevelDesc index
-    int x0, y0;  // strip origin: kStripW x kStripH pixels, one wave
+    int x0, y0;  // strip origin: kStripW x the plan's strip height in pixels, one wave
 };
 
 struct BlurTaps {
@@ -77,8 +77,9 @@ __device__ __forceinline__ int reflect101(int i, int n) {
 }
 
 // ---------------------------------------------------------------------------
-// Strip kernels: a wave owns kStripW x kStripH pixels of one level, each lane
-// 4 horizontally adjacent pixels (one u32 of a pitched row).
+// Strip kernels: a wave owns kStripW x sh pixels of one level (sh: the plan's
+// strip height), each lane 4 horizontally adjacent pixels (one u32 of a
+// pitched row).
 // kXcd: consecutive workgroups land on one XCD (shared L2 for the row halos
 // of neighbouring strips); without it the dispatcher's round robin spreads
 // consecutive strips over the 8 XCDs, which balances uneven per-strip work.
@@ -91,9 +92,9 @@ __device__ __forceinline__ int reflect101(int i, int n) {
     const Strip S = (tab)[sidx];                                    \
     const LevelDesc L = lv[S.lvl];                                  \
     const int x = S.x0 + 4 * lane;                                  \
-    const int yend = min(S.y0 + kStripH, L.h);
+    const int yend = min(S.y0 + sh, L.h);
 
-__global__ __launch_bounds__(256) void k_copy_level0(const Strip* st, int n, const LevelDesc* lv,
+__global__ __launch_bounds__(256) void k_copy_level0(const Strip* st, int n, int sh, const LevelDesc* lv,
                                                      const uint8_t* const* src, const int* src_stride,
                                                      uint8_t* __restrict__ pyr) {
     STRIP_SETUP(st, n, true)
@@ -101,7 +102,11 @@ __global__ __launch_bounds__(256) void k_copy_level0(const Strip* st, int n, con
     const uint8_t* s = src[L.img];
     const long long stride = src_stride[L.img];
     uint8_t* d = pyr + L.pix;  // row y, column x at byte y * pitch + x
-    const bool vec = x + 4 <= L.w && ((reinterpret_cast<uintptr_t>(s) | (uintptr_t)stride | (uintptr_t)x) & 3) == 0;
+    // a whole word of the row, at any alignment of the caller's image (byte
+    // loads of rows that are no multiple of 4 wide took 25 us where this takes
+    // 5, 6 images of about 1240 x 730)
+    typedef uint32_t __attribute__((aligned(1))) u32_any;
+    const bool vec = x + 4 <= L.w;
     // 8 rows in flight: all loads of a group before its stores
     for (int y0 = S.y0; y0 < yend; y0 += 8) {
         uint32_t v[8];
@@ -112,7 +117,7 @@ __global__ __launch_bounds__(256) void k_copy_level0(const Strip* st, int n, con
             if (y < yend) {
                 const uint8_t* sr = s + y * stride + x;
                 if (vec) {
-                    v[u] = *reinterpret_cast<const uint32_t*>(sr);
+                    v[u] = *reinterpret_cast<const u32_any*>(sr);
                 } else {
                     for (int k = 0; k < 4 && x + k < L.w; k++) v[u] |= (uint32_t)sr[k] << (8 * k);
                 }
@@ -143,7 +148,7 @@ __global__ __launch_bounds__(64) void k_resize(const Strip* st, int n, const Lev
     const LevelDesc L = lv[S.lvl];
     const LevelDesc SL = lv[L.src];
     const int x = S.x0 + 4 * lane;
-    const int ny = min(S.y0 + kStripH, L.h) - S.y0;
+    const int ny = min(S.y0 + kResizeH, L.h) - S.y0;
     const uint8_t* sp = pyr + SL.pix;
     // the strip's row coefficients, lane k for output row S.y0 + k
     int2 cyl = make_int2(0, 0);
@@ -260,7 +265,7 @@ __device__ __forceinline__ EdgeGather edge_gather(int x, int w, int pitch) {
 // horizontal sum < 2^16: 24-bit multiplies), out = (sum + 2^15) >> 16.  Each lane keeps the last 7 horizontal rows of its
 // 4 columns in registers while walking down the strip.  Two walks compute
 // the same bytes: kFixed = false stops at the level's last row; kFixed =
-// true always covers kStripH + 6 rows (row indices reflect, stores past the
+// true always covers kH + 6 rows (row indices reflect, stores past the
 // level end are skipped).  kEdge: the wave has a lane near a level edge and
 // reads its rows through EdgeGather.
 template <bool kFixed, bool kEdge>
@@ -283,7 +288,7 @@ __device__ __forceinline__ void blur_load_row(const uint8_t* __restrict__ src, c
     }
 }
 
-template <bool kFixed, bool kEdge>
+template <bool kFixed, bool kEdge, int kH>
 __device__ __forceinline__ void blur_strip(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
                                            const LevelDesc& L, int x, int y0, int yend, const BlurTaps& taps,
                                            const EdgeGather& eg) {
@@ -300,11 +305,11 @@ __device__ __forceinline__ void blur_strip(const uint8_t* __restrict__ src, uint
     uint32_t n0, n1, n2;
     blur_load_row<kFixed, kEdge>(src, L, x, y0 - 3, eg, n0, n1, n2);
 #pragma unroll
-    for (int r = 0; r < kStripH + 6; r++) {
+    for (int r = 0; r < kH + 6; r++) {
         const int yi = y0 - 3 + r;
         if (!kFixed && yi - 3 >= yend) break;
         const uint32_t w0 = n0, w1 = n1, w2 = n2;
-        if (r + 1 < kStripH + 6) blur_load_row<kFixed, kEdge>(src, L, x, yi + 1, eg, n0, n1, n2);
+        if (r + 1 < kH + 6) blur_load_row<kFixed, kEdge>(src, L, x, yi + 1, eg, n0, n1, n2);
         uint32_t h[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -334,19 +339,20 @@ __device__ __forceinline__ void blur_strip(const uint8_t* __restrict__ src, uint
     }
 }
 
-template <bool kFixed>
+template <bool kFixed, int kH>
 __global__ __launch_bounds__(256) void k_blur(const Strip* st, int n, const LevelDesc* lv,
                                               const uint8_t* __restrict__ pyr, uint8_t* __restrict__ blur,
                                               BlurTaps taps) {
+    constexpr int sh = kH;
     STRIP_SETUP(st, n, true)
     if (x >= L.w) return;
     // a wave with no lane near a level edge reads its 3 words directly
     const bool interior = x >= 4 && x + 8 <= L.pitch && x + 6 < L.w;
     if (__all(interior)) {
-        blur_strip<kFixed, false>(pyr + L.pix, blur + L.pix, L, x, S.y0, yend, taps, EdgeGather{});
+        blur_strip<kFixed, false, kH>(pyr + L.pix, blur + L.pix, L, x, S.y0, yend, taps, EdgeGather{});
     } else {
         const EdgeGather eg = edge_gather(x, L.w, L.pitch);
-        blur_strip<kFixed, true>(pyr + L.pix, blur + L.pix, L, x, S.y0, yend, taps, eg);
+        blur_strip<kFixed, true, kH>(pyr + L.pix, blur + L.pix, L, x, S.y0, yend, taps, eg);
     }
 }
 
@@ -494,7 +500,7 @@ constexpr int kBlk = 4;                   // rows per group (prefetch) and per s
 // rows (stored at the group's end) without overwriting a row the group reads
 static_assert(2 * kBlk + 6 <= kRing, "FAST ring too small for the prefetch group");
 
-__global__ __launch_bounds__(256) void k_fast_score(const Strip* st, int n, const LevelDesc* lv, const uint8_t* pyr,
+__global__ __launch_bounds__(256) void k_fast_score(const Strip* st, int n, int sh, const LevelDesc* lv, const uint8_t* pyr,
                                                     uint8_t* score, int t_lo) {
     __shared__ uint32_t s_ring[4][kRing + kRingG][kRingW];
     __shared__ uint16_t s_queue[4][64 + kStripW];

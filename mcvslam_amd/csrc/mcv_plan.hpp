@@ -11,10 +11,22 @@ constexpr int kMaxLevels = 16;
 constexpr int kOctreeDepth = 15;        // quadtree depths encoded per candidate
 constexpr int kSortCapLds = 4096;       // candidates per level sorted in LDS (more: pool memory)
 constexpr int kHeapTabLds = 2048;       // node-table entries per level the octree heap replay stages in LDS
-constexpr long long kOctLargePixels = 600000;  // levels this large get 1024-thread octree builds
+// Octree builds take 1024 threads a level, not 256, up to kOctWideLevels levels
+// (us, all 1024 / mixed: 24 levels 57 / 99, 384 62 / 107, 768 101 / 112, 1536
+// 179 / 123), beyond that on the levels of at least kOctLargePixels pixels.
+constexpr int kOctWideLevels = 768;
+constexpr long long kOctLargePixels = 600000;
 constexpr int kMaxWin = 96;             // max FAST cell window side (pixels)
-constexpr int kStripW = 256;            // strip kernels: one wave per 256 x 32 pixels,
-constexpr int kStripH = 32;             //   4 adjacent pixels per lane
+// Strip kernels: one wave per kStripW x kStripH pixels, 4 adjacent pixels per
+// lane.  A wave walks its strip down, so a batch of few strips waits on the
+// walk: below kStripMin strips they are kStripHLow rows high (FAST and blur,
+// us, 32 / 8 rows: 1 rig frame 43 + 20 / 26 + 14, 8 frames 110 + 40 / 99 + 45,
+// 16 frames 179 + 66 / 182 + 82).  k_resize's strips are always kResizeH high.
+constexpr int kStripW = 256;
+constexpr int kStripH = 32;
+constexpr int kStripHLow = 8;
+constexpr int kStripMin = 8192;
+constexpr int kResizeH = 8;
 constexpr int kPitchAlign = 64;         // level rows start on 64-byte boundaries
 
 struct LevelDesc {

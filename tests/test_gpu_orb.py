@@ -210,3 +210,16 @@ def test_orb_octree_candidate_counts(own_ctx, levels, repeats):
     if repeats == 1:
         _check_distinct(orb, [np.full((250, 300), 128, np.uint8), synth.blob_image(8, 400, 300),
                               rng.integers(0, 256, (720, 960), dtype=np.uint8)], 1)
+
+
+@pytest.mark.parametrize("repeats", [1, 60])
+def test_orb_strip_edges(own_ctx, repeats):
+    """Level sizes around the strips' edges (columns and rows that are no
+    multiple of 4 or of the strip height, one more and one less than a strip)
+    from images at odd strides, with low strips (2 images) and high ones (120
+    images: more than 8192 strips of 32 rows)."""
+    orb = ORB(1000, 1.2, 8, 20, 7, ctx=own_ctx)
+    _check_distinct(orb, [synth.blob_image(70, 769, 481), synth.blob_image(71, 767, 511)], repeats)
+    if repeats == 1:
+        _check_distinct(orb, [synth.blob_image(72 + i, w, h) for i, (w, h) in
+                              enumerate([(257, 230), (255, 240), (239, 239), (514, 225), (330, 227)])], 1)
