@@ -1178,7 +1178,7 @@ __global__ __launch_bounds__(kOctThreads) void k_octree_build(OrbGlobals g, cons
 // without children, at the deepest depth, carries its own index instead),
 // so a popped node's children are known without another lookup.
 //
-// The whole wave runs the heap (ParHeap: one LDS round trip per gathered
+// The whole wave runs the heap (push_rows, heap_pop_wave: one LDS round trip per gathered
 // chain or 5-level subtree), and lanes 0..4 fetch the counts and child
 // ranges of a popped node's children together from the node tables in
 // global memory.  The workgroup's LDS is the heap alone (8 bytes per entry),
@@ -1249,50 +1249,39 @@ __device__ __forceinline__ void tab_children(const NodeTabs& nt, const TabPrefix
 }
 
 // libstdc++ binary heap (push_heap / pop_heap, keys compared alone) run by a
-// whole wave on LDS arrays: every sift gathers, in one round trip, either the
-// ancestor chain of the hole (sift-up) or the 5-level subtree below it
-// (62 nodes, sift-down), and the path is then decided in registers, so a pop
-// over a 1000-entry heap costs about three LDS round trips instead of one per
-// level.  Entries: key (count << 3 | children) and payload in two arrays.
-struct ParHeap {
-    uint32_t* key;
-    uint32_t* pay;
-};
-
+// whole wave on LDS entries of 8 bytes: .x the key (count << 3 | children), .y
+// the payload.  Entries sit in slots from 1 on (children of slot s: 2 s and
+// 2 s + 1); slot 0 holds a key above every real one.  The replay is one wave's
+// chain of dependent steps, so what counts are the LDS round trips and the
+// instructions on that chain.
 __device__ __forceinline__ uint32_t hkey(uint32_t k) { return k >> 3; }
 
-// push_heap's __push_heap(first, hole, 0, value): move parents down while
-// parent < value, then place value.  Lane l reads the l-th ancestor of the
-// hole; the run of ancestors smaller than the value (ancestor keys never
-// decrease upwards) moves down one step each.  All lanes take part; the
-// wave's LDS accesses execute in order, so only the compiler is fenced.
-__device__ __forceinline__ void par_sift_up(ParHeap& H, int hole, uint32_t vk, uint32_t vp) {
-    const int lane = threadIdx.x & 63;
-    // c_l = ((hole + 1) >> l) - 1 is the l-th node of the chain (c_0 = hole)
-    const int cl = ((hole + 1) >> lane) - 1;
-    const int cp = ((hole + 1) >> (lane + 1)) - 1;
-    uint32_t pk = 0xFFFFFFFFu, pp = 0;
-    if (lane < 31 && cl >= 1) {
-        pk = H.key[cp];
-        pp = H.pay[cp];
-    }
-    const unsigned long long go = __ballot(hkey(pk) < hkey(vk));
-    const int L = (int)__builtin_ctzll(~go);  // first step that does not move
-    if (lane < L) {
-        H.key[cl] = pk;
-        H.pay[cl] = pp;
-    }
-    if (lane == 0) {
-        const int final_hole = ((hole + 1) >> L) - 1;
-        H.key[final_hole] = vk;
-        H.pay[final_hole] = vp;
-    }
-    lds_order();
-}
+// lanes of a mask, as a lane condition (the mask becomes the execution mask)
+__device__ __forceinline__ bool in_lanes(unsigned long long m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
-__device__ __forceinline__ void par_push(ParHeap& H, int& len, uint32_t vk, uint32_t vp) {
-    par_sift_up(H, len, vk, vp);
-    len++;
+// push_heap's __push_heap(first, hole, 0, value) for `n` <= 4 values in a row,
+// the j-th pushed by row j of 16 lanes (every lane of a row holds its value
+// v): move parents down while parent < value, then place the value.  Lane l of
+// a row reads the l-th parent above the new slot; the run of parents smaller
+// than the value (keys never decrease upwards) moves down one step each, and
+// the lane past the run holds the value's place.  A value that stays in its
+// slot leaves the later rows' parents as they were read, so one round trip
+// serves all values up to and including the first that moves (in a heap of
+// fewer than 3 a later row's parent may be an earlier row's new slot: those
+// rows wait for the next round).  Returns how many were pushed.
+__device__ __forceinline__ int push_rows(uint2* H, int len, int n, uint2 v) {
+    const int lane = threadIdx.x & 63, l = lane & 15;
+    n = min(n, len + 1);
+    const uint32_t s0 = (uint32_t)(len + 1 + (lane >> 4)) >> l;  // the l-th slot of the row's chain
+    const uint2 p = H[s0 >> 1];
+    const bool go = hkey(p.x) < hkey(v.x);
+    const unsigned long long G = __ballot(go) & (~0ull >> (64 - 16 * n));
+    const int m = G ? __builtin_ctzll(G) >> 4 : n - 1;  // rows 0 .. m
+    const unsigned long long rows = ~0ull >> (48 - 16 * m);
+    // the first lane of each row and, in row m, the lanes above the moved parents'
+    if (in_lanes((0x0001000100010001ull | (G << 1)) & rows)) H[s0] = go ? p : v;
+    lds_order();
+    return m + 1;
 }
 
 // 5-level subtrees gathered in one LDS round trip: lane (2^d - 2) + k holds
@@ -1302,42 +1291,14 @@ __device__ __forceinline__ int subtree_depth(int lane) {
     return lane < 2 ? 1 : lane < 6 ? 2 : lane < 14 ? 3 : lane < 30 ? 4 : 5;
 }
 
-// The reads a pop starts with, in one LDS round trip: the top, the last
-// entry and the 5-level subtree below the root.
-struct PopReads {
-    uint32_t tk, tp, lk, lp, sk, sp;
-};
-
-__device__ __forceinline__ PopReads par_pop_reads(const ParHeap& H, int len) {
-    const int lane = threadIdx.x & 63;
-    const int d = subtree_depth(lane);
-    const int idx = (1 << d) - 1 + (lane - ((1 << d) - 2));
-    const int last = len - 1;
-    PopReads r;
-    r.tk = H.key[0];
-    r.tp = H.pay[0];
-    r.lk = H.key[last];
-    r.lp = H.pay[last];
-    r.sk = 0;
-    r.sp = 0;
-    if (lane < 62 && idx < last) {
-        r.sk = H.key[idx];
-        r.sp = H.pay[idx];
-    }
-    r.tk = __builtin_amdgcn_readfirstlane(r.tk);
-    r.tp = __builtin_amdgcn_readfirstlane(r.tp);
-    r.lk = __builtin_amdgcn_readfirstlane(r.lk);
-    r.lp = __builtin_amdgcn_readfirstlane(r.lp);
-    return r;
-}
-
 // Per-lane constants of the 5-level subtree layout: the lane's depth and
-// offset, whether it is a right child, and its own and its ancestors' lanes
-// as a 64-bit lane mask (lanes 62 and 63 hold no node: their mask names
-// lane 63, which no ballot below ever sets).
+// offset, its slot in the root's subtree (lane 62: the root), whether it is a
+// right child, and its own and its ancestors' lanes as a 64-bit lane mask.
+// Lanes 62 and 63 hold no node.
 struct SubLanes {
-    int d, k;
-    bool valid, right;
+    int d, k, slot0;
+    bool valid;
+    uint32_t right, keep;
     uint32_t am_lo, am_hi;
 };
 
@@ -1347,8 +1308,10 @@ __device__ __forceinline__ SubLanes sub_lanes() {
     S.d = subtree_depth(lane);
     S.k = lane - ((1 << S.d) - 2);
     S.valid = lane < 62;
-    S.right = (lane & 1) != 0;
-    unsigned long long am = 1ull << 63;
+    S.slot0 = S.valid ? (1 << S.d) + S.k : 1;
+    S.right = lane & 1;
+    S.keep = lane == 62 ? 7u : ~0u;
+    unsigned long long am = 1ull << 63;  // lanes 62, 63: a bit no walk ever sets
     if (S.valid) {
         am = 0;
         for (int e = 1; e <= S.d; e++) am |= 1ull << ((1 << e) - 2 + (S.k >> (S.d - e)));
@@ -1358,58 +1321,57 @@ __device__ __forceinline__ SubLanes sub_lanes() {
     return S;
 }
 
-// pop_heap with its reads done, as one top-down pass.  pop_heap moves the
-// hole from the root to a leaf along the max-child path of the heap without
-// its last element x (the right child unless it is smaller than the left;
-// the single child at the end of an even-length heap) and then pushes x up
-// from that leaf while the parent is smaller.  The path values never
-// increase, so the same result comes from walking the path down while the
-// next path value is >= x, moving each such value up one level, and placing
-// x where the walk stops.  Each round gathers the 5-level subtree below the
-// hole (the root's came with the reads; absent nodes read as key 0, below
-// every real key).  A lane is on the walk when it and each of its ancestors
-// in the subtree is the chosen child of its parent and >= x: one ballot and
-// a compare against the lane's ancestor mask, no per-level walk.
-__device__ __forceinline__ void par_pop(ParHeap& H, int& len, const PopReads& r, const SubLanes& S) {
-    const int L = len - 1;  // entries left; x was entry L
-    len = L;
-    if (L == 0) return;
-    constexpr unsigned long long kValid = (1ull << 62) - 1, kRight = 0xAAAAAAAAAAAAAAAAull & kValid;
-    const uint32_t xk = hkey(r.lk);
-    uint32_t sk = r.sk, sp = r.sp;
-    int hole = 0;
-    for (bool first = true;; first = false) {
-        const int idx = ((hole + 1) << S.d) - 1 + S.k;
-        if (!first) {
-            sk = 0;
-            sp = 0;
-            if (S.valid && idx < L) {
-                sk = H.key[idx];
-                sp = H.pay[idx];
-            }
+// pop_heap, as one top-down pass; the popped entry comes back in `top`.
+// pop_heap moves the hole from the root to a leaf along the max-child path of
+// the heap without its last element x (the right child unless it is smaller
+// than the left; the single child at the end of an even-length heap) and then
+// pushes x up from that leaf while the parent is smaller.  The path values
+// never increase, so the same result comes from walking the path down while
+// the next path value is >= x, moving each such value up one level, and
+// placing x where the walk stops.  Each round gathers the 5-level subtree
+// below the hole in one LDS read (lanes 62 and 63 read the top and x in the
+// first).  A lane is on the walk when it and each of its ancestors in the
+// subtree is the chosen child of its parent and >= x: with c = 2 count +
+// (right child), 0 or 1 where the heap has no entry, a child is chosen iff c >
+// its sibling's c, and >= x iff c > 2 x - 1, so both are one comparison with
+// the larger of the two; the ancestors are one ballot and the lane's ancestor
+// mask.  The round's moves are one store; in the last one lane 63 stores x and
+// lane 62 the popped entry, with count 0, in the freed slot, where the drain
+// keeps it.  (The key and payload in two arrays, the moves, x and the drained
+// word in stores of their own: 455 ns a pop, 330 ns so; with the pushes one
+// by one 1.1 us a split, 0.7 us so.)
+__device__ __forceinline__ void heap_pop_wave(uint2* H, int& len, const SubLanes& S, uint2& top) {
+    const int lane = threadIdx.x & 63;
+    const int n = len;
+    len = n - 1;
+    int slot = S.slot0;
+    uint2 s = H[lane == 63 ? n : slot];
+    const uint32_t x2 = 2 * hkey(__builtin_amdgcn_readlane(s.x, 63)) - 1;  // counts are at least 1
+    top.x = __builtin_amdgcn_readlane(s.x, 62);
+    top.y = __builtin_amdgcn_readlane(s.y, 62);
+    s.x &= S.keep;  // lane 62: the children count alone
+    int hole = 1;
+    for (;;) {
+        const uint32_t k = S.valid && slot < n ? s.x : 0u;
+        const uint32_t c = ((k >> 2) & ~1u) | S.right;
+        // the sibling's (lane swap within pairs: DPP quad_perm [1, 0, 3, 2])
+        const uint32_t cs = (uint32_t)__builtin_amdgcn_mov_dpp((int)c, 0xB1, 0xF, 0xF, false);
+        const unsigned long long M = ~__ballot(c > max(cs, x2));
+        const unsigned long long P = __ballot((((uint32_t)M & S.am_lo) | ((uint32_t)(M >> 32) & S.am_hi)) == 0);
+        if (P) hole = __builtin_amdgcn_readlane(slot, 63 - __builtin_clzll(P));  // the deepest node of the walk
+        // a walk through all 5 levels (its last node: a lane of depth 5) may go on
+        if ((P >> 30) == 0 || 2 * hole >= n) {
+            int to = slot >> 1;
+            to = lane == 62 ? n : lane == 63 ? hole : to;
+            if (in_lanes(P | (3ull << 62))) H[to] = s;
+            lds_order();
+            break;
         }
-        const uint32_t hk = hkey(sk);
-        // the sibling's key (lane swap within pairs: DPP quad_perm [1, 0, 3, 2])
-        const uint32_t hs = (uint32_t)__builtin_amdgcn_mov_dpp((int)hk, 0xB1, 0xF, 0xF, false);
-        // chosen child: the right one unless it is smaller than the left
-        const unsigned long long chosen = (__ballot(hk >= hs) & kRight) | (__ballot(hk > hs) & ~kRight);
-        const unsigned long long M = chosen & __ballot(hk >= xk) & kValid;
-        const unsigned long long P =
-            __ballot(((uint32_t)M & S.am_lo) == S.am_lo) & __ballot(((uint32_t)(M >> 32) & S.am_hi) == S.am_hi);
-        if ((P >> (threadIdx.x & 63)) & 1ull) {
-            const int parent = (idx - 1) >> 1;
-            H.key[parent] = sk;
-            H.pay[parent] = sp;
-        }
-        if (P == 0) break;
-        hole = __builtin_amdgcn_readlane(idx, 63 - __builtin_clzll(P));  // the deepest node of the walk
-        if (__builtin_popcountll(P) < 5) break;
+        if (in_lanes(P)) H[slot >> 1] = s;
+        lds_order();
+        slot = (hole << S.d) + S.k;
+        if (S.valid) s = H[min(slot, n)];
     }
-    if ((threadIdx.x & 63) == 0) {
-        H.key[hole] = r.lk;
-        H.pay[hole] = r.lp;
-    }
-    lds_order();
 }
 
 // heap entry of node c from start[c], start[c+1], child[c], child[c+1]
@@ -1420,18 +1382,62 @@ __device__ __forceinline__ uint2 node_entry(uint32_t c, uint32_t s0, uint32_t s1
 
 __device__ __forceinline__ uint32_t lane_val(uint32_t v, int k) { return __builtin_amdgcn_readlane(v, k); }
 
+// the first entries of a level's node tables in LDS, as (start, child)
+__device__ __forceinline__ int tab_pairs_load(const NodeTabs& nt, uint2* T, int cap, int total) {
+    const int lane = threadIdx.x & 63, n = min(total, cap);
+    // 8 entries per lane in flight
+    for (int i0 = 0; i0 < n; i0 += 512) {
+        uint2 a[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int i = min(i0 + 64 * u + lane, n - 1);
+            a[u] = make_uint2(nt.start[i], nt.child[i]);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (i0 + 64 * u + lane < n) T[i0 + 64 * u + lane] = a[u];
+    }
+    wave_lds_sync();
+    return n;
+}
+
+// pushes the nodes c0 .. c0 + nch - 1 (at most 4), in that order: row j of 16
+// lanes reads the table entries of the j-th left to push, in the round trip
+// that reads its parents
+__device__ __forceinline__ void push_nodes(uint2* H, int& len, const NodeTabs& nt, const uint2* T, int tn, uint32_t c0,
+                                           int nch) {
+    const bool in_lds = (int)c0 + nch < tn;  // wave-uniform
+    while (nch > 0) {
+        const int row = min((int)(threadIdx.x & 63) >> 4, nch - 1);
+        const uint32_t c = c0 + (uint32_t)row;
+        uint2 a, b;
+        if (in_lds) {
+            a = T[c];
+            b = T[c + 1];
+        } else {
+            a = make_uint2(__builtin_nontemporal_load(nt.start + c), __builtin_nontemporal_load(nt.child + c));
+            b = make_uint2(__builtin_nontemporal_load(nt.start + c + 1), __builtin_nontemporal_load(nt.child + c + 1));
+        }
+        const int k = push_rows(H, len, nch, node_entry(c, a.x, b.x, a.y, b.y));
+        len += k;
+        c0 += (uint32_t)k;
+        nch -= k;
+    }
+}
+
 // The order the keypoint kernels visit a level's slots in: the kept nodes
-// (candidate words in `words`, LDS) by 16-row band of the level (then in any
+// (candidate words in `words`, LDS, `step` apart) by 16-row band of the level (then in any
 // order within a band), seed and unused slots last.  Neighbouring keypoints
 // are then processed by neighbouring waves, which share their disk and patch
 // rows in L2.  Only the processing order: every slot's outputs stay where
 // they are.  One wave; the LDS executes the wave's DS instructions in order.
-__device__ __forceinline__ void slot_order(const OrbGlobals& g, const LevelDesc& L, int nkeep, const uint32_t* words) {
+__device__ __forceinline__ void slot_order(const OrbGlobals& g, const LevelDesc& L, int nkeep, const uint32_t* words,
+                                           int step) {
     const int lane = threadIdx.x & 63;
     __shared__ int s_band[256];
     for (int b = lane; b < 256; b += 64) s_band[b] = 0;
     lds_order();
-    for (int jj = lane; jj < nkeep; jj += 64) atomicAdd(&s_band[(words[jj] >> 16) & 0xFF], 1);
+    for (int jj = lane; jj < nkeep; jj += 64) atomicAdd(&s_band[(words[jj * step] >> 16) & 0xFF], 1);
     lds_order();
     {
         int c4[4], sum = 0;
@@ -1457,7 +1463,7 @@ __device__ __forceinline__ void slot_order(const OrbGlobals& g, const LevelDesc&
     const int nslot = L.out_cap + L.seed_count;
     for (int jj = lane; jj < nslot; jj += 64) {
         int pos = jj;
-        if (jj < nkeep) pos = atomicAdd(&s_band[(words[jj] >> 16) & 0xFF], 1);
+        if (jj < nkeep) pos = atomicAdd(&s_band[(words[jj * step] >> 16) & 0xFF], 1);
         g.perm_out[L.kp_slot + pos] = L.kp_slot + jj;
     }
 }
@@ -1467,11 +1473,10 @@ __device__ __forceinline__ void slot_order_identity(const OrbGlobals& g, const L
     for (int j = threadIdx.x & 63; j < L.out_cap + L.seed_count; j += 64) g.perm_out[L.kp_slot + j] = L.kp_slot + j;
 }
 
-
-
 __global__ __launch_bounds__(64) void k_octree_heap(OrbGlobals g, const int* order, int cap, int tab_cap) {
     extern __shared__ uint32_t heap_lds[];
-    ParHeap H{heap_lds, heap_lds + cap};
+    uint2* H = reinterpret_cast<uint2*>(heap_lds);
+    uint2* T = H + cap;
     const SubLanes SL = sub_lanes();
     const int lane = threadIdx.x;
     const int li = order[blockIdx.x];
@@ -1485,51 +1490,23 @@ __global__ __launch_bounds__(64) void k_octree_heap(OrbGlobals g, const int* ord
     NodeTabs nt;
     nt.start = g.pool + O->tab;
     nt.child = nt.start + O->total;
-    const TabPrefix TP = tab_prefix_load(nt, heap_lds + 2 * cap, tab_cap, (uint32_t)O->total);
+    if (lane == 0) H[0] = make_uint2(0xFFFFFFFFu, 0u);
+    const int tn = tab_pairs_load(nt, T, tab_cap, O->total);
     const int nr = O->n_roots;
     int len = 0;
-    {
-        uint32_t s_l = 0, c_l = 0;
-        if (lane <= nr) {
-            s_l = nt.st(lane);
-            c_l = nt.ch(lane);
-        }
-        for (int k = 0; k < nr; k++) {
-            const uint2 e = node_entry((uint32_t)k, lane_val(s_l, k), lane_val(s_l, k + 1), lane_val(c_l, k),
-                                       lane_val(c_l, k + 1));
-            par_push(H, len, e.x, e.y);
-        }
-    }
+    for (int k = 0; k < nr; k += 4) push_nodes(H, len, nt, T, tn, (uint32_t)k, min(4, nr - k));
     const int N = min(L.nfeat, cap - 8);
-    while (len < N && len > 0) {
-        const PopReads pr = par_pop_reads(H, len);
-        const uint32_t tk = pr.tk, tp = pr.tp;
-        if (hkey(tk) == 1) break;
-        const uint32_t c0 = tp, nch = tk & 7u;
-        uint32_t s_l, c_l;
-        // the children's table entries are requested before the pop and used
-        // after it: their LDS latency passes during the pop's first round,
-        // which needs nothing new from LDS
-        tab_children(nt, TP, c0, nch, s_l, c_l);
-        par_pop(H, len, pr, SL);
-#pragma unroll
-        for (uint32_t k = 0; k < 4; k++) {
-            if (k < nch) {
-                const uint2 e = node_entry(c0 + k, lane_val(s_l, k), lane_val(s_l, k + 1), lane_val(c_l, k),
-                                           lane_val(c_l, k + 1));
-                par_push(H, len, e.x, e.y);
-            }
-        }
+    uint2 top;
+    while (len > 0 && len < N) {
+        // the largest node; one with a single keypoint ends the splitting
+        if (hkey(__builtin_amdgcn_readfirstlane(H[1].x)) == 1) break;
+        heap_pop_wave(H, len, SL, top);
+        push_nodes(H, len, nt, T, tn, top.y, (int)(top.x & 7u));
     }
-    // drain: the j-th popped node's word goes to key[len] once the pop has
-    // freed that slot, i.e. node j ends at key[n0 - 1 - j]
+    // drain: the j-th popped node ends in the slot that its pop frees, n0 - j,
+    // its key's count 0
     const int n0 = len;
-    while (len > 0) {
-        const PopReads pr = par_pop_reads(H, len);
-        const uint32_t w = (pr.tp << 3) | (pr.tk & 7u);
-        par_pop(H, len, pr, SL);
-        if (lane == 0) H.key[len] = w;
-    }
+    while (len > 1) heap_pop_wave(H, len, SL, top);
     wave_lds_sync();
     const int nkeep = min(n0, L.out_cap);
     if (lane == 0) O->nout = nkeep;
@@ -1540,8 +1517,8 @@ __global__ __launch_bounds__(64) void k_octree_heap(OrbGlobals g, const int* ord
     const uint32_t* sorted = g.pool + O->sorted;
     const uint32_t* cand = g.lvl_cand + L.cand_base;
     for (int jj = lane; jj < nkeep; jj += 64) {
-        const uint32_t nw = H.key[n0 - 1 - jj];
-        const uint32_t ny = nw >> 3, nch = max(nw & 7u, 1u);
+        const uint2 e = H[n0 - jj];
+        const uint32_t ny = e.y, nch = max(e.x & 7u, 1u);
         const uint32_t s0 = nt.st(ny), s1 = nt.st(ny + nch);
         uint32_t best = 0, bi = 0;
         for (uint32_t p = s0; p < s1; p++) {
@@ -1553,9 +1530,9 @@ __global__ __launch_bounds__(64) void k_octree_heap(OrbGlobals g, const int* ord
             }
         }
         g.nodes_out[L.kp_slot + jj] = best;
-        H.pay[jj] = best;  // the drained heap's payload array is free
+        H[n0 - jj].x = best;  // the slot's word, for slot_order
     }
-    slot_order(g, L, nkeep, H.pay);
+    slot_order(g, L, nkeep, &H[n0].x, -2);
 }
 
 // ---------------------------------------------------------------------------
@@ -1851,7 +1828,7 @@ __global__ __launch_bounds__(64) void k_octree_heap_r(OrbGlobals g, const int* o
             H.p[jj] = best;
         }
     }
-    slot_order(g, L, nkeep, H.p);
+    slot_order(g, L, nkeep, H.p, 1);
 }
 
 // ---------------------------------------------------------------------------

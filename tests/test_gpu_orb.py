@@ -223,3 +223,15 @@ def test_orb_strip_edges(own_ctx, repeats):
     if repeats == 1:
         _check_distinct(orb, [synth.blob_image(72 + i, w, h) for i, (w, h) in
                               enumerate([(257, 230), (255, 240), (239, 239), (514, 225), (330, 227)])], 1)
+
+
+@pytest.mark.parametrize("nfeatures", [1, 2, 5, 60, 4000, 9000])
+def test_orb_heap_sizes(own_ctx, nfeatures):
+    """The octree's heap from one entry to thousands (a heap of 1 or 2
+    entries takes its pushes one by one; beyond 2048 nodes the tables are
+    read from memory), on a wide image that starts with several roots and on
+    a tall one without any split."""
+    orb = ORB(nfeatures, 1.2, 3, 12, 5, ctx=own_ctx)
+    rng = np.random.default_rng(9)
+    _check(orb, rng.integers(0, 256, (240, 900), dtype=np.uint8))
+    _check(orb, synth.blob_image(17, 300, 420))
