@@ -49,6 +49,8 @@ int mcv_use_own_stream(mcv_ctx* ctx);
 int mcv_synchronize(mcv_ctx* ctx);
 /* Synchronous device -> host copy of `bytes` on the context's stream. */
 int mcv_copy_to_host(mcv_ctx* ctx, void* dst, const void* d_src, uint64_t bytes);
+/* n such copies with one wait. */
+int mcv_copy_parts_to_host(mcv_ctx* ctx, int n, void* const* dst, const void* const* d_src, const uint64_t* bytes);
 
 /* ---- ORB extraction ---------------------------------------------------
  * Replaces ORB_SLAM3::ORBextractor::init (modules/local_feature/ORB/

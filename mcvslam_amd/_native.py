@@ -40,6 +40,7 @@ SIGNATURES = {
     "mcv_use_own_stream": (I, [P]),
     "mcv_synchronize": (I, [P]),
     "mcv_copy_to_host": (I, [P, P, P, ctypes.c_uint64]),
+    "mcv_copy_parts_to_host": (I, [P, I, P, P, P]),
     "mcv_orb_configure": (I, [P, I, F, I, I, I]),
     "mcv_orb_tables": (I, [P, P, P, P, P, P]),
     "mcv_orb_capacity": (I, [P, I, I, I, P]),

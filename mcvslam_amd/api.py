@@ -80,6 +80,15 @@ class Context:
         check(self.h, lib().mcv_copy_to_host(self.h, _p(out), ctypes.c_void_p(d_ptr), out.nbytes))
         return out
 
+    def to_host_all(self, parts):
+        """Host copies of several device arrays (pointer, dtype, shape)."""
+        outs = [np.empty(shape, dtype) for _, dtype, shape in parts]
+        n = len(outs)
+        check(self.h, lib().mcv_copy_parts_to_host(self.h, n, (ctypes.c_void_p * n)(*[o.ctypes.data for o in outs]),
+                                                   (ctypes.c_void_p * n)(*[p for p, _, _ in parts]),
+                                                   (ctypes.c_uint64 * n)(*[o.nbytes for o in outs])))
+        return outs
+
 
 _default_ctx = None
 
@@ -422,8 +431,7 @@ class RigBatch:
         ptrs = [ctypes.c_void_p() for _ in range(3)]
         check(self.ctx.h, lib().mcv_rig_stereo_outputs(self.h, *[ctypes.byref(p) for p in ptrs]))
         shape = (self.n_frames, self.cap)
-        return (self.ctx.to_host(ptrs[0].value, np.float32, shape), self.ctx.to_host(ptrs[1].value, np.float32, shape),
-                self.ctx.to_host(ptrs[2].value, np.int32, shape))
+        return tuple(self.ctx.to_host_all([(p.value, t, shape) for p, t in zip(ptrs, (np.float32, np.float32, np.int32))]))
 
     def octree_stats(self):
         """(FAST candidates, node-table entries, nodes emitted) of the last run."""
@@ -446,12 +454,9 @@ class RigBatch:
         matches [3n][cap][3], match counts [3n], knn [3n][cap][4])."""
         check(self.ctx.h, lib().mcv_rig_check(self.h))
         n, c = 3 * self.n_frames, self.cap
-        kps = self.ctx.to_host(self.d_kps, np.float32, (n, c, 6))
-        desc = self.ctx.to_host(self.d_desc, np.uint8, (n, c, 32))
-        counts = self.ctx.to_host(self.d_counts, np.int32, (n,))
-        matches = self.ctx.to_host(self.d_matches, np.int32, (n, c, 3))
-        mcounts = self.ctx.to_host(self.d_mcounts, np.int32, (n,))
-        knn = self.ctx.to_host(self.d_knn, np.int32, (n, c, 4))
+        kps, desc, counts, matches, mcounts, knn = self.ctx.to_host_all([
+            (self.d_kps, np.float32, (n, c, 6)), (self.d_desc, np.uint8, (n, c, 32)), (self.d_counts, np.int32, (n,)),
+            (self.d_matches, np.int32, (n, c, 3)), (self.d_mcounts, np.int32, (n,)), (self.d_knn, np.int32, (n, c, 4))])
         return kp_records(kps), desc, counts, matches, mcounts, knn
 
 

@@ -47,6 +47,9 @@ __global__ void k_zero_words(uint32_t* p, int n) {
 // held until the process ends.  After set-up host code uses only the device
 // address that hipGetSymbolAddress returns for it (once per device, in
 // mcv_create); the array's name is not a device address in host code.
+constexpr size_t kPinBytes = 4u << 20;   // pinned host memory of a context
+constexpr int kCopyParts = 8;            // ranges one launch copies
+constexpr uint32_t kCopyBlock = 16384;   // bytes per workgroup of k_copy_parts
 constexpr int kNoAllocMaxQueries = 65536;
 static __device__ __align__(256) int scratch[2 * kNoAllocMaxQueries];
 
@@ -930,8 +933,15 @@ struct mcv_ctx {
         if (!sums) HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&sums), kPoseSums * sizeof(double), hipHostMallocDefault));
         return sums;
     }
+    // pinned host memory for HostIO
+    char* pin = nullptr;
+    char* pinned() {
+        if (!pin) HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&pin), kPinBytes, hipHostMallocDefault));
+        return pin;
+    }
     ~mcv_ctx() {
         if (sums) (void)hipHostFree(sums);
+        if (pin) (void)hipHostFree(pin);
     }
 
     const SinCosTables tables() {
@@ -1126,6 +1136,137 @@ static int fail(mcv_ctx* ctx, const Fail& f) {
     return f.code;
 }
 
+// Copies of up to kCopyParts ranges in one launch, one workgroup per kCopyBlock
+// bytes, at any alignment (4 loads of 16 bytes in flight per lane).
+struct CopyPart {
+    const void* src;
+    void* dst;
+    uint32_t bytes, first;  // first workgroup
+};
+struct CopyParts {
+    int n;
+    uint32_t blocks;
+    CopyPart p[kCopyParts];
+};
+
+__global__ __launch_bounds__(256) void k_copy_parts(CopyParts a) {
+    int k = 0;
+    while (k + 1 < a.n && blockIdx.x >= a.p[k + 1].first) k++;
+    const CopyPart P = a.p[k];
+    const char* src = static_cast<const char*>(P.src);
+    char* dst = static_cast<char*>(P.dst);
+    struct __attribute__((packed)) B16 {
+        uint32_t v[4];
+    };
+    const uint32_t base = (blockIdx.x - P.first) * kCopyBlock + threadIdx.x * 16;
+    B16 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint32_t o = base + u * 4096;
+        if (o + 16 <= P.bytes) v[u] = *reinterpret_cast<const B16*>(src + o);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint32_t o = base + u * 4096;
+        if (o + 16 <= P.bytes) *reinterpret_cast<B16*>(dst + o) = v[u];
+        else
+            for (uint32_t b = o; b < P.bytes; b++) dst[b] = src[b];
+    }
+}
+
+// A call's host arrays to the device and back through the context's pinned
+// memory: the inputs of a call go up in one kernel launch, its outputs come
+// back in one, with one wait.  A copy of pageable memory costs 10 to 30 us of
+// the call each, whatever its size, and a two-dimensional one a transfer per
+// row (4.3 ms for 640 x 480).  What does not fit (kPinBytes, kCopyParts) is
+// copied as pageable memory.  Used within one call at a time; when it ends,
+// nothing of the stream touches the pinned memory any more.
+class HostIO {
+public:
+    explicit HostIO(mcv_ctx* ctx) : c(ctx) {}
+    HostIO(const HostIO&) = delete;
+    HostIO& operator=(const HostIO&) = delete;
+    ~HostIO() {
+        if (pending) (void)hipStreamSynchronize(c->stream);
+    }
+    // n bytes of pinned memory, or null
+    char* room(size_t n) {
+        const size_t at = (used + 255) / 256 * 256;
+        if (n == 0 || n > kPinBytes || at > kPinBytes - n) return nullptr;
+        used = at + n;
+        return c->pinned() + at;
+    }
+    void up(void* dev, const void* host, size_t n) {
+        if (n == 0) return;
+        char* p = in.n < kCopyParts ? room(n) : nullptr;
+        if (!p) {
+            HIP_OK(hipMemcpyAsync(dev, host, n, hipMemcpyHostToDevice, c->stream));
+            return;
+        }
+        std::memcpy(p, host, n);
+        add(in, dev, p, n);
+    }
+    template <typename T>
+    void up(DevBuf& b, const std::vector<T>& v) {
+        b.ensure(std::max<size_t>(v.size() * sizeof(T), 16));
+        up(b.p, v.data(), v.size() * sizeof(T));
+    }
+    // everything given to up(), before the kernels that read it
+    void send() { launch(in); }
+    // n bytes of the device, where peek() finds them after fetch()
+    void down(void* host, const void* dev, size_t n) {
+        if (n == 0) return;
+        char* p = out.n < kCopyParts ? room(n) : nullptr;
+        if (!p) {
+            if (host) HIP_OK(hipMemcpyAsync(host, dev, n, hipMemcpyDeviceToHost, c->stream));
+            return;
+        }
+        back[out.n] = Back{host, p, n};
+        add(out, p, dev, n);
+    }
+    // down() without a host array yet: where the bytes are after fetch(), or null
+    const char* peek(const void* dev, size_t n) {
+        const int k = out.n;
+        down(nullptr, dev, n);
+        return out.n > k ? back[k].pin : nullptr;
+    }
+    void fetch() {
+        const int n = out.n;
+        launch(out);
+        HIP_OK(hipStreamSynchronize(c->stream));
+        pending = false;
+        for (int k = 0; k < n; k++)
+            if (back[k].host) std::memcpy(back[k].host, back[k].pin, back[k].n);
+    }
+    // the pinned memory is used from here (by a kernel that reads it)
+    void hold() { pending = true; }
+
+private:
+    struct Back {
+        void* host;
+        const char* pin;
+        size_t n;
+    };
+    mcv_ctx* c;
+    size_t used = 0;
+    bool pending = false;
+    CopyParts in{}, out{};
+    Back back[kCopyParts];
+
+    static void add(CopyParts& a, void* dst, const void* src, size_t n) {
+        a.p[a.n] = CopyPart{src, dst, (uint32_t)n, a.blocks};
+        a.blocks += (uint32_t)((n + kCopyBlock - 1) / kCopyBlock);
+        a.n++;
+    }
+    void launch(CopyParts& a) {
+        if (a.n == 0) return;
+        pending = true;
+        hipLaunchKernelGGL(k_copy_parts, dim3(a.blocks), dim3(256), 0, c->stream, a);
+        HIP_OK(hipGetLastError());
+        a = CopyParts{};
+    }
+};
+
 #define API_BEGIN(ctxp) \
     mcv_ctx* api_ctx_ = (ctxp); \
     try {
@@ -1205,6 +1346,18 @@ int mcv_copy_to_host(mcv_ctx* c, void* dst, const void* src, uint64_t bytes) {
     API_END
 }
 
+int mcv_copy_parts_to_host(mcv_ctx* c, int n, void* const* dst, const void* const* src, const uint64_t* bytes) {
+    API_BEGIN(c)
+    REQUIRE(c && n >= 0 && (n == 0 || (dst && src && bytes)), MCV_ERR_INVALID, "null copy list");
+    for (int k = 0; k < n; k++)
+        REQUIRE(bytes[k] == 0 || (dst[k] && src[k]), MCV_ERR_INVALID, "null copy buffer");
+    c->set_device();
+    HostIO io(c);
+    for (int k = 0; k < n; k++) io.down(dst[k], src[k], (size_t)bytes[k]);
+    io.fetch();
+    API_END
+}
+
 int mcv_orb_configure(mcv_ctx* c, int nf, float sf, int nl, int ini, int mn) {
     API_BEGIN(c)
     REQUIRE(c, MCV_ERR_INVALID, "null context");
@@ -1269,23 +1422,42 @@ int mcv_orb_extract(mcv_ctx* c, const uint8_t* image, int w, int h, int stride, 
     }
     OrbPlan& P = *c->single;
     const SinCosTables tb = c->tables();
-    c->in_img.ensure((size_t)w * h);
-    HIP_OK(hipMemcpy2DAsync(c->in_img.p, w, image, stride, w, h, hipMemcpyHostToDevice, c->stream));
-    const uint8_t* src = c->in_img.as<uint8_t>();
+    HostIO io(c);
+    // the level-0 copy reads the image from pinned memory, or from a device copy
+    const uint8_t* src;
     const int st = w;
-    HIP_OK(hipMemcpyAsync(P.d_src.p, &src, sizeof(src), hipMemcpyHostToDevice, c->stream));
-    HIP_OK(hipMemcpyAsync(P.d_stride.p, &st, sizeof(st), hipMemcpyHostToDevice, c->stream));
+    if (char* pin = io.room((size_t)w * h)) {
+        if (stride == w) std::memcpy(pin, image, (size_t)w * h);
+        else
+            for (int y = 0; y < h; y++) std::memcpy(pin + (size_t)y * w, image + (size_t)y * stride, (size_t)w);
+        io.hold();
+        src = reinterpret_cast<const uint8_t*>(pin);
+    } else {
+        c->in_img.ensure((size_t)w * h);
+        if (stride == w) HIP_OK(hipMemcpyAsync(c->in_img.p, image, (size_t)w * h, hipMemcpyHostToDevice, c->stream));
+        else
+            HIP_OK(hipMemcpy2DAsync(c->in_img.p, w, image, stride, w, h, hipMemcpyHostToDevice, c->stream));
+        src = c->in_img.as<uint8_t>();
+    }
+    io.up(P.d_src.p, &src, sizeof(src));
+    io.up(P.d_stride.p, &st, sizeof(st));
+    io.send();
     c->out_kps.ensure((size_t)P.cap * sizeof(mcv_keypoint));
     c->out_desc.ensure((size_t)P.cap * 32);
     c->out_cnt.ensure(16);
     int n = 0;
+    const size_t kps_bytes = (size_t)P.cap * sizeof(mcv_keypoint), desc_bytes = (size_t)P.cap * 32;
+    const char *h_kps = nullptr, *h_desc = nullptr;
     for (int attempt = 0;; attempt++) {
+        io.hold();
         P.enqueue(c->orb, tb, c->stream, c->out_kps.as<mcv_keypoint>(), c->out_desc.as<uint8_t>(), P.cap,
                   c->out_cnt.as<int>());
         unsigned long long st[2] = {0, 0};  // pool words requested, error bits
-        HIP_OK(hipMemcpyAsync(&n, c->out_cnt.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        HIP_OK(hipMemcpyAsync(st, P.d_used.p, 16, hipMemcpyDeviceToHost, c->stream));
-        HIP_OK(hipStreamSynchronize(c->stream));
+        io.down(&n, c->out_cnt.p, sizeof(int));
+        io.down(st, P.d_used.p, 16);
+        h_kps = kps ? io.peek(c->out_kps.p, kps_bytes) : nullptr;
+        h_desc = desc ? io.peek(c->out_desc.p, desc_bytes) : nullptr;
+        io.fetch();
         const int err = (int)(st[1] & 0xFFFFFFFFu);
         if (err == 0) break;
         REQUIRE(!(err & 2), MCV_ERR_STATE, "a pyramid level has more FAST candidates than its cell capacity");
@@ -1297,8 +1469,12 @@ int mcv_orb_extract(mcv_ctx* c, const uint8_t* image, int w, int h, int stride, 
     *count = n;
     if (n > capacity) throw Fail{MCV_ERR_CAPACITY, "keypoint capacity too small"};
     if (n > 0) {
-        if (kps) HIP_OK(hipMemcpy(kps, c->out_kps.p, (size_t)n * sizeof(mcv_keypoint), hipMemcpyDeviceToHost));
-        if (desc) HIP_OK(hipMemcpy(desc, c->out_desc.p, (size_t)n * 32, hipMemcpyDeviceToHost));
+        if (h_kps) std::memcpy(kps, h_kps, (size_t)n * sizeof(mcv_keypoint));
+        else if (kps)
+            HIP_OK(hipMemcpy(kps, c->out_kps.p, (size_t)n * sizeof(mcv_keypoint), hipMemcpyDeviceToHost));
+        if (h_desc) std::memcpy(desc, h_desc, (size_t)n * 32);
+        else if (desc)
+            HIP_OK(hipMemcpy(desc, c->out_desc.p, (size_t)n * 32, hipMemcpyDeviceToHost));
     }
     API_END
 }
@@ -1500,14 +1676,16 @@ int mcv_distinctive_descriptors(mcv_ctx* c, const uint8_t* desc, const int32_t* 
     c->d_ptr.ensure((size_t)(n + 1) * 4);
     c->d_best.ensure((size_t)n * 4);
     c->d_desc_out.ensure((size_t)n * 32);
-    if (total) HIP_OK(hipMemcpyAsync(c->d_desc_in.p, desc, (size_t)total * 32, hipMemcpyHostToDevice, s));
-    HIP_OK(hipMemcpyAsync(c->d_ptr.p, ptr, (size_t)(n + 1) * 4, hipMemcpyHostToDevice, s));
+    HostIO io(c);
+    io.up(c->d_desc_in.p, desc, (size_t)total * 32);
+    io.up(c->d_ptr.p, ptr, (size_t)(n + 1) * 4);
+    io.send();
     hipLaunchKernelGGL(k_distinctive, dim3(n), dim3(64), 0, s, c->d_desc_in.as<uint8_t>(), c->d_ptr.as<int>(), n,
                        c->d_best.as<int>(), out_desc ? c->d_desc_out.as<uint8_t>() : nullptr);
     HIP_OK(hipGetLastError());
-    HIP_OK(hipMemcpyAsync(best, c->d_best.p, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-    if (out_desc) HIP_OK(hipMemcpyAsync(out_desc, c->d_desc_out.p, (size_t)n * 32, hipMemcpyDeviceToHost, s));
-    HIP_OK(hipStreamSynchronize(s));
+    io.down(best, c->d_best.p, (size_t)n * 4);
+    if (out_desc) io.down(out_desc, c->d_desc_out.p, (size_t)n * 32);
+    io.fetch();
     API_END
 }
 
@@ -1530,20 +1708,23 @@ int mcv_match_filter_orientation(mcv_ctx* c, const int32_t* matches, int n, cons
     c->o_a2.ensure((size_t)std::max(n2, 1) * 4);
     c->o_out.ensure((size_t)n * 12);
     c->o_cnt.ensure(4);
-    HIP_OK(hipMemcpyAsync(c->o_m.p, matches, (size_t)n * 12, hipMemcpyHostToDevice, s));
-    HIP_OK(hipMemcpyAsync(c->o_a1.p, angle1, (size_t)n1 * 4, hipMemcpyHostToDevice, s));
-    HIP_OK(hipMemcpyAsync(c->o_a2.p, angle2, (size_t)n2 * 4, hipMemcpyHostToDevice, s));
-    std::vector<OrientJob> jobs{OrientJob{c->o_m.as<int32_t>(), n, c->o_a1.as<float>(), c->o_a2.as<float>(),
-                                          c->o_out.as<int32_t>(), c->o_cnt.as<int>()}};
-    upload(c->o_jobs, jobs, s);
+    HostIO io(c);
+    io.up(c->o_m.p, matches, (size_t)n * 12);
+    io.up(c->o_a1.p, angle1, (size_t)n1 * 4);
+    io.up(c->o_a2.p, angle2, (size_t)n2 * 4);
+    io.up(c->o_jobs, std::vector<OrientJob>{OrientJob{c->o_m.as<int32_t>(), n, c->o_a1.as<float>(), c->o_a2.as<float>(),
+                                                      c->o_out.as<int32_t>(), c->o_cnt.as<int>()}});
+    io.send();
     hipLaunchKernelGGL(k_filter_orientation, dim3(1), dim3(256), 0, s, c->o_jobs.as<OrientJob>());
     HIP_OK(hipGetLastError());
     int k = 0;
-    HIP_OK(hipMemcpyAsync(&k, c->o_cnt.p, 4, hipMemcpyDeviceToHost, s));
-    HIP_OK(hipStreamSynchronize(s));
+    io.down(&k, c->o_cnt.p, 4);
+    const char* h_out = io.peek(c->o_out.p, (size_t)n * 12);
+    io.fetch();
     if (k > 0) {
-        HIP_OK(hipMemcpyAsync(out, c->o_out.p, (size_t)k * 12, hipMemcpyDeviceToHost, s));
-        HIP_OK(hipStreamSynchronize(s));
+        if (h_out) std::memcpy(out, h_out, (size_t)k * 12);
+        else
+            HIP_OK(hipMemcpy(out, c->o_out.p, (size_t)k * 12, hipMemcpyDeviceToHost));
     }
     *out_n = k;
     API_END
@@ -1565,12 +1746,14 @@ int mcv_match_knn2(mcv_ctx* c, const uint8_t* q, int nq, const uint8_t* t, int n
     c->m_q.ensure((size_t)nq * 32);
     c->m_t.ensure((size_t)std::max(nt, 1) * 32);
     c->m_out.ensure((size_t)nq * 16);
-    HIP_OK(hipMemcpyAsync(c->m_q.p, q, (size_t)nq * 32, hipMemcpyHostToDevice, c->stream));
-    if (nt) HIP_OK(hipMemcpyAsync(c->m_t.p, t, (size_t)nt * 32, hipMemcpyHostToDevice, c->stream));
+    HostIO io(c);
+    io.up(c->m_q.p, q, (size_t)nq * 32);
+    io.up(c->m_t.p, t, (size_t)nt * 32);
+    io.send();
     launch_knn(c, MatchPair{c->m_q.as<uint8_t>(), c->m_t.as<uint8_t>(), nullptr, nullptr, nq, nt,
                             c->m_out.as<int32_t>()});
-    HIP_OK(hipMemcpyAsync(out, c->m_out.p, (size_t)nq * 16, hipMemcpyDeviceToHost, c->stream));
-    HIP_OK(hipStreamSynchronize(c->stream));
+    io.down(out, c->m_out.p, (size_t)nq * 16);
+    io.fetch();
     API_END
 }
 
@@ -1585,16 +1768,23 @@ int mcv_match_filter(mcv_ctx* c, const int32_t* knn, int nq, float ratio, int th
     c->f_out.ensure((size_t)nq * 12);
     c->f_cnt.ensure(16);
     c->f_scr.ensure((size_t)nq * 8);
-    HIP_OK(hipMemcpyAsync(c->f_knn.p, knn, (size_t)nq * 16, hipMemcpyHostToDevice, c->stream));
+    HostIO io(c);
+    io.up(c->f_knn.p, knn, (size_t)nq * 16);
     FilterJob j{c->f_knn.as<int32_t>(), nullptr, nq, ratio, th, c->f_out.as<int32_t>(), c->f_cnt.as<int>(),
                 c->f_scr.as<int>()};
-    upload(c->f_jobs, std::vector<FilterJob>{j}, c->stream);
+    io.up(c->f_jobs, std::vector<FilterJob>{j});
+    io.send();
     hipLaunchKernelGGL(k_filter, dim3(1), dim3(1024), 0, c->stream, c->f_jobs.as<FilterJob>());
     HIP_OK(hipGetLastError());
     int n = 0;
-    HIP_OK(hipMemcpyAsync(&n, c->f_cnt.p, 4, hipMemcpyDeviceToHost, c->stream));
-    HIP_OK(hipStreamSynchronize(c->stream));
-    if (n > 0) HIP_OK(hipMemcpy(out, c->f_out.p, (size_t)n * 12, hipMemcpyDeviceToHost));
+    io.down(&n, c->f_cnt.p, 4);
+    const char* h_out = io.peek(c->f_out.p, (size_t)nq * 12);
+    io.fetch();
+    if (n > 0) {
+        if (h_out) std::memcpy(out, h_out, (size_t)n * 12);
+        else
+            HIP_OK(hipMemcpy(out, c->f_out.p, (size_t)n * 12, hipMemcpyDeviceToHost));
+    }
     *count = n;
     API_END
 }
@@ -2345,13 +2535,13 @@ int mcv_window_search(mcv_ctx* c, const float* points, const uint8_t* pdesc, con
     c->w_kxy.ensure((size_t)std::max(K, 1) * 8);
     c->w_kdesc.ensure((size_t)std::max(K, 1) * 32);
     c->w_out.ensure((size_t)P * 24);
-    HIP_OK(hipMemcpyAsync(c->w_pts.p, points, (size_t)P * 12, hipMemcpyHostToDevice, s));
-    HIP_OK(hipMemcpyAsync(c->w_pdesc.p, pdesc, (size_t)P * 32, hipMemcpyHostToDevice, s));
-    HIP_OK(hipMemcpyAsync(c->w_plev.p, plevel, (size_t)P * 4, hipMemcpyHostToDevice, s));
-    if (K) {
-        HIP_OK(hipMemcpyAsync(c->w_kxy.p, kxy, (size_t)K * 8, hipMemcpyHostToDevice, s));
-        HIP_OK(hipMemcpyAsync(c->w_kdesc.p, kdesc, (size_t)K * 32, hipMemcpyHostToDevice, s));
-    }
+    HostIO io(c);
+    io.up(c->w_pts.p, points, (size_t)P * 12);
+    io.up(c->w_pdesc.p, pdesc, (size_t)P * 32);
+    io.up(c->w_plev.p, plevel, (size_t)P * 4);
+    io.up(c->w_kxy.p, kxy, (size_t)K * 8);
+    io.up(c->w_kdesc.p, kdesc, (size_t)K * 32);
+    io.send();
     float Rt[12];
     for (int i = 0; i < 9; i++) Rt[i] = R[i];
     for (int i = 0; i < 3; i++) Rt[9 + i] = t[i];
@@ -2371,8 +2561,8 @@ int mcv_window_search(mcv_ctx* c, const float* points, const uint8_t* pdesc, con
     q.ratio = ratio;
     q.th = th;
     window_run(c, 1, q, sz, &kx, nullptr, &kd, &K, c->w_out.as<int32_t>());
-    HIP_OK(hipMemcpyAsync(out, c->w_out.p, (size_t)P * 24, hipMemcpyDeviceToHost, s));
-    HIP_OK(hipStreamSynchronize(s));
+    io.down(out, c->w_out.p, (size_t)P * 24);
+    io.fetch();
     API_END
 }
 
@@ -2478,14 +2668,16 @@ int mcv_bow_transform(mcv_bow_vocab* v, const uint8_t* feats, int n, int levelsu
         v->word.ensure((size_t)n * 4);
         v->weight.ensure((size_t)n * 8);
         v->nid.ensure((size_t)n * 4);
-        HIP_OK(hipMemcpyAsync(v->feats.p, feats, (size_t)n * 32, hipMemcpyHostToDevice, s));
+        HostIO io(c);
+        io.up(v->feats.p, feats, (size_t)n * 32);
+        io.send();
         const int rc = mcv_bow_transform_dev(v, v->feats.as<uint8_t>(), n, levelsup, v->word.as<int32_t>(),
                                              v->weight.as<double>(), v->nid.as<int32_t>());
         if (rc != MCV_OK) return rc;
-        HIP_OK(hipMemcpyAsync(w.data(), v->word.p, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-        HIP_OK(hipMemcpyAsync(wt.data(), v->weight.p, (size_t)n * 8, hipMemcpyDeviceToHost, s));
-        HIP_OK(hipMemcpyAsync(nd.data(), v->nid.p, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-        HIP_OK(hipStreamSynchronize(s));
+        io.down(w.data(), v->word.p, (size_t)n * 4);
+        io.down(wt.data(), v->weight.p, (size_t)n * 8);
+        io.down(nd.data(), v->nid.p, (size_t)n * 4);
+        io.fetch();
     }
     if (word) std::copy(w.begin(), w.end(), word);
     if (weight) std::copy(wt.begin(), wt.end(), weight);
@@ -2496,53 +2688,64 @@ int mcv_bow_transform(mcv_bow_vocab* v, const uint8_t* feats, int n, int levelsu
     // skipped; FeatureVector::addFeature (FeatureVector.cpp:31-45); the
     // scoring's normalisation (ScoringObject.h: L2 for L2 scoring, L1 for the
     // others but the dot product) or, without one, TF weights / v.size()
-    std::map<int32_t, double> bv;
-    std::map<int32_t, std::vector<int32_t>> fv;
+    // The features by (word, feature) and by (node, feature): runs of a sorted
+    // list hold what a map from words and one from nodes would, with each
+    // word's weights added in feature order.
     const bool must = v->scoring != 5, l2 = v->scoring == 1;
+    std::vector<uint64_t> by_word, by_node;
+    auto entry = [](int32_t id, int i) { return (uint64_t)((uint32_t)id ^ 0x80000000u) << 32 | (uint32_t)i; };
+    auto id_of = [](uint64_t e) { return (int32_t)((uint32_t)(e >> 32) ^ 0x80000000u); };
+    by_word.reserve(n);
+    by_node.reserve(n);
     for (int i = 0; i < n; i++) {
         if (!(wt[i] > 0)) continue;
-        if (v->weighting <= 1) bv[w[i]] += wt[i];
-        else bv.emplace(w[i], wt[i]);
-        fv[nd[i]].push_back(i);
+        by_word.push_back(entry(w[i], i));
+        by_node.push_back(entry(nd[i], i));
     }
-    if (v->weighting <= 1 && !bv.empty() && !must) {
-        const double m = (double)bv.size();
-        for (auto& kv : bv) kv.second /= m;
+    std::sort(by_word.begin(), by_word.end());
+    std::sort(by_node.begin(), by_node.end());
+    std::vector<int32_t> bw;
+    std::vector<double> bx;
+    for (size_t e = 0; e < by_word.size(); e++) {
+        const int32_t word_e = id_of(by_word[e]);
+        const double x = wt[(uint32_t)by_word[e]];
+        if (bw.empty() || bw.back() != word_e) {
+            bw.push_back(word_e);
+            bx.push_back(x);
+        } else if (v->weighting <= 1) {
+            bx.back() += x;
+        }
+    }
+    if (v->weighting <= 1 && !bx.empty() && !must) {
+        const double m = (double)bx.size();
+        for (double& x : bx) x /= m;
     }
     if (must) {
         double norm = 0.0;
         if (!l2) {
-            for (auto& kv : bv) norm += std::fabs(kv.second);
+            for (double x : bx) norm += std::fabs(x);
         } else {
-            for (auto& kv : bv) norm += kv.second * kv.second;
+            for (double x : bx) norm += x * x;
             norm = std::sqrt(norm);
         }
         if (norm > 0.0)
-            for (auto& kv : bv) kv.second /= norm;
+            for (double& x : bx) x /= norm;
     }
-    if (n_words) *n_words = (int32_t)bv.size();
-    if (bv_words || bv_vals) {
-        int k = 0;
-        for (auto& kv : bv) {
-            if (bv_words) bv_words[k] = kv.first;
-            if (bv_vals) bv_vals[k] = kv.second;
-            k++;
-        }
-    }
-    if (n_nodes) *n_nodes = (int32_t)fv.size();
-    if (fv_nodes || fv_ptr || fv_feats) {
-        int m = 0, t = 0;
-        if (fv_ptr) fv_ptr[0] = 0;
-        for (auto& kv : fv) {
-            if (fv_nodes) fv_nodes[m] = kv.first;
-            for (int32_t i : kv.second) {
-                if (fv_feats) fv_feats[t] = i;
-                t++;
-            }
+    if (n_words) *n_words = (int32_t)bw.size();
+    if (bv_words) std::copy(bw.begin(), bw.end(), bv_words);
+    if (bv_vals) std::copy(bx.begin(), bx.end(), bv_vals);
+    int m = 0;
+    if (fv_ptr) fv_ptr[0] = 0;
+    for (size_t e = 0; e < by_node.size(); e++) {
+        const int32_t node = id_of(by_node[e]);
+        if (e == 0 || node != id_of(by_node[e - 1])) {
+            if (fv_nodes) fv_nodes[m] = node;
             m++;
-            if (fv_ptr) fv_ptr[m] = t;
         }
+        if (fv_feats) fv_feats[e] = (int32_t)(uint32_t)by_node[e];
+        if (fv_ptr) fv_ptr[m] = (int32_t)e + 1;
     }
+    if (n_nodes) *n_nodes = m;
     API_END
 }
 
@@ -2585,15 +2788,17 @@ int mcv_bow_match(mcv_ctx* c, const uint8_t* d1, int n1, int m1, const int32_t* 
     c->b_d1.ensure((size_t)n1 * 32);
     c->b_d2.ensure((size_t)n2 * 32);
     c->b_out.ensure((size_t)nj * 20);
-    HIP_OK(hipMemcpyAsync(c->b_d1.p, d1, (size_t)n1 * 32, hipMemcpyHostToDevice, s));
-    HIP_OK(hipMemcpyAsync(c->b_d2.p, d2, (size_t)n2 * 32, hipMemcpyHostToDevice, s));
-    upload(c->b_f2, std::vector<int32_t>(feats2, feats2 + ptr2[m2]), s);
-    upload(c->b_jobs, jobs, s);
+    HostIO io(c);
+    io.up(c->b_d1.p, d1, (size_t)n1 * 32);
+    io.up(c->b_d2.p, d2, (size_t)n2 * 32);
+    io.up(c->b_f2, std::vector<int32_t>(feats2, feats2 + ptr2[m2]));
+    io.up(c->b_jobs, jobs);
+    io.send();
     hipLaunchKernelGGL(k_bow_match, dim3((nj + 3) / 4), dim3(256), 0, s, c->b_jobs.as<BowJob>(), nj,
                        c->b_d1.as<uint32_t>(), c->b_d2.as<uint32_t>(), c->b_f2.as<int32_t>(), c->b_out.as<int32_t>());
     HIP_OK(hipGetLastError());
-    HIP_OK(hipMemcpyAsync(out, c->b_out.p, (size_t)nj * 20, hipMemcpyDeviceToHost, s));
-    HIP_OK(hipStreamSynchronize(s));
+    io.down(out, c->b_out.p, (size_t)nj * 20);
+    io.fetch();
     *count = nj;
     API_END
 }

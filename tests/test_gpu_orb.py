@@ -176,7 +176,7 @@ def test_orb_batch_seeds(orb_default):
 
 
 @pytest.fixture(scope="module")
-def own_ctx():
+def own_ctx(gpu_ctx):
     """A context whose extractor settings no other test shares."""
     from mcvslam_amd import Context
     ctx = Context(0)
