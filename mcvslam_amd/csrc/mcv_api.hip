@@ -910,7 +910,7 @@ struct mcv_ctx {
     DevBuf m_q, m_t, m_out, m_part, f_knn, f_out, f_cnt, f_scr, f_jobs;
     DevBuf d_desc_in, d_ptr, d_best, d_desc_out;
     DevBuf o_m, o_a1, o_a2, o_out, o_cnt, o_jobs;
-    DevBuf w_pts, w_pdesc, w_plev, w_kxy, w_kdesc, w_cs, w_ci, w_out, w_view, w_cams;
+    DevBuf w_pts, w_pdesc, w_plev, w_kxy, w_kdesc, w_cs, w_ci, w_cxy, w_out;
     DevBuf b_d1, b_d2, b_f2, b_jobs, b_out;
     DevBuf sb_work;  // ba_build_schur
     std::map<std::string, std::unique_ptr<OrbPlan>> plans;
@@ -2388,8 +2388,8 @@ int mcv_rig_pyramid_dev(mcv_rig* r, int image, int level, int blurred, const uin
 }
 
 // ---- window search ----------------------------------------------------------
-// One launch of k_window_knn over n_cams cameras (each with its own keypoint
-// set and grid): map points (d_pts) or direct positions (d_uv).
+// k_window_knn over n_cams cameras (each with its own keypoint set and grid),
+// kWindowCams to a launch: map points (d_pts) or direct positions (d_uv).
 struct WindowQuery {
     const float* d_pts = nullptr;
     const float* d_uv = nullptr;
@@ -2423,34 +2423,8 @@ static void window_run(mcv_ctx* c, int n_cams, const WindowQuery& q, const int32
                                                  "a level-filtered query needs keypoint octaves");
     c->w_cs.ensure((size_t)n_cams * (kGridCells + 1) * 4);
     c->w_ci.ensure((size_t)std::max(total_k, 1) * 4);
-    std::vector<GridView> views(n_cams);
-    std::vector<WindowCam> wc(n_cams);
-    int off = 0;
-    for (int k = 0; k < n_cams; k++) {
-        GridView& g = views[k];
-        g.kxy = d_kxy[k];
-        g.koct = level_filter ? d_koct[k] : nullptr;
-        g.kdesc = d_kdesc[k];
-        g.n = n_kps[k];
-        g.width = sizes[2 * k];
-        g.height = sizes[2 * k + 1];
-        g.inv_w = (float)(30.0 / g.width);
-        g.inv_h = (float)(30.0 / g.height);
-        g.cell_start = c->w_cs.as<int>() + (size_t)k * (kGridCells + 1);
-        g.cell_items = c->w_ci.as<int>() + off;
-        off += n_kps[k];
-        WindowCam& w = wc[k];
-        w.grid = g;
-        if (q.d_pts) {
-            for (int i = 0; i < 9; i++) w.R[i] = q.Rt[12 * k + i];
-            for (int i = 0; i < 3; i++) w.t[i] = q.Rt[12 * k + 9 + i];
-            w.fx = q.cams[4 * k]; w.fy = q.cams[4 * k + 1]; w.cx = q.cams[4 * k + 2]; w.cy = q.cams[4 * k + 3];
-        }
-        w.out = d_out + (size_t)k * q.P * 6;
-    }
-    upload(c->w_view, views, s);
-    upload(c->w_cams, wc, s);
-    hipLaunchKernelGGL(k_grid_build, dim3(n_cams), dim3(1024), 0, s, c->w_view.as<GridView>());
+    c->w_cxy.ensure((size_t)std::max(total_k, 1) * 8);
+    WindowCams wc{};
     WindowPoints wp{};
     wp.pts = q.d_pts;
     wp.uv = q.d_uv;
@@ -2464,8 +2438,33 @@ static void window_run(mcv_ctx* c, int n_cams, const WindowQuery& q, const int32
     wp.min_level = q.min_level;
     wp.max_level = q.max_level;
     for (int i = 0; i < q.nl && i < 16; i++) wp.scales[i] = q.scales[i];
-    if (q.P > 0)
-        hipLaunchKernelGGL(k_window_knn, dim3((q.P + 3) / 4, n_cams), dim3(256), 0, s, c->w_cams.as<WindowCam>(), wp);
+    int off = 0;
+    for (int k = 0; k < n_cams; k++) {
+        WindowCam& w = wc.c[k % kWindowCams];
+        GridView& g = w.grid;
+        g.kxy = d_kxy[k];
+        g.koct = level_filter ? d_koct[k] : nullptr;
+        g.kdesc = d_kdesc[k];
+        g.n = n_kps[k];
+        g.width = sizes[2 * k];
+        g.height = sizes[2 * k + 1];
+        g.inv_w = (float)(30.0 / g.width);
+        g.inv_h = (float)(30.0 / g.height);
+        g.cell_start = c->w_cs.as<int>() + (size_t)k * (kGridCells + 1);
+        g.cell_items = c->w_ci.as<int>() + off;
+        g.cell_xy = c->w_cxy.as<float2>() + off;
+        off += n_kps[k];
+        if (q.d_pts) {
+            for (int i = 0; i < 9; i++) w.R[i] = q.Rt[12 * k + i];
+            for (int i = 0; i < 3; i++) w.t[i] = q.Rt[12 * k + 9 + i];
+            w.fx = q.cams[4 * k]; w.fy = q.cams[4 * k + 1]; w.cx = q.cams[4 * k + 2]; w.cy = q.cams[4 * k + 3];
+        }
+        w.out = d_out + (size_t)k * q.P * 6;
+        const int m = k % kWindowCams + 1;
+        if (m < kWindowCams && k + 1 < n_cams) continue;
+        hipLaunchKernelGGL(k_grid_build, dim3(m), dim3(1024), 0, s, wc);
+        if (q.P > 0) hipLaunchKernelGGL(k_window_knn, dim3((q.P + 15) / 16, m), dim3(256), 0, s, wc, wp);
+    }
     HIP_OK(hipGetLastError());
 }
 

@@ -11,7 +11,7 @@
 //                  query of Tracker::Wnd_Track (src/Tracker.cpp:339-353):
 //                  GetFeaturesInArea(kp.pt, r, minLevel, maxLevel) then the
 //                  same top-2 and filters.
-// Included by mcv_api.hip (shares bitonic_sort with the ORB kernels).
+// Included by mcv_api.hip.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -30,44 +30,8 @@ struct GridView {
     float inv_w, inv_h;     // (float)(30.0 / cols), (float)(30.0 / rows)
     int* cell_start;        // 901 entries
     int* cell_items;        // n entries (keypoint indices grouped by cell)
+    float2* cell_xy;        // their positions
 };
-
-__global__ __launch_bounds__(1024) void k_grid_build(const GridView* views) {
-    __shared__ uint32_t keys[kGridSortCap];
-    __shared__ int cnt[kGridCells + 1];
-    const GridView G = views[blockIdx.x];
-    int n2 = 1;
-    while (n2 < G.n) n2 <<= 1;
-    for (int i = threadIdx.x; i < n2; i += blockDim.x) {
-        uint32_t k = 0xFFFFFFFFu;
-        if (i < G.n) {
-            const float x = G.kxy[2 * i], y = G.kxy[2 * i + 1];
-            const int px = (int)roundf((x - 0.f) * G.inv_w);
-            const int py = (int)roundf((y - 0.f) * G.inv_h);
-            if (px >= 0 && px < kGrid && py >= 0 && py < kGrid) k = ((uint32_t)(px * kGrid + py) << 16) | (uint32_t)i;
-        }
-        keys[i] = k;
-    }
-    for (int c = threadIdx.x; c <= kGridCells; c += blockDim.x) cnt[c] = 0;
-    __syncthreads();
-    bitonic_sort(keys, n2);
-    for (int i = threadIdx.x; i < G.n; i += blockDim.x) {
-        const uint32_t k = keys[i];
-        if (k != 0xFFFFFFFFu) {
-            G.cell_items[i] = (int)(k & 0xFFFF);
-            atomicAdd(&cnt[k >> 16], 1);
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int acc = 0;
-        for (int c = 0; c < kGridCells; c++) {
-            G.cell_start[c] = acc;
-            acc += cnt[c];
-        }
-        G.cell_start[kGridCells] = acc;
-    }
-}
 
 struct WindowCam {
     GridView grid;
@@ -75,6 +39,96 @@ struct WindowCam {
     float fx, fy, cx, cy;
     int32_t* out;           // n_points x 6
 };
+
+// the cameras of one launch, as kernel arguments
+constexpr int kWindowCams = 8;
+struct WindowCams {
+    WindowCam c[kWindowCams];
+};
+
+// A stable counting sort by cell, one workgroup per camera: the keypoints are
+// cut into one contiguous run per wave, each wave counts its run's cells
+// (LDS), the counts are scanned over (cell, wave), and each wave places its
+// run 64 keypoints at a time, the lanes of one cell ranked by ballots of the
+// cell's bits.  Latency bound (one workgroup per camera, two trips to memory);
+// a bitonic sort of (cell, index) with a one-thread scan took 75 us for 3
+// cameras of 2000 keypoints.
+__global__ __launch_bounds__(1024) void k_grid_build(WindowCams cams) {
+    constexpr int kWaves = 16, kIter = kGridSortCap / 1024;
+    __shared__ int s_cnt[kWaves][kGridCells];
+    __shared__ int s_base[kGridCells];
+    __shared__ int s_sum[kWaves];
+    const GridView& G = cams.c[blockIdx.x].grid;
+    const int n = G.n;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int run = (n + 1023) / 1024 * 64;  // keypoints per wave: at most kIter * 64
+    const int i0 = wv * run;
+    for (int c = threadIdx.x; c < kWaves * kGridCells; c += 1024) s_cnt[0][c] = 0;
+    float2 xy[kIter];
+    int cell[kIter];
+#pragma unroll
+    for (int u = 0; u < kIter; u++) {
+        const int i = i0 + 64 * u + lane;
+        cell[u] = -1;
+        if (64 * u < run && i < n) {
+            const float x = G.kxy[2 * i], y = G.kxy[2 * i + 1];
+            const int px = (int)roundf((x - 0.f) * G.inv_w);
+            const int py = (int)roundf((y - 0.f) * G.inv_h);
+            if (px >= 0 && px < kGrid && py >= 0 && py < kGrid) cell[u] = px * kGrid + py;
+            xy[u] = make_float2(x, y);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kIter; u++)
+        if (cell[u] >= 0) atomicAdd(&s_cnt[wv][cell[u]], 1);
+    __syncthreads();
+    {
+        int sum = 0;
+        if (threadIdx.x < kGridCells)
+            for (int w = 0; w < kWaves; w++) {
+                const int k = s_cnt[w][threadIdx.x];
+                s_cnt[w][threadIdx.x] = sum;
+                sum += k;
+            }
+        int incl = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+        }
+        if (lane == 63) s_sum[wv] = incl;
+        __syncthreads();
+        int start = incl - sum;
+        for (int w = 0; w < wv; w++) start += s_sum[w];
+        // thread kGridCells, past the last cell: the total
+        if (threadIdx.x <= kGridCells) G.cell_start[threadIdx.x] = start;
+        if (threadIdx.x < kGridCells) s_base[threadIdx.x] = start;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kIter; u++) {
+        if (64 * u >= run) continue;  // wave-uniform
+        const int c = cell[u];
+        unsigned long long m = __ballot(c >= 0);
+#pragma unroll
+        for (int b = 0; b < 10; b++) {
+            const unsigned long long on = __ballot((c >> b) & 1);
+            m &= ((c >> b) & 1) ? on : ~on;
+        }
+        if (c >= 0) {
+            const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+            const int done = s_cnt[wv][c];
+            // one wave's DS instructions run in order: the reads, then the first lanes' writes
+            asm volatile("" ::: "memory");
+            if (rank == 0) s_cnt[wv][c] = done + __builtin_popcountll(m);
+            asm volatile("" ::: "memory");
+            const int pos = s_base[c] + done + rank;
+            G.cell_items[pos] = i0 + 64 * u + lane;
+            G.cell_xy[pos] = xy[u];
+        }
+    }
+}
 
 struct WindowPoints {
     const float* pts;       // P x 3 map points, or null for direct positions
@@ -89,15 +143,20 @@ struct WindowPoints {
     float scales[16];
 };
 
-// One wave per (camera, query).  Output row: (kp0, d0, kp1, d1, n_candidates,
-// match); a map point whose level is outside [0, nl) gets n_candidates = -1
-// and no match (the reference indexes mvScaleFactor with it).
-__global__ __launch_bounds__(256) void k_window_knn(const WindowCam* cams, WindowPoints W) {
-    const int wave = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    const int p = wave;
+// 16 lanes per (camera, query).  The grid's items are ordered by (column of
+// cells, row, keypoint), the order candidates are visited in, so the window is
+// one run of items per column and an item's place in the grid orders it among
+// the candidates; the lanes take the items of all columns together.  Output
+// row: (kp0, d0, kp1, d1, n_candidates, match); a map point whose level is
+// outside [0, nl) gets n_candidates = -1 and no match (the reference indexes
+// mvScaleFactor with it).  Bound by the chain cell ranges -> positions ->
+// descriptors of a query.  A wave per query that walked the cells one by one
+// took 67 us for 3 cameras of 5000 queries and 2000 keypoints.
+__global__ __launch_bounds__(256) void k_window_knn(WindowCams cams, WindowPoints W) {
+    const int lane = threadIdx.x & 15;
+    const int p = blockIdx.x * 16 + (threadIdx.x >> 4);
     if (p >= W.P) return;
-    const WindowCam& C = cams[blockIdx.y];
+    const WindowCam& C = cams.c[blockIdx.y];
     const GridView& G = C.grid;
     int32_t* o = C.out + 6 * (long long)p;
     float u = 0.f, v = 0.f, r = 0.f;
@@ -146,63 +205,70 @@ __global__ __launch_bounds__(256) void k_window_knn(const WindowCam* cams, Windo
         if (!(nMinX < kGrid && nMaxX >= 0 && nMinY < kGrid && nMaxY >= 0)) nMaxX = -1;
     }
     if (nMaxX >= nMinX && nMaxY >= nMinY) {
-        uint32_t q[8];
-        const uint32_t* qd = reinterpret_cast<const uint32_t*>(W.pdesc + 32 * (long long)p);
+        // 32 bytes at any 4-byte alignment
+        typedef uint32_t __attribute__((ext_vector_type(4), aligned(4))) u32x4;
+        const u32x4* qd = reinterpret_cast<const u32x4*>(W.pdesc + 32 * (long long)p);
+        const u32x4 qa = qd[0], qb = qd[1];
+        const int ncols = nMaxX - nMinX + 1;
+        for (int j0 = 0; j0 < ncols; j0 += 16) {
+            // lane j: column j0 + j's run of items
+            const int nc = min(16, ncols - j0);
+            int a = 0, len = 0;
+            if (lane < nc) {
+                const int* cs = G.cell_start + (nMinX + j0 + lane) * kGrid;
+                a = cs[nMinY];
+                len = cs[nMaxY + 1] - a;
+            }
+            int incl = len;
 #pragma unroll
-        for (int k = 0; k < 8; k++) q[k] = qd[k];
-        // enumerate cells ix-major, then iy; candidate order index c
-        int base = 0;
-        const int ny = nMaxY - nMinY + 1;
-        const int ncells = (nMaxX - nMinX + 1) * ny;
-        for (int cc = 0; cc < ncells; cc++) {
-            const int ix = nMinX + cc / ny, iy = nMinY + cc % ny;
-            const int cell = ix * kGrid + iy;
-            const int s0 = G.cell_start[cell], s1 = G.cell_start[cell + 1];
-            for (int s = s0 + lane; s < s1; s += 64) {
+            for (int s = 1; s < 16; s <<= 1) {
+                const int y = __shfl_up(incl, s, 16);
+                if (lane >= s) incl += y;
+            }
+            const int total = __shfl(incl, 15, 16);
+            const int first = incl - len;  // items of the columns before
+            for (int t0 = 0; t0 < total; t0 += 16) {
+                const int t = t0 + lane;
+                int s = 0;
+                for (int j = 0; j < nc; j++) {
+                    const int fj = __shfl(first, j, 16), aj = __shfl(a, j, 16);
+                    if (t >= fj) s = aj + (t - fj);
+                }
+                if (t >= total) continue;
                 const int idx = G.cell_items[s];
-                const float dx = G.kxy[2 * idx] - u, dy = G.kxy[2 * idx + 1] - v;
+                const float2 xy = G.cell_xy[s];
+                const float dx = xy.x - u, dy = xy.y - v;
                 bool in = fabsf(dx) < r && fabsf(dy) < r;
                 if (check_levels) {
                     const int oct = G.koct[idx];
                     if (oct < W.min_level || (W.max_level >= 0 && oct > W.max_level)) in = false;
                 }
                 if (in) {
-                    const uint32_t* kd = reinterpret_cast<const uint32_t*>(G.kdesc + 32 * (long long)idx);
+                    const u32x4* kd = reinterpret_cast<const u32x4*>(G.kdesc + 32 * (long long)idx);
+                    const u32x4 ka = kd[0] ^ qa, kb = kd[1] ^ qb;
                     uint32_t d = 0;
 #pragma unroll
-                    for (int k = 0; k < 8; k++) d += __builtin_popcount(q[k] ^ kd[k]);
-                    const uint32_t key = (d << 22) | (uint32_t)(base + (s - s0));
+                    for (int k = 0; k < 4; k++) d += __builtin_popcount(ka[k]) + __builtin_popcount(kb[k]);
+                    const uint32_t key = (d << 22) | (uint32_t)s;
                     k1 = min(k1, max(k0, key));
                     k0 = min(k0, key);
                     ncand++;
                 }
             }
-            base += s1 - s0;
         }
     }
     // merge the lanes' top-2 keys and candidate counts
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const uint32_t b0 = __shfl_xor(k0, off, 64), b1 = __shfl_xor(k1, off, 64);
+    for (int off = 8; off > 0; off >>= 1) {
+        const uint32_t b0 = __shfl_xor(k0, off, 16), b1 = __shfl_xor(k1, off, 16);
         const uint32_t n1 = min(max(k0, b0), min(k1, b1));
         k0 = min(k0, b0);
         k1 = n1;
-        ncand += __shfl_xor(ncand, off, 64);
+        ncand += __shfl_xor(ncand, off, 16);
     }
     if (lane != 0) return;
-    // candidate order index -> keypoint index (the same cell walk)
     auto kp_of = [&](uint32_t key) -> int {
-        if ((key >> 22) == 999u) return -1;
-        const int c = (int)(key & ((1u << 22) - 1));
-        const int ny = nMaxY - nMinY + 1;
-        int base = 0;
-        for (int cc = 0; cc < (nMaxX - nMinX + 1) * ny; cc++) {
-            const int cell = (nMinX + cc / ny) * kGrid + nMinY + cc % ny;
-            const int s0 = G.cell_start[cell], s1 = G.cell_start[cell + 1];
-            if (c < base + (s1 - s0)) return G.cell_items[s0 + (c - base)];
-            base += s1 - s0;
-        }
-        return -1;
+        return (key >> 22) == 999u ? -1 : G.cell_items[key & ((1u << 22) - 1)];
     };
     const int d0 = (int)(k0 >> 22), d1 = (int)(k1 >> 22);
     const int kp0 = kp_of(k0), kp1 = kp_of(k1);

@@ -148,3 +148,44 @@ def test_window_edges(gpu_ctx):
     for kx, kd in [(kxy, kdesc), (kxy[:0], kdesc[:0])]:
         oargs = (pts, pdesc, plevel, R, t, K, scales, 15.0, 0.9, 120, kx, koct[:len(kx)], kd, w, h)
         np.testing.assert_array_equal(window_search(*_gpu_args(oargs), ctx=gpu_ctx), oracle.project_search(*oargs))
+
+
+@pytest.mark.parametrize("n,spread", [(1, 1.0), (63, 0.02), (1024, 1.0), (1025, 0.3), (5000, 0.02), (16384, 1.0)])
+def test_window_keypoint_counts(gpu_ctx, n, spread):
+    """Keypoint counts around the grid build's runs (one wave's 64, one more
+    than a round of the workgroup, the largest accepted), spread over the image or
+    crowded into a few cells; windows of one cell and of every column; equal
+    descriptors, so that the candidate order decides."""
+    import torch
+    rng = np.random.default_rng(n)
+    w, h = 640, 480
+    kxy = (np.array([w, h]) * (0.5 + spread * rng.uniform(-0.52, 0.52, (n, 2)))).astype(np.float32)
+    kdesc = rng.integers(0, 4, (n, 32), dtype=np.uint8) // 3
+    koct = rng.integers(0, 4, n).astype(np.int32)
+    uv = (np.array([w, h]) * rng.uniform(0.0, 1.0, (40, 2))).astype(np.float32)
+    uv[:20] = kxy[rng.integers(0, n, 20)]
+    qdesc = rng.integers(0, 4, (40, 32), dtype=np.uint8) // 3
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    for r, lo, hi in [(9.0, -1, -1), (1000.0, 1, 2)]:
+        got = window_search_uv_dev(dev(uv), dev(qdesc), r, dev(kxy), dev(koct), dev(kdesc), w, h, lo, hi, 0.9, 250,
+                                   ctx=gpu_ctx).cpu().numpy()
+        np.testing.assert_array_equal(got, _wnd_oracle(uv, qdesc, r, kxy, koct, kdesc, w, h, lo, hi, 0.9, 250))
+
+
+def test_window_more_cameras_than_one_launch(gpu_ctx):
+    """9 cameras (a launch takes 8), one of them without keypoints."""
+    import torch
+    sc = synth.projection_scene(seed=23, n_points=300, n_kps=500)
+    scales = oracle.orb_tables()["scale"]
+    oargs = [list(_oracle_args(sc, k % 3, scales, 0.7, 50)) for k in range(9)]
+    for i in (10, 11, 12):
+        oargs[4][i] = oargs[4][i][:0]
+    dev = lambda a, dt: torch.from_numpy(np.ascontiguousarray(a, dt)).cuda()
+    Rt = np.stack([np.concatenate([np.asarray(a[3], np.float32).ravel(), np.asarray(a[4], np.float32)]) for a in oargs])
+    out = window_search_dev(dev(sc.points, np.float32), dev(sc.pdesc, np.uint8), dev(sc.plevel, np.int32), Rt,
+                            np.stack([a[5] for a in oargs]), np.array([a[13:15] for a in oargs], np.int32), scales,
+                            15.0, 0.7, 50, [dev(a[10], np.float32) for a in oargs],
+                            [dev(a[12], np.uint8) for a in oargs], ctx=gpu_ctx)
+    got = out.cpu().numpy()
+    for k in range(9):
+        np.testing.assert_array_equal(got[k], oracle.project_search(*oargs[k]), err_msg=f"camera {k}")
