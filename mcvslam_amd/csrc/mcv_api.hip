@@ -428,7 +428,7 @@ constexpr int kFastSplitLevel = 3;
 struct Tuning {
     int knn = 0;   // launch_knn2 variant (0: its rule)
     int blur = 0;  // 0: k_blur<false>, 1: k_blur<true>
-    int kp = 2;    // keypoints per wave: 0: one (k_keypoints), 1: 8, 2: 16, 3: 32 (k_keypoints_k<K>)
+    int kp = 2;    // keypoints per wave: 0: one (k_keypoints), 1: 8, 2: 16, 3: 32 (k_keypoints_k<K>); a plan's: kp_rule
     int heap = 1;  // 0: k_octree_heap_r (register top), 1: k_octree_heap (LDS), the faster one measured
     bool operator==(const Tuning& o) const { return knn == o.knn && blur == o.blur && kp == o.kp && heap == o.heap; }
 };
@@ -577,6 +577,7 @@ struct OrbPlan {
             max_slots_img = std::max(max_slots_img, img_slots);
         }
         n_slots = slot;
+        tune.kp = kp_rule(n_slots);
         cap = max_slots_img;
         heap_cap = 16;
         for (const LevelDesc& d : lv) heap_cap = std::max(heap_cap, std::max(d.nfeat, d.n_ini) + 16);
@@ -1846,7 +1847,7 @@ int mcv_rig_create(mcv_ctx* c, int n_frames, const int32_t* w3, const int32_t* h
             for (int i = 0; i < 3 * n_frames; i++) key += ":" + std::to_string(nfeatures[i]);
         r->shape_key = key;
         auto it = c->tuned.find(key);
-        if (it != c->tuned.end()) r->tune = it->second;
+        r->tune = it != c->tuned.end() ? it->second : r->batch->tune;
         r->batch->tune = r->tune;
     }
     const int n = 3 * n_frames;

@@ -2107,6 +2107,10 @@ constexpr int kHeapVariants = 2;
 inline const char* heap_variant_name(int v) { return v == 1 ? "lds-heap" : "register-top"; }
 
 constexpr int kKpVariants = 4;  // keypoints per wave: 1 (k_keypoints), 8, 16, 32
+// The untuned choice by the plan's keypoint slots: few slots want one wave
+// each, many want their set-up shared (us at 6, 12, 24, 49, 98 thousand slots:
+// 1/wave 17 25 37 62 126, 8/wave 27 31 36 46 98, 16/wave 38 38 45 51 90).
+constexpr int kp_rule(int n_slots) { return n_slots <= 20000 ? 0 : n_slots <= 70000 ? 1 : 2; }
 constexpr int kKpGroup = 256;   // waves that share slot windows in k_keypoints_k
 inline const char* kp_variant_name(int v) {
     return v == 1 ? "8/wave" : v == 2 ? "16/wave" : v == 3 ? "32/wave" : "1/wave";
