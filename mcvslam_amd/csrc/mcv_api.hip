@@ -993,7 +993,8 @@ struct mcv_rig {
     bool last_batched = false;
     Tuning tune;
     std::string shape_key;
-    DevBuf st_u, st_d, st_sad, st_keys, st_jobs;
+    DevBuf st_u, st_d, st_sad, st_jobs;
+    std::vector<StereoJob> st_hjobs;  // as last uploaded
     // destroys every captured graph (buffers moved, or the variants were retimed)
     void drop_graphs() {
         for (auto& e : graphs)
@@ -2283,8 +2284,7 @@ int mcv_rig_stereo(mcv_rig* r, float bf, float baseline) {
     r->st_u.ensure((size_t)nf * cap * 4);
     r->st_d.ensure((size_t)nf * cap * 4);
     r->st_sad.ensure((size_t)nf * cap * 4);
-    r->st_keys.ensure((size_t)nf * cap * 8);
-    std::vector<StereoJob> jobs(nf);
+    std::vector<StereoJob> jobs(nf, StereoJob{});
     for (int f = 0; f < nf; f++) {
         StereoJob& j = jobs[f];
         const int il = 3 * f, ir = 3 * f + 1;
@@ -2299,9 +2299,13 @@ int mcv_rig_stereo(mcv_rig* r, float bf, float baseline) {
         j.u_right = r->st_u.as<float>() + (size_t)f * cap;
         j.depth = r->st_d.as<float>() + (size_t)f * cap;
         j.sad = r->st_sad.as<int>() + (size_t)f * cap;
-        j.keys = r->st_keys.as<unsigned long long>() + (size_t)f * cap;
     }
-    upload(r->st_jobs, jobs, s);
+    // the jobs hold the rig's own buffers alone: the same every time, unless a buffer grew
+    if (r->st_hjobs.size() != jobs.size() || std::memcmp(r->st_hjobs.data(), jobs.data(), nf * sizeof(StereoJob))) {
+        r->st_hjobs.clear();
+        upload(r->st_jobs, jobs, s);
+        r->st_hjobs = jobs;
+    }
     StereoParams sp{};
     for (int l = 0; l < nl; l++) {
         sp.scale[l] = c->orb.scale[l];
@@ -2310,10 +2314,10 @@ int mcv_rig_stereo(mcv_rig* r, float bf, float baseline) {
     sp.bf = bf;
     sp.b = baseline;
     sp.cap = cap;
-    REQUIRE(cap <= kStereoSortCap, MCV_ERR_INVALID, "too many keypoints per image for the stereo median");
+    REQUIRE(cap <= kStereoMedianCap, MCV_ERR_INVALID, "too many keypoints per image for the stereo median");
     hipLaunchKernelGGL(k_stereo, dim3((cap + 3) / 4, nf), dim3(256), 0, s, r->st_jobs.as<StereoJob>(),
                        r->batch->d_lv.as<LevelDesc>(), r->batch->d_pyr.as<uint8_t>(), sp);
-    hipLaunchKernelGGL(k_stereo_median, dim3(nf), dim3(256), 0, s, r->st_jobs.as<StereoJob>(), sp);
+    hipLaunchKernelGGL(k_stereo_median, dim3(nf), dim3(1024), 0, s, r->st_jobs.as<StereoJob>(), sp);
     HIP_OK(hipGetLastError());
     API_END
 }

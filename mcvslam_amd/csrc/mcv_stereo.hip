@@ -4,9 +4,9 @@
 //                   disparity gating of the right keypoints in index order,
 //                   top-2 Hamming, ratio 0.70 / threshold 34, 11x11 SAD over
 //                   11 shifts on the pyramid level, parabola sub-pixel fit
-//   k_stereo_median one workgroup per pair: sort the accepted (SAD, index)
-//                   pairs, drop those beyond 1.6x / below 0.4x the median
-// Included by mcv_api.hip (uses LevelDesc, bitonic_sort, wave_sum).
+//   k_stereo_median one workgroup per pair: the median of the accepted SADs,
+//                   those beyond 1.6x / below 0.4x of it dropped
+// Included by mcv_api.hip (uses LevelDesc, wave_sum).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -22,8 +22,7 @@ struct StereoJob {
     int lvl_l, lvl_r;       // LevelDesc index of level 0 of the left / right image
     float* u_right;         // per left keypoint, -1 when unmatched
     float* depth;
-    int* sad;
-    unsigned long long* keys;  // per left keypoint: sad << 32 | index, or ~0
+    int* sad;               // per left keypoint, -1 when unmatched
 };
 
 struct StereoParams {
@@ -47,7 +46,6 @@ __global__ __launch_bounds__(256) void k_stereo(const StereoJob* jobs, const Lev
         J.u_right[iL] = -1.f;
         J.depth[iL] = -1.f;
         J.sad[iL] = -1;
-        J.keys[iL] = ~0ull;
     }
     const int rowL = (int)vL;
     const float minZ = sp.b, minD = 1.f;
@@ -145,49 +143,80 @@ __global__ __launch_bounds__(256) void k_stereo(const StereoJob* jobs, const Lev
         J.depth[iL] = sp.bf / disparity;
         J.u_right[iL] = bestuR;
         J.sad[iL] = bestDist;
-        J.keys[iL] = ((unsigned long long)(uint32_t)bestDist << 32) | (unsigned)iL;
     }
 }
 
-constexpr int kStereoSortCap = 8192;
+constexpr int kStereoMedianCap = 8192;
 
-__global__ __launch_bounds__(256) void k_stereo_median(const StereoJob* jobs, StereoParams sp) {
-    __shared__ unsigned long long s[kStereoSortCap];
-    __shared__ int s_n;
+// The reference sorts the accepted (SAD, index) pairs and drops entries from
+// the end while the SAD exceeds 1.6 times that of the middle entry (n / 2) and
+// from the start while it is below 0.4 times: SADs of the middle one's size
+// always stay, so both are a test of each entry alone and only the middle SAD
+// is needed.  A SAD is below 2^16 (121 pixels of at most 510), so two counts
+// of 256 bins find it; the SADs stay in registers.  Latency bound: one
+// workgroup per pair (sorting 2000 pairs took 52 us).
+__global__ __launch_bounds__(1024) void k_stereo_median(const StereoJob* jobs, StereoParams sp) {
+    constexpr int kPer = kStereoMedianCap / 1024;
+    __shared__ int s_bin[2][256];
+    __shared__ int s_sel[2], s_rank[2];
     const StereoJob J = jobs[blockIdx.x];
-    const int nl = min(min(*J.nl, sp.cap), kStereoSortCap);
-    int n2 = 1;
-    while (n2 < nl) n2 <<= 1;
-    for (int i = threadIdx.x; i < n2; i += 256) s[i] = i < nl ? J.keys[i] : ~0ull;
-    if (threadIdx.x == 0) s_n = 0;
+    const int nl = min(min(*J.nl, sp.cap), kStereoMedianCap);
+    int sad[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; u++) {
+        const int i = u * 1024 + threadIdx.x;
+        sad[u] = i < nl ? J.sad[i] : -1;
+    }
+    if (threadIdx.x < 512) s_bin[0][threadIdx.x] = 0;
     __syncthreads();
-    bitonic_sort(s, n2);
-    // number of accepted entries = first sentinel position
-    for (int i = threadIdx.x; i < n2; i += 256)
-        if (s[i] != ~0ull && (i + 1 == n2 || s[i + 1] == ~0ull)) s_n = i + 1;
-    __syncthreads();
-    const int n = s_n;
-    if (n == 0) return;
-    const float median = (float)(int)(s[n / 2] >> 32);
+#pragma unroll
+    for (int pass = 0; pass < 2; pass++) {
+#pragma unroll
+        for (int u = 0; u < kPer; u++)
+            if (sad[u] >= 0 && (pass == 0 || (sad[u] >> 8) == s_sel[0]))
+                atomicAdd(&s_bin[pass][pass == 0 ? sad[u] >> 8 : sad[u] & 255], 1);
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            // lane l: bins 4 l .. 4 l + 3
+            const int l = threadIdx.x;
+            int c[4], sum = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                c[k] = s_bin[pass][4 * l + k];
+                sum += c[k];
+            }
+            int incl = sum;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(incl, o, 64);
+                if (l >= o) incl += y;
+            }
+            const int rank = pass == 0 ? __shfl(incl, 63, 64) / 2 : s_rank[0];
+            // the bin that holds the rank-th entry (no lane when there is none)
+            int before = incl - sum;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                if (rank >= before && rank < before + c[k]) {
+                    s_sel[pass] = 4 * l + k;
+                    s_rank[pass] = rank - before;
+                }
+                before += c[k];
+            }
+            if (pass == 0 && l == 63 && incl == 0) s_sel[0] = -1;
+        }
+        __syncthreads();
+        if (s_sel[0] < 0) return;  // nothing accepted
+    }
+    const float median = (float)(s_sel[0] << 8 | s_sel[1]);
     const float th_max = 1.6f * median;
     const float th_min = (float)(0.4 * (double)median);
-    // r: last kept from the end; l: first kept from the start (l < r)
-    __shared__ int s_r, s_l;
-    if (threadIdx.x == 0) {
-        int r = n - 1;
-        while (r >= 0 && (float)(int)(s[r] >> 32) > th_max) r--;
-        int l = 0;
-        while (l < r && (float)(int)(s[l] >> 32) < th_min) l++;
-        s_r = r;
-        s_l = l;
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += 256) {
-        if (i > s_r || i < s_l) {
-            const int idx = (int)(s[i] & 0xFFFFFFFFu);
-            J.u_right[idx] = -1.f;
-            J.depth[idx] = -1.f;
-            J.sad[idx] = -1;
+#pragma unroll
+    for (int u = 0; u < kPer; u++) {
+        const int i = u * 1024 + threadIdx.x;
+        if (sad[u] >= 0 && ((float)sad[u] > th_max || (float)sad[u] < th_min)) {
+            J.u_right[i] = -1.f;
+            J.depth[i] = -1.f;
+            J.sad[i] = -1;
         }
     }
 }
