@@ -322,6 +322,11 @@ int mcv_ba_set_observations(mcv_ba* ba, const float* uv, const int32_t* point, c
  * world (qx qy qz qw tx ty tz); cams C x 12 (fx fy cx cy, camera-from-body
  * qx qy qz qw tx ty tz, Huber delta). */
 int mcv_ba_set_state(mcv_ba* ba, const double* points, const double* frames, const double* cams);
+/* The same state after g2o's oplus of every vertex (VertexSE3Expmap: T <-
+ * exp(delta) T, VertexSBAPointXYZ: P <- P + delta) with increments on the
+ * device: F x 6 and P x 3, float or (fp64 != 0) double. */
+int mcv_ba_set_state_increments(mcv_ba* ba, const double* points, const double* frames, const double* cams,
+                                const void* d_pose, int pose_fp64, const void* d_point, int point_fp64);
 /* Linearize every edge into 22 device planes of M floats: e_u, e_v, chi2,
  * Huber weight, J_pose (2x6 row-major), J_point (2x3 row-major).  mode:
  * MCV_BA_FULL every plane; MCV_BA_RESIDUAL the first four only (the LM
@@ -377,6 +382,8 @@ int mcv_ba_planes(mcv_ba* ba, float** d_planes, int64_t* stride);
 int mcv_ba_read_planes(mcv_ba* ba, int first, int count, float* host);
 /* Device-to-device copy of planes [first, first + count) (enqueued). */
 int mcv_ba_copy_planes_dev(mcv_ba* ba, int first, int count, float* d_dst);
+/* The residuals of the last linearization as M rows (e_u, e_v). */
+int mcv_ba_copy_residuals_dev(mcv_ba* ba, float* d_dst);
 /* Adjoint of the residual: grad_pose[F x 6] = sum J_pose^T g and
  * grad_point[P x 3] = sum J_point^T g over the last linearization, with
  * d_g an M x 2 device array; outputs are device arrays. */

@@ -81,6 +81,7 @@ SIGNATURES = {
     "mcv_ba_destroy": (None, [P]),
     "mcv_ba_set_observations": (I, [P, P, P, P, P, P]),
     "mcv_ba_set_state": (I, [P, P, P, P]),
+    "mcv_ba_set_state_increments": (I, [P, P, P, P, P, I, P, I]),
     "mcv_ba_linearize": (I, [P, I]),
     "mcv_ba_set_variant": (I, [P, I]),
     "mcv_ba_autotune": (I, [P, I, P, I]),
@@ -93,6 +94,7 @@ SIGNATURES = {
     "mcv_ba_planes": (I, [P, P, P]),
     "mcv_ba_read_planes": (I, [P, I, I, P]),
     "mcv_ba_copy_planes_dev": (I, [P, I, I, P]),
+    "mcv_ba_copy_residuals_dev": (I, [P, P]),
     "mcv_ba_adjoint_dev": (I, [P, P, P, P]),
     "mcv_ba_set_fixed": (I, [P, P]),
     "mcv_ba_schur": (I, [P, F]),

@@ -40,6 +40,7 @@ class Context:
         if code != 0:
             raise MCVError(code, f"mcv_create(device={device}) failed")
         self.h = h
+        self.device = device
 
     def close(self):
         if getattr(self, "h", None):
@@ -602,6 +603,16 @@ class BALinearizer:
              np.ascontiguousarray(cams, np.float64)]
         check(self.ctx.h, lib().mcv_ba_set_state(self.h, *[_p(x) for x in a]))
 
+    def set_state_increments(self, points, frames, cams, pose_delta, point_delta):
+        """The state after the increments pose_delta (F x 6) and point_delta
+        (P x 3): contiguous float32 or float64 tensors on this device."""
+        a = [np.ascontiguousarray(points, np.float64), np.ascontiguousarray(frames, np.float64),
+             np.ascontiguousarray(cams, np.float64)]
+        d = []
+        for t in (pose_delta, point_delta):
+            d += [ctypes.c_void_p(t.data_ptr()), int(t.element_size() == 8)]
+        check(self.ctx.h, lib().mcv_ba_set_state_increments(self.h, *[_p(x) for x in a], *d))
+
     FULL, RESIDUAL, POSE_ONLY = 0, 1, 2
 
     def linearize(self, residual_only: bool = False, mode: int | None = None):
@@ -742,6 +753,9 @@ class BALinearizer:
 
     def copy_planes_dev(self, first: int, count: int, d_ptr: int):
         check(self.ctx.h, lib().mcv_ba_copy_planes_dev(self.h, first, count, ctypes.c_void_p(d_ptr)))
+
+    def copy_residuals_dev(self, d_ptr: int):
+        check(self.ctx.h, lib().mcv_ba_copy_residuals_dev(self.h, ctypes.c_void_p(d_ptr)))
 
     def adjoint_dev(self, g_ptr: int, gpose_ptr: int, gpoint_ptr: int):
         check(self.ctx.h, lib().mcv_ba_adjoint_dev(self.h, ctypes.c_void_p(g_ptr), ctypes.c_void_p(gpose_ptr),

@@ -4,8 +4,8 @@ Reprojection.apply(pose_delta [F, 6], point_delta [P, 3], lin, state) -> e [M, 2
 
 forward applies the increments the way g2o's vertices do (VertexSE3Expmap:
 T <- exp(delta) * T, types_six_dof_expmap.h:98-101; VertexSBAPointXYZ:
-P <- P + delta, types_sba.h:146-149) to the FP64 state on the host, loads it,
-and evaluates EdgeSE3XYZ2Camera::computeError for every edge on the GPU
+P <- P + delta, types_sba.h:146-149) to the FP64 state, the frames on the host
+and the points on the device, and evaluates EdgeSE3XYZ2Camera::computeError for every edge on the GPU
 (include/OptimizeTypes.hpp:80-86).  backward runs the hand-written adjoint
 kernels k_ba_pose_adj / k_ba_point_adj: grad_pose[f] = sum of J_pose^T g over
 frame f's edges, grad_point[p] = sum of J_point^T g over point p's edges,
@@ -77,21 +77,40 @@ def apply_increments(points, frames, pose_delta, point_delta):
     return np.asarray(points, np.float64) + point_delta, fr
 
 
+def _on_device(d, shape, device):
+    return (d.is_cuda and d.device.index == device and tuple(d.shape) == shape
+            and d.dtype in (torch.float32, torch.float64))
+
+
 class Reprojection(torch.autograd.Function):
     @staticmethod
     def forward(ctx, pose_delta: torch.Tensor, point_delta: torch.Tensor, lin: BALinearizer, state):
         points, frames, cams = state
-        pts, frs = apply_increments(points, frames, pose_delta.detach().double().cpu().numpy(),
-                                    point_delta.detach().double().cpu().numpy())
-        lin.ctx.use_torch_stream()
-        lin.set_state(pts, frs, cams)
-        lin.linearize()
-        e = torch.empty((2, lin.M), dtype=torch.float32, device=pose_delta.device)
-        lin.copy_planes_dev(0, 2, e.data_ptr())
+        # increments of other kinds (another type, broadcast rows, another
+        # device or the host) are applied on the host
+        native = (_on_device(pose_delta, (lin.F, 6), lin.ctx.device)
+                  and _on_device(point_delta, (lin.P, 3), lin.ctx.device)
+                  and np.shape(points) == (lin.P, 3) and np.shape(frames) == (lin.F, 7))
+        if native:
+            dp, dx = pose_delta.detach().contiguous(), point_delta.detach().contiguous()
+            lin.ctx.use_torch_stream()
+            lin.set_state_increments(points, frames, cams, dp, dx)
+            lin.linearize()
+            e = torch.empty((lin.M, 2), dtype=torch.float32, device=pose_delta.device)
+            lin.copy_residuals_dev(e.data_ptr())
+        else:
+            pts, frs = apply_increments(points, frames, pose_delta.detach().double().cpu().numpy(),
+                                        point_delta.detach().double().cpu().numpy())
+            lin.ctx.use_torch_stream()
+            lin.set_state(pts, frs, cams)
+            lin.linearize()
+            e = torch.empty((2, lin.M), dtype=torch.float32, device=pose_delta.device)
+            lin.copy_planes_dev(0, 2, e.data_ptr())
+            e = e.t().contiguous()
         ctx.lin = lin
         ctx.gen = lin.generation()
         ctx.dtypes = (pose_delta.dtype, point_delta.dtype)
-        return e.t().contiguous()
+        return e
 
     @staticmethod
     def backward(ctx, g: torch.Tensor):

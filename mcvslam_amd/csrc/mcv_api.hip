@@ -1213,6 +1213,8 @@ public:
         b.ensure(std::max<size_t>(v.size() * sizeof(T), 16));
         up(b.p, v.data(), v.size() * sizeof(T));
     }
+    // what has been handed out so far stays past fetch()
+    void keep() { base = used; }
     // everything given to up(), before the kernels that read it
     void send() { launch(in); }
     // n bytes of the device, where peek() finds them after fetch()
@@ -1226,7 +1228,8 @@ public:
         back[out.n] = Back{host, p, n};
         add(out, p, dev, n);
     }
-    // down() without a host array yet: where the bytes are after fetch(), or null
+    // down() without a host array yet: where the bytes are after fetch() until
+    // the next up() or down(), or null
     const char* peek(const void* dev, size_t n) {
         const int k = out.n;
         down(nullptr, dev, n);
@@ -1237,6 +1240,7 @@ public:
         launch(out);
         HIP_OK(hipStreamSynchronize(c->stream));
         pending = false;
+        used = base;
         for (int k = 0; k < n; k++)
             if (back[k].host) std::memcpy(back[k].host, back[k].pin, back[k].n);
     }
@@ -1250,7 +1254,7 @@ private:
         size_t n;
     };
     mcv_ctx* c;
-    size_t used = 0;
+    size_t used = 0, base = 0;
     bool pending = false;
     CopyParts in{}, out{};
     Back back[kCopyParts];
@@ -1444,6 +1448,7 @@ int mcv_orb_extract(mcv_ctx* c, const uint8_t* image, int w, int h, int stride, 
     io.up(P.d_src.p, &src, sizeof(src));
     io.up(P.d_stride.p, &st, sizeof(st));
     io.send();
+    io.keep();
     c->out_kps.ensure((size_t)P.cap * sizeof(mcv_keypoint));
     c->out_desc.ensure((size_t)P.cap * 32);
     c->out_cnt.ensure(16);
@@ -2947,27 +2952,35 @@ static void ba_frame_records(const mcv_ba* b, const double* fq, BAPair* pr, Fram
 }
 
 // every frame's records to the device
-static void ba_upload_frames(mcv_ba* b, hipStream_t s) {
+static void ba_upload_frames(mcv_ba* b, HostIO& io) {
     std::vector<BAPair> pr((size_t)b->F * b->C);
     std::vector<FramePose> fp(b->F);
     for (int f = 0; f < b->F; f++) ba_frame_records(b, b->h_frames.data() + 7 * (size_t)f, &pr[(size_t)f * b->C], fp[f]);
-    upload(b->pairs, pr, s);
-    upload(b->fposes, fp, s);
+    io.up(b->pairs, pr);
+    io.up(b->fposes, fp);
+    io.send();
     const double* sc = b->h_scam;
     b->scam = StereoCam{(float)sc[0], (float)sc[1], (float)sc[2], (float)sc[3], (float)sc[4],
                         b->robust ? (float)sc[5] : INFINITY};
 }
 
-// FP64 points to the device and their float pairs
-static void ba_upload_points(mcv_ba* b, const double* points, hipStream_t s) {
+}  // extern "C"
+
+// FP64 points to the device and their float pairs; d_delta (device, P x 3,
+// or null): added first
+template <typename T>
+static void ba_upload_points(mcv_ba* b, const double* points, const T* d_delta, HostIO& io, hipStream_t s) {
     b->p64.ensure((size_t)b->P * 24);
     b->phi.ensure((size_t)b->P * 16);
     b->plo.ensure((size_t)b->P * 16);
-    HIP_OK(hipMemcpyAsync(b->p64.p, points, (size_t)b->P * 24, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_ba_points_apply, dim3((b->P + 255) / 256), dim3(256), 0, s, b->p64.as<double>(),
-                       (const float*)nullptr, (const uint8_t*)nullptr, b->P, b->phi.as<float4>(), b->plo.as<float4>());
+    io.up(b->p64.p, points, (size_t)b->P * 24);
+    io.send();
+    hipLaunchKernelGGL(k_ba_points_apply<T>, dim3((b->P + 255) / 256), dim3(256), 0, s, b->p64.as<double>(), d_delta,
+                       (const uint8_t*)nullptr, b->P, b->phi.as<float4>(), b->plo.as<float4>());
     HIP_OK(hipGetLastError());
 }
+
+extern "C" {
 
 int mcv_ba_set_state(mcv_ba* b, const double* points, const double* frames, const double* cams) {
     mcv_ctx* c = b ? b->ctx : nullptr;
@@ -2977,8 +2990,47 @@ int mcv_ba_set_state(mcv_ba* b, const double* points, const double* frames, cons
     hipStream_t s = c->stream;
     b->h_frames.assign(frames, frames + 7 * (size_t)b->F);
     b->h_cams.assign(cams, cams + 12 * (size_t)b->C);
-    ba_upload_points(b, points, s);
-    ba_upload_frames(b, s);
+    HostIO io(c);
+    ba_upload_points(b, points, (const float*)nullptr, io, s);
+    ba_upload_frames(b, io);
+    HIP_OK(hipStreamSynchronize(s));
+    b->have_state = true;
+    b->touched(-1);
+    API_END
+}
+
+static void se3_oplus(double* frame, const double* xi);
+
+int mcv_ba_set_state_increments(mcv_ba* b, const double* points, const double* frames, const double* cams,
+                                const void* d_pose, int pose_fp64, const void* d_point, int point_fp64) {
+    mcv_ctx* c = b ? b->ctx : nullptr;
+    API_BEGIN(c)
+    REQUIRE(b && points && frames && cams && d_pose && d_point, MCV_ERR_INVALID, "null state arrays");
+    c->set_device();
+    hipStream_t s = c->stream;
+    HostIO io(c);
+    if (point_fp64) ba_upload_points(b, points, static_cast<const double*>(d_point), io, s);
+    else ba_upload_points(b, points, static_cast<const float*>(d_point), io, s);
+    const size_t nx = 6 * (size_t)b->F;
+    std::vector<double> xi(nx);
+    if (pose_fp64) {
+        io.down(xi.data(), d_pose, nx * 8);
+        io.fetch();
+    } else {
+        std::vector<float> xf(nx);
+        io.down(xf.data(), d_pose, nx * 4);
+        io.fetch();
+        std::copy(xf.begin(), xf.end(), xi.begin());
+    }
+    b->h_frames.assign(frames, frames + 7 * (size_t)b->F);
+    b->h_cams.assign(cams, cams + 12 * (size_t)b->C);
+    for (int f = 0; f < b->F; f++) {
+        const double* d = &xi[6 * (size_t)f];
+        bool any = false;
+        for (int k = 0; k < 6; k++) any = any || d[k] != 0;
+        if (any) se3_oplus(&b->h_frames[7 * (size_t)f], d);
+    }
+    ba_upload_frames(b, io);
     HIP_OK(hipStreamSynchronize(s));
     b->have_state = true;
     b->touched(-1);
@@ -3434,7 +3486,8 @@ int mcv_ba_set_robust(mcv_ba* b, int enabled) {
     REQUIRE(b && b->have_state, MCV_ERR_STATE, "set the state first");
     c->set_device();
     b->robust = enabled != 0;
-    ba_upload_frames(b, c->stream);
+    HostIO io(c);
+    ba_upload_frames(b, io);
     HIP_OK(hipStreamSynchronize(c->stream));
     b->touched(-1);
     API_END
@@ -3745,7 +3798,8 @@ static int ba_optimize_pose(mcv_ba* b, int frame, int iterations, double tau, in
         it_done++;
         if (qmax == max_trials || rho == 0 || !std::isfinite(lambda)) break;
     }
-    ba_upload_frames(b, s);
+    HostIO io(c);
+    ba_upload_frames(b, io);
     HIP_OK(hipStreamSynchronize(s));
     return it_done;
 }
@@ -3837,13 +3891,16 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
                 hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, s, b->partial.as<double>(), bblocks,
                                    b->dsum.as<double>() + 1);
                 // update: points on the device, frames on the host
-                hipLaunchKernelGGL(k_ba_points_apply, dim3(std::max(pblocks, 1)), dim3(256), 0, s,
+                hipLaunchKernelGGL(k_ba_points_apply<float>, dim3(std::max(pblocks, 1)), dim3(256), 0, s,
                                    b->p64.as<double>(), b->xl.as<float>(), pfix, P, b->phi.as<float4>(),
                                    b->plo.as<float4>());
                 HIP_OK(hipGetLastError());
                 for (int f = 0; f < b->F; f++)
                     if (fidx[f] >= 0) se3_oplus(&b->h_frames[7 * (size_t)f], &xp[6 * (size_t)fidx[f]]);
-                ba_upload_frames(b, s);
+                {
+                    HostIO io(c);
+                    ba_upload_frames(b, io);
+                }
                 scale += ba_read_double(b, s, 1);
             }
             // computeActiveErrors at the new state
@@ -3864,9 +3921,12 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
                 ni *= 2;
                 // pop
                 b->h_frames = frames0;
-                ba_upload_frames(b, s);
+                {
+                    HostIO io(c);
+                    ba_upload_frames(b, io);
+                }
                 HIP_OK(hipMemcpyAsync(b->p64.p, b->p64_bak.p, (size_t)P * 24, hipMemcpyDeviceToDevice, s));
-                hipLaunchKernelGGL(k_ba_points_apply, dim3(std::max(pblocks, 1)), dim3(256), 0, s,
+                hipLaunchKernelGGL(k_ba_points_apply<float>, dim3(std::max(pblocks, 1)), dim3(256), 0, s,
                                    b->p64.as<double>(), (const float*)nullptr, (const uint8_t*)nullptr, P,
                                    b->phi.as<float4>(), b->plo.as<float4>());
                 HIP_OK(hipGetLastError());
@@ -3934,6 +3994,18 @@ int mcv_ba_copy_planes_dev(mcv_ba* b, int first, int count, float* d_dst) {
     API_END
 }
 
+int mcv_ba_copy_residuals_dev(mcv_ba* b, float* d_dst) {
+    mcv_ctx* c = b ? b->ctx : nullptr;
+    API_BEGIN(c)
+    REQUIRE(b && (d_dst || b->M == 0), MCV_ERR_INVALID, "null residual buffer");
+    c->set_device();
+    if (b->M)
+        hipLaunchKernelGGL(k_ba_residual_rows, dim3((b->M + 255) / 256), dim3(256), 0, c->stream, b->planes.as<float>(),
+                           (long long)b->M, reinterpret_cast<float2*>(d_dst));
+    HIP_OK(hipGetLastError());
+    API_END
+}
+
 int mcv_ba_adjoint_dev(mcv_ba* b, const float* d_g, float* d_gpose, float* d_gpoint) {
     mcv_ctx* c = b ? b->ctx : nullptr;
     API_BEGIN(c)
@@ -3943,7 +4015,7 @@ int mcv_ba_adjoint_dev(mcv_ba* b, const float* d_g, float* d_gpose, float* d_gpo
     hipStream_t s = c->stream;
     hipLaunchKernelGGL(k_ba_point_adj, dim3((b->P + 255) / 256), dim3(256), 0, s, b->planes.as<float>(), (long long)b->M,
                        reinterpret_cast<const float2*>(d_g), b->pptr.as<int>(), b->P, d_gpoint);
-    hipLaunchKernelGGL(k_ba_pose_adj, dim3(b->F), dim3(256), 0, s, b->planes.as<float>(), (long long)b->M,
+    hipLaunchKernelGGL(k_ba_pose_adj, dim3(b->F, 6), dim3(kPoseAdjThreads), 0, s, b->planes.as<float>(), (long long)b->M,
                        reinterpret_cast<const float2*>(d_g), b->fptr.as<int>(), b->fobs.as<int>(), d_gpose);
     HIP_OK(hipGetLastError());
     API_END

@@ -447,30 +447,49 @@ __global__ __launch_bounds__(256) void k_ba_point_adj(const float* planes, long 
     gout[3 * p + 2] = a2;
 }
 
-// grad_pose[f] = sum over the observations of frame f of J_pose^T g.  One
-// workgroup per frame; each thread sums a strided slice, then a fixed-order
-// tree reduction: deterministic for a given launch shape.
-__global__ __launch_bounds__(256) void k_ba_pose_adj(const float* planes, long long S, const float2* g,
-                                                     const int* fptr, const int* fobs, float* gout) {
-    __shared__ float red[6][256];
-    const int f = blockIdx.x;
-    float a[6] = {0, 0, 0, 0, 0, 0};
-    for (int k = fptr[f] + threadIdx.x; k < fptr[f + 1]; k += 256) {
-        const int i = fobs[k];
-        const float2 gi = g[i];
+// grad_pose[f][c] = sum over the observations of frame f of row c of J_pose^T
+// g, one workgroup per (frame, c); each thread sums a strided slice, then a
+// fixed-order tree reduction: deterministic.  A frame's observations lie some
+// 10 apart in the planes, so a workgroup pulls whole planes through its CU:
+// that bounds it, hence the cut by component (two planes of the twelve each;
+// a workgroup per frame took 84 us for 10 frames of 15 thousand) and 4 loads
+// in flight per thread.
+constexpr int kPoseAdjThreads = 1024;
+__global__ __launch_bounds__(kPoseAdjThreads) void k_ba_pose_adj(const float* planes, long long S, const float2* g,
+                                                                 const int* fptr, const int* fobs, float* gout) {
+    __shared__ float red[kPoseAdjThreads / 64];
+    const int f = blockIdx.x, c = blockIdx.y;
+    const float* pu = planes + (4 + c) * S;
+    const float* pv = planes + (10 + c) * S;
+    const int k1 = fptr[f + 1];
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int k = fptr[f] + threadIdx.x; k < k1; k += 4 * kPoseAdjThreads) {
+        int i[4];
 #pragma unroll
-        for (int c = 0; c < 6; c++) a[c] += planes[(4 + c) * S + i] * gi.x + planes[(10 + c) * S + i] * gi.y;
+        for (int u = 0; u < 4; u++) i[u] = k + u * kPoseAdjThreads < k1 ? fobs[k + u * kPoseAdjThreads] : -1;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (i[u] >= 0) {
+                const float2 gi = g[i[u]];
+                a[u] += pu[i[u]] * gi.x + pv[i[u]] * gi.y;
+            }
     }
+    float s = (a[0] + a[1]) + (a[2] + a[3]);
 #pragma unroll
-    for (int c = 0; c < 6; c++) red[c][threadIdx.x] = a[c];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s)
-#pragma unroll
-            for (int c = 0; c < 6; c++) red[c][threadIdx.x] += red[c][threadIdx.x + s];
-        __syncthreads();
+    if (threadIdx.x == 0) {
+        float t = 0.f;
+        for (int w = 0; w < kPoseAdjThreads / 64; w++) t += red[w];
+        gout[6 * f + c] = t;
     }
-    if (threadIdx.x < 6) gout[6 * f + threadIdx.x] = red[threadIdx.x][0];
+}
+
+// the residual planes as rows (e_u, e_v)
+__global__ __launch_bounds__(256) void k_ba_residual_rows(const float* planes, long long S, float2* out) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i < S) out[i] = make_float2(planes[i], planes[S + i]);
 }
 
 }  // namespace mcv
@@ -1518,7 +1537,8 @@ __global__ __launch_bounds__(256) void k_max_partials(const float* partial, int 
 
 // FP64 point estimates -> (hi, lo) float pairs; with xl, first the additive
 // update P += x_l of the free points (VertexSBAPointXYZ::oplusImpl)
-__global__ __launch_bounds__(256) void k_ba_points_apply(double* p64, const float* xl, const uint8_t* fixed, int P,
+template <typename T>
+__global__ __launch_bounds__(256) void k_ba_points_apply(double* p64, const T* xl, const uint8_t* fixed, int P,
                                                          float4* hi, float4* lo) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= P) return;

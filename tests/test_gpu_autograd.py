@@ -117,3 +117,61 @@ def test_adjoint_at_150k_observations(gpu_ctx):
         print(f"adjoint 150k: max rel err {err.max():.2e}", flush=True)
         assert err.max() < 1e-5
     lin.close()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+def test_increments_on_the_device(gpu_ctx, dtype):
+    """Increments applied on the device against the host's: full tensors of
+    both types, strided ones, one frame's increment zero; broadcast and
+    half-precision increments still take the host's way."""
+    import torch
+    prob = _problem()
+    lin = BALinearizer.from_problem(prob, ctx=gpu_ctx)
+    F, P = len(prob.frames), len(prob.points)
+    dt = getattr(torch, dtype)
+    rng = np.random.default_rng(2)
+    dp = torch.from_numpy(rng.normal(size=(F, 6)) * 1e-2).to(dt).cuda()
+    dp[1] = 0
+    dx = torch.from_numpy(rng.normal(size=(P, 3)) * 1e-2).to(dt).cuda()
+    state = (prob.points, prob.frames, prob.cams)
+
+    def check(a, b):
+        e = reprojection(a, b, lin, state)
+        assert e.shape == (lin.M, 2) and e.is_contiguous()
+        re = _oracle_e(prob, a.double().cpu().numpy(), b.double().cpu().numpy())
+        err = np.linalg.norm(e.cpu().numpy() - re, axis=1) / np.maximum(np.linalg.norm(re, axis=1), 1e-9)
+        assert err.max() < 1e-5
+        pts, frs = apply_increments(prob.points, prob.frames, a.double().cpu().numpy(), b.double().cpu().numpy())
+        got_pts, got_frs = lin.get_state()
+        np.testing.assert_array_equal(got_pts, pts)
+        assert np.abs(got_frs - frs * np.where(frs[:, 3:4] < 0, np.array([[-1.] * 4 + [1.] * 3]), 1.0)).max() < 1e-13
+
+    check(dp, dx)
+    check(dp.repeat(1, 2)[:, ::2], dx.t().contiguous().t())
+    check(dp, dx[:1])                     # one increment for every point
+    if dtype == "float32":
+        check(dp.half(), dx)
+    lin.close()
+
+
+@pytest.mark.parametrize("n_kf,n_points,obs", [(1, 40, 40), (2, 900, 1500), (1, 4200, 4200)])
+def test_pose_adjoint_sizes(gpu_ctx, n_kf, n_points, obs):
+    """Frames of fewer observations than the adjoint's workgroup has threads,
+    and of a little more than one round of it.  Bound: sums of n float32
+    products in any order, n eps sum |J^T g|."""
+    import torch
+    prob = synth.ba_problem(seed=50 + n_kf, n_kf=n_kf, n_points=n_points, target_obs=obs)
+    lin = BALinearizer.from_problem(prob, ctx=gpu_ctx)
+    F, P, M = len(prob.frames), len(prob.points), len(prob.obs_pt)
+    z = lambda n, k: torch.zeros((n, k), dtype=torch.float32, device="cuda", requires_grad=True)
+    dpose, dpoint = z(F, 6), z(P, 3)
+    e = reprojection(dpose, dpoint, lin, (prob.points, prob.frames, prob.cams))
+    G = np.random.default_rng(1).normal(size=(M, 2)).astype(np.float32)
+    (e * torch.from_numpy(G).cuda()).sum().backward()
+    J = lin.results()[3].astype(np.float64)
+    terms = np.einsum("mij,mi->mj", J, G.astype(np.float64))
+    want, mag = np.zeros((F, 6)), np.zeros((F, 6))
+    np.add.at(want, prob.obs_frame, terms)
+    np.add.at(mag, prob.obs_frame, np.einsum("mij,mi->mj", np.abs(J), np.abs(G).astype(np.float64)))
+    assert (np.abs(dpose.grad.cpu().numpy() - want) <= M * 2.0 ** -24 * mag + 1e-30).all()
+    lin.close()
