@@ -2975,8 +2975,8 @@ static void ba_upload_points(mcv_ba* b, const double* points, const T* d_delta, 
     b->plo.ensure((size_t)b->P * 16);
     io.up(b->p64.p, points, (size_t)b->P * 24);
     io.send();
-    hipLaunchKernelGGL(k_ba_points_apply<T>, dim3((b->P + 255) / 256), dim3(256), 0, s, b->p64.as<double>(), d_delta,
-                       (const uint8_t*)nullptr, b->P, b->phi.as<float4>(), b->plo.as<float4>());
+    hipLaunchKernelGGL(k_ba_points_apply<T>, dim3((b->P + 255) / 256), dim3(256), 0, s, b->p64.as<double>(),
+                       (double*)nullptr, false, d_delta, (const uint8_t*)nullptr, b->P, b->phi.as<float4>(), b->plo.as<float4>());
     HIP_OK(hipGetLastError());
 }
 
@@ -3835,6 +3835,7 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
     const uint8_t* pfix = b->point_fixed.empty() ? nullptr : b->pfix_d.as<uint8_t>();
     const int pblocks = (P + 255) / 256;
     std::vector<float> Sf((size_t)n * n), bsf(n), bpf(n), xpf(n);
+    HostIO io(c);
     std::vector<double> S((size_t)n * n), bs(n), bp(n), xp(n);
     double lambda = 0, ni = 2;
     int it_done = 0;
@@ -3842,8 +3843,7 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
         // computeActiveErrors + activeRobustChi2 + buildSystem's linearization
         ba_lin_all(b, full_mode, s);
         ba_enqueue_rho(b, s, 0);
-        double currentChi = ba_read_double(b, s, 0);
-        if (stats) stats[4 * it] = currentChi;
+        double currentChi = 0;  // read with the first trial's system
         if (it == 0) {
             // computeLambdaInit: tau * the largest diagonal entry of H
             ba_enqueue_schur(b, 1.f, s, false);
@@ -3855,24 +3855,25 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
                                mblocks, b->fmax.as<float>());
             HIP_OK(hipGetLastError());
             float mx = 0;
-            HIP_OK(hipMemcpyAsync(&mx, b->fmax.p, 4, hipMemcpyDeviceToHost, s));
-            HIP_OK(hipStreamSynchronize(s));
+            io.down(&mx, b->fmax.p, 4);
+            io.fetch();
             lambda = tau * (double)mx;
             ni = 2;
         }
         double rho = 0;
         int qmax = 0;
         do {
-            // push
+            // push (the points' part goes with their update)
             const std::vector<double> frames0 = b->h_frames;
-            HIP_OK(hipMemcpyAsync(b->p64_bak.p, b->p64.p, (size_t)P * 24, hipMemcpyDeviceToDevice, s));
             ba_enqueue_schur(b, (float)lambda, s);
             if (n) {
-                HIP_OK(hipMemcpyAsync(Sf.data(), b->sargs.Sout, Sf.size() * 4, hipMemcpyDeviceToHost, s));
-                HIP_OK(hipMemcpyAsync(bsf.data(), b->sargs.bs, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-                HIP_OK(hipMemcpyAsync(bpf.data(), b->sargs.bp, (size_t)n * 4, hipMemcpyDeviceToHost, s));
+                io.down(Sf.data(), b->sargs.Sout, Sf.size() * 4);
+                io.down(bsf.data(), b->sargs.bs, (size_t)n * 4);
+                io.down(bpf.data(), b->sargs.bp, (size_t)n * 4);
             }
-            HIP_OK(hipStreamSynchronize(s));
+            if (qmax == 0) io.down(&currentChi, b->dsum.as<double>(), 8);
+            io.fetch();
+            if (qmax == 0 && stats) stats[4 * it] = currentChi;
             for (size_t k = 0; k < Sf.size(); k++) S[k] = Sf[k];
             for (int k = 0; k < n; k++) { bs[k] = bsf[k]; bp[k] = bpf[k]; }
             // FP64 Cholesky of the reduced camera system
@@ -3883,7 +3884,10 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
                     xpf[k] = (float)xp[k];
                     scale += xp[k] * (lambda * xp[k] + bp[k]);
                 }
-                if (n) HIP_OK(hipMemcpyAsync(b->xp.p, xpf.data(), (size_t)n * 4, hipMemcpyHostToDevice, s));
+                for (int f = 0; f < b->F; f++)
+                    if (fidx[f] >= 0) se3_oplus(&b->h_frames[7 * (size_t)f], &xp[6 * (size_t)fidx[f]]);
+                io.up(b->xp.p, xpf.data(), (size_t)n * 4);
+                ba_upload_frames(b, io);
                 const SchurArgs a = ba_schur_args(b, (float)lambda);
                 const int bblocks = (P + 31) / 32;
                 hipLaunchKernelGGL(k_schur_backsub, dim3(bblocks), dim3(256), 0, s, a, b->xp.as<float>(),
@@ -3892,22 +3896,18 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
                                    b->dsum.as<double>() + 1);
                 // update: points on the device, frames on the host
                 hipLaunchKernelGGL(k_ba_points_apply<float>, dim3(std::max(pblocks, 1)), dim3(256), 0, s,
-                                   b->p64.as<double>(), b->xl.as<float>(), pfix, P, b->phi.as<float4>(),
-                                   b->plo.as<float4>());
+                                   b->p64.as<double>(), b->p64_bak.as<double>(), false, b->xl.as<float>(), pfix, P,
+                                   b->phi.as<float4>(), b->plo.as<float4>());
                 HIP_OK(hipGetLastError());
-                for (int f = 0; f < b->F; f++)
-                    if (fidx[f] >= 0) se3_oplus(&b->h_frames[7 * (size_t)f], &xp[6 * (size_t)fidx[f]]);
-                {
-                    HostIO io(c);
-                    ba_upload_frames(b, io);
-                }
-                scale += ba_read_double(b, s, 1);
             }
             // computeActiveErrors at the new state
             ba_lin_all(b, kBaResidual, s);
             ba_enqueue_rho(b, s, 2);
-            double tempChi = ba_read_double(b, s, 2);
-            if (!ok2) tempChi = DBL_MAX;
+            double sums[2];  // x_l's part of the scale, chi2
+            io.down(sums, b->dsum.as<double>() + 1, 16);
+            io.fetch();
+            const double tempChi = ok2 ? sums[1] : DBL_MAX;
+            if (ok2) scale += sums[0];
             scale += 1e-3;
             rho = (currentChi - tempChi) / scale;
             if (rho > 0 && std::isfinite(tempChi)) {
@@ -3920,16 +3920,14 @@ int mcv_ba_optimize(mcv_ba* b, int iterations, double tau, int max_trials, doubl
                 lambda *= ni;
                 ni *= 2;
                 // pop
-                b->h_frames = frames0;
-                {
-                    HostIO io(c);
+                if (ok2) {
+                    b->h_frames = frames0;
                     ba_upload_frames(b, io);
+                    hipLaunchKernelGGL(k_ba_points_apply<float>, dim3(std::max(pblocks, 1)), dim3(256), 0, s,
+                                       b->p64.as<double>(), b->p64_bak.as<double>(), true, (const float*)nullptr,
+                                       (const uint8_t*)nullptr, P, b->phi.as<float4>(), b->plo.as<float4>());
+                    HIP_OK(hipGetLastError());
                 }
-                HIP_OK(hipMemcpyAsync(b->p64.p, b->p64_bak.p, (size_t)P * 24, hipMemcpyDeviceToDevice, s));
-                hipLaunchKernelGGL(k_ba_points_apply<float>, dim3(std::max(pblocks, 1)), dim3(256), 0, s,
-                                   b->p64.as<double>(), (const float*)nullptr, (const uint8_t*)nullptr, P,
-                                   b->phi.as<float4>(), b->plo.as<float4>());
-                HIP_OK(hipGetLastError());
                 if (!std::isfinite(lambda)) break;
             }
             qmax++;

@@ -1536,13 +1536,20 @@ __global__ __launch_bounds__(256) void k_max_partials(const float* partial, int 
 }
 
 // FP64 point estimates -> (hi, lo) float pairs; with xl, first the additive
-// update P += x_l of the free points (VertexSBAPointXYZ::oplusImpl)
+// update P += x_l of the free points (VertexSBAPointXYZ::oplusImpl).  bak keeps
+// the estimates from before it; restore: they come back from there.
 template <typename T>
-__global__ __launch_bounds__(256) void k_ba_points_apply(double* p64, const T* xl, const uint8_t* fixed, int P,
-                                                         float4* hi, float4* lo) {
+__global__ __launch_bounds__(256) void k_ba_points_apply(double* p64, double* bak, bool restore, const T* xl,
+                                                         const uint8_t* fixed, int P, float4* hi, float4* lo) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= P) return;
-    double v[3] = {p64[3 * p], p64[3 * p + 1], p64[3 * p + 2]};
+    const double* src = restore ? bak : p64;
+    double* dst = restore ? p64 : bak;
+    double v[3] = {src[3 * p], src[3 * p + 1], src[3 * p + 2]};
+    if (dst) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) dst[3 * p + k] = v[k];
+    }
     if (xl && !(fixed && fixed[p])) {
 #pragma unroll
         for (int k = 0; k < 3; k++) {
