@@ -581,6 +581,8 @@ struct OrbPlan {
         cap = max_slots_img;
         heap_cap = 16;
         for (const LevelDesc& d : lv) heap_cap = std::max(heap_cap, std::max(d.nfeat, d.n_ini) + 16);
+        // the slots that pop_pairs reads
+        heap_cap = heap_cap <= 128 ? 128 : heap_cap <= 256 ? 256 : std::max(heap_cap, 512);
         // octree workgroups of 1024 threads: every level of a small batch, the
         // large levels (the most FAST candidates) of a larger one
         build_levels.clear();

@@ -1178,7 +1178,7 @@ __global__ __launch_bounds__(kOctThreads) void k_octree_build(OrbGlobals g, cons
 // without children, at the deepest depth, carries its own index instead),
 // so a popped node's children are known without another lookup.
 //
-// The whole wave runs the heap (push_rows, heap_pop_wave: one LDS round trip per gathered
+// The whole wave runs the heap (push_rows, pop_pairs: one LDS round trip per gathered
 // chain or 5-level subtree), and lanes 0..4 fetch the counts and child
 // ranges of a popped node's children together from the node tables in
 // global memory.  The workgroup's LDS is the heap alone (8 bytes per entry),
@@ -1264,24 +1264,42 @@ __device__ __forceinline__ bool in_lanes(unsigned long long m) { return __builti
 // v): move parents down while parent < value, then place the value.  Lane l of
 // a row reads the l-th parent above the new slot; the run of parents smaller
 // than the value (keys never decrease upwards) moves down one step each, and
-// the lane past the run holds the value's place.  A value that stays in its
-// slot leaves the later rows' parents as they were read, so one round trip
-// serves all values up to and including the first that moves (in a heap of
-// fewer than 3 a later row's parent may be an earlier row's new slot: those
-// rows wait for the next round).  Returns how many were pushed.
+// the lane past the run holds the value's place.  One round trip serves all
+// rows: what a row moves, the later rows' parents take over from its lanes.
+// (In a heap of fewer than 3 a later row's parent may be an earlier row's new
+// slot: those rows wait for the next call.)  Returns how many were pushed.
 __device__ __forceinline__ int push_rows(uint2* H, int len, int n, uint2 v) {
     const int lane = threadIdx.x & 63, l = lane & 15;
     n = min(n, len + 1);
     const uint32_t s0 = (uint32_t)(len + 1 + (lane >> 4)) >> l;  // the l-th slot of the row's chain
-    const uint2 p = H[s0 >> 1];
-    const bool go = hkey(p.x) < hkey(v.x);
-    const unsigned long long G = __ballot(go) & (~0ull >> (64 - 16 * n));
-    const int m = G ? __builtin_ctzll(G) >> 4 : n - 1;  // rows 0 .. m
-    const unsigned long long rows = ~0ull >> (48 - 16 * m);
-    // the first lane of each row and, in row m, the lanes above the moved parents'
-    if (in_lanes((0x0001000100010001ull | (G << 1)) & rows)) H[s0] = go ? p : v;
+    uint2 p = H[s0 >> 1];
+    unsigned long long rows = ~0ull >> (64 - 16 * n);  // still to push
+    for (;;) {
+        const bool go = hkey(p.x) < hkey(v.x);
+        const unsigned long long G = __ballot(go) & rows;
+        const uint2 w = go ? p : v;
+        if (G == 0) {
+            if (in_lanes(0x0001000100010001ull & rows)) H[s0] = w;
+            break;
+        }
+        // up to the first row that moves: the first lane of each row and, in
+        // that row, the lanes above the moved parents'
+        const int m = __builtin_ctzll(G) >> 4;
+        const unsigned long long done = ~0ull >> (48 - 16 * m), run = (G << 1) & done;
+        if (in_lanes(((0x0001000100010001ull & rows) | run) & done)) H[s0] = w;
+        rows &= ~done;
+        if (rows == 0) break;
+        for (unsigned long long b = run; b; b &= b - 1) {
+            const int j = __builtin_ctzll(b);
+            const uint32_t c = __builtin_amdgcn_readlane(s0, j), wx = __builtin_amdgcn_readlane(w.x, j),
+                           wy = __builtin_amdgcn_readlane(w.y, j);
+            const bool same = (s0 >> 1) == c;
+            p.x = same ? wx : p.x;
+            p.y = same ? wy : p.y;
+        }
+    }
     lds_order();
-    return m + 1;
+    return n;
 }
 
 // 5-level subtrees gathered in one LDS round trip: lane (2^d - 2) + k holds
@@ -1337,9 +1355,7 @@ __device__ __forceinline__ SubLanes sub_lanes() {
 // the larger of the two; the ancestors are one ballot and the lane's ancestor
 // mask.  The round's moves are one store; in the last one lane 63 stores x and
 // lane 62 the popped entry, with count 0, in the freed slot, where the drain
-// keeps it.  (The key and payload in two arrays, the moves, x and the drained
-// word in stores of their own: 455 ns a pop, 330 ns so; with the pushes one
-// by one 1.1 us a split, 0.7 us so.)
+// keeps it.  For the heaps that pop_pairs does not take.
 __device__ __forceinline__ void heap_pop_wave(uint2* H, int& len, const SubLanes& S, uint2& top) {
     const int lane = threadIdx.x & 63;
     const int n = len;
@@ -1374,6 +1390,97 @@ __device__ __forceinline__ void heap_pop_wave(uint2* H, int& len, const SubLanes
     }
 }
 
+// Per-lane constants of pop_pairs: as a parent p = lane of the heap's top, its
+// ancestors as bits and which of them are left to the right.
+struct PairLanes {
+    uint32_t anc, dir;
+};
+
+__device__ __forceinline__ PairLanes pair_lanes() {
+    const uint32_t lane = threadIdx.x & 63;
+    PairLanes S{0, 0};
+    if (lane == 0) S.anc = S.dir = 1;  // no parent: slot 0 is never smaller than slot 1, so the test fails
+    for (uint32_t p = lane; p > 1; p >>= 1) {
+        S.anc |= 1u << (p >> 1);
+        S.dir |= (p & 1) << (p >> 1);
+    }
+    return S;
+}
+
+// heap_pop_wave for heaps of fewer than 128 R entries, 128 R slots of which are
+// readable: the whole heap comes in one LDS round trip, lane l holding the
+// children of the parents 64 r + l as pairs.  x, the last entry, leaves its slot
+// first; free slots have count 0, which is never the larger child nor >= x.
+// Per parent: the larger child, and whether that is >= x.  A parent below 64
+// is on the walk when each of its ancestors moves its larger child and that
+// leads here; below that the walk goes on by bit tests.  A wave alone issues an
+// instruction every 5 cycles or so, and that is what a pop costs: draining 434
+// entries 890 cycles each by two rounds of heap_pop_wave, 510 so.
+template <int R>
+__device__ __forceinline__ void pop_pairs(uint2* H, int& len, const PairLanes& S, uint2& top) {
+    const int lane = threadIdx.x & 63;
+    const int n = len;
+    len = n - 1;
+    const uint2 x = H[n];
+    lds_order();
+    if (n == 1) {
+        top.x = __builtin_amdgcn_readfirstlane(x.x);
+        top.y = __builtin_amdgcn_readfirstlane(x.y);
+        return;
+    }
+    if (lane == 0) H[n] = make_uint2(0, 0);
+    lds_order();
+    uint2 big[R];
+    unsigned long long right[R], go[R];
+    uint4 q[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) q[r] = reinterpret_cast<const uint4*>(H)[64 * r + lane];
+    lds_order();
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const bool rt = (q[r].z | 7u) >= q[r].x;  // by counts alone
+        right[r] = __ballot(rt);
+        big[r] = rt ? make_uint2(q[r].z, q[r].w) : make_uint2(q[r].x, q[r].y);
+        go[r] = __ballot((big[r].x | 7u) >= x.x);
+    }
+    top.x = __builtin_amdgcn_readlane(q[0].z, 0);
+    top.y = __builtin_amdgcn_readlane(q[0].w, 0);
+    const unsigned long long walk = __ballot(((((uint32_t)right[0] ^ S.dir) | ~(uint32_t)go[0]) & S.anc) == 0);
+    const unsigned long long moved = walk & go[0];
+    if (in_lanes(moved)) H[lane] = big[0];
+    int hole = 63 - __builtin_clzll(walk);
+    if ((moved >> hole) & 1) {
+        hole = 2 * hole + (int)((right[0] >> hole) & 1);  // 64 .. 127
+        if constexpr (R > 1) {
+            int k = hole - 64;
+            if ((go[1] >> k) & 1) {
+                if (lane == k) H[hole] = big[1];
+                hole = 2 * hole + (int)((right[1] >> k) & 1);  // 128 .. 255
+                if constexpr (R > 2) {
+                    k = hole & 63;
+                    const bool hi = hole >= 192;
+                    if (((hi ? go[3] : go[2]) >> k) & 1) {
+                        if (lane == k) H[hole] = hi ? big[3] : big[2];
+                        hole = 2 * hole + (int)(((hi ? right[3] : right[2]) >> k) & 1);
+                    }
+                }
+            }
+        }
+    }
+    if (lane == 0) {
+        H[hole] = x;
+        H[n] = make_uint2(q[0].z & 7u, q[0].w);  // the popped entry, for the drain
+    }
+    lds_order();
+}
+
+__device__ __forceinline__ void heap_pop(uint2* H, int& len, const SubLanes& SL, const PairLanes& PL, uint2& top) {
+    if (len < 128) pop_pairs<1>(H, len, PL, top);
+    else if (len < 256) pop_pairs<2>(H, len, PL, top);
+    else if (len < 512) pop_pairs<4>(H, len, PL, top);
+    else heap_pop_wave(H, len, SL, top);
+}
+
 // heap entry of node c from start[c], start[c+1], child[c], child[c+1]
 __device__ __forceinline__ uint2 node_entry(uint32_t c, uint32_t s0, uint32_t s1, uint32_t c0, uint32_t c1) {
     const uint32_t nch = c1 - c0;
@@ -1401,27 +1508,41 @@ __device__ __forceinline__ int tab_pairs_load(const NodeTabs& nt, uint2* T, int 
     return n;
 }
 
-// pushes the nodes c0 .. c0 + nch - 1 (at most 4), in that order: row j of 16
-// lanes reads the table entries of the j-th left to push, in the round trip
-// that reads its parents
+// The table entries of the nodes c0 .. c0 + n - 1 (n <= 4), row j of 16 lanes
+// the j-th's, asked for; entry() is what to push.
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+struct NodeRows {
+    uint32_t c;
+    u32x2 a, b;  // (start, child) of c and of c + 1
+    __device__ __forceinline__ uint2 entry() const { return node_entry(c, a.x, b.x, a.y, b.y); }
+};
+
+__device__ __forceinline__ NodeRows node_rows(const NodeTabs& nt, const uint2* T, int tn, uint32_t c0, int n) {
+    NodeRows N;
+    N.c = c0 + (uint32_t)min((int)(threadIdx.x & 63) >> 4, max(n, 1) - 1);
+    if ((int)c0 + n < tn) {  // wave-uniform
+        // as LDS by type: merged with the other way's into loads of a generic
+        // address they would be several times slower
+        const __attribute__((address_space(3))) u32x2* t = (const __attribute__((address_space(3))) u32x2*)T;
+        N.a = t[N.c];
+        N.b = t[N.c + 1];
+    } else {
+        const uint32_t c1 = N.c + (n > 0 ? 1u : 0u);
+        N.a = u32x2{nt.start[N.c], nt.child[N.c]};
+        N.b = u32x2{nt.start[c1], nt.child[c1]};
+    }
+    return N;
+}
+
+// pushes the nodes c0 .. c0 + n - 1 (at most 4), in that order; N: their rows
 __device__ __forceinline__ void push_nodes(uint2* H, int& len, const NodeTabs& nt, const uint2* T, int tn, uint32_t c0,
-                                           int nch) {
-    const bool in_lds = (int)c0 + nch < tn;  // wave-uniform
-    while (nch > 0) {
-        const int row = min((int)(threadIdx.x & 63) >> 4, nch - 1);
-        const uint32_t c = c0 + (uint32_t)row;
-        uint2 a, b;
-        if (in_lds) {
-            a = T[c];
-            b = T[c + 1];
-        } else {
-            a = make_uint2(__builtin_nontemporal_load(nt.start + c), __builtin_nontemporal_load(nt.child + c));
-            b = make_uint2(__builtin_nontemporal_load(nt.start + c + 1), __builtin_nontemporal_load(nt.child + c + 1));
-        }
-        const int k = push_rows(H, len, nch, node_entry(c, a.x, b.x, a.y, b.y));
+                                           int n, NodeRows N) {
+    while (n > 0) {
+        const int k = push_rows(H, len, n, N.entry());
         len += k;
         c0 += (uint32_t)k;
-        nch -= k;
+        n -= k;
+        if (n > 0) N = node_rows(nt, T, tn, c0, n);
     }
 }
 
@@ -1473,11 +1594,35 @@ __device__ __forceinline__ void slot_order_identity(const OrbGlobals& g, const L
     for (int j = threadIdx.x & 63; j < L.out_cap + L.seed_count; j += 64) g.perm_out[L.kp_slot + j] = L.kp_slot + j;
 }
 
+// A kept node's keypoint: of the candidates sorted[s0 .. s1) the one with the
+// largest response, the first in candidate order among equals (DistributeOctTree's
+// scan, ORBextractor.cc:569-574), as its word (response << 24 | y << 12 | x).
+// 8 candidates in flight: the nodes of 3500 candidates took 34 us one by one,
+// 13 so.
+__device__ __forceinline__ uint32_t node_winner(const uint32_t* sorted, const uint32_t* cand, uint32_t s0, uint32_t s1) {
+    uint32_t best = 0, bi = 0xFFFFFFFFu;
+    for (uint32_t p = s0; p < s1; p += 8) {
+        uint32_t idx[8], w[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) idx[u] = sorted[min(p + u, s1 - 1)];
+#pragma unroll
+        for (int u = 0; u < 8; u++) w[u] = cand[idx[u]];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (bi == 0xFFFFFFFFu || (w[u] >> 24) > (best >> 24) || ((w[u] >> 24) == (best >> 24) && idx[u] < bi)) {
+                best = w[u];
+                bi = idx[u];
+            }
+    }
+    return best;
+}
+
 __global__ __launch_bounds__(64) void k_octree_heap(OrbGlobals g, const int* order, int cap, int tab_cap) {
     extern __shared__ uint32_t heap_lds[];
     uint2* H = reinterpret_cast<uint2*>(heap_lds);
     uint2* T = H + cap;
     const SubLanes SL = sub_lanes();
+    const PairLanes PL = pair_lanes();
     const int lane = threadIdx.x;
     const int li = order[blockIdx.x];
     const LevelDesc L = g.lv[li];
@@ -1490,45 +1635,44 @@ __global__ __launch_bounds__(64) void k_octree_heap(OrbGlobals g, const int* ord
     NodeTabs nt;
     nt.start = g.pool + O->tab;
     nt.child = nt.start + O->total;
-    if (lane == 0) H[0] = make_uint2(0xFFFFFFFFu, 0u);
+    // slot 0 above every key, the others free
+    for (int i = lane; i < cap; i += 64) H[i] = make_uint2(i == 0 ? 0xFFFFFFFFu : 0u, 0u);
+    lds_order();
     const int tn = tab_pairs_load(nt, T, tab_cap, O->total);
     const int nr = O->n_roots;
     int len = 0;
-    for (int k = 0; k < nr; k += 4) push_nodes(H, len, nt, T, tn, (uint32_t)k, min(4, nr - k));
+    for (int k = 0; k < nr; k += 4)
+        push_nodes(H, len, nt, T, tn, (uint32_t)k, min(4, nr - k), node_rows(nt, T, tn, (uint32_t)k, min(4, nr - k)));
     const int N = min(L.nfeat, cap - 8);
     uint2 top;
     while (len > 0 && len < N) {
         // the largest node; one with a single keypoint ends the splitting
-        if (hkey(__builtin_amdgcn_readfirstlane(H[1].x)) == 1) break;
-        heap_pop_wave(H, len, SL, top);
-        push_nodes(H, len, nt, T, tn, top.y, (int)(top.x & 7u));
+        top = H[1];
+        top.x = __builtin_amdgcn_readfirstlane(top.x);
+        if (hkey(top.x) == 1) break;
+        // its children's table entries, asked for before the pop
+        const uint32_t c0 = __builtin_amdgcn_readfirstlane(top.y);
+        const int nch = (int)(top.x & 7u);
+        const NodeRows kids = node_rows(nt, T, tn, c0, nch);
+        heap_pop(H, len, SL, PL, top);
+        push_nodes(H, len, nt, T, tn, c0, nch, kids);
     }
     // drain: the j-th popped node ends in the slot that its pop frees, n0 - j,
     // its key's count 0
     const int n0 = len;
-    while (len > 1) heap_pop_wave(H, len, SL, top);
+    while (len >= 512) heap_pop_wave(H, len, SL, top);
+    while (len >= 256) pop_pairs<4>(H, len, PL, top);
+    while (len >= 128) pop_pairs<2>(H, len, PL, top);
+    while (len > 1) pop_pairs<1>(H, len, PL, top);
     wave_lds_sync();
     const int nkeep = min(n0, L.out_cap);
     if (lane == 0) O->nout = nkeep;
-    // each kept node's keypoint, one node per lane: the candidate with the
-    // largest response, the first in candidate order among equals
-    // (DistributeOctTree's scan, ORBextractor.cc:569-574); its candidate
-    // word (response << 24 | y << 12 | x) is the slot's output
     const uint32_t* sorted = g.pool + O->sorted;
     const uint32_t* cand = g.lvl_cand + L.cand_base;
     for (int jj = lane; jj < nkeep; jj += 64) {
         const uint2 e = H[n0 - jj];
         const uint32_t ny = e.y, nch = max(e.x & 7u, 1u);
-        const uint32_t s0 = nt.st(ny), s1 = nt.st(ny + nch);
-        uint32_t best = 0, bi = 0;
-        for (uint32_t p = s0; p < s1; p++) {
-            const uint32_t idx = sorted[p];
-            const uint32_t r = cand[idx];
-            if (p == s0 || (r >> 24) > (best >> 24) || ((r >> 24) == (best >> 24) && idx < bi)) {
-                best = r;
-                bi = idx;
-            }
-        }
+        const uint32_t best = node_winner(sorted, cand, nt.st(ny), nt.st(ny + nch));
         g.nodes_out[L.kp_slot + jj] = best;
         H[n0 - jj].x = best;  // the slot's word, for slot_order
     }

@@ -225,11 +225,12 @@ def test_orb_strip_edges(own_ctx, repeats):
                               enumerate([(257, 230), (255, 240), (239, 239), (514, 225), (330, 227)])], 1)
 
 
-@pytest.mark.parametrize("nfeatures", [1, 2, 5, 60, 4000, 9000])
+@pytest.mark.parametrize("nfeatures", [1, 2, 5, 60, 1284, 1292, 2000, 2580, 2600, 4000, 9000])
 def test_orb_heap_sizes(own_ctx, nfeatures):
     """The octree's heap from one entry to thousands (a heap of 1 or 2
-    entries takes its pushes one by one; beyond 2048 nodes the tables are
-    read from memory), on a wide image that starts with several roots and on
+    entries takes its pushes one by one; up to 511 and up to 1023 entries run
+    in registers; beyond the first thousands of nodes the tables are read from
+    memory), on a wide image that starts with several roots and on
     a tall one without any split."""
     orb = ORB(nfeatures, 1.2, 3, 12, 5, ctx=own_ctx)
     rng = np.random.default_rng(9)
