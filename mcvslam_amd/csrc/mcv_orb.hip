@@ -368,6 +368,9 @@ inline const char* blur_variant_name(int v) {
     return (v >= 0 && v < 4) ? names[v] : "?";
 }
 
+// lanes of a mask, as a lane condition (the mask becomes the execution mask)
+__device__ __forceinline__ bool in_lanes(unsigned long long m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
 // ---------------------------------------------------------------------------
 // FAST 9/16.  best(p) = max over the 16 arcs of 9 contiguous circle pixels
 // of min(v - p_k) (darker arc) or min(p_k - v) (brighter arc).  A pixel is a
@@ -426,7 +429,11 @@ __device__ __forceinline__ int byte_of(uint32_t w, int j) { return (int)((w >> (
 // bound rejects most pixels: every 9-arc holds two consecutive compass
 // points (0,4,8,12), so a corner at t needs such a pair both darker than
 // v - t or both brighter than v + t; the test runs on 2 pixels per packed
-// u16 operation.  Survivors queue up in LDS and are scored 64 at a time by
+// u16 operation (10 of them) and its compares are the survivors' lane masks.
+// Bound by instruction issue, some 130 per row and wave, with the survivors'
+// byte reads next: 64 frames of 3 cameras 619 us with pairwise extrema and the
+// survivors as per-lane bits, 540 so (with the circle read as 7 unaligned
+// words instead of 17 bytes 964).  Survivors queue up in LDS and are scored 64 at a time by
 // the whole wave from the ring; the group's score rows are zeroed when the
 // group starts and each score above t_lo is stored as a byte (no LDS tile,
 // so that six workgroups fit a CU's LDS).
@@ -434,23 +441,14 @@ __device__ __forceinline__ int byte_of(uint32_t w, int j) { return (int)((w >> (
 typedef short mcv_s2 __attribute__((ext_vector_type(2)));
 
 // compass test for two pixels held in the 16-bit lanes of the arguments
-// (values 0..255).  With d = p - v, a pair of neighbouring compass points is
-// darker than v - t iff max(d_a, d_b) < -t and brighter than v + t iff
-// min(d_a, d_b) > t; a lane of the result is > 0 iff some pair qualifies.
-// nt = -t in both lanes.
-__device__ __forceinline__ uint32_t compass2(mcv_us2 v, mcv_us2 s, mcv_us2 e, mcv_us2 n, mcv_us2 w, mcv_s2 t,
-                                             mcv_s2 nt) {
-    const mcv_s2 vs = __builtin_bit_cast(mcv_s2, v);
-    const mcv_s2 ds = __builtin_bit_cast(mcv_s2, s) - vs, de = __builtin_bit_cast(mcv_s2, e) - vs;
-    const mcv_s2 dn = __builtin_bit_cast(mcv_s2, n) - vs, dw = __builtin_bit_cast(mcv_s2, w) - vs;
-    const mcv_s2 mx = __builtin_elementwise_min(
-        __builtin_elementwise_min(__builtin_elementwise_max(ds, de), __builtin_elementwise_max(de, dn)),
-        __builtin_elementwise_min(__builtin_elementwise_max(dn, dw), __builtin_elementwise_max(dw, ds)));
-    const mcv_s2 mn = __builtin_elementwise_max(
-        __builtin_elementwise_max(__builtin_elementwise_min(ds, de), __builtin_elementwise_min(de, dn)),
-        __builtin_elementwise_max(__builtin_elementwise_min(dn, dw), __builtin_elementwise_min(dw, ds)));
-    const mcv_s2 r = __builtin_elementwise_max(__builtin_elementwise_max(mn - t, nt - mx), mcv_s2{0, 0});
-    return __builtin_bit_cast(uint32_t, r);
+// (values 0..255): a lane of the result is > t iff some pair of neighbouring
+// compass points is darker than v - t or brighter than v + t.  Neighbours are
+// one of north and south with one of east and west, so the darkest pair's
+// larger value is max(min(n, s), min(e, w)), and likewise for the bright one.
+__device__ __forceinline__ mcv_us2 compass2(mcv_us2 v, mcv_us2 s, mcv_us2 e, mcv_us2 n, mcv_us2 w) {
+    const mcv_us2 dark = __builtin_elementwise_max(__builtin_elementwise_min(n, s), __builtin_elementwise_min(e, w));
+    const mcv_us2 bright = __builtin_elementwise_min(__builtin_elementwise_max(n, s), __builtin_elementwise_max(e, w));
+    return __builtin_elementwise_max(__builtin_elementwise_sub_sat(v, dark), __builtin_elementwise_sub_sat(bright, v));
 }
 
 // exact best of the pixel at base[3 * kRowB]: base points into row -3 of 7
@@ -510,12 +508,10 @@ __global__ __launch_bounds__(256) void k_fast_score(const Strip* st, int n, int 
     uint16_t* queue = s_queue[wv];
     const uint8_t* img = pyr + L.pix;
     const bool own = x < L.w;
-    const mcv_s2 tt = {(short)t_lo, (short)t_lo}, ntt = {(short)-t_lo, (short)-t_lo};
-    // this lane's columns inside the detection range [3, w - 3)
-    int bmask = 0;
+    // the lanes whose column j is inside the detection range [3, w - 3)
+    unsigned long long cols[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-        if (x + j >= 3 && x + j < L.w - 3) bmask |= 1 << j;
+    for (int j = 0; j < 4; j++) cols[j] = __ballot(x + j >= 3 && x + j < L.w - 3);
     // one level row into registers: this lane's u32, plus the word left of
     // the strip (lane 0) or right of it (lane 63); rows clamp to the level
     auto load_row = [&](int r, uint32_t& a, uint32_t& e) {
@@ -567,7 +563,6 @@ __global__ __launch_bounds__(256) void k_fast_score(const Strip* st, int n, int 
         for (int y = yg; y < ye; y++) {
             const int tb = y - yg;
             wave_lds_sync();
-            int surv = 0;
             if (y >= 3 && y < L.h - 3) {
                 const uint32_t* C = ring[y & (kRing - 1)];
                 const uint32_t c0 = C[lane], c1 = C[lane + 1], c2 = C[lane + 2];
@@ -578,24 +573,22 @@ __global__ __launch_bounds__(256) void k_fast_score(const Strip* st, int n, int 
                 // south bytes and the east (x+3) and west (x-3) neighbours out of
                 // the adjacent words (selector 0x0c: zero byte)
                 const uint32_t m = 0x00FF00FFu, odd = 0x0c030c01u;
-                const uint32_t ev = compass2(as_us2(c1 & m), as_us2(dn & m), as_us2(__builtin_amdgcn_perm(c2, c1, 0x0c050c03u)),
-                                             as_us2(up & m), as_us2(__builtin_amdgcn_perm(c1, c0, 0x0c030c01u)), tt, ntt);
-                const uint32_t od = compass2(as_us2(__builtin_amdgcn_perm(0u, c1, odd)), as_us2(__builtin_amdgcn_perm(0u, dn, odd)),
+                const mcv_us2 ev = compass2(as_us2(c1 & m), as_us2(dn & m), as_us2(__builtin_amdgcn_perm(c2, c1, 0x0c050c03u)),
+                                             as_us2(up & m), as_us2(__builtin_amdgcn_perm(c1, c0, 0x0c030c01u)));
+                const mcv_us2 od = compass2(as_us2(__builtin_amdgcn_perm(0u, c1, odd)), as_us2(__builtin_amdgcn_perm(0u, dn, odd)),
                                              as_us2(__builtin_amdgcn_perm(c2, c1, 0x0c060c04u)),
                                              as_us2(__builtin_amdgcn_perm(0u, up, odd)),
-                                             as_us2(__builtin_amdgcn_perm(c1, c0, 0x0c040c02u)), tt, ntt);
-                // each 16-bit lane capped at 1, then bit 0 / 16 of ev and od
-                // moved to bits 0..3 (pixel order 0, 1, 2, 3)
-                const uint32_t e1 = as_u32(__builtin_elementwise_min(as_us2(ev), mcv_us2{1, 1}));
-                const uint32_t o1 = as_u32(__builtin_elementwise_min(as_us2(od), mcv_us2{1, 1}));
-                const uint32_t t2 = e1 | (o1 << 1);
-                surv = (int)(((t2 & 3u) | ((t2 >> 14) & 12u)) & (uint32_t)bmask);
-            }
+                                             as_us2(__builtin_amdgcn_perm(c1, c0, 0x0c040c02u)));
+                // pixel j's survivors as a lane mask, straight from the compare
+                const unsigned long long surv[4] = {__ballot(ev.x > t_lo) & cols[0], __ballot(od.x > t_lo) & cols[1],
+                                                    __ballot(ev.y > t_lo) & cols[2], __ballot(od.y > t_lo) & cols[3]};
+                if (surv[0] | surv[1] | surv[2] | surv[3]) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const unsigned long long b = __ballot((surv >> j) & 1);
-                if ((surv >> j) & 1) queue[qlen + lanes_below(b)] = (uint16_t)((tb << 8) | (4 * lane + j));
-                qlen += __popcll(b);
+                    for (int j = 0; j < 4; j++) {
+                        if (in_lanes(surv[j])) queue[qlen + lanes_below(surv[j])] = (uint16_t)((tb << 8) | (4 * lane + j));
+                        qlen += __popcll(surv[j]);
+                    }
+                }
             }
             const bool block_end = y == ye - 1;
             while (qlen >= 64 || (block_end && qlen > 0)) {
@@ -1255,9 +1248,6 @@ __device__ __forceinline__ void tab_children(const NodeTabs& nt, const TabPrefix
 // chain of dependent steps, so what counts are the LDS round trips and the
 // instructions on that chain.
 __device__ __forceinline__ uint32_t hkey(uint32_t k) { return k >> 3; }
-
-// lanes of a mask, as a lane condition (the mask becomes the execution mask)
-__device__ __forceinline__ bool in_lanes(unsigned long long m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
 // push_heap's __push_heap(first, hole, 0, value) for `n` <= 4 values in a row,
 // the j-th pushed by row j of 16 lanes (every lane of a row holds its value
