@@ -930,11 +930,11 @@ struct mcv_ctx {
         return side;
     }
 
-    // host memory the device writes k_pose_eval's sums to
-    double* sums = nullptr;
-    double* pose_sums() {
-        if (!sums) HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&sums), kPoseSums * sizeof(double), hipHostMallocDefault));
-        return sums;
+    // host memory the device writes a pose optimization's outcome to
+    void* pose = nullptr;
+    void* pose_out() {
+        if (!pose) HIP_OK(hipHostMalloc(&pose, sizeof(PoseRun) + 4 * kPoseIters * sizeof(double), hipHostMallocDefault));
+        return pose;
     }
     // pinned host memory for HostIO
     char* pin = nullptr;
@@ -943,7 +943,7 @@ struct mcv_ctx {
         return pin;
     }
     ~mcv_ctx() {
-        if (sums) (void)hipHostFree(sums);
+        if (pose) (void)hipHostFree(pose);
         if (pin) (void)hipHostFree(pin);
     }
 
@@ -2894,63 +2894,14 @@ int mcv_ba_set_observations(mcv_ba* b, const float* uv, const int32_t* pt, const
     API_END
 }
 
-// double -> (hi, lo) float pair
-static inline void split(double v, float& hi, float& lo) {
-    hi = (float)v;
-    lo = (float)(v - (double)hi);
-}
-
-static void quat_to_R(const double* q, double R[9]) {
-    const double x = q[0], y = q[1], z = q[2], w = q[3];
-    const double tx = 2 * x, ty = 2 * y, tz = 2 * z;
-    const double twx = tx * w, twy = ty * w, twz = tz * w;
-    const double txx = tx * x, txy = ty * x, txz = tz * x;
-    const double tyy = ty * y, tyz = tz * y, tzz = tz * z;
-    R[0] = 1 - (tyy + tzz); R[1] = txy - twz; R[2] = txz + twy;
-    R[3] = txy + twz; R[4] = 1 - (txx + tzz); R[5] = tyz - twx;
-    R[6] = txz - twy; R[7] = tyz + twx; R[8] = 1 - (txx + tyy);
-}
 
 // One frame's (frame, camera) records of the mono edges and its pose for the
-// stereo edges from its FP64 state; without the robust kernel the Huber
-// deltas are infinite (w = 1, rho = chi2).
+// stereo edges from its FP64 state
 static void ba_frame_records(const mcv_ba* b, const double* fq, BAPair* pr, FramePose& fp) {
-    const double* cams = b->h_cams.data();
     double Rbw[9];
-    // g2o SE3Quat keeps a normalised quaternion with w >= 0 (se3quat.h:280-285)
-    double q[4] = {fq[0], fq[1], fq[2], fq[3]};
-    double qn = std::sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
-    for (double& v : q) v /= qn;
-    quat_to_R(q, Rbw);
-    const double* tbw = fq + 4;
-    for (int i = 0; i < 9; i++) split(Rbw[i], fp.Rh[i], fp.Rl[i]);
-    for (int i = 0; i < 3; i++) split(tbw[i], fp.th[i], fp.tl[i]);
-    for (int k = 0; k < b->C; k++) {
-        const double* cm = cams + 12 * k;
-        double Rcb[9];
-        double qc[4] = {cm[4], cm[5], cm[6], cm[7]};
-        double qcn = std::sqrt(qc[0] * qc[0] + qc[1] * qc[1] + qc[2] * qc[2] + qc[3] * qc[3]);
-        for (double& v : qc) v /= qcn;
-        quat_to_R(qc, Rcb);
-        const double* tcb = cm + 8;
-        BAPair& P = pr[k];
-        // Tcw = Tcb * Tbw
-        for (int r = 0; r < 3; r++) {
-            for (int cc = 0; cc < 3; cc++) {
-                double v = 0;
-                for (int m = 0; m < 3; m++) v += Rcb[3 * r + m] * Rbw[3 * m + cc];
-                split(v, P.Rh[3 * r + cc], P.Rl[3 * r + cc]);
-            }
-            double tv = tcb[r];
-            for (int m = 0; m < 3; m++) tv += Rcb[3 * r + m] * tbw[m];
-            split(tv, P.th[r], P.tl[r]);
-        }
-        for (int i = 0; i < 9; i++) { P.Rbw[i] = (float)Rbw[i]; P.Rcb[i] = (float)Rcb[i]; }
-        for (int i = 0; i < 3; i++) P.tbw[i] = (float)tbw[i];
-        P.fx = (float)cm[0]; P.fy = (float)cm[1]; P.cx = (float)cm[2]; P.cy = (float)cm[3];
-        P.delta = b->robust ? (float)cm[11] : INFINITY;
-        P.pad[0] = P.pad[1] = P.pad[2] = 0.f;
-    }
+    frame_rotation(fq, Rbw);
+    pose_record(Rbw, fq + 4, fp);
+    for (int k = 0; k < b->C; k++) pair_record(Rbw, fq + 4, b->h_cams.data() + 12 * k, b->robust, pr[k]);
 }
 
 // every frame's records to the device
@@ -3000,8 +2951,6 @@ int mcv_ba_set_state(mcv_ba* b, const double* points, const double* frames, cons
     b->touched(-1);
     API_END
 }
-
-static void se3_oplus(double* frame, const double* xi);
 
 int mcv_ba_set_state_increments(mcv_ba* b, const double* points, const double* frames, const double* cams,
                                 const void* d_pose, int pose_fp64, const void* d_point, int point_fp64) {
@@ -3563,90 +3512,6 @@ int mcv_solve_llt(int n, const double* S, const double* b, double* x) {
 }  // extern "C"
 
 // ---- Levenberg-Marquardt over the GPU data ------------------------------------
-// Pose increment T <- exp(x) * T of VertexSE3Expmap::oplusImpl
-// (types/sba/types_six_dof_expmap.h:98-101): SE3Quat::exp
-// (types/slam3d/se3quat.h:218-257) with Eigen's matrix -> quaternion
-// conversion, then the product with a normalised (w >= 0) quaternion.
-struct Qd { double x, y, z, w; };
-
-static Qd qd_mul(const Qd& a, const Qd& b) {
-    return Qd{a.w * b.x + a.x * b.w + a.y * b.z - a.z * b.y, a.w * b.y + a.y * b.w + a.z * b.x - a.x * b.z,
-              a.w * b.z + a.z * b.w + a.x * b.y - a.y * b.x, a.w * b.w - a.x * b.x - a.y * b.y - a.z * b.z};
-}
-
-static void qd_rotate(const Qd& q, const double v[3], double o[3]) {
-    double uv[3] = {q.y * v[2] - q.z * v[1], q.z * v[0] - q.x * v[2], q.x * v[1] - q.y * v[0]};
-    for (double& c : uv) c += c;
-    o[0] = v[0] + q.w * uv[0] + (q.y * uv[2] - q.z * uv[1]);
-    o[1] = v[1] + q.w * uv[1] + (q.z * uv[0] - q.x * uv[2]);
-    o[2] = v[2] + q.w * uv[2] + (q.x * uv[1] - q.y * uv[0]);
-}
-
-static void qd_normalize(Qd& q) {
-    if (q.w < 0) q = Qd{-q.x, -q.y, -q.z, -q.w};
-    const double n = std::sqrt(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w);
-    q = Qd{q.x / n, q.y / n, q.z / n, q.w / n};
-}
-
-static Qd qd_from_R(const double* m) {
-    Qd q{};
-    double t = m[0] + m[4] + m[8];
-    if (t > 0) {
-        t = std::sqrt(t + 1.0);
-        q.w = 0.5 * t;
-        t = 0.5 / t;
-        q.x = (m[7] - m[5]) * t;
-        q.y = (m[2] - m[6]) * t;
-        q.z = (m[3] - m[1]) * t;
-    } else {
-        int i = 0;
-        if (m[4] > m[0]) i = 1;
-        if (m[8] > m[4 * i]) i = 2;
-        const int j = (i + 1) % 3, k = (j + 1) % 3;
-        double c[3];
-        t = std::sqrt(m[4 * i] - m[4 * j] - m[4 * k] + 1.0);
-        c[i] = 0.5 * t;
-        t = 0.5 / t;
-        q.w = (m[3 * k + j] - m[3 * j + k]) * t;
-        c[j] = (m[3 * j + i] + m[3 * i + j]) * t;
-        c[k] = (m[3 * k + i] + m[3 * i + k]) * t;
-        q.x = c[0]; q.y = c[1]; q.z = c[2];
-    }
-    return q;
-}
-
-static void se3_oplus(double* frame, const double* xi) {
-    const double w[3] = {xi[0], xi[1], xi[2]};
-    const double th = std::sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]);
-    const double W[9] = {0, -w[2], w[1], w[2], 0, -w[0], -w[1], w[0], 0};
-    double W2[9];
-    for (int r = 0; r < 3; r++)
-        for (int c = 0; c < 3; c++) W2[3 * r + c] = W[3 * r] * W[c] + W[3 * r + 1] * W[3 + c] + W[3 * r + 2] * W[6 + c];
-    double R[9], V[9];
-    for (int k = 0; k < 9; k++) {
-        const double I = (k % 4 == 0) ? 1.0 : 0.0;
-        if (th < 0.00001) {
-            R[k] = I + W[k] + 0.5 * W2[k];
-            V[k] = I + 0.5 * W[k] + (1.0 / 6.0) * W2[k];
-        } else {
-            R[k] = I + std::sin(th) / th * W[k] + (1 - std::cos(th)) / (th * th) * W2[k];
-            V[k] = I + (1 - std::cos(th)) / (th * th) * W[k] + (th - std::sin(th)) / std::pow(th, 3) * W2[k];
-        }
-    }
-    Qd dq = qd_from_R(R);
-    qd_normalize(dq);
-    double dt[3];
-    for (int r = 0; r < 3; r++) dt[r] = V[3 * r] * xi[3] + V[3 * r + 1] * xi[4] + V[3 * r + 2] * xi[5];
-    // exp(x) * T
-    const Qd q{frame[0], frame[1], frame[2], frame[3]};
-    double rt[3];
-    qd_rotate(dq, frame + 4, rt);
-    Qd nq = qd_mul(dq, q);
-    qd_normalize(nq);
-    frame[0] = nq.x; frame[1] = nq.y; frame[2] = nq.z; frame[3] = nq.w;
-    for (int r = 0; r < 3; r++) frame[4 + r] = dt[r] + rt[r];
-}
-
 // both edge sets linearized at the current state (mode as k_ba_linearize)
 static void ba_lin_all(mcv_ba* b, int mode, hipStream_t s) {
     ba_enqueue_linearize(b, b->variant, mode, s);
@@ -3697,7 +3562,7 @@ int mcv_ba_robust_chi2(mcv_ba* b, double* chi2) {
 }  // extern "C"
 
 // The frame of a problem whose only unknown is its pose and that fits
-// k_pose_eval, else -1.  (Points without edges would allow it too; the rule
+// k_pose_optimize, else -1.  (Points without edges would allow it too; the rule
 // asks for what PoseOptimization sets up, every point fixed.)
 static int ba_single_pose(const mcv_ba* b) {
     const int E = b->M + (b->have_stereo ? b->Ms : 0);
@@ -3711,11 +3576,8 @@ static int ba_single_pose(const mcv_ba* b) {
     return frame;
 }
 
-// The optimizer on a problem whose only unknown is one keyframe's pose: the
-// same iterations, trials and rules as mcv_ba_optimize, with one launch and
-// one wait per trial.  k_pose_eval gives chi2, H_pp and b_p of a state at
-// once, so a trial that is accepted has already linearized the next
-// iteration, and one that is rejected leaves the last H_pp and b_p in hand.
+// The optimizer on a problem whose only unknown is one keyframe's pose, on the
+// device (k_pose_optimize), kPoseIters iterations to a launch.
 static int ba_optimize_pose(mcv_ba* b, int frame, int iterations, double tau, int max_trials, double* stats,
                             hipStream_t s) {
     mcv_ctx* c = b->ctx;
@@ -3732,73 +3594,30 @@ static int ba_optimize_pose(mcv_ba* b, int frame, int iterations, double tau, in
     a.scam = b->scam;
     a.frame = frame;
     a.C = b->C;
-    double* sums = c->pose_sums();
-    a.out = sums;
+    PoseSetup q{};
+    std::copy(b->h_cams.begin(), b->h_cams.begin() + 12 * (size_t)b->C, q.cams);
+    q.tau = tau;
+    q.max_trials = max_trials;
+    q.robust = b->robust;
+    // where the kernel writes: host memory
+    PoseRun* run = reinterpret_cast<PoseRun*>(c->pose_out());
+    double* st = reinterpret_cast<double*>(run + 1);
     double* fr = &b->h_frames[7 * (size_t)frame];
-    struct Eval {
-        double chi2, S[36], b[6];
-    };
-    auto eval = [&]() {
-        PoseState st{};
-        ba_frame_records(b, fr, st.pair, st.pose);
-        hipLaunchKernelGGL(k_pose_eval, dim3(1), dim3(kPoseThreads), 0, s, a, st);
+    PoseRun in{};
+    in.ni = 2;
+    in.stop = 1;
+    int it_done = 0;
+    while (it_done < iterations) {
+        std::copy(fr, fr + 7, in.fr);
+        in.iters = std::min(iterations - it_done, kPoseIters);
+        hipLaunchKernelGGL(k_pose_optimize, dim3(1), dim3(kPoseThreads), 0, s, a, q, in, run, st);
         HIP_OK(hipGetLastError());
         HIP_OK(hipStreamSynchronize(s));
-        Eval e;
-        for (int r = 0, o = 0; r < 6; r++) {
-            for (int k = r; k < 6; k++, o++) e.S[6 * r + k] = e.S[6 * k + r] = sums[o];
-            e.b[r] = sums[o++];
-        }
-        e.chi2 = sums[27];
-        return e;
-    };
-    Eval cur = eval();
-    double lambda = 0, ni = 2;
-    int it_done = 0;
-    for (int it = 0; it < iterations; it++) {
-        if (stats) stats[4 * it] = cur.chi2;
-        if (it == 0) {
-            double mx = 0;
-            for (int k = 0; k < 6; k++) mx = std::max(mx, std::fabs(cur.S[7 * k]));
-            lambda = tau * mx;
-        }
-        double rho = 0;
-        int qmax = 0;
-        do {
-            double fr0[7], S[36], x[6];
-            std::memcpy(fr0, fr, sizeof fr0);
-            std::memcpy(S, cur.S, sizeof S);
-            for (int k = 0; k < 6; k++) S[7 * k] += lambda;
-            const bool ok = mcv_solve_llt(6, S, cur.b, x) == MCV_OK;
-            double scale = 1e-3;
-            Eval e = cur;
-            if (ok) {
-                for (int k = 0; k < 6; k++) scale += x[k] * (lambda * x[k] + cur.b[k]);
-                se3_oplus(fr, x);
-                e = eval();
-            } else {
-                e.chi2 = DBL_MAX;
-            }
-            rho = (cur.chi2 - e.chi2) / scale;
-            if (rho > 0 && std::isfinite(e.chi2)) {
-                lambda *= std::max(1. / 3., std::min(1. - std::pow(2 * rho - 1, 3), 2. / 3.));
-                ni = 2;
-                cur = e;
-            } else {
-                lambda *= ni;
-                ni *= 2;
-                std::memcpy(fr, fr0, sizeof fr0);
-                if (!std::isfinite(lambda)) break;
-            }
-            qmax++;
-        } while (rho < 0 && qmax < max_trials);
-        if (stats) {
-            stats[4 * it + 1] = cur.chi2;
-            stats[4 * it + 2] = lambda;
-            stats[4 * it + 3] = qmax;
-        }
-        it_done++;
-        if (qmax == max_trials || rho == 0 || !std::isfinite(lambda)) break;
+        in = *run;
+        std::copy(in.fr, in.fr + 7, fr);
+        if (stats) std::copy(st, st + 4 * (size_t)in.iters, stats + 4 * (size_t)it_done);
+        it_done += in.iters;
+        if (in.stop) break;
     }
     HostIO io(c);
     ba_upload_frames(b, io);

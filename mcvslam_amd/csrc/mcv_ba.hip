@@ -1374,18 +1374,169 @@ __global__ __launch_bounds__(256) void k_ba_rho_sum(const float* chi2, const uin
     if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
-// One evaluation of a problem whose only unknown is one keyframe's pose
-// (every point fixed, every other frame fixed): from the frame's state, sum of
-// rho(chi2), H_pp (upper triangle by rows, each row followed by b_p's entry)
-// in FP64 sums of the edges' FP32 terms, in a fixed order, written to host
-// memory.  Linearization, robust chi2 and normal equations in one launch of
-// one workgroup: a frame has at most a few thousand edges, so a trial of the
-// optimizer is bound by launches and by the host's wait (12 launches and 3
-// waits, 0.2 ms, before; see mcv_ba_optimize), not by the edges' arithmetic.
-constexpr int kPoseThreads = 1024;
-constexpr int kPoseCams = 8;       // cameras whose records fit the kernel arguments
+// ---- a keyframe's pose, on the host and on the device --------------------------
+// double -> (hi, lo) float pair
+__host__ __device__ inline void split(double v, float& hi, float& lo) {
+    hi = (float)v;
+    lo = (float)(v - (double)hi);
+}
+
+__host__ __device__ inline void quat_to_R(const double* q, double R[9]) {
+    const double x = q[0], y = q[1], z = q[2], w = q[3];
+    const double tx = 2 * x, ty = 2 * y, tz = 2 * z;
+    const double twx = tx * w, twy = ty * w, twz = tz * w;
+    const double txx = tx * x, txy = ty * x, txz = tz * x;
+    const double tyy = ty * y, tyz = tz * y, tzz = tz * z;
+    R[0] = 1 - (tyy + tzz); R[1] = txy - twz; R[2] = txz + twy;
+    R[3] = txy + twz; R[4] = 1 - (txx + tzz); R[5] = tyz - twx;
+    R[6] = txz - twy; R[7] = tyz + twx; R[8] = 1 - (txx + tyy);
+}
+
+// One frame's records from its FP64 state: the pose for the stereo edges, and
+// per camera (cm: fx fy cx cy, quaternion, translation, Huber delta) that of the
+// mono edges.  Without the robust kernel the Huber deltas are infinite (w = 1,
+// rho = chi2).
+__host__ __device__ inline void frame_rotation(const double* fq, double Rbw[9]) {
+    // g2o SE3Quat keeps a normalised quaternion with w >= 0 (se3quat.h:280-285)
+    const double qn = sqrt(fq[0] * fq[0] + fq[1] * fq[1] + fq[2] * fq[2] + fq[3] * fq[3]);
+    const double q[4] = {fq[0] / qn, fq[1] / qn, fq[2] / qn, fq[3] / qn};
+    quat_to_R(q, Rbw);
+}
+
+__host__ __device__ inline void pose_record(const double Rbw[9], const double* tbw, FramePose& fp) {
+    for (int i = 0; i < 9; i++) split(Rbw[i], fp.Rh[i], fp.Rl[i]);
+    for (int i = 0; i < 3; i++) split(tbw[i], fp.th[i], fp.tl[i]);
+}
+
+__host__ __device__ inline void pair_record(const double Rbw[9], const double* tbw, const double* cm, bool robust,
+                                            BAPair& P) {
+    double Rcb[9];
+    const double qn = sqrt(cm[4] * cm[4] + cm[5] * cm[5] + cm[6] * cm[6] + cm[7] * cm[7]);
+    const double qc[4] = {cm[4] / qn, cm[5] / qn, cm[6] / qn, cm[7] / qn};
+    quat_to_R(qc, Rcb);
+    const double* tcb = cm + 8;
+    // Tcw = Tcb * Tbw
+    for (int r = 0; r < 3; r++) {
+        for (int cc = 0; cc < 3; cc++) {
+            double v = 0;
+            for (int m = 0; m < 3; m++) v += Rcb[3 * r + m] * Rbw[3 * m + cc];
+            split(v, P.Rh[3 * r + cc], P.Rl[3 * r + cc]);
+        }
+        double tv = tcb[r];
+        for (int m = 0; m < 3; m++) tv += Rcb[3 * r + m] * tbw[m];
+        split(tv, P.th[r], P.tl[r]);
+    }
+    for (int i = 0; i < 9; i++) { P.Rbw[i] = (float)Rbw[i]; P.Rcb[i] = (float)Rcb[i]; }
+    for (int i = 0; i < 3; i++) P.tbw[i] = (float)tbw[i];
+    P.fx = (float)cm[0]; P.fy = (float)cm[1]; P.cx = (float)cm[2]; P.cy = (float)cm[3];
+    P.delta = robust ? (float)cm[11] : INFINITY;
+    P.pad[0] = P.pad[1] = P.pad[2] = 0.f;
+}
+
+// Pose increment T <- exp(x) * T of VertexSE3Expmap::oplusImpl
+// (types/sba/types_six_dof_expmap.h:98-101): SE3Quat::exp
+// (types/slam3d/se3quat.h:218-257) with Eigen's matrix -> quaternion
+// conversion, then the product with a normalised (w >= 0) quaternion.
+struct Qd { double x, y, z, w; };
+
+__host__ __device__ inline Qd qd_mul(const Qd& a, const Qd& b) {
+    return Qd{a.w * b.x + a.x * b.w + a.y * b.z - a.z * b.y, a.w * b.y + a.y * b.w + a.z * b.x - a.x * b.z,
+              a.w * b.z + a.z * b.w + a.x * b.y - a.y * b.x, a.w * b.w - a.x * b.x - a.y * b.y - a.z * b.z};
+}
+
+__host__ __device__ inline void qd_rotate(const Qd& q, const double v[3], double o[3]) {
+    double uv[3] = {q.y * v[2] - q.z * v[1], q.z * v[0] - q.x * v[2], q.x * v[1] - q.y * v[0]};
+    for (double& c : uv) c += c;
+    o[0] = v[0] + q.w * uv[0] + (q.y * uv[2] - q.z * uv[1]);
+    o[1] = v[1] + q.w * uv[1] + (q.z * uv[0] - q.x * uv[2]);
+    o[2] = v[2] + q.w * uv[2] + (q.x * uv[1] - q.y * uv[0]);
+}
+
+__host__ __device__ inline void qd_normalize(Qd& q) {
+    if (q.w < 0) q = Qd{-q.x, -q.y, -q.z, -q.w};
+    const double n = sqrt(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w);
+    q = Qd{q.x / n, q.y / n, q.z / n, q.w / n};
+}
+
+// the case of the largest diagonal entry I (indices known when compiled: the
+// device keeps no array in memory)
+template <int I>
+__host__ __device__ inline Qd qd_from_diagonal(const double* m) {
+    constexpr int J = (I + 1) % 3, K = (J + 1) % 3;
+    double c[3];
+    double t = sqrt(m[4 * I] - m[4 * J] - m[4 * K] + 1.0);
+    c[I] = 0.5 * t;
+    t = 0.5 / t;
+    c[J] = (m[3 * J + I] + m[3 * I + J]) * t;
+    c[K] = (m[3 * K + I] + m[3 * I + K]) * t;
+    return Qd{c[0], c[1], c[2], (m[3 * K + J] - m[3 * J + K]) * t};
+}
+
+__host__ __device__ inline Qd qd_from_R(const double* m) {
+    Qd q{};
+    double t = m[0] + m[4] + m[8];
+    if (t > 0) {
+        t = sqrt(t + 1.0);
+        q.w = 0.5 * t;
+        t = 0.5 / t;
+        q.x = (m[7] - m[5]) * t;
+        q.y = (m[2] - m[6]) * t;
+        q.z = (m[3] - m[1]) * t;
+    } else {
+        const bool y = m[4] > m[0];
+        if (m[8] > (y ? m[4] : m[0])) q = qd_from_diagonal<2>(m);
+        else q = y ? qd_from_diagonal<1>(m) : qd_from_diagonal<0>(m);
+    }
+    return q;
+}
+
+__host__ __device__ inline void se3_oplus(double* frame, const double* xi) {
+    const double w[3] = {xi[0], xi[1], xi[2]};
+    const double th = sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]);
+    const double W[9] = {0, -w[2], w[1], w[2], 0, -w[0], -w[1], w[0], 0};
+    double W2[9];
+    for (int r = 0; r < 3; r++)
+        for (int c = 0; c < 3; c++) W2[3 * r + c] = W[3 * r] * W[c] + W[3 * r + 1] * W[3 + c] + W[3 * r + 2] * W[6 + c];
+    double R[9], V[9];
+    for (int k = 0; k < 9; k++) {
+        const double I = (k % 4 == 0) ? 1.0 : 0.0;
+        if (th < 0.00001) {
+            R[k] = I + W[k] + 0.5 * W2[k];
+            V[k] = I + 0.5 * W[k] + (1.0 / 6.0) * W2[k];
+        } else {
+            R[k] = I + sin(th) / th * W[k] + (1 - cos(th)) / (th * th) * W2[k];
+            V[k] = I + (1 - cos(th)) / (th * th) * W[k] + (th - sin(th)) / (th * th * th) * W2[k];
+        }
+    }
+    Qd dq = qd_from_R(R);
+    qd_normalize(dq);
+    double dt[3];
+    for (int r = 0; r < 3; r++) dt[r] = V[3 * r] * xi[3] + V[3 * r + 1] * xi[4] + V[3 * r + 2] * xi[5];
+    // exp(x) * T
+    const Qd q{frame[0], frame[1], frame[2], frame[3]};
+    double rt[3];
+    qd_rotate(dq, frame + 4, rt);
+    Qd nq = qd_mul(dq, q);
+    qd_normalize(nq);
+    frame[0] = nq.x; frame[1] = nq.y; frame[2] = nq.z; frame[3] = nq.w;
+    for (int r = 0; r < 3; r++) frame[4 + r] = dt[r] + rt[r];
+}
+
+// The optimizer on a problem whose only unknown is one keyframe's pose (every
+// point and every other frame fixed), in one launch of one workgroup: the
+// iterations, trials and rules of mcv_ba_optimize.  An evaluation of a state
+// gives chi2 (sum of rho), H_pp and b_p at once, FP64 sums of the edges' FP32
+// terms in a fixed order, so a trial that is accepted has already linearized
+// the next iteration, and one that is rejected leaves the last H_pp and b_p in
+// hand.  Wave 0 solves the 6 x 6 system, moves the frame and writes its records;
+// all waves evaluate.  A frame has at most a few thousand edges, so a trial is
+// bound by its chain, not by the edges' arithmetic: with the optimizer on the
+// host and a launch and a wait per trial it took 26 us.
+constexpr int kPoseThreads = 512;
+constexpr int kPoseCams = 8;       // cameras whose records fit the workgroup's state
 constexpr int kPoseMaxEdges = 16384;
-constexpr int kPoseSums = 28;
+constexpr int kPoseSums = 28;      // H_pp's upper triangle by rows, each row followed by b_p's entry; chi2
+constexpr int kPoseIters = 64;     // iterations of one launch
 
 struct PoseState {
     BAPair pair[kPoseCams];  // (frame, camera) records of the free frame
@@ -1401,7 +1552,18 @@ struct PoseArgs {
     const uint8_t *act_m, *act_s;  // or null
     StereoCam scam;
     int frame, C;            // the free frame
-    double* out;             // kPoseSums
+};
+
+struct PoseRun {             // in: where the optimizer stands; out: where it stopped
+    double fr[7], lambda, ni;
+    int iters;               // in: to run (at most kPoseIters); out: run
+    int stop;                // in: nonzero on a problem's first launch; out: no further iteration
+};
+
+struct PoseSetup {
+    double cams[12 * kPoseCams];
+    double tau;
+    int max_trials, robust;
 };
 
 template <int kCtrl, int N>
@@ -1415,38 +1577,64 @@ __device__ __forceinline__ void sum_fold_d(double* v, int hi) {
     }
 }
 
-__global__ __launch_bounds__(kPoseThreads) void k_pose_eval(PoseArgs a, PoseState st) {
-    __shared__ float s_state[sizeof(PoseState) / 4];
-    __shared__ double s_sum[kPoseThreads / 64][32];
-    for (int k = threadIdx.x; k < (int)(sizeof(PoseState) / 4); k += kPoseThreads)
-        s_state[k] = reinterpret_cast<const float*>(&st)[k];
-    __syncthreads();
-    const PoseState& S = *reinterpret_cast<const PoseState*>(s_state);
-    double acc[32];
+// acc += W times the outer products of kRows rows of J with themselves (upper
+// triangle by rows) and, negated, with e, in FP64
+template <int kRows>
+__device__ __forceinline__ void pose_terms(double (&acc)[32], const float* J, const float* e, float W) {
 #pragma unroll
-    for (int k = 0; k < 32; k++) acc[k] = 0.0;
-    for (int i = threadIdx.x; i < a.ob.M; i += kPoseThreads) {
-        if (a.act_m && !a.act_m[i]) continue;
-        BAIn in;
-        ba_load_obs(i, a.ob, in);
-        ba_load_point(a.hi, a.lo, in);
-        const int f = (int)in.pair / a.C, c = (int)in.pair - f * a.C;
-        const BAPair& T = f == a.frame ? S.pair[c] : a.pairs[in.pair];
-        const BAEdge E = ba_residual(in, T);
-        acc[27] += huber_rho(E.chi2, T.delta);
-        if (f != a.frame) continue;
-        float J[12];
-        ba_jpose(in, E, T, J);
-        const float W = E.w * in.isig;
+    for (int row = 0; row < kRows; row++) {
+        double j[6], w[6];
+#pragma unroll
+        for (int r = 0; r < 6; r++) {
+            j[r] = (double)J[6 * row + r];
+            w[r] = (double)W * j[r];
+        }
+        const double m = -(double)e[row];
         int o = 0;
 #pragma unroll
         for (int r = 0; r < 6; r++) {
 #pragma unroll
-            for (int k = r; k < 6; k++, o++) acc[o] += (double)(W * (J[r] * J[k])) + (double)(W * (J[6 + r] * J[6 + k]));
-            acc[o++] -= (double)(W * (J[r] * E.e0)) + (double)(W * (J[6 + r] * E.e1));
+            for (int k = r; k < 6; k++, o++) acc[o] = __builtin_fma(w[r], j[k], acc[o]);
+            acc[o] = __builtin_fma(w[r], m, acc[o]);
+            o++;
         }
     }
-    for (int i = threadIdx.x; i < a.so.M; i += kPoseThreads) {
+}
+
+// The sums of state S into sums (LDS).  The mono edges go to the threads in
+// order, kPoseBatch of them loaded at once, the stereo edges from the last
+// thread down, whose waves have fewer.
+constexpr int kPoseBatch = 3;
+__device__ __forceinline__ void pose_eval(const PoseArgs& a, const PoseState& S, double (*s_sum)[32], double* sums) {
+    double acc[32];
+#pragma unroll
+    for (int k = 0; k < 32; k++) acc[k] = 0.0;
+    for (int i0 = threadIdx.x; i0 < a.ob.M; i0 += kPoseBatch * kPoseThreads) {
+        BAIn in[kPoseBatch];
+        bool on[kPoseBatch];
+#pragma unroll
+        for (int u = 0; u < kPoseBatch; u++) {
+            const int i = i0 + u * kPoseThreads;
+            on[u] = i < a.ob.M && !(a.act_m && !a.act_m[i]);
+            ba_load_obs(min(i, a.ob.M - 1), a.ob, in[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kPoseBatch; u++) ba_load_point(a.hi, a.lo, in[u]);
+#pragma unroll
+        for (int u = 0; u < kPoseBatch; u++) {
+            if (!on[u]) continue;
+            const int f = (int)in[u].pair / a.C, c = (int)in[u].pair - f * a.C;
+            const BAPair& T = f == a.frame ? S.pair[c] : a.pairs[in[u].pair];
+            const BAEdge E = ba_residual(in[u], T);
+            acc[27] += huber_rho(E.chi2, T.delta);
+            if (f != a.frame) continue;
+            float J[12];
+            ba_jpose(in[u], E, T, J);
+            const float e[2] = {E.e0, E.e1};
+            pose_terms<2>(acc, J, e, E.w * in[u].isig);
+        }
+    }
+    for (int i = kPoseThreads - 1 - threadIdx.x; i < a.so.M; i += kPoseThreads) {
         if (a.act_s && !a.act_s[i]) continue;
         const int f = (int)a.so.fr[i];
         const FramePose& T = f == a.frame ? S.pose : a.poses[f];
@@ -1455,16 +1643,7 @@ __global__ __launch_bounds__(kPoseThreads) void k_pose_eval(PoseArgs a, PoseStat
         if (f != a.frame) continue;
         float J[18];
         stereo_jpose(E, a.scam, J);
-        const float W = E.w * a.so.isig[i];
-        int o = 0;
-#pragma unroll
-        for (int r = 0; r < 6; r++) {
-#pragma unroll
-            for (int k = r; k < 6; k++, o++)
-                acc[o] += (double)(W * (J[r] * J[k])) + (double)(W * (J[6 + r] * J[6 + k])) +
-                          (double)(W * (J[12 + r] * J[12 + k]));
-            acc[o++] -= (double)(W * (J[r] * E.e[0])) + (double)(W * (J[6 + r] * E.e[1])) + (double)(W * (J[12 + r] * E.e[2]));
-        }
+        pose_terms<3>(acc, J, E.e, E.w * a.so.isig[i]);
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     sum_fold_d<0x140, 16>(acc, lane & 8);
@@ -1486,7 +1665,170 @@ __global__ __launch_bounds__(kPoseThreads) void k_pose_eval(PoseArgs a, PoseStat
         double v = 0.0;
 #pragma unroll
         for (int w = 0; w < kPoseThreads / 64; w++) v += s_sum[w][threadIdx.x];
-        a.out[threadIdx.x] = v;
+        sums[threadIdx.x] = v;
+    }
+}
+
+// x = S^-1 b by Cholesky (mcv_solve_llt for n = 6, with the diagonal's
+// reciprocals: a chain of 33 divisions otherwise), S = H_pp + lambda I from the
+// sums of an evaluation; false when S is not positive definite
+__device__ __forceinline__ bool pose_solve(const double* sums, double lambda, double (&b)[6], double (&x)[6]) {
+    double L[6][6], inv[6];
+    int o = 0;
+#pragma unroll
+    for (int r = 0; r < 6; r++) {
+#pragma unroll
+        for (int k = r; k < 6; k++) L[k][r] = sums[o++];
+        L[r][r] += lambda;
+        b[r] = sums[o++];
+    }
+#pragma unroll
+    for (int j = 0; j < 6; j++) {
+        double d = L[j][j];
+#pragma unroll
+        for (int k = 0; k < j; k++) d -= L[j][k] * L[j][k];
+        if (!(d > 0)) return false;
+        inv[j] = 1.0 / sqrt(d);
+#pragma unroll
+        for (int i = j + 1; i < 6; i++) {
+            double v = L[i][j];
+#pragma unroll
+            for (int k = 0; k < j; k++) v -= L[i][k] * L[j][k];
+            L[i][j] = v * inv[j];
+        }
+    }
+    double y[6];
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        double v = b[i];
+#pragma unroll
+        for (int k = 0; k < i; k++) v -= L[i][k] * y[k];
+        y[i] = v * inv[i];
+    }
+#pragma unroll
+    for (int i = 5; i >= 0; i--) {
+        double v = y[i];
+#pragma unroll
+        for (int k = i + 1; k < 6; k++) v -= L[k][i] * x[k];
+        x[i] = v * inv[i];
+    }
+    return true;
+}
+
+// the optimizer's state, in LDS between its steps (the evaluations need the
+// registers)
+struct PoseStep {
+    double fr[7], fr0[7], lambda, ni, rho, scale;
+    int it, qmax;
+    bool begin, pending, done, stop;
+};
+
+__global__ __launch_bounds__(kPoseThreads) void k_pose_optimize(PoseArgs a, PoseSetup q, PoseRun in, PoseRun* out,
+                                                                double* stats) {
+    __shared__ PoseState s_state;
+    __shared__ double s_sum[kPoseThreads / 64][32];
+    __shared__ double s_new[kPoseSums], s_cur[kPoseSums];
+    __shared__ PoseStep s_step;
+    const int lane = threadIdx.x & 63;
+    const bool ctl = threadIdx.x < 64;  // wave 0: the optimizer, every lane alike
+    // the frame's records: camera `lane`, or the pose
+    auto records = [&](const double* fr) {
+        double Rbw[9];
+        frame_rotation(fr, Rbw);
+        if (lane < a.C) pair_record(Rbw, fr + 4, q.cams + 12 * lane, q.robust != 0, s_state.pair[lane]);
+        else if (lane == kPoseCams) pose_record(Rbw, fr + 4, s_state.pose);
+    };
+    if (ctl) {
+        records(in.fr);
+        PoseStep T{};
+#pragma unroll
+        for (int k = 0; k < 7; k++) T.fr[k] = in.fr[k];
+        T.lambda = in.lambda;
+        T.ni = in.ni;
+        T.begin = true;
+        if (lane == 0) s_step = T;
+    }
+    __syncthreads();
+    pose_eval(a, s_state, s_sum, s_cur);
+    for (;;) {
+        __syncthreads();
+        if (ctl) {
+            PoseStep T = s_step;
+            // the trial's verdict; at an iteration's end, whether to go on
+            auto judge = [&](double chi) {
+                T.rho = (s_cur[27] - chi) / T.scale;
+                bool last = false;
+                if (T.rho > 0 && isfinite(chi)) {
+                    const double g = 2 * T.rho - 1;
+                    T.lambda *= fmax(1. / 3., fmin(1. - g * g * g, 2. / 3.));
+                    T.ni = 2;
+                    wave_lds_sync();
+                    if (lane < kPoseSums) s_cur[lane] = s_new[lane];
+                    wave_lds_sync();
+                } else {
+                    T.lambda *= T.ni;
+                    T.ni *= 2;
+#pragma unroll
+                    for (int k = 0; k < 7; k++) T.fr[k] = T.fr0[k];
+                    last = !isfinite(T.lambda);
+                }
+                if (!last) {
+                    T.qmax++;
+                    if (T.rho < 0 && T.qmax < q.max_trials) return;
+                }
+                if (lane == 0) {
+                    stats[4 * T.it + 1] = s_cur[27];
+                    stats[4 * T.it + 2] = T.lambda;
+                    stats[4 * T.it + 3] = T.qmax;
+                }
+                T.it++;
+                T.stop = T.qmax == q.max_trials || T.rho == 0 || !isfinite(T.lambda);
+                T.done = T.stop || T.it == in.iters;
+                T.begin = true;
+            };
+            if (T.pending) judge(s_new[27]);
+            T.pending = false;
+            while (!T.done) {
+                if (T.begin) {
+                    T.begin = false;
+                    if (lane == 0) stats[4 * T.it] = s_cur[27];
+                    if (in.stop && T.it == 0) {
+                        // computeLambdaInit: the diagonal entries of H_pp
+                        const double mx =
+                            fmax(fmax(fmax(fabs(s_cur[0]), fabs(s_cur[7])), fmax(fabs(s_cur[13]), fabs(s_cur[18]))),
+                                 fmax(fabs(s_cur[22]), fabs(s_cur[25])));
+                        T.lambda = q.tau * mx;
+                    }
+                    T.rho = 0;
+                    T.qmax = 0;
+                }
+#pragma unroll
+                for (int k = 0; k < 7; k++) T.fr0[k] = T.fr[k];
+                double b[6], x[6];
+                T.scale = 1e-3;
+                if (pose_solve(s_cur, T.lambda, b, x)) {
+#pragma unroll
+                    for (int k = 0; k < 6; k++) T.scale += x[k] * (T.lambda * x[k] + b[k]);
+                    se3_oplus(T.fr, x);
+                    records(T.fr);
+                    T.pending = true;
+                    break;
+                }
+                judge(DBL_MAX);
+            }
+            if (lane == 0) s_step = T;
+        }
+        __syncthreads();
+        if (!s_step.pending) break;
+        pose_eval(a, s_state, s_sum, s_new);
+    }
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int k = 0; k < 7; k++) out->fr[k] = s_step.fr[k];
+        out->lambda = s_step.lambda;
+        out->ni = s_step.ni;
+        out->iters = s_step.it;
+        out->stop = s_step.stop;
     }
 }
 
