@@ -1536,7 +1536,7 @@ constexpr int kPoseThreads = 512;
 constexpr int kPoseCams = 8;       // cameras whose records fit the workgroup's state
 constexpr int kPoseMaxEdges = 16384;
 constexpr int kPoseSums = 28;      // H_pp's upper triangle by rows, each row followed by b_p's entry; chi2
-constexpr int kPoseIters = 64;     // iterations of one launch
+constexpr int kPoseIters = 16;     // iterations of one launch
 
 struct PoseState {
     BAPair pair[kPoseCams];  // (frame, camera) records of the free frame

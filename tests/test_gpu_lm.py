@@ -249,3 +249,29 @@ def test_single_pose_route_vs_oracle_and_general_route(gpu_ctx, n_kf, n_points, 
     for a, b in zip(out[0][2], out[1][2]):
         if a is not None:
             assert (a != b).sum() <= max(2, len(a) // 1000)
+
+
+def test_single_pose_more_iterations_than_one_launch(gpu_ctx):
+    """A first lambda so large that the steps stay small for some 20
+    iterations: more than one launch of the one-frame optimizer runs (16).
+    Against the general route, which the same problem takes when a point
+    without edges is left free; tolerances as above."""
+    lp = synth.local_ba_problem(seed=77, n_kf=1, n_points=700, target_obs=500, stereo_frac=0.5, fixed_point_frac=1.0,
+                                perturb_pose=0.0)
+    mono = lp.mono
+    mono.frame_fixed = np.zeros(1, np.int32)
+    mono.frames[0] = oracle.se3_oplus(mono.frames[0], np.random.default_rng(5).normal(0, 0.01, 6))
+    mono.points = np.concatenate([mono.points, [[0.0, 0.0, 5.0]]])       # seen by no edge
+    out = []
+    for last in (1, 0):
+        pfix = np.ones(len(mono.points), np.int32)
+        pfix[-1] = last
+        lin = local_ba_linearizer(mono, lp.stereo, pfix, ctx=gpu_ctx)
+        stats, n = lin.optimize(40, tau=1e8)
+        out.append((stats, n, lin.get_state()[1]))
+        lin.close()
+    assert out[0][1] > 17 and out[1][1] > 17
+    k = 17                                # the iterations around the second launch's start
+    np.testing.assert_allclose(out[0][0][:k + 1, :3], out[1][0][:k + 1, :3], rtol=1e-3)
+    assert np.abs(out[0][2][0, 4:] - out[1][2][0, 4:]).max() < 1e-5
+    assert np.abs(out[0][2][0, :4] - out[1][2][0, :4]).max() < 1e-6
