@@ -871,11 +871,10 @@ __device__ __forceinline__ unsigned long long path_code(int x, int y, const Leve
     int uly = 0, by = L.maxBY - L.minBY;
     unsigned long long code = (unsigned long long)root;
     for (int d = 1; d <= kOctreeDepth; d++) {
-        const int halfX = (int)ceilf((float)(urx - ulx) / 2.f);
-        const int halfY = (int)ceilf((float)(by - uly) / 2.f);
-        const int mx = ulx + halfX, my = uly + halfY;
-        const int qx = ((float)x < (float)mx) ? 0 : 1;
-        const int qy = ((float)y < (float)my) ? 0 : 1;
+        // ceilf(d / 2.f) and the float compares are exact on these integers
+        const int mx = ulx + ((urx - ulx + 1) >> 1), my = uly + ((by - uly + 1) >> 1);
+        const int qx = x < mx ? 0 : 1;
+        const int qy = y < my ? 0 : 1;
         if (qx) ulx = mx; else urx = mx;
         if (qy) uly = my; else by = my;
         code = (code << 2) | (unsigned long long)(qx + 2 * qy);
@@ -1329,7 +1328,8 @@ __device__ __forceinline__ SubLanes sub_lanes() {
     return S;
 }
 
-// pop_heap, as one top-down pass; the popped entry comes back in `top`.
+// pop_heap, as one top-down pass.  on_top gets the entry to be popped as soon as
+// it is known and says whether to go on; if not, the heap stays as it is.
 // pop_heap moves the hole from the root to a leaf along the max-child path of
 // the heap without its last element x (the right child unless it is smaller
 // than the left; the single child at the end of an even-length heap) and then
@@ -1346,15 +1346,15 @@ __device__ __forceinline__ SubLanes sub_lanes() {
 // mask.  The round's moves are one store; in the last one lane 63 stores x and
 // lane 62 the popped entry, with count 0, in the freed slot, where the drain
 // keeps it.  For the heaps that pop_pairs does not take.
-__device__ __forceinline__ void heap_pop_wave(uint2* H, int& len, const SubLanes& S, uint2& top) {
+template <typename F>
+__device__ __forceinline__ void heap_pop_wave(uint2* H, int& len, const SubLanes& S, F&& on_top) {
     const int lane = threadIdx.x & 63;
     const int n = len;
-    len = n - 1;
     int slot = S.slot0;
     uint2 s = H[lane == 63 ? n : slot];
     const uint32_t x2 = 2 * hkey(__builtin_amdgcn_readlane(s.x, 63)) - 1;  // counts are at least 1
-    top.x = __builtin_amdgcn_readlane(s.x, 62);
-    top.y = __builtin_amdgcn_readlane(s.y, 62);
+    if (!on_top(make_uint2(__builtin_amdgcn_readlane(s.x, 62), __builtin_amdgcn_readlane(s.y, 62)))) return;
+    len = n - 1;
     s.x &= S.keep;  // lane 62: the children count alone
     int hole = 1;
     for (;;) {
@@ -1406,16 +1406,14 @@ __device__ __forceinline__ PairLanes pair_lanes() {
 // leads here; below that the walk goes on by bit tests.  A wave alone issues an
 // instruction every 5 cycles or so, and that is what a pop costs: draining 434
 // entries 890 cycles each by two rounds of heap_pop_wave, 510 so.
-template <int R>
-__device__ __forceinline__ void pop_pairs(uint2* H, int& len, const PairLanes& S, uint2& top) {
+template <int R, typename F>
+__device__ __forceinline__ void pop_pairs(uint2* H, int& len, const PairLanes& S, F&& on_top) {
     const int lane = threadIdx.x & 63;
     const int n = len;
-    len = n - 1;
     const uint2 x = H[n];
     lds_order();
     if (n == 1) {
-        top.x = __builtin_amdgcn_readfirstlane(x.x);
-        top.y = __builtin_amdgcn_readfirstlane(x.y);
+        if (on_top(make_uint2(__builtin_amdgcn_readfirstlane(x.x), __builtin_amdgcn_readfirstlane(x.y)))) len = 0;
         return;
     }
     if (lane == 0) H[n] = make_uint2(0, 0);
@@ -1426,6 +1424,12 @@ __device__ __forceinline__ void pop_pairs(uint2* H, int& len, const PairLanes& S
 #pragma unroll
     for (int r = 0; r < R; r++) q[r] = reinterpret_cast<const uint4*>(H)[64 * r + lane];
     lds_order();
+    if (!on_top(make_uint2(__builtin_amdgcn_readlane(q[0].z, 0), __builtin_amdgcn_readlane(q[0].w, 0)))) {
+        if (lane == 0) H[n] = x;
+        lds_order();
+        return;
+    }
+    len = n - 1;
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const bool rt = (q[r].z | 7u) >= q[r].x;  // by counts alone
@@ -1433,8 +1437,6 @@ __device__ __forceinline__ void pop_pairs(uint2* H, int& len, const PairLanes& S
         big[r] = rt ? make_uint2(q[r].z, q[r].w) : make_uint2(q[r].x, q[r].y);
         go[r] = __ballot((big[r].x | 7u) >= x.x);
     }
-    top.x = __builtin_amdgcn_readlane(q[0].z, 0);
-    top.y = __builtin_amdgcn_readlane(q[0].w, 0);
     const unsigned long long walk = __ballot(((((uint32_t)right[0] ^ S.dir) | ~(uint32_t)go[0]) & S.anc) == 0);
     const unsigned long long moved = walk & go[0];
     if (in_lanes(moved)) H[lane] = big[0];
@@ -1464,11 +1466,39 @@ __device__ __forceinline__ void pop_pairs(uint2* H, int& len, const PairLanes& S
     lds_order();
 }
 
-__device__ __forceinline__ void heap_pop(uint2* H, int& len, const SubLanes& SL, const PairLanes& PL, uint2& top) {
-    if (len < 128) pop_pairs<1>(H, len, PL, top);
-    else if (len < 256) pop_pairs<2>(H, len, PL, top);
-    else if (len < 512) pop_pairs<4>(H, len, PL, top);
-    else heap_pop_wave(H, len, SL, top);
+template <typename F>
+__device__ __forceinline__ void heap_pop(uint2* H, int& len, const SubLanes& SL, const PairLanes& PL, F&& on_top) {
+    if (len < 128) pop_pairs<1>(H, len, PL, on_top);
+    else if (len < 256) pop_pairs<2>(H, len, PL, on_top);
+    else if (len < 512) pop_pairs<4>(H, len, PL, on_top);
+    else heap_pop_wave(H, len, SL, on_top);
+}
+
+// The drain of a heap whose m entries all have the same count, at once: with
+// ties the right child moves up, so a pop takes the front of the queue formed by
+// the slots 1, 3, 7, .. (the right spine), and the last entry joins its back.
+// The slots from m down that are not on the spine therefore follow the spine's
+// in order, except that where the spine's deepest slot 2^j - 1 leaves, slot
+// 2^j - 2 comes in before the queue's last entry.  The k-th popped entry ends in
+// slot m - k, its count 0.  tmp: m + 1 entries of LDS.
+__device__ __forceinline__ void drain_ties(uint2* H, uint2* tmp, int m) {
+    const int lane = threadIdx.x & 63;
+    for (int n = 1 + lane; n <= m; n += 64) {
+        const int j = 31 - __builtin_clz((uint32_t)n + 1);  // floor(log2(n + 1))
+        int k;
+        if (((n + 1) & n) == 0) {
+            k = j - 1;                                       // on the spine
+            if (n > 1 && n == m) k++;                        // slot n - 1 came in before it
+        } else {
+            k = m - n + j;
+            if (((n + 2) & (n + 1)) == 0 && n + 1 <= m) k--;  // slot 2^j - 2
+            else if (n > 2 && (n & (n - 1)) == 0) k++;        // slot 2^j, last when that came in
+        }
+        tmp[m - k] = make_uint2(H[n].x & 7u, H[n].y);
+    }
+    wave_lds_sync();
+    for (int n = 1 + lane; n <= m; n += 64) H[n] = tmp[n];
+    wave_lds_sync();
 }
 
 // heap entry of node c from start[c], start[c+1], child[c], child[c+1]
@@ -1634,26 +1664,42 @@ __global__ __launch_bounds__(64) void k_octree_heap(OrbGlobals g, const int* ord
     for (int k = 0; k < nr; k += 4)
         push_nodes(H, len, nt, T, tn, (uint32_t)k, min(4, nr - k), node_rows(nt, T, tn, (uint32_t)k, min(4, nr - k)));
     const int N = min(L.nfeat, cap - 8);
-    uint2 top;
     while (len > 0 && len < N) {
-        // the largest node; one with a single keypoint ends the splitting
-        top = H[1];
-        top.x = __builtin_amdgcn_readfirstlane(top.x);
-        if (hkey(top.x) == 1) break;
-        // its children's table entries, asked for before the pop
-        const uint32_t c0 = __builtin_amdgcn_readfirstlane(top.y);
-        const int nch = (int)(top.x & 7u);
-        const NodeRows kids = node_rows(nt, T, tn, c0, nch);
-        heap_pop(H, len, SL, PL, top);
+        uint32_t c0 = 0;
+        int nch = -1;
+        NodeRows kids;
+        heap_pop(H, len, SL, PL, [&](uint2 top) {
+            // the largest node; one with a single keypoint ends the splitting
+            if (hkey(top.x) == 1) return false;
+            // its children's table entries, asked for while the pop goes on
+            c0 = top.y;
+            nch = (int)(top.x & 7u);
+            kids = node_rows(nt, T, tn, c0, nch);
+            return true;
+        });
+        if (nch < 0) break;
         push_nodes(H, len, nt, T, tn, c0, nch, kids);
     }
     // drain: the j-th popped node ends in the slot that its pop frees, n0 - j,
     // its key's count 0
     const int n0 = len;
-    while (len >= 512) heap_pop_wave(H, len, SL, top);
-    while (len >= 256) pop_pairs<4>(H, len, PL, top);
-    while (len >= 128) pop_pairs<2>(H, len, PL, top);
-    while (len > 1) pop_pairs<1>(H, len, PL, top);
+    bool ties = false;
+    auto popped = [&](uint2 top) {
+        ties = hkey(top.x) == 1;  // then all others have one keypoint too
+        return true;
+    };
+    if (n0 <= tab_cap) {
+        while (len >= 512 && !ties) heap_pop_wave(H, len, SL, popped);
+        while (len >= 256 && !ties) pop_pairs<4>(H, len, PL, popped);
+        while (len >= 128 && !ties) pop_pairs<2>(H, len, PL, popped);
+        while (len > 1 && !ties) pop_pairs<1>(H, len, PL, popped);
+        if (len > 1) {
+            wave_lds_sync();
+            drain_ties(H, T, len);
+        }
+    } else {
+        while (len > 1) heap_pop(H, len, SL, PL, popped);
+    }
     wave_lds_sync();
     const int nkeep = min(n0, L.out_cap);
     if (lane == 0) O->nout = nkeep;

@@ -236,3 +236,13 @@ def test_orb_heap_sizes(own_ctx, nfeatures):
     rng = np.random.default_rng(9)
     _check(orb, rng.integers(0, 256, (240, 900), dtype=np.uint8))
     _check(orb, synth.blob_image(17, 300, 420))
+
+
+@pytest.mark.parametrize("nfeatures,size", [(1200, (400, 300)), (3000, (500, 320)), (9000, (640, 400))])
+def test_orb_heap_of_ties(own_ctx, nfeatures, size):
+    """More features asked for than there are candidates: every kept node
+    holds one keypoint, so the whole drain is one run of ties (from some tens
+    to thousands of entries)."""
+    orb = ORB(nfeatures, 1.2, 4, 30, 25, ctx=own_ctx)
+    _check(orb, synth.blob_image(61, *size))
+    _check(orb, np.ascontiguousarray(synth.blob_image(62, *size)[::-1]))
