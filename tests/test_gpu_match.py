@@ -185,3 +185,15 @@ def test_knn2_dev(gpu_ctx, nq, nt):
                                               ctypes.c_void_p(dt.data_ptr()), nt, ctypes.c_void_p(out.data_ptr())))
     torch.cuda.synchronize()
     np.testing.assert_array_equal(out.cpu().numpy(), oracle.knn2(q, t))
+
+
+@pytest.mark.parametrize("n", [1, 3, 1023, 1024, 1025, 4095, 4097, 9001])
+def test_filter_list_lengths(gpu_ctx, n):
+    """Lists around the runs of rows a thread takes (one row each, 4 loads at
+    a time, more), with many rows refused by each of the two filters."""
+    rng = np.random.default_rng(n)
+    for hi, ratio, th in [(100, 0.8, 50), (60, 1.0, 5), (256, 0.3, 250)]:
+        d = np.sort(rng.integers(0, hi, (n, 2)), axis=1).astype(np.int32)
+        knn = np.stack([rng.integers(0, 5000, n), d[:, 0], rng.integers(0, 5000, n), d[:, 1]], 1).astype(np.int32)
+        got = Matcher.filter(knn, ratio, th, ctx=gpu_ctx)
+        np.testing.assert_array_equal(got, oracle.filter_ratio_threshold(knn, ratio, th))
