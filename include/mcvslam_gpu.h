@@ -152,7 +152,7 @@ int mcv_match_filter(mcv_ctx* ctx, const int32_t* knn, int nq, float ratio, int 
  * that cannot allocate device memory (work under HIP graph capture, tight
  * serving loops).  d_knn: nq x 4 knn rows, d_out: nq x 3, *d_count: the
  * filtered length, all device memory; enqueued on the context's stream.
- * The filter's scratch is a fixed per-GPU array of the library (512 KiB,
+ * The filter's scratch is a fixed per-GPU array of the library (256 KiB,
  * held until the process ends) shared by every call on that GPU, so calls
  * that overlap on one GPU (other contexts or streams) race.  nq may be at
  * most 65536 (MCV_ERR_CAPACITY above). */

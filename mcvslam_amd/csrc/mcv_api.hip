@@ -42,16 +42,16 @@ __global__ void k_zero_words(uint32_t* p, int n) {
 }
 }  // namespace mcv
 
-// Scratch of mcv_match_filter_noalloc_dev: the ratio survivors and the
-// threshold holes of one list, 2 * kNoAllocMaxQueries ints (512 KiB) per GPU,
-// held until the process ends.  After set-up host code uses only the device
-// address that hipGetSymbolAddress returns for it (once per device, in
-// mcv_create); the array's name is not a device address in host code.
 constexpr size_t kPinBytes = 4u << 20;   // pinned host memory of a context
 constexpr int kCopyParts = 8;            // ranges one launch copies
 constexpr uint32_t kCopyBlock = 16384;   // bytes per workgroup of k_copy_parts
+
+// Scratch of mcv_match_filter_noalloc_dev: the threshold holes of one list,
+// kNoAllocMaxQueries ints (256 KiB) per GPU, held until the process ends.  After set-up host code uses only the device
+// address that hipGetSymbolAddress returns for it (once per device, in
+// mcv_create); the array's name is not a device address in host code.
 constexpr int kNoAllocMaxQueries = 65536;
-static __device__ __align__(256) int scratch[2 * kNoAllocMaxQueries];
+static __device__ __align__(256) int scratch[kNoAllocMaxQueries];
 
 namespace {
 
@@ -1776,7 +1776,7 @@ int mcv_match_filter(mcv_ctx* c, const int32_t* knn, int nq, float ratio, int th
     c->f_knn.ensure((size_t)nq * 16);
     c->f_out.ensure((size_t)nq * 12);
     c->f_cnt.ensure(16);
-    c->f_scr.ensure((size_t)nq * 8);
+    c->f_scr.ensure((size_t)nq * 4);
     HostIO io(c);
     io.up(c->f_knn.p, knn, (size_t)nq * 16);
     FilterJob j{c->f_knn.as<int32_t>(), nullptr, nq, ratio, th, c->f_out.as<int32_t>(), c->f_cnt.as<int>(),
@@ -1865,7 +1865,7 @@ int mcv_rig_create(mcv_ctx* c, int n_frames, const int32_t* w3, const int32_t* h
     r->knn.ensure((size_t)n * r->cap * 16);
     r->matches.ensure((size_t)n * r->cap * 12);
     r->mcounts.ensure((size_t)n * 4);
-    r->scratch.ensure((size_t)n * r->cap * 8);
+    r->scratch.ensure((size_t)n * r->cap * 4);
     r->porder.ensure((size_t)(2 * n + 1) * sizeof(int));
     // segment keys of the fp4 top-2: the batched launch's or one pair's
     r->part.ensure(std::max(knn_part_bytes(0, n, r->cap, r->cap), knn_part_bytes(0, 1, r->cap, r->cap)));
@@ -1891,7 +1891,7 @@ int mcv_rig_create(mcv_ctx* c, int n_frames, const int32_t* w3, const int32_t* h
             j.th = th;
             j.out = r->matches.as<int32_t>() + (size_t)pi * r->cap * 3;
             j.count = r->mcounts.as<int>() + pi;
-            j.scratch = r->scratch.as<int>() + (size_t)pi * r->cap * 2;
+            j.scratch = r->scratch.as<int>() + (size_t)pi * r->cap;
             r->hj.push_back(j);
         }
     upload(r->pairs, r->hp, c->stream);
