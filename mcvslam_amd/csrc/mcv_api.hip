@@ -441,7 +441,7 @@ struct ImageSpec {
 
 // A batch plan: geometry and work tables for a list of images.
 struct OrbPlan {
-    int n_images = 0, nlevels = 0, cap = 0, n_slots = 0, strip_h = kStripH;
+    int n_images = 0, nlevels = 0, cap = 0, n_slots = 0, strip_h = kStripH, resize_h = kResizeH;
     std::vector<LevelDesc> lv;
     std::vector<CellDesc> cells;
     std::vector<Strip> strips;
@@ -622,7 +622,8 @@ struct OrbPlan {
             begin[nlevels] = (int)out.size();
         };
         cut(strip_h, strips, strip_begin);
-        cut(kResizeH, rstrips, rstrip_begin);
+        resize_h = tall < kResizeMin ? kResizeHLow : kResizeH;
+        cut(resize_h, rstrips, rstrip_begin);
         // k_resize: the source bytes of 4 adjacent outputs (both taps)
         // lie in the 12 bytes from the first one's aligned word
         for (const LevelDesc& d : lv) {
@@ -822,7 +823,8 @@ void OrbPlan::enqueue(const OrbConfig& c, const SinCosTables& tb, hipStream_t s,
             const int n = rstrip_begin[l + 1] - rstrip_begin[l];
             if (n > 0) {
                 hipLaunchKernelGGL(k_resize, dim3(xcd_grid(n)), dim3(64), 0, s,
-                                   d_rstrips.as<Strip>() + rstrip_begin[l], n, g.lv, d_coef.as<int2>(), g.pyr);
+                                   d_rstrips.as<Strip>() + rstrip_begin[l], n, resize_h, g.lv, d_coef.as<int2>(),
+                                   g.pyr);
                 mark("k_resize");
             }
         }

@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256) void k_copy_level0(const Strip* st, int n, int
 // once per source row.  The wave walks the strip's source rows in order, 4
 // rows per step with the next 4 rows' loads in flight, and stores an output
 // row once both of its source rows are done.
-__global__ __launch_bounds__(64) void k_resize(const Strip* st, int n, const LevelDesc* lv, const int2* coef,
+__global__ __launch_bounds__(64) void k_resize(const Strip* st, int n, int sh, const LevelDesc* lv, const int2* coef,
                                                uint8_t* pyr) {
     const int sidx = xcd_block(n);
     if (sidx < 0) return;
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(64) void k_resize(const Strip* st, int n, const Lev
     const LevelDesc L = lv[S.lvl];
     const LevelDesc SL = lv[L.src];
     const int x = S.x0 + 4 * lane;
-    const int ny = min(S.y0 + kResizeH, L.h) - S.y0;
+    const int ny = min(S.y0 + sh, L.h) - S.y0;
     const uint8_t* sp = pyr + SL.pix;
     // the strip's row coefficients, lane k for output row S.y0 + k
     int2 cyl = make_int2(0, 0);

@@ -21,12 +21,16 @@ constexpr int kMaxWin = 96;             // max FAST cell window side (pixels)
 // lane.  A wave walks its strip down, so a batch of few strips waits on the
 // walk: below kStripMin strips they are kStripHLow rows high (FAST and blur,
 // us, 32 / 8 rows: 1 rig frame 43 + 20 / 26 + 14, 8 frames 110 + 40 / 99 + 45,
-// 16 frames 179 + 66 / 182 + 82).  k_resize's strips are always kResizeH high.
+// 16 frames 179 + 66 / 182 + 82).  k_resize's strips are kResizeHLow rows high
+// below kResizeMin strips (the 7 launches, us, 8 / 4 / 2 rows: 1 frame 58 / 48 / 46,
+// 4 frames 63 / 54 / 51, 16 frames 91 / 87 / 88 but the whole step 858 / 859 / 866).
 constexpr int kStripW = 256;
 constexpr int kStripH = 32;
 constexpr int kStripHLow = 8;
 constexpr int kStripMin = 8192;
 constexpr int kResizeH = 8;
+constexpr int kResizeHLow = 2;
+constexpr int kResizeMin = 4096;
 constexpr int kPitchAlign = 64;         // level rows start on 64-byte boundaries
 
 struct LevelDesc {
