@@ -92,7 +92,8 @@ class Reprojection(torch.autograd.Function):
                   and _on_device(point_delta, (lin.P, 3), lin.ctx.device)
                   and np.shape(points) == (lin.P, 3) and np.shape(frames) == (lin.F, 7))
         if native:
-            dp, dx = pose_delta.detach().contiguous(), point_delta.detach().contiguous()
+            # as memory: dense, and without a negation that is still to be done
+            dp, dx = (d.detach().resolve_neg().contiguous() for d in (pose_delta, point_delta))
             lin.ctx.use_torch_stream()
             lin.set_state_increments(points, frames, cams, dp, dx)
             lin.linearize()
@@ -121,7 +122,7 @@ class Reprojection(torch.autograd.Function):
             # are gone, and the adjoint would use another state's
             raise RuntimeError("Reprojection.backward: the BALinearizer was relinearized after this forward; "
                                "use one BALinearizer per forward that is still to be differentiated")
-        g = g.contiguous().float()
+        g = g.resolve_neg().contiguous().float()
         gpose = torch.empty((lin.F, 6), dtype=torch.float32, device=g.device)
         gpoint = torch.empty((lin.P, 3), dtype=torch.float32, device=g.device)
         lin.ctx.use_torch_stream()

@@ -175,3 +175,26 @@ def test_pose_adjoint_sizes(gpu_ctx, n_kf, n_points, obs):
     np.add.at(mag, prob.obs_frame, np.einsum("mij,mi->mj", np.abs(J), np.abs(G).astype(np.float64)))
     assert (np.abs(dpose.grad.cpu().numpy() - want) <= M * 2.0 ** -24 * mag + 1e-30).all()
     lin.close()
+
+
+def test_negated_views(gpu_ctx):
+    """Tensors whose negation is a flag on shared memory (what the imaginary
+    part of a conjugated complex tensor is): increments and an incoming
+    gradient of that kind give what their values in memory of their own give."""
+    import torch
+    prob = _problem()
+    lin = BALinearizer.from_problem(prob, ctx=gpu_ctx)
+    F, P = len(prob.frames), len(prob.points)
+    rng = np.random.default_rng(4)
+    dp = torch.from_numpy(rng.normal(size=(F, 6)) * 1e-2).float().cuda()
+    dx = torch.from_numpy(rng.normal(size=(P, 3)) * 1e-2).float().cuda()
+    g = torch.from_numpy(rng.normal(size=(lin.M, 2))).float().cuda()
+    out = []
+    for neg in (torch._neg_view, torch.neg):
+        a, b = neg(dp).requires_grad_(), neg(dx).requires_grad_()
+        assert a.is_neg() == (neg is torch._neg_view)
+        e = reprojection(a, b, lin, (prob.points, prob.frames, prob.cams))
+        out.append((e, *torch.autograd.grad(e, (a, b), neg(g))))
+    for x, y in zip(*out):
+        np.testing.assert_array_equal(x.detach().cpu().numpy(), y.detach().cpu().numpy())
+    lin.close()
