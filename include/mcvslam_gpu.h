@@ -410,6 +410,9 @@ int mcv_ba_set_active(mcv_ba* ba, const uint8_t* active_mono, const uint8_t* act
 /* enabled = 0 drops the Huber kernels of every edge (setRobustKernel(0),
  * src/PoseEstimation.cpp:117): weight 1 and rho(chi2) = chi2. */
 int mcv_ba_set_robust(mcv_ba* ba, int enabled);
+/* lambda: the damping, not negative.  Where H_ll + lambda I of a point is
+ * singular in FP32 (lambda = 0 and a point of one mono edge, or seen under no
+ * parallax), the singular directions are left out, as by a pseudo-inverse. */
 int mcv_ba_schur(mcv_ba* ba, float lambda);
 /* Host copy of S (row-major, full symmetric) and b_schur as double. */
 int mcv_ba_read_schur(mcv_ba* ba, double* S, double* b_schur, int32_t* n);

@@ -979,16 +979,26 @@ __global__ __launch_bounds__(256) void k_schur_points(SchurArgs a) {
     h11 = sum8(h11); h12 = sum8(h12); h22 = sum8(h22);
     b0 = sum8(b0); b1 = sum8(b1); b2 = sum8(b2);
     if (p >= a.P) return;
-    // D = H_ll + lambda I = C C^T; a pivot of D is at least lambda (H_ll is
-    // positive semidefinite), which also holds it against cancellation
+    // D = H_ll + lambda I = C C^T.  H_ll is positive semidefinite, so a pivot of
+    // D is at least lambda, which holds it against cancellation.  Where it is
+    // within rounding of zero all the same (lambda of 0 or next to it: a point
+    // of one mono edge has an H_ll of rank 2) its direction carries nothing and
+    // is left out, as in a pseudo-inverse: the rounding error over such a
+    // pivot's root would reach S and b_schur of every frame that sees the point.
+    // (A lambda below zero that leaves D indefinite gives NaN.)
     float c10 = 0.f, c20 = 0.f, c21 = 0.f, i00 = 0.f, i11 = 0.f, i22 = 0.f;
     if (e1 > e0) {
-        i00 = 1.f / sqrtf(h00 + a.lambda);
+        auto inv_root = [&](float pivot, float diag) {
+            const float v = fmaxf(pivot, a.lambda);
+            return a.lambda >= 0.f && v <= __FLT_EPSILON__ * diag ? 0.f : 1.f / sqrtf(v);
+        };
+        const float d0 = h00 + a.lambda, d1 = h11 + a.lambda, d2 = h22 + a.lambda;
+        i00 = inv_root(d0, d0);
         c10 = h01 * i00;
         c20 = h02 * i00;
-        i11 = 1.f / sqrtf(fmaxf(h11 + a.lambda - c10 * c10, a.lambda));
+        i11 = inv_root(d1 - c10 * c10, d1);
         c21 = (h12 - c20 * c10) * i11;
-        i22 = 1.f / sqrtf(fmaxf(h22 + a.lambda - c20 * c20 - c21 * c21, a.lambda));
+        i22 = inv_root(d2 - c20 * c20 - c21 * c21, d2);
     }
     const float y0 = b0 * i00, y1 = (b1 - c10 * y0) * i11, y2 = (b2 - c20 * y0 - c21 * y1) * i22;
     if (g == 0) {

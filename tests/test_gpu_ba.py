@@ -119,6 +119,63 @@ def test_schur_vs_fp64(gpu_ctx, lam):
     b.close()
 
 
+def _without_damping(seed):
+    """Points of one edge, whose H_ll has rank 2, among points whose H_ll has
+    a condition number below 300; per point (frames, J_pose, J_point, W, e)."""
+    prob = synth.ba_problem(seed=seed, n_kf=5, n_points=700, target_obs=7000)
+    e, _, w, Jp, Jx = oracle.ba_linearize(prob)
+    W = w * prob.obs_isig
+    Hll = np.zeros((len(prob.points), 3, 3))
+    np.add.at(Hll, prob.obs_pt, W[:, None, None] * np.einsum("mri,mrj->mij", Jx, Jx))
+    good = np.linalg.cond(Hll) < 300
+    first = np.r_[True, prob.obs_pt[1:] != prob.obs_pt[:-1]]
+    keep = good[prob.obs_pt] | first
+    for k in ("obs_uv", "obs_pt", "obs_frame", "obs_cam", "obs_level", "obs_isig"):
+        setattr(prob, k, getattr(prob, k)[keep])
+    n = np.bincount(prob.obs_pt, minlength=len(prob.points))
+    assert (n == 1).sum() > 100 and (n > 1).sum() > 100
+    return prob, n
+
+
+def test_schur_without_damping(gpu_ctx):
+    """lambda = 0, the default: points of one edge contribute what the
+    pseudo-inverse of their H_ll does, and keep S and b_schur finite.  Bound:
+    16 roundings of 2^-24 at a condition number of 300, of the sums of the
+    magnitudes (a pivot left out lies under 2^-23 of its diagonal and what
+    remains of its column within 16 roundings, so it would add less)."""
+    prob, n = _without_damping(36)
+    lin = BALinearizer.from_problem(prob, ctx=gpu_ctx)
+    lin.linearize()
+    S, bs = lin.schur()
+    e, _, w, Jp, Jx = oracle.ba_linearize(prob)
+    free = np.nonzero(prob.frame_fixed == 0)[0]
+    col = {f: 6 * k for k, f in enumerate(free)}
+    m = 6 * len(free)
+    want, mag = (np.zeros((m, m + 1)) for _ in range(2))
+    for p in np.unique(prob.obs_pt):
+        i = np.nonzero(prob.obs_pt == p)[0]
+        W = (w[i] * prob.obs_isig[i]).repeat(2)[:, None]
+        A = np.zeros((2 * len(i), m))
+        for k, j in enumerate(i):
+            if prob.obs_frame[j] in col:
+                c = col[prob.obs_frame[j]]
+                A[2 * k:2 * k + 2, c:c + 6] = Jp[j]
+        B, r = Jx[i].reshape(-1, 3), e[i].reshape(-1, 1)
+        AB = (W * A).T @ B
+        rest = np.linalg.pinv((W * B).T @ B, rcond=1e-9) @ np.c_[AB.T, -(W * B).T @ r]
+        want += np.c_[(W * A).T @ A, -(W * A).T @ r] - AB @ rest
+        mag += np.c_[np.abs(W * A).T @ np.abs(A), np.abs(W * A).T @ np.abs(r)] + np.abs(AB) @ np.abs(rest)
+    assert np.isfinite(S).all() and np.isfinite(bs).all()
+    tol = 16 * 2.0 ** -24 * 300
+    assert np.linalg.norm(S - want[:, :m]) < tol * np.linalg.norm(mag[:, :m])
+    assert np.linalg.norm(bs - want[:, m]) < tol * np.linalg.norm(mag[:, m])
+    # undamped steps: points without parallax no longer stop the optimizer
+    stats, _ = lin.optimize(3, tau=0.0)
+    assert np.isfinite(stats).all() and stats[-1, 1] < stats[0, 0]
+    assert all(np.isfinite(x).all() for x in lin.get_state())
+    lin.close()
+
+
 def test_stereo_edge_vs_oracle(gpu_ctx):
     """EdgeStereoSE3ProjectXYZ on the GPU against the FP64 oracle: residual,
     chi2, Huber weight and the 3x6 / 3x3 Jacobians within 1e-5."""
