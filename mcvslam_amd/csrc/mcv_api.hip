@@ -3191,6 +3191,7 @@ int mcv_ba_generation(mcv_ba* b, int64_t* gen) {
 // reads them after the final synchronization.
 static void ba_build_schur(mcv_ba* b, hipStream_t s) {
     mcv_ctx* c = b->ctx;
+    b->schur_done = false;  // S and b_schur lie in the same allocation
     const int P = b->P, F = b->F, M = b->M, Ms = b->have_stereo ? b->Ms : 0, E = M + Ms;
     if (b->fixed.empty()) b->fixed.assign(F, 0);
     std::vector<int> fidx(F, -1);
@@ -3382,13 +3383,18 @@ static void ba_enqueue_schur(mcv_ba* b, float lambda, hipStream_t s, bool blocks
     HIP_OK(hipGetLastError());
 }
 
-static void ba_require_schur_inputs(mcv_ba* b) {
+// what the lists need not be built for: asked first, so that a refused call
+// leaves the last S and b_schur readable
+static void ba_require_linearized(const mcv_ba* b) {
+    REQUIRE(b->pose_linearized, MCV_ERR_STATE, "linearize before the Schur complement");
+    REQUIRE(!(b->have_stereo && b->Ms > 0) || b->stereo_pose_linearized, MCV_ERR_STATE,
+            "linearize the stereo edges before the Schur complement");
+}
+
+static void ba_require_schur_inputs(const mcv_ba* b) {
     REQUIRE(b->linearized || !b->free_points_with_edges, MCV_ERR_STATE,
             "a pose-only linearization leaves no J_point for the free points");
-    const bool stereo_edges = b->have_stereo && b->Ms > 0;
-    REQUIRE(!stereo_edges || b->stereo_pose_linearized, MCV_ERR_STATE,
-            "linearize the stereo edges before the Schur complement");
-    REQUIRE(!stereo_edges || !b->free_points_with_edges || b->stereo_full, MCV_ERR_STATE,
+    REQUIRE(!(b->have_stereo && b->Ms > 0) || !b->free_points_with_edges || b->stereo_full, MCV_ERR_STATE,
             "a pose-only stereo linearization leaves no J_point for the free points");
 }
 
@@ -3452,7 +3458,7 @@ int mcv_ba_schur(mcv_ba* b, float lambda) {
     REQUIRE(b, MCV_ERR_INVALID, "null BA object");
     c->set_device();
     hipStream_t s = c->stream;
-    REQUIRE(b->pose_linearized, MCV_ERR_STATE, "linearize before the Schur complement");
+    ba_require_linearized(b);
     if (!b->schur_ready) ba_build_schur(b, s);
     ba_require_schur_inputs(b);
     ba_enqueue_schur(b, lambda, s);

@@ -275,3 +275,27 @@ def test_single_pose_more_iterations_than_one_launch(gpu_ctx):
     np.testing.assert_allclose(out[0][0][:k + 1, :3], out[1][0][:k + 1, :3], rtol=1e-3)
     assert np.abs(out[0][2][0, 4:] - out[1][2][0, 4:]).max() < 1e-5
     assert np.abs(out[0][2][0, :4] - out[1][2][0, :4]).max() < 1e-6
+
+
+def test_schur_stays_readable_after_a_refused_call(gpu_ctx):
+    """Stereo edges set but not linearized: the Schur complement is refused and
+    the last one is still what is read; after the linearization it is theirs."""
+    import ctypes
+    from mcvslam_amd import MCVError
+    from mcvslam_amd._native import lib
+    lp = synth.local_ba_problem(seed=78, n_kf=5, n_points=300, target_obs=3000, stereo_frac=0.5)
+    lin = BALinearizer.from_problem(lp.mono, ctx=gpu_ctx)
+    lin.linearize()
+    S, bs = lin.schur(1e3)
+    s = lp.stereo
+    lin.set_stereo(s.obs, s.obs_pt, s.obs_frame, s.obs_isig, s.cam)
+    with pytest.raises(MCVError):
+        lin.schur(1e3)
+    got, gb, n = np.zeros_like(S), np.zeros_like(bs), ctypes.c_int32()
+    ptr = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    assert lib().mcv_ba_read_schur(lin.h, ptr(got), ptr(gb), ctypes.byref(n)) == 0 and n.value == len(bs)
+    np.testing.assert_array_equal(got, S)
+    np.testing.assert_array_equal(gb, bs)
+    lin.linearize_stereo()
+    assert not np.array_equal(lin.schur(1e3)[0], S)
+    lin.close()
