@@ -752,15 +752,11 @@ void OrbPlan::enqueue(const OrbConfig& c, const SinCosTables& tb, hipStream_t s,
     taps.hi3 = (uint32_t)c.gauss[4] | (uint32_t)c.gauss[5] << 8 | (uint32_t)c.gauss[6] << 16;
     const int ns = (int)strips.size();
     auto blur = [&](hipStream_t bs) {
-        if (strip_h == kStripHLow)
-            hipLaunchKernelGGL((k_blur<false, kStripHLow>), strip_grid(ns), dim3(256), 0, bs, st, ns, g.lv, g.pyr,
-                               g.blur, taps);
-        else if (tune.blur & 1)
-            hipLaunchKernelGGL((k_blur<true, kStripH>), strip_grid(ns), dim3(256), 0, bs, st, ns, g.lv, g.pyr, g.blur,
-                               taps);
-        else
-            hipLaunchKernelGGL((k_blur<false, kStripH>), strip_grid(ns), dim3(256), 0, bs, st, ns, g.lv, g.pyr, g.blur,
-                               taps);
+        // the walk (tune.blur bit 0) at the plan's strip height
+        const bool fixed = (tune.blur & 1) != 0;
+        const auto kernel = strip_h == kStripHLow ? (fixed ? k_blur<true, kStripHLow> : k_blur<false, kStripHLow>)
+                                                  : (fixed ? k_blur<true, kStripH> : k_blur<false, kStripH>);
+        hipLaunchKernelGGL(kernel, strip_grid(ns), dim3(256), 0, bs, st, ns, g.lv, g.pyr, g.blur, taps);
         mark("k_blur");
     };
     // dynamic LDS: the heap (8 B per entry), then the node-table prefix (8 B per entry)

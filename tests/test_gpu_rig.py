@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import oracle
+from kernel_check import device_events
 from mcvslam_amd import RigBatch, synth
 
 pytestmark = pytest.mark.gpu
@@ -205,3 +206,30 @@ def test_rigs_in_flight(orb_default):
             rg.close()
         for cx in ctxs:
             cx.close()
+
+
+@pytest.mark.parametrize("n_frames,strip", [(2, 8), (10, 32)])
+def test_blur_walks_at_both_strip_heights(orb_default, n_frames, strip):
+    """Both walks of the blur, before FAST and beside the heap replay, on plans
+    of low strips (fewer than 8192 of 32 rows) and of 32-row ones (the frames
+    repeated): the walk asked for is the one that runs, the outputs are those
+    of the first one, and in the first frames the oracle's."""
+    import torch
+    frames = [synth.rig_frame(1100 + 10 * f) for f in range(2)]
+    imgs = [torch.from_numpy(im).cuda() for fr in frames for im in fr]
+    ptrs = [im.data_ptr() for im in imgs] * (n_frames // 2)
+    rig = RigBatch(orb_default, n_frames, ratio=0.7, th=50)
+    before = None
+    for blur in (0, 1, 2, 3):
+        rig.set_variants(1, blur, 2, 1)
+        names = {n.split("(")[0] for n in device_events(lambda: rig.run_timed(ptrs)) if "k_blur" in n}
+        assert names == {f"void mcv::k_blur<{'true' if blur & 1 else 'false'}, {strip}>"}
+        rig.run(ptrs, graph=True)
+        out = rig.read()
+        before = before or out
+        assert_same_outputs(before, out)
+    for i, im in enumerate(im for fr in frames for im in fr):
+        rk, rd = oracle.orb_extract(im)
+        assert before[2][i] == len(rk)
+        np.testing.assert_array_equal(before[1][i, :len(rk)], rd)
+    rig.close()
