@@ -3838,8 +3838,14 @@ int mcv_ba_adjoint_dev(mcv_ba* b, const float* d_g, float* d_gpose, float* d_gpo
     hipStream_t s = c->stream;
     hipLaunchKernelGGL(k_ba_point_adj, dim3((b->P + 255) / 256), dim3(256), 0, s, b->planes.as<float>(), (long long)b->M,
                        reinterpret_cast<const float2*>(d_g), b->pptr.as<int>(), b->P, d_gpoint);
-    hipLaunchKernelGGL(k_ba_pose_adj, dim3(b->F, 6), dim3(kPoseAdjThreads), 0, s, b->planes.as<float>(), (long long)b->M,
-                       reinterpret_cast<const float2*>(d_g), b->fptr.as<int>(), b->fobs.as<int>(), d_gpose);
+    const PoseAdjShape sh = pose_adj_shape(b->M, b->F);
+    const auto pose_adj = sh.threads == 1024 ? k_ba_pose_adj<1024, 1>
+                          : sh.comps == 1    ? k_ba_pose_adj<256, 1>
+                          : sh.comps == 3    ? k_ba_pose_adj<256, 3>
+                                             : k_ba_pose_adj<256, 6>;
+    hipLaunchKernelGGL(pose_adj, dim3(b->F, 6 / sh.comps), dim3(sh.threads), 0, s, b->planes.as<float>(),
+                       (long long)b->M, reinterpret_cast<const float2*>(d_g), b->fptr.as<int>(), b->fobs.as<int>(),
+                       d_gpose);
     HIP_OK(hipGetLastError());
     API_END
 }

@@ -448,42 +448,66 @@ __global__ __launch_bounds__(256) void k_ba_point_adj(const float* planes, long 
 }
 
 // grad_pose[f][c] = sum over the observations of frame f of row c of J_pose^T
-// g, one workgroup per (frame, c); each thread sums a strided slice, then a
-// fixed-order tree reduction: deterministic.  A frame's observations lie some
-// 10 apart in the planes, so a workgroup pulls whole planes through its CU:
-// that bounds it, hence the cut by component (two planes of the twelve each;
-// a workgroup per frame took 84 us for 10 frames of 15 thousand) and 4 loads
-// in flight per thread.
-constexpr int kPoseAdjThreads = 1024;
-__global__ __launch_bounds__(kPoseAdjThreads) void k_ba_pose_adj(const float* planes, long long S, const float2* g,
-                                                                 const int* fptr, const int* fobs, float* gout) {
-    __shared__ float red[kPoseAdjThreads / 64];
-    const int f = blockIdx.x, c = blockIdx.y;
-    const float* pu = planes + (4 + c) * S;
-    const float* pv = planes + (10 + c) * S;
+// g, one workgroup per frame and kC of the six components; each thread sums a
+// strided slice, then a fixed-order tree reduction: deterministic.  A frame's
+// observations lie some F apart in the planes, so what bounds it is whole lines
+// of the planes pulled through a CU for a few values each.  The cut by component
+// spreads them over more CUs, 4 loads in flight per thread; it costs the
+// observation list and g once per component (pose_adj_shape).
+template <int kThreads, int kC>
+__global__ __launch_bounds__(kThreads) void k_ba_pose_adj(const float* planes, long long S, const float2* g,
+                                                          const int* fptr, const int* fobs, float* gout) {
+    constexpr int kLoads = kC == 1 ? 4 : 2;
+    __shared__ float red[kC][kThreads / 64];
+    const int f = blockIdx.x, c0 = kC * blockIdx.y;
+    const float* pu = planes + (4 + c0) * S;
+    const float* pv = planes + (10 + c0) * S;
     const int k1 = fptr[f + 1];
-    float a[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int k = fptr[f] + threadIdx.x; k < k1; k += 4 * kPoseAdjThreads) {
-        int i[4];
+    float a[kC][kLoads] = {};
+    for (int k = fptr[f] + threadIdx.x; k < k1; k += kLoads * kThreads) {
+        int i[kLoads];
 #pragma unroll
-        for (int u = 0; u < 4; u++) i[u] = k + u * kPoseAdjThreads < k1 ? fobs[k + u * kPoseAdjThreads] : -1;
+        for (int u = 0; u < kLoads; u++) i[u] = k + u * kThreads < k1 ? fobs[k + u * kThreads] : -1;
 #pragma unroll
-        for (int u = 0; u < 4; u++)
+        for (int u = 0; u < kLoads; u++)
             if (i[u] >= 0) {
                 const float2 gi = g[i[u]];
-                a[u] += pu[i[u]] * gi.x + pv[i[u]] * gi.y;
+#pragma unroll
+                for (int c = 0; c < kC; c++) a[c][u] += pu[c * S + i[u]] * gi.x + pv[c * S + i[u]] * gi.y;
             }
     }
-    float s = (a[0] + a[1]) + (a[2] + a[3]);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float t = 0.f;
-        for (int w = 0; w < kPoseAdjThreads / 64; w++) t += red[w];
-        gout[6 * f + c] = t;
+    for (int c = 0; c < kC; c++) {
+        float s = 0.f;
+        if constexpr (kLoads == 4) s = (a[c][0] + a[c][1]) + (a[c][2] + a[c][3]);
+        else s = a[c][0] + a[c][1];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        if ((threadIdx.x & 63) == 0) red[c][threadIdx.x >> 6] = s;
     }
+    __syncthreads();
+    if (threadIdx.x < kC) {
+        float t = 0.f;
+        for (int w = 0; w < kThreads / 64; w++) t += red[threadIdx.x][w];
+        gout[6 * f + c0 + threadIdx.x] = t;
+    }
+}
+
+// Components per workgroup and threads.  Below about 500k observations the
+// planes stay in L2 and the cut by component pays at any number of frames; above,
+// only while it does not make more workgroups than CUs, which otherwise pull the
+// same lines at different times.  us of an adjoint, <256, 6> / <256, 3> / <256, 1>
+// / <1024, 1>: 10 frames of 15k observations 86 59 36 31, 5 of 300k 991 673 523
+// 275, 42 of 36k 408 259 142 211, 100 of 20k 306 201 304 397, 200 of 10k 203 320
+// 369 394, 1000 of 1000 194 206 241 239, 400 of 250 19 18 18 22, 2000 of 200 83
+// 78 66 79.
+struct PoseAdjShape {
+    int threads, comps;
+};
+inline PoseAdjShape pose_adj_shape(int M, int F) {
+    if (F <= 21) return {1024, 1};
+    if (F <= 42 || M <= 500000) return {256, 1};
+    return {256, F <= 128 ? 3 : 6};
 }
 
 // the residual planes as rows (e_u, e_v)

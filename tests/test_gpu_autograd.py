@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import oracle
+from kernel_check import device_events
 from mcvslam_amd import BALinearizer, synth
 from mcvslam_amd.autograd import apply_increments, reprojection
 
@@ -197,4 +198,37 @@ def test_negated_views(gpu_ctx):
         out.append((e, *torch.autograd.grad(e, (a, b), neg(g))))
     for x, y in zip(*out):
         np.testing.assert_array_equal(x.detach().cpu().numpy(), y.detach().cpu().numpy())
+    lin.close()
+
+
+@pytest.mark.parametrize("F,M,shape", [(21, 3000, "1024, 1"), (22, 3000, "256, 1"), (42, 500001, "256, 1"),
+                                       (43, 500000, "256, 1"), (43, 500001, "256, 3"), (128, 500001, "256, 3"),
+                                       (129, 500001, "256, 6"), (300, 900, "256, 1")])
+def test_pose_adjoint_shapes(gpu_ctx, F, M, shape):
+    """Both sides of every line between the pose adjoint's launch shapes, the
+    last frame without observations.  Bound as above, n the frame's own
+    observations and the roundings of a term."""
+    import torch
+    rng = np.random.default_rng(F + M)
+    P = M // 8
+    fr = rng.integers(0, F - 1, M)
+    lin = BALinearizer(M, P, F, 1, gpu_ctx)
+    lin.set_observations(rng.uniform(0, 600, (M, 2)), np.sort(rng.integers(0, P, M)), fr, np.zeros(M), np.ones(M))
+    lin.set_state(np.c_[rng.uniform(-2, 2, (P, 2)), rng.uniform(3, 9, P)], np.tile([0, 0, 0, 1., 0, 0, 0], (F, 1)),
+                  [[700, 700, 640, 360, 0, 0, 0, 1., 0, 0, 0, 2.]])
+    G = rng.normal(size=(M, 2)).astype(np.float32)
+    g = torch.from_numpy(G).cuda()
+    pose, point = torch.full((F, 6), 9.0, device="cuda"), torch.empty((P, 3), device="cuda")
+    lin.ctx.use_torch_stream()
+    lin.linearize()
+    names = device_events(lambda: lin.adjoint_dev(g.data_ptr(), pose.data_ptr(), point.data_ptr()))
+    assert [n for n in names if f"k_ba_pose_adj<{shape}>" in n]
+    J = lin.read(4, 12).astype(np.float64).reshape(2, 6, M)
+    G = G.T.astype(np.float64)
+    got = pose.cpu().numpy()
+    n = np.bincount(fr, minlength=F)
+    for c in range(6):
+        want = np.bincount(fr, J[0, c] * G[0] + J[1, c] * G[1], F)
+        mag = np.bincount(fr, np.abs(J[0, c] * G[0]) + np.abs(J[1, c] * G[1]), F)
+        assert (np.abs(got[:, c] - want) <= (n + 2) * 2.0 ** -24 * mag + 1e-30).all()
     lin.close()
