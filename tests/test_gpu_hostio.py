@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import oracle
+from kernel_check import device_events
 from mcvslam_amd import Context, Matcher, ORB, synth
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +49,24 @@ def test_large_image(own_ctx):
     for f in ("x", "y", "size", "angle", "response", "octave"):
         np.testing.assert_array_equal(kps[f], rk[f], err_msg=f)
     np.testing.assert_array_equal(desc, rd)
+
+
+@pytest.mark.parametrize("total,pageable", [(120000, False), (131072, True)])
+def test_outputs_take_the_place_of_inputs(own_ctx, total, pageable):
+    """3.84 MB of descriptors in and 0.72 MB of results out: each fits the
+    pinned memory, so no copy of pageable memory is made.  4 MiB of
+    descriptors leave no room for their offsets."""
+    from mcvslam_amd import distinctive_descriptors
+    rng = np.random.default_rng(8)
+    n = 20000
+    ptr = np.concatenate([[0], np.sort(rng.choice(np.arange(1, total), n - 1, replace=False)), [total]])
+    desc = rng.integers(0, 256, (total, 32), dtype=np.uint8)
+    assert np.diff(ptr).max() <= 256
+    got = []
+    names = device_events(lambda: got.append(distinctive_descriptors(desc, ptr, ctx=own_ctx)))
+    assert any("k_distinctive" in n for n in names)
+    assert any("Memcpy" in n for n in names) == pageable, names
+    best, out = got[0]
+    want = oracle.distinctive(desc, ptr.astype(np.int32))
+    np.testing.assert_array_equal(best, want)
+    np.testing.assert_array_equal(out, desc[ptr[:-1] + want])
