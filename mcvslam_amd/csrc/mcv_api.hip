@@ -2484,7 +2484,13 @@ static void window_run(mcv_ctx* c, int n_cams, const WindowQuery& q, const int32
         const int m = k % kWindowCams + 1;
         if (m < kWindowCams && k + 1 < n_cams) continue;
         hipLaunchKernelGGL(k_grid_build, dim3(m), dim3(1024), 0, s, wc);
-        if (q.P > 0) hipLaunchKernelGGL(k_window_knn, dim3((q.P + 15) / 16, m), dim3(256), 0, s, wc, wp);
+        if (q.P > 0) {
+            const int lanes = window_lanes((long long)q.P * m), per = 256 / lanes;
+            hipLaunchKernelGGL(lanes == 64   ? k_window_knn<64>
+                               : lanes == 32 ? k_window_knn<32>
+                                             : k_window_knn<16>,
+                               dim3(q.P / per + (q.P % per != 0), m), dim3(256), 0, s, wc, wp);
+        }
     }
     HIP_OK(hipGetLastError());
 }

@@ -143,7 +143,7 @@ struct WindowPoints {
     float scales[16];
 };
 
-// 16 lanes per (camera, query).  The grid's items are ordered by (column of
+// kLanes lanes per (camera, query).  The grid's items are ordered by (column of
 // cells, row, keypoint), the order candidates are visited in, so the window is
 // one run of items per column and an item's place in the grid orders it among
 // the candidates; the lanes take the items of all columns together.  Output
@@ -152,9 +152,21 @@ struct WindowPoints {
 // mvScaleFactor with it).  Bound by the chain cell ranges -> positions ->
 // descriptors of a query.  A wave per query that walked the cells one by one
 // took 67 us for 3 cameras of 5000 queries and 2000 keypoints.
+//
+// Lanes by the queries of a launch: few queries leave lanes idle, so a query
+// takes more of them, which shortens its walk over many candidates; from some
+// ten thousand on they are better spent on queries.  us of a search, 16 / 32 / 64
+// lanes: 1000 queries, 8000 keypoints in a twelfth of the image each way, radius
+// 100: 489 / - / 137; 5000 so 488 / 250 / 158, 15000 512 / 362 / 402; 2000
+// keypoints over the image, radius 400: 5000 queries 117 / 86 / 61, 10000 122 /
+// 112 / 98, 15000 137 / 163 / 123; radius 15: 8000 queries 14.8 / 14.8 / 17.1,
+// 20000 14.8 / 15.8 / 19.7.
+constexpr int window_lanes(long long queries) { return queries <= 4096 ? 64 : queries <= 10240 ? 32 : 16; }
+
+template <int kLanes>
 __global__ __launch_bounds__(256) void k_window_knn(WindowCams cams, WindowPoints W) {
-    const int lane = threadIdx.x & 15;
-    const int p = blockIdx.x * 16 + (threadIdx.x >> 4);
+    const int lane = threadIdx.x % kLanes;
+    const int p = blockIdx.x * (256 / kLanes) + threadIdx.x / kLanes;
     if (p >= W.P) return;
     const WindowCam& C = cams.c[blockIdx.y];
     const GridView& G = C.grid;
@@ -210,9 +222,9 @@ __global__ __launch_bounds__(256) void k_window_knn(WindowCams cams, WindowPoint
         const u32x4* qd = reinterpret_cast<const u32x4*>(W.pdesc + 32 * (long long)p);
         const u32x4 qa = qd[0], qb = qd[1];
         const int ncols = nMaxX - nMinX + 1;
-        for (int j0 = 0; j0 < ncols; j0 += 16) {
+        for (int j0 = 0; j0 < ncols; j0 += kLanes) {
             // lane j: column j0 + j's run of items
-            const int nc = min(16, ncols - j0);
+            const int nc = min(kLanes, ncols - j0);
             int a = 0, len = 0;
             if (lane < nc) {
                 const int* cs = G.cell_start + (nMinX + j0 + lane) * kGrid;
@@ -221,17 +233,17 @@ __global__ __launch_bounds__(256) void k_window_knn(WindowCams cams, WindowPoint
             }
             int incl = len;
 #pragma unroll
-            for (int s = 1; s < 16; s <<= 1) {
-                const int y = __shfl_up(incl, s, 16);
+            for (int s = 1; s < kLanes; s <<= 1) {
+                const int y = __shfl_up(incl, s, kLanes);
                 if (lane >= s) incl += y;
             }
-            const int total = __shfl(incl, 15, 16);
+            const int total = __shfl(incl, kLanes - 1, kLanes);
             const int first = incl - len;  // items of the columns before
-            for (int t0 = 0; t0 < total; t0 += 16) {
+            for (int t0 = 0; t0 < total; t0 += kLanes) {
                 const int t = t0 + lane;
                 int s = 0;
                 for (int j = 0; j < nc; j++) {
-                    const int fj = __shfl(first, j, 16), aj = __shfl(a, j, 16);
+                    const int fj = __shfl(first, j, kLanes), aj = __shfl(a, j, kLanes);
                     if (t >= fj) s = aj + (t - fj);
                 }
                 if (t >= total) continue;
@@ -259,12 +271,12 @@ __global__ __launch_bounds__(256) void k_window_knn(WindowCams cams, WindowPoint
     }
     // merge the lanes' top-2 keys and candidate counts
 #pragma unroll
-    for (int off = 8; off > 0; off >>= 1) {
-        const uint32_t b0 = __shfl_xor(k0, off, 16), b1 = __shfl_xor(k1, off, 16);
+    for (int off = kLanes / 2; off > 0; off >>= 1) {
+        const uint32_t b0 = __shfl_xor(k0, off, kLanes), b1 = __shfl_xor(k1, off, kLanes);
         const uint32_t n1 = min(max(k0, b0), min(k1, b1));
         k0 = min(k0, b0);
         k1 = n1;
-        ncand += __shfl_xor(ncand, off, 16);
+        ncand += __shfl_xor(ncand, off, kLanes);
     }
     if (lane != 0) return;
     auto kp_of = [&](uint32_t key) -> int {

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import oracle
+from kernel_check import device_events
 from mcvslam_amd import MCVError, synth, window_search
 from mcvslam_amd.api import window_search_dev, window_search_uv_dev
 
@@ -189,3 +190,27 @@ def test_window_more_cameras_than_one_launch(gpu_ctx):
     got = out.cpu().numpy()
     for k in range(9):
         np.testing.assert_array_equal(got[k], oracle.project_search(*oargs[k]), err_msg=f"camera {k}")
+
+
+@pytest.mark.parametrize("P,lanes", [(1, 64), (4096, 64), (4097, 32), (10240, 32), (10241, 16)])
+def test_window_lanes_per_query(gpu_ctx, P, lanes):
+    """Both sides of every line between the numbers of lanes a query takes:
+    keypoints crowded into a few cells and spread, windows of one cell and of
+    every column (30, more than 16 lanes), equal descriptors among them, so
+    that the candidate order decides."""
+    import torch
+    rng = np.random.default_rng(P)
+    w, h, n = 640, 480, 700
+    koct = rng.integers(0, 4, n).astype(np.int32)
+    kdesc = rng.integers(0, 4, (n, 32), dtype=np.uint8) // 3
+    uv = (np.array([w, h]) * rng.uniform(0.0, 1.0, (P, 2))).astype(np.float32)
+    qdesc = rng.integers(0, 4, (P, 32), dtype=np.uint8) // 3
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    for spread, r, lo, hi in [(1.0, 25.0, -1, -1), (0.05, 60.0, 1, 2), (1.0, 1000.0, -1, -1)]:
+        kxy = (np.array([w, h]) * (0.5 + spread * rng.uniform(-0.52, 0.52, (n, 2)))).astype(np.float32)
+        args = (dev(uv), dev(qdesc), r, dev(kxy), dev(koct), dev(kdesc), w, h, lo, hi, 0.9, 250)
+        got = []
+        names = device_events(lambda: got.append(window_search_uv_dev(*args, ctx=gpu_ctx)))
+        assert [x for x in names if f"k_window_knn<{lanes}>" in x]
+        want = _wnd_oracle(uv, qdesc, r, kxy, koct, kdesc, w, h, lo, hi, 0.9, 250)
+        np.testing.assert_array_equal(got[0].cpu().numpy(), want)
