@@ -3200,8 +3200,10 @@ int mcv_ba_generation(mcv_ba* b, int64_t* gen) {
 
 // The edge lists of the Schur complement over the active edges, free points
 // and free frames (mcv_ba.hip, SchurBuild), and the division of the pair
-// blocks' items into chunks.  The work arrays are the context's; nothing
-// reads them after the final synchronization.
+// blocks' items into chunks.  The work arrays are the context's (larger ones
+// than kSchurWorkKept are given back); nothing reads them after the final
+// synchronization.
+constexpr size_t kSchurWorkKept = 64u << 20;
 static void ba_build_schur(mcv_ba* b, hipStream_t s) {
     mcv_ctx* c = b->ctx;
     b->schur_done = false;  // S and b_schur lie in the same allocation
@@ -3236,7 +3238,9 @@ static void ba_build_schur(mcv_ba* b, hipStream_t s) {
     // threads that share a frame sum in k_schur_edges: its 512 threads cover
     // the 27 Fp sums once
     a.esub = Fp > 0 ? std::max(1, 512 / (kFrameSums * Fp)) : 1;
-    const size_t np = P, fp = Fp;
+    const size_t np = P, fp = Fp, erow = a.esub * kFrameSums * fp * 4;
+    a.egroup = erow ? std::max(1, (int)(((size_t)nec * erow + kEpartBytes - 1) / kEpartBytes)) : 1;
+    a.nerow = (nec + a.egroup - 1) / a.egroup;
     carve(b->sb_lists, [&](Carver& t) {
         t(B.pe_ptr, np + 1);
         t(B.pf_ptr, np + 1);
@@ -3250,7 +3254,7 @@ static void ba_build_schur(mcv_ba* b, hipStream_t s) {
         t(a.prec, np * kPointRec);
         t(a.hd, np * 3);
         t(a.Z, (size_t)E * kZRow);
-        t(a.epart, (size_t)nec * a.esub * kFrameSums * fp);
+        t(a.epart, (size_t)a.nerow * a.esub * kFrameSums * fp);
         t(a.Hpp, fp * 36);
         t(a.bs, fp * 6);
         t(a.bp, fp * 6);
@@ -3344,6 +3348,7 @@ static void ba_build_schur(mcv_ba* b, hipStream_t s) {
     if (nitem > 0) hipLaunchKernelGGL(k_sb_items<true>, dim3((rtiles + 3) / 4), dim3(256), 0, s, B);
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(s));  // the uploads' host arrays end here
+    if (c->sb_work.bytes > kSchurWorkKept) c->sb_work.release();
     a.M = M;
     a.Ms = Ms;
     a.S = M;
@@ -3386,7 +3391,9 @@ static void ba_enqueue_schur(mcv_ba* b, float lambda, hipStream_t s, bool blocks
     const SchurArgs a = ba_schur_args(b, lambda);
     hipLaunchKernelGGL(k_schur_points, dim3(xcd_grid((b->P + 31) / 32)), dim3(256), 0, s, a);
     if (b->Fp > 0) {
-        if (a.nechunk > 0) hipLaunchKernelGGL(k_schur_edges, dim3(a.nechunk), dim3(512), 0, s, a);
+        if (a.nechunk > 0)
+            hipLaunchKernelGGL(a.egroup > 1 ? k_schur_edges<true> : k_schur_edges<false>, dim3(a.nerow), dim3(512), 0, s,
+                               a);
         hipLaunchKernelGGL(k_schur_edge_sums, dim3((kFrameSums * b->Fp + 15) / 16), dim3(1024), 0, s, a);
         if (blocks) {
             if (a.nichunk > 0) hipLaunchKernelGGL(k_schur_items, dim3(xcd_grid((a.nichunk + 3) / 4)), dim3(256), 0, s, a);

@@ -551,6 +551,10 @@ constexpr int kPointRec = 12;      // floats per point: c10 c20 c21, 1/c00 1/c11
 constexpr int kEdgeChunk = 512;    // edges per workgroup of k_schur_edges
 constexpr int kItemSums = 40;      // sums of an item chunk (36, or 27 on the diagonal)
 constexpr int kFrameSums = 27;     // per frame: H_pp upper triangle by rows, each row followed by b_p's entry
+// Rows of frame sums take 0.2 Fp bytes an edge with one per chunk.  Below this
+// bound every chunk has its own (1.5M edges, 50 frames: 16 MB); it leaves a row
+// for each CU up to kMaxFreeFrames.
+constexpr size_t kEpartBytes = 256u << 20;
 
 struct ItemChunk {
     int i0, i1;  // items [i0, i1) of one frame-pair block
@@ -904,11 +908,12 @@ struct SchurArgs {
     const int* blk_chunk;   // per block: its first item chunk (nblk + 1)
     const int2* items;      // (row_i, row_j), by block, then by point
     int P, Fp, nechunk, esub, nichunk;
+    int egroup, nerow;      // chunks per workgroup of k_schur_edges, its workgroups
     float lambda;
     float* prec;            // P x kPointRec
     float* hd;              // P x 3: diagonal of H_ll
     float* Z;               // npf x kZRow
-    float* epart;           // (nechunk * esub) x (kFrameSums * Fp)
+    float* epart;           // (nerow * esub) x (kFrameSums * Fp)
     float* ipart;           // nichunk x kItemSums
     float* Hpp;             // Fp x 36 (without lambda)
     float* bs;              // Fp x 6 (b_schur)
@@ -1083,48 +1088,59 @@ __global__ __launch_bounds__(256) void k_schur_points(SchurArgs a) {
 // that different edges start in different banks), then a thread takes one of
 // a frame's 27 sums and walks the frame's edges of the chunk.  With few
 // frames, esub threads share a sum.  (A frame's edges gathered straight from
-// the planes put every 4-byte read in a line of its own.)
+// the planes put every 4-byte read in a line of its own.)  A workgroup takes
+// egroup chunks in turn and adds their sums in its row of epart: one, unless a
+// row per chunk would take more than kEpartBytes (kMany; with the loop for every
+// problem 47.0 us instead of 45.5, 50 frames and 1.5M edges).
+template <bool kMany>
 __global__ __launch_bounds__(512) void k_schur_edges(SchurArgs a) {
     constexpr int kWords = 23;  // 1 + 7 * 3 rows, and one to make it odd
     __shared__ float s_e[kEdgeChunk * kWords];
     __shared__ uint16_t s_list[kEdgeChunk];
-    const bool st = (int)blockIdx.x >= a.nchunk_m;
-    const int rows = st ? 3 : 2, words = st ? kWords : 15;
-    const int e0 = (int)(st ? blockIdx.x - a.nchunk_m : blockIdx.x) * kEdgeChunk, n = min(kEdgeChunk, (st ? a.Ms : a.M) - e0);
-    const uint16_t* ptr = a.eptr + (long long)blockIdx.x * (a.Fp + 1);
-    const int nl = ptr[a.Fp];
-    for (int i = threadIdx.x; i < nl; i += 512) s_list[i] = a.elist[(long long)blockIdx.x * kEdgeChunk + i];
-    for (int i = threadIdx.x; i < n; i += 512) {
-        const EdgeRef E = edge_ref(a, st ? a.M + e0 + i : e0 + i);
-        float* o = s_e + i * words;
-        o[0] = E.W;
-        for (int r = 0; r < rows; r++) {
-#pragma unroll
-            for (int k = 0; k < 6; k++) o[1 + 7 * r + k] = E.Jp(r, k);
-            o[7 + 7 * r] = E.e(r);
-        }
-    }
-    __syncthreads();
     const int cols = kFrameSums * a.Fp;
-    for (int t = threadIdx.x; t < cols * a.esub; t += 512) {
-        const int sub = t / cols, col = t - sub * cols, f = col / kFrameSums;
-        // sum k of a frame is element (i, c) of the rows (i, i .. 6), i = 0..5
-        int i = 0, c = col - kFrameSums * f;
-        while (c >= 7 - i) {
-            c -= 7 - i;
-            i++;
+    const int c0 = kMany ? (int)blockIdx.x * a.egroup : (int)blockIdx.x;
+    const int c1 = kMany ? min(a.nechunk, c0 + a.egroup) : c0 + 1;
+    for (int chunk = c0; chunk < c1; chunk++) {
+        const bool st = chunk >= a.nchunk_m;
+        const int rows = st ? 3 : 2, words = st ? kWords : 15;
+        const int e0 = (st ? chunk - a.nchunk_m : chunk) * kEdgeChunk, n = min(kEdgeChunk, (st ? a.Ms : a.M) - e0);
+        const uint16_t* ptr = a.eptr + (long long)chunk * (a.Fp + 1);
+        const int nl = ptr[a.Fp];
+        if (kMany && chunk > c0) __syncthreads();  // the previous chunk's LDS is read
+        for (int i = threadIdx.x; i < nl; i += 512) s_list[i] = a.elist[(long long)chunk * kEdgeChunk + i];
+        for (int i = threadIdx.x; i < n; i += 512) {
+            const EdgeRef E = edge_ref(a, st ? a.M + e0 + i : e0 + i);
+            float* o = s_e + i * words;
+            o[0] = E.W;
+            for (int r = 0; r < rows; r++) {
+#pragma unroll
+                for (int k = 0; k < 6; k++) o[1 + 7 * r + k] = E.Jp(r, k);
+                o[7 + 7 * r] = E.e(r);
+            }
         }
-        c += i;
-        float acc = 0.f;
-        const int l1 = ptr[f + 1];
-        for (int l = ptr[f] + sub; l < l1; l += a.esub) {
-            const float* e = s_e + (int)s_list[l] * words;
-            const float W = e[0];
-            acc += W * (e[1 + i] * e[1 + c]);
-            acc += W * (e[8 + i] * e[8 + c]);
-            if (rows == 3) acc += W * (e[15 + i] * e[15 + c]);
+        __syncthreads();
+        for (int t = threadIdx.x; t < cols * a.esub; t += 512) {
+            const int sub = t / cols, col = t - sub * cols, f = col / kFrameSums;
+            // sum k of a frame is element (i, c) of the rows (i, i .. 6), i = 0..5
+            int i = 0, c = col - kFrameSums * f;
+            while (c >= 7 - i) {
+                c -= 7 - i;
+                i++;
+            }
+            c += i;
+            float acc = 0.f;
+            const int l1 = ptr[f + 1];
+            for (int l = ptr[f] + sub; l < l1; l += a.esub) {
+                const float* e = s_e + (int)s_list[l] * words;
+                const float W = e[0];
+                acc += W * (e[1 + i] * e[1 + c]);
+                acc += W * (e[8 + i] * e[8 + c]);
+                if (rows == 3) acc += W * (e[15 + i] * e[15 + c]);
+            }
+            if (c == 6) acc = -acc;
+            float* sum = a.epart + ((long long)blockIdx.x * a.esub + sub) * cols + col;
+            *sum = !kMany || chunk == c0 ? acc : *sum + acc;
         }
-        a.epart[((long long)blockIdx.x * a.esub + sub) * cols + col] = c == 6 ? -acc : acc;
     }
 }
 
@@ -1132,7 +1148,7 @@ __global__ __launch_bounds__(512) void k_schur_edges(SchurArgs a) {
 // sum, chunk order fixed
 __global__ __launch_bounds__(1024) void k_schur_edge_sums(SchurArgs a) {
     __shared__ float red[64][17];
-    const int cols = kFrameSums * a.Fp, rows = a.nechunk * a.esub;
+    const int cols = kFrameSums * a.Fp, rows = a.nerow * a.esub;
     const int cl = threadIdx.x & 15, sl = threadIdx.x >> 4;
     const int col = blockIdx.x * 16 + cl;
     float acc = 0.f;

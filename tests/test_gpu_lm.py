@@ -299,3 +299,120 @@ def test_schur_stays_readable_after_a_refused_call(gpu_ctx):
     lin.linearize_stereo()
     assert not np.array_equal(lin.schur(1e3)[0], S)
     lin.close()
+
+
+def _many_frames(n_kf, n_points, seen, seed):
+    """Keyframes side by side before a wall of points.  Every point is seen by
+    keyframes 0, 1 and 2 (pairs with more shared points than one chunk of
+    items) and by `seen` others, some of them with two cameras."""
+    rng = np.random.default_rng(seed)
+    q = rng.normal(0, 0.02, (n_kf, 4)) + [0, 0, 0, 1.0]
+    frames = np.c_[q / np.linalg.norm(q, axis=1)[:, None], rng.uniform(-1, 1, (n_kf, 2)), rng.uniform(-0.3, 0.3, n_kf)]
+    points = np.c_[rng.uniform(-2, 2, (n_points, 2)), rng.uniform(4, 8, n_points)]
+    cams = np.array([[500, 500, 320, 240, 0, 0, 0, 1.0, 0.1 * k, 0, 0, 2.4] for k in range(2)])
+    rows = [(p, f, c) for p in range(n_points)
+            for f in np.r_[0, 1, 2, rng.choice(np.arange(3, n_kf), seen, replace=False)]
+            for c in range(1 + (rng.random() < 0.2))]
+    pt, fr, cam = np.array(rows).T
+    R = _rotations(frames)
+    x = np.einsum("mij,mj->mi", R[fr], points[pt]) + frames[fr, 4:]
+    x[:, 0] += 0.1 * cam
+    uv = (500 * x[:, :2] / x[:, 2:] + [320, 240] + rng.normal(0, 1.0, (len(pt), 2))).astype(np.float32)
+    fixed = np.zeros(n_kf, np.int32)
+    fixed[-1] = 1
+    return synth.BAProblem(uv, pt.astype(np.int32), fr.astype(np.int32), cam.astype(np.int32), np.zeros(len(pt), np.int32),
+                           np.ones(len(pt), np.float32), points, frames, cams, fixed)
+
+
+def _rotations(frames):
+    x, y, z, w = frames[:, :4].T
+    return np.array([[1 - 2 * (y * y + z * z), 2 * (x * y - z * w), 2 * (x * z + y * w)],
+                     [2 * (x * y + z * w), 1 - 2 * (x * x + z * z), 2 * (y * z - x * w)],
+                     [2 * (x * z - y * w), 2 * (y * z + x * w), 1 - 2 * (x * x + y * y)]]).transpose(2, 0, 1)
+
+
+def _check_schur_fp64(lin, prob):
+    """The Schur complement of a linearized _many_frames problem against the
+    FP64 sums over its points; tolerances as the dense comparisons above."""
+    n_kf = len(prob.frames)
+    e, _, w, Jp, Jx = oracle.ba_linearize(prob)
+    W = w * prob.obs_isig
+    m = 6 * (n_kf - 1)
+    for lam in (1e2, 1e4):
+        S_ref, bs_ref = lam * np.eye(m), np.zeros(m)
+        for p in range(len(prob.points)):
+            i = np.nonzero(prob.obs_pt == p)[0]
+            B, r, ww = Jx[i].reshape(-1, 3), e[i].ravel(), W[i].repeat(2)[:, None]
+            A = np.zeros((2 * len(i), n_kf, 6))
+            A[np.arange(2 * len(i)), prob.obs_frame[i].repeat(2)] = Jp[i].reshape(-1, 6)
+            used = np.unique(prob.obs_frame[i])
+            used = used[used < n_kf - 1]
+            A = A[:, used].reshape(2 * len(i), -1)
+            D = (ww * B).T @ B + lam * np.eye(3)
+            C, bl = (ww * A).T @ B, -(ww * B).T @ r
+            at = (6 * used[:, None] + np.arange(6)).ravel()
+            S_ref[np.ix_(at, at)] += (ww * A).T @ A - C @ np.linalg.solve(D, C.T)
+            bs_ref[at] += -(ww * A).T @ r - C @ np.linalg.solve(D, bl)
+        S, bs = lin.schur(lam)
+        assert np.linalg.norm(S - S_ref) < 1e-5 * np.linalg.norm(S_ref)
+        assert np.linalg.norm(bs - bs_ref) < 1e-4 * np.linalg.norm(bs_ref)
+        np.testing.assert_array_equal(lin.schur(lam)[0], S)
+
+
+@pytest.mark.parametrize("n_kf", [65, 66, 71, 131])
+def test_schur_many_frames_vs_fp64(gpu_ctx, n_kf):
+    """64 free keyframes and more: masks of more than one 64-bit word."""
+    prob = _many_frames(n_kf, 700, 8, n_kf)
+    lin = BALinearizer.from_problem(prob, ctx=gpu_ctx)
+    lin.linearize()
+    _check_schur_fp64(lin, prob)
+    lin.close()
+
+
+def test_schur_frame_sums_of_many_chunks(gpu_ctx):
+    """1000 free keyframes with 2M mono and 0.6M stereo edges: a row of frame
+    sums per chunk would take 550 MB, so workgroups take several chunks, mono
+    and stereo ones among them.  Every point is fixed, so S is H_pp + lambda I.
+    Bound: sums of n FP32 products in any order.  What stays allocated: 116
+    bytes an edge of lists and entry rows, S, at most 256 MiB of frame sums."""
+    import torch
+    from mcvslam_amd import Context
+    ctx = Context(0)
+    F, P, M, Ms = 1000, 5000, 2_000_000, 600_000
+    rng = np.random.default_rng(79)
+    fr, sfr = rng.integers(0, F, M), rng.integers(0, F, Ms)
+    lin = BALinearizer(M, P, F, 1, ctx)
+    lin.set_observations(rng.uniform(0, 640, (M, 2)), np.sort(rng.integers(0, P, M)), fr, np.zeros(M), np.ones(M))
+    cam = [500, 500, 320, 240, 0, 0, 0, 1.0, 0, 0, 0, 2.4]
+    lin.set_state(np.c_[rng.uniform(-1, 1, (P, 2)), rng.uniform(4, 8, P)], np.tile([0, 0, 0, 1.0, 0, 0, 0], (F, 1)), [cam])
+    obs = rng.uniform(0, 640, (Ms, 3))
+    lin.set_stereo(obs, rng.integers(0, P, Ms), sfr, np.ones(Ms), [500, 500, 320, 240, 50, 2.8])
+    lin.set_fixed(np.zeros(F))
+    lin.set_point_fixed(np.ones(P))
+    lin.linearize()
+    lin.linearize_stereo()
+    ctx.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    S, bs = lin.schur(10.0)
+    assert free - torch.cuda.mem_get_info()[0] < 116 * (M + Ms) + 144e6 + (256 << 20) + 40e6
+    e, _, w, Jp, _ = lin.results()
+    se, _, sw, sJp, _ = lin.stereo_results()
+    f64 = lambda a: np.asarray(a, np.float64)
+    blocks = S.reshape(F, 6, F, 6)
+    got = blocks[np.arange(F), :, np.arange(F)]
+    n = np.bincount(fr, minlength=F) * 2 + np.bincount(sfr, minlength=F) * 3
+    for i in range(6):
+        for j in range(i, 7):
+            want, mag = np.zeros(F), np.zeros(F)
+            for J, r, W, f in ((Jp, e, w, fr), (sJp, se, sw, sfr)):
+                t = f64(W)[:, None] * f64(J[:, :, i]) * (f64(J[:, :, j]) if j < 6 else -f64(r))
+                want += np.bincount(f, t.sum(1), F)
+                mag += np.bincount(f, np.abs(t).sum(1), F)
+            if j == i:
+                want += 10.0
+            x = got[:, i, j] if j < 6 else bs.reshape(F, 6)[:, i]
+            assert (np.abs(x - want) <= (n + 4) * 2.0 ** -24 * (mag + 10.0)).all(), (i, j)
+    blocks[np.arange(F), :, np.arange(F)] = 0
+    assert not S.any()
+    lin.close()
+    ctx.close()
