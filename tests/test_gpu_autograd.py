@@ -221,8 +221,9 @@ def test_pose_adjoint_shapes(gpu_ctx, F, M, shape):
     pose, point = torch.full((F, 6), 9.0, device="cuda"), torch.empty((P, 3), device="cuda")
     lin.ctx.use_torch_stream()
     lin.linearize()
-    names = device_events(lambda: lin.adjoint_dev(g.data_ptr(), pose.data_ptr(), point.data_ptr()))
-    assert [n for n in names if f"k_ba_pose_adj<{shape}>" in n]
+    kernel = f"k_ba_pose_adj<{shape}>"
+    names = device_events(lambda: lin.adjoint_dev(g.data_ptr(), pose.data_ptr(), point.data_ptr()), [kernel])
+    assert {n.split("(")[0] for n in names if "k_ba_pose_adj" in n} == {"void mcv::" + kernel}
     J = lin.read(4, 12).astype(np.float64).reshape(2, 6, M)
     G = G.T.astype(np.float64)
     got = pose.cpu().numpy()

@@ -210,7 +210,8 @@ def test_window_lanes_per_query(gpu_ctx, P, lanes):
         kxy = (np.array([w, h]) * (0.5 + spread * rng.uniform(-0.52, 0.52, (n, 2)))).astype(np.float32)
         args = (dev(uv), dev(qdesc), r, dev(kxy), dev(koct), dev(kdesc), w, h, lo, hi, 0.9, 250)
         got = []
-        names = device_events(lambda: got.append(window_search_uv_dev(*args, ctx=gpu_ctx)))
-        assert [x for x in names if f"k_window_knn<{lanes}>" in x]
+        kernel = f"k_window_knn<{lanes}>"
+        names = device_events(lambda: got.append(window_search_uv_dev(*args, ctx=gpu_ctx)), [kernel])
+        assert {x.split("(")[0] for x in names if "k_window_knn" in x} == {"void mcv::" + kernel}
         want = _wnd_oracle(uv, qdesc, r, kxy, koct, kdesc, w, h, lo, hi, 0.9, 250)
         np.testing.assert_array_equal(got[0].cpu().numpy(), want)
