@@ -913,7 +913,7 @@ struct mcv_ctx {
     DevBuf o_m, o_a1, o_a2, o_out, o_cnt, o_jobs;
     DevBuf w_pts, w_pdesc, w_plev, w_kxy, w_kdesc, w_cs, w_ci, w_cxy, w_out;
     DevBuf b_d1, b_d2, b_f2, b_jobs, b_out;
-    DevBuf sb_work;  // ba_build_schur
+    DevBuf sb_work, sb_cut;  // ba_build_schur
     std::map<std::string, std::unique_ptr<OrbPlan>> plans;
 
     void set_device() { HIP_OK(hipSetDevice(device)); }
@@ -3204,6 +3204,7 @@ int mcv_ba_generation(mcv_ba* b, int64_t* gen) {
 // than kSchurWorkKept are given back); nothing reads them after the final
 // synchronization.
 constexpr size_t kSchurWorkKept = 64u << 20;
+constexpr int kMinItems = 128, kMinCut = 192;  // items of a chunk; of a block that is cut
 static void ba_build_schur(mcv_ba* b, hipStream_t s) {
     mcv_ctx* c = b->ctx;
     b->schur_done = false;  // S and b_schur lie in the same allocation
@@ -3217,6 +3218,11 @@ static void ba_build_schur(mcv_ba* b, hipStream_t s) {
     const int nb = (P + 255) / 256, etiles = std::max((E + 255) / 256, 1), rtiles = E / 64 + Fp + 1;
     const int nblk = Fp * (Fp + 1) / 2, ncm = (M + kEdgeChunk - 1) / kEdgeChunk;
     const int nec = Fp > 0 ? ncm + (Ms + kEdgeChunk - 1) / kEdgeChunk : 0;
+    // The host cuts the blocks' items by windows of their rows: every block's in
+    // one table while that stays below 1 MiB, else the totals first and the
+    // windows of the blocks that are cut (1500 frames, 300k edges: the table
+    // is 150 MB, all but a few blocks without items).
+    const bool all_windows = (size_t)nblk * (kWindows + 1) <= 1u << 18;
     // entries are at most the edges, so all lists but the items have a bound here
     SchurBuild B{};
     SchurArgs a{};
@@ -3233,8 +3239,10 @@ static void ba_build_schur(mcv_ba* b, hipStream_t s) {
         t(B.fbase, Fp + 1);
         t(B.tbase, Fp + 1);
         t(B.tcount, (size_t)rtiles * Fp);
-        t(B.win, (size_t)nblk * (kWindows + 1));
+        t(B.win, all_windows ? (size_t)nblk * (kWindows + 1) : 0);
+        t(B.btotal, all_windows ? 0 : (size_t)nblk);
     });
+    if (!all_windows) B.win = nullptr;
     // threads that share a frame sum in k_schur_edges: its 512 threads cover
     // the 27 Fp sums once
     a.esub = Fp > 0 ? std::max(1, 512 / (kFrameSums * Fp)) : 1;
@@ -3294,9 +3302,11 @@ static void ba_build_schur(mcv_ba* b, hipStream_t s) {
     }
     HIP_OK(hipGetLastError());
     // the items' windows and the totals come back; the host cuts the chunks
-    std::vector<int> win((size_t)nblk * (kWindows + 1));
+    const int wstep = all_windows ? kWindows + 1 : 1;  // a block's total is its last int
+    std::vector<int> win((size_t)nblk * wstep);
     int tot[3] = {0, 0, 0};
-    if (nblk) HIP_OK(hipMemcpyAsync(win.data(), B.win, win.size() * 4, hipMemcpyDeviceToHost, s));
+    if (nblk)
+        HIP_OK(hipMemcpyAsync(win.data(), all_windows ? B.win : B.btotal, win.size() * 4, hipMemcpyDeviceToHost, s));
     HIP_OK(hipMemcpyAsync(tot, B.btot + 3 * nb, 12, hipMemcpyDeviceToHost, s));
     HIP_OK(hipStreamSynchronize(s));
     // one upload: every block's first item, its first chunk, then the chunks
@@ -3304,23 +3314,57 @@ static void ba_build_schur(mcv_ba* b, hipStream_t s) {
     int* blk_ptr = up.data();
     int* blk_chunk = blk_ptr + nblk + 1;
     for (int k = 0; k < nblk; k++) {
-        const long long n = (long long)blk_ptr[k] + win[(size_t)k * (kWindows + 1) + kWindows];
+        const long long n = (long long)blk_ptr[k] + win[(size_t)k * wstep + wstep - 1];
         REQUIRE(n <= INT32_MAX, MCV_ERR_CAPACITY, "more than 2^31 frame-pair products");
         blk_ptr[k + 1] = (int)n;
     }
     const int nitem = blk_ptr[nblk];
+    std::vector<int> some;  // the windows of the blocks that are cut
+    if (!all_windows) {
+        std::vector<int2> cutb;
+        for (int i = 0, k = 0; i < Fp; i++)
+            for (int j = i; j < Fp; j++, k++)
+                if (win[k] >= kMinCut) cutb.push_back(make_int2(i, j));
+        const int n = (int)cutb.size();
+        if (n) {
+            int2* d_cut = nullptr;
+            int* d_win = nullptr;
+            carve(c->sb_cut, [&](Carver& t) {
+                t(d_cut, n);
+                t(d_win, (size_t)n * kWindows);
+            });
+            some.resize((size_t)n * kWindows);
+            HIP_OK(hipMemcpyAsync(d_cut, cutb.data(), (size_t)n * sizeof(int2), hipMemcpyHostToDevice, s));
+            hipLaunchKernelGGL(k_sb_windows, dim3((n * kWindows + 255) / 256), dim3(256), 0, s, B, d_cut, n, d_win);
+            HIP_OK(hipGetLastError());
+            HIP_OK(hipMemcpyAsync(some.data(), d_win, some.size() * 4, hipMemcpyDeviceToHost, s));
+            HIP_OK(hipStreamSynchronize(s));
+        }
+    }
     // Chunks of a block's items, one wave each: whole windows up to at least
-    // 128 items, at most csz items (about 16384 waves), launched in the order
+    // kMinItems items, at most csz items (about 16384 waves), launched in the order
     // of their first window (see k_schur_items).
     const int csz = std::min(2048, std::max(256, (nitem / 16384 + 63) / 64 * 64));
     std::vector<ItemChunk> cut;
     std::vector<int> first, cnt(kWindows + 1, 0);
+    int wbuf[kWindows + 1];
+    const int* next = some.data();
     for (int i = 0, k = 0; i < Fp; i++)
         for (int j = i; j < Fp; j++, k++) {
             const int* w = win.data() + (size_t)k * (kWindows + 1);
+            if (!all_windows) {
+                wbuf[kWindows] = win[k];
+                if (win[k] >= kMinCut) {
+                    std::copy(next, next + kWindows, wbuf);
+                    next += kWindows;
+                } else {
+                    std::fill(wbuf, wbuf + kWindows, 0);  // one chunk
+                }
+                w = wbuf;
+            }
             for (int x = 0, y = 0; x < kWindows && w[kWindows] > 0; x = y) {
-                for (y = x + 1; y < kWindows && w[y] - w[x] < 128; y++) {}
-                if (y < kWindows && w[kWindows] - w[y] < 64) y = kWindows;  // no remainder of its own
+                for (y = x + 1; y < kWindows && w[y] - w[x] < kMinItems; y++) {}
+                if (y < kWindows && w[kWindows] - w[y] < kMinCut - kMinItems) y = kWindows;  // no remainder of its own
                 for (int i0 = w[x]; i0 < w[y]; i0 += csz) {
                     cut.push_back(ItemChunk{blk_ptr[k] + i0, blk_ptr[k] + std::min(i0 + csz, w[y]), (int)cut.size(),
                                             i == j ? 1 : 0});
@@ -3348,7 +3392,8 @@ static void ba_build_schur(mcv_ba* b, hipStream_t s) {
     if (nitem > 0) hipLaunchKernelGGL(k_sb_items<true>, dim3((rtiles + 3) / 4), dim3(256), 0, s, B);
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(s));  // the uploads' host arrays end here
-    if (c->sb_work.bytes > kSchurWorkKept) c->sb_work.release();
+    for (DevBuf* w : {&c->sb_work, &c->sb_cut})
+        if (w->bytes > kSchurWorkKept) w->release();
     a.M = M;
     a.Ms = Ms;
     a.S = M;

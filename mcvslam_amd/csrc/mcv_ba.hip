@@ -594,7 +594,8 @@ struct SchurBuild {
     int* fbase;               // Fp + 1: first row of a frame
     int* tbase;               // Fp + 1: first 64-row tile of a frame
     int* tcount;              // row tiles x Fp
-    int* win;                 // nblk x (kWindows + 1): items before each window
+    int* win;                 // nblk x (kWindows + 1): items before each window, then all; or null:
+    int* btotal;              // nblk: all items
     const int* blk_ptr;       // nblk
     int2* items;
     uint16_t *eptr, *elist;
@@ -822,7 +823,8 @@ __global__ __launch_bounds__(64) void k_sb_blocks(SchurBuild b) {
     const int i = blockIdx.y, j = blockIdx.x;
     if (j < i) return;
     const int t0 = b.tbase[i], nt = b.tbase[i + 1] - t0, lane = threadIdx.x;
-    int* win = b.win + (long long)block_of(i, j, b.Fp) * (kWindows + 1);
+    const int blk = block_of(i, j, b.Fp);
+    int* win = b.win ? b.win + (long long)blk * (kWindows + 1) : nullptr;
     int run = 0;
     for (int k0 = 0; k0 < nt; k0 += 64) {
         const int k = k0 + lane;
@@ -837,14 +839,28 @@ __global__ __launch_bounds__(64) void k_sb_blocks(SchurBuild b) {
         if (k < nt) {
             *c = run + x - v;
             // windows whose first tile (w * nt / kWindows) is k
-            for (int w = (int)(((long long)k * kWindows + nt - 1) / nt);
-                 w < kWindows && (int)((long long)w * nt / kWindows) == k; w++)
-                win[w] = run + x - v;
+            if (win)
+                for (int w = (int)(((long long)k * kWindows + nt - 1) / nt);
+                     w < kWindows && (int)((long long)w * nt / kWindows) == k; w++)
+                    win[w] = run + x - v;
         }
         run += __shfl(x, 63, 64);
     }
+    if (!win) {
+        if (lane == 0) b.btotal[blk] = run;
+        return;
+    }
     if (nt == 0 && lane < kWindows) win[lane] = 0;
     if (lane == 0) win[kWindows] = run;
+}
+
+// the windows of some blocks (i, j) that have items, from the tiles' offsets
+__global__ __launch_bounds__(256) void k_sb_windows(SchurBuild b, const int2* blocks, int n, int* win) {
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k >= n * kWindows) return;
+    const int2 ij = blocks[k / kWindows];
+    const int w = k % kWindows, t0 = b.tbase[ij.x], nt = b.tbase[ij.x + 1] - t0;
+    win[k] = b.tcount[(t0 + (long long)w * nt / kWindows) * b.Fp + ij.y];
 }
 
 // the frame-sorted edge lists of k_schur_edges' chunks

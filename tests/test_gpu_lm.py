@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import oracle
+from kernel_check import device_events
 from lm_check import dense_schur, dense_system
 from mcvslam_amd import BALinearizer, synth
 from mcvslam_amd.ba import bundle_adjustment, local_ba_linearizer, pose_optimization
@@ -416,3 +417,22 @@ def test_schur_frame_sums_of_many_chunks(gpu_ctx):
     assert not S.any()
     lin.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("n_kf,fetched", [(126, False), (127, True), (160, True)])
+def test_schur_windows_of_cut_pairs(gpu_ctx, n_kf, fetched):
+    """125 free keyframes and fewer: the windows of every keyframe pair come to
+    the host in one table; more: those of the pairs whose items are cut into
+    chunks alone (the pairs of keyframes 0, 1 and 2 here)."""
+    prob = _many_frames(n_kf, 700, 8, n_kf)
+    lin = BALinearizer.from_problem(prob, ctx=gpu_ctx)
+    lin.linearize()
+
+    def build():
+        lin.set_active(np.ones(lin.M, np.uint8))          # the lists are built anew
+        lin.schur(1e2)
+
+    names = device_events(build, ["k_sb_blocks"] + ["k_sb_windows"] * fetched)
+    assert any("k_sb_windows" in n for n in names) == fetched
+    _check_schur_fp64(lin, prob)
+    lin.close()
