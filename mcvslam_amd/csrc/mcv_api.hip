@@ -2097,9 +2097,9 @@ int mcv_rig_autotune(mcv_rig* r, const uint8_t* const* d_images, int reps, char*
     std::string rep;
     char line[160];
     {
-        int best = 0;
+        int best = 1;
         float bt = 1e30f;
-        for (int v = 0; v < kKnnVariants; v++) {
+        for (int v = 1; v < kKnnVariants; v++) {  // 0 stands for one of them
             r->tune.knn = v;
             const float t = time_kernel("k_knn2");
             snprintf(line, sizeof line, "k_knn2 %s %.4f ms\n", knn_variant_name(v), t);

@@ -234,3 +234,16 @@ def test_blur_walks_at_both_strip_heights(orb_default, n_frames, strip):
         assert before[2][i] == len(rk)
         np.testing.assert_array_equal(before[1][i, :len(rk)], rd)
     rig.close()
+
+
+def test_autotune_times_each_top2_kernel_once(orb_default):
+    """Every top-2 kernel appears once in the report, and the library's rule
+    (variant 0), which stands for one of them, not at all."""
+    import torch
+    imgs = [torch.from_numpy(im).cuda() for im in synth.rig_frame(1300)]
+    rig = RigBatch(orb_default, 1, ratio=0.7, th=50)
+    report = rig.autotune([im.data_ptr() for im in imgs], reps=1)
+    names = [line.split()[1] for line in report.splitlines() if line.startswith("k_knn2 ")]
+    assert len(names) == len(set(names)) == 11 and "rule" not in names
+    assert rig.variants()[0] != 0
+    rig.close()
