@@ -137,9 +137,9 @@ int mcv_distinctive_descriptors(mcv_ctx* ctx, const uint8_t* desc, const int32_t
  * (0 .. 11: 0, the default, the library's choice (currently 10); 1-3, 5-7
  * popcount kernels with scalar-loaded trains, 4 LDS-tiled, 8-9 distances on
  * the int8 matrix cores, 10-11 on the fp4 ones, which cut large train sets
- * into segments when there are few queries; no counterpart in the reference:
- * the autotuner's choice, also settable for testing).  Every variant returns
- * the same rows. */
+ * into segments when there are few queries; no counterpart in the reference).
+ * A rig's variants, tuned or fixed, are its own.  Every variant returns the
+ * same rows. */
 int mcv_match_set_variant(mcv_ctx* ctx, int variant);
 int mcv_match_knn2_dev(mcv_ctx* ctx, const uint8_t* d_q, int nq, const uint8_t* d_t, int nt, int32_t* d_out);
 /* Replaces MatchResKnn::FilterRatio(ratio).FilterThreshold(th)

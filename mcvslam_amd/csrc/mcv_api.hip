@@ -895,7 +895,7 @@ struct mcv_ctx {
     hipStream_t own = nullptr;
     hipStream_t cap = nullptr;  // graph capture only (the null stream cannot capture)
     hipStream_t side = nullptr; // graph capture only: the blur branch
-    int knn_variant = 0;        // for mcv_match_knn2*: the last rig tuning's choice
+    int knn_variant = 0;        // for mcv_match_knn2* (mcv_match_set_variant)
     std::map<std::string, Tuning> tuned;  // rig shape -> autotuned choices
     hipStream_t stream = nullptr;
     std::string err;
@@ -2207,7 +2207,6 @@ int mcv_rig_autotune(mcv_rig* r, const uint8_t* const* d_images, int reps, char*
     P.tune = r->tune;
     for (auto& sp : r->single) sp->tune = r->tune;
     c->tuned[r->shape_key] = r->tune;
-    c->knn_variant = r->tune.knn;
     r->drop_graphs();
     if (report && report_cap > 0) {
         strncpy(report, rep.c_str(), (size_t)report_cap - 1);

@@ -5,7 +5,7 @@ import pytest
 
 import oracle
 from kernel_check import device_events
-from mcvslam_amd import RigBatch, synth
+from mcvslam_amd import Context, Matcher, ORB, RigBatch, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -247,3 +247,23 @@ def test_autotune_times_each_top2_kernel_once(orb_default):
     assert len(names) == len(set(names)) == 11 and "rule" not in names
     assert rig.variants()[0] != 0
     rig.close()
+
+
+def test_autotune_leaves_the_matcher_alone(gpu_ctx):
+    """The matcher's top-2 kernel is the one set on the context, whatever a
+    rig's autotuner finds the fastest for the rig."""
+    import torch
+    ctx = Context(0)
+    ctx.set_match_variant(5)
+    imgs = [torch.from_numpy(im).cuda() for im in synth.rig_frame(1301)]
+    torch.cuda.synchronize()
+    rig = RigBatch(ORB(2000, 1.2, 8, 20, 7, ctx=ctx), 1, ratio=0.7, th=50)
+    rig.autotune([im.data_ptr() for im in imgs], reps=1)
+    rng = np.random.default_rng(1)
+    q, t = (rng.integers(0, 256, (n, 32), dtype=np.uint8) for n in (300, 400))
+    rows = []
+    names = device_events(lambda: rows.append(Matcher.KnnMatch(q, t, ctx=ctx).rows), ["k_knn2_s<2, 8>"])
+    assert {n.split("(")[0] for n in names if "k_knn2" in n} == {"void mcv::k_knn2_s<2, 8>"}
+    np.testing.assert_array_equal(rows[0], oracle.knn2(q, t))
+    rig.close()
+    ctx.close()
