@@ -43,7 +43,11 @@ int mcv_create(mcv_ctx** ctx, int device);
 void mcv_destroy(mcv_ctx* ctx);
 const char* mcv_last_error(const mcv_ctx* ctx);
 /* hipStream_t to enqueue on; NULL is the null (default) stream.  A new
- * context enqueues on a non-blocking stream of its own. */
+ * context enqueues on a non-blocking stream of its own.  A context's calls
+ * share its work buffers (the segment keys of mcv_match_knn2_dev, the grids of
+ * mcv_window_search_dev, ...) for as long as their kernels run, so work that is
+ * enqueued on another stream has to be ordered after what the context enqueued
+ * before; work that is to overlap takes contexts of its own. */
 int mcv_set_stream(mcv_ctx* ctx, void* hip_stream);
 int mcv_use_own_stream(mcv_ctx* ctx);
 int mcv_synchronize(mcv_ctx* ctx);

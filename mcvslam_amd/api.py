@@ -54,7 +54,9 @@ class Context:
             pass
 
     def set_stream(self, stream_handle: int | None):
-        """hipStream_t handle (0 / None: the null stream)."""
+        """hipStream_t handle (0 / None: the null stream).  Work enqueued before
+        on another stream shares the context's buffers: order the two, or use a
+        context for each."""
         check(self.h, lib().mcv_set_stream(self.h, ctypes.c_void_p(stream_handle or 0)))
 
     def use_own_stream(self):
