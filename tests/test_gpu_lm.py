@@ -436,3 +436,62 @@ def test_schur_windows_of_cut_pairs(gpu_ctx, n_kf, fetched):
     assert any("k_sb_windows" in n for n in names) == fetched
     _check_schur_fp64(lin, prob)
     lin.close()
+
+
+def _one_frame(n_edges, n_cams, n_stereo, seed):
+    """One keyframe before a wall of fixed points, the last one unseen: exactly
+    n_edges mono edges over n_cams cameras and n_stereo stereo edges, from a
+    perturbed pose."""
+    rng = np.random.default_rng(seed)
+    P = max(-(-n_edges // n_cams), n_stereo) + 1
+    points = np.c_[rng.uniform(-2, 2, (P, 2)), rng.uniform(4, 8, P)]
+    cams = np.array([[500, 500, 320, 240, 0, 0, 0, 1.0, 0.05 * k, -0.02 * k, 0, 2.4] for k in range(n_cams)])
+    pt, cam = np.repeat(np.arange(P - 1), n_cams)[:n_edges], np.tile(np.arange(n_cams), P - 1)[:n_edges]
+    x = points[pt] + cams[cam, 8:11]
+    uv = 500 * x[:, :2] / x[:, 2:] + [320, 240] + rng.normal(0, 1.0, (n_edges, 2))
+    frame = oracle.se3_oplus(np.array([0, 0, 0, 1.0, 0, 0, 0]), rng.normal(0, 0.01, 6))[None]
+    i32, z = np.int32, np.zeros
+    mono = synth.BAProblem(uv.astype(np.float32), pt.astype(i32), z(n_edges, i32), cam.astype(i32), z(n_edges, i32),
+                           np.ones(n_edges, np.float32), points, frame, cams, z(1, i32))
+    spt = np.sort(rng.choice(P - 1, n_stereo, replace=False)).astype(i32)
+    xs = points[spt]
+    obs = np.c_[500 * xs[:, :2] / xs[:, 2:] + [320, 240], 500 * xs[:, 0] / xs[:, 2] + 320 - 50 / xs[:, 2]]
+    obs = (obs + rng.normal(0, 1.0, obs.shape)).astype(np.float32)
+    stereo = synth.StereoProblem(obs, spt, z(n_stereo, i32), np.ones(n_stereo, np.float32), points, frame,
+                                 np.array([500, 500, 320, 240, 50, 2.8]))
+    return mono, stereo
+
+
+@pytest.mark.parametrize("n_edges,n_cams,n_stereo,one_launch",
+                         [(511, 1, 0, True), (512, 2, 0, True), (513, 3, 2, True), (1535, 3, 511, True),
+                          (1536, 3, 512, True), (1537, 3, 513, True), (16384, 8, 0, True), (15000, 8, 1384, True),
+                          (16385, 8, 0, False), (15000, 8, 1385, False), (900, 8, 40, True), (900, 9, 40, False)])
+def test_single_pose_route_limits(gpu_ctx, n_edges, n_cams, n_stereo, one_launch):
+    """The one-launch optimizer at the edges of its division of the edges (512
+    threads, 3 mono edges each at a time) and on both sides of its limits (16384
+    edges, 8 cameras), against the FP64 oracle and the general route, which the
+    same problem takes when the unseen point is left free.  Tolerances as
+    test_single_pose_route_vs_oracle_and_general_route."""
+    mono, stereo = _one_frame(n_edges, n_cams, n_stereo, n_edges + n_cams)
+    stereo = stereo if n_stereo else None
+    out = []
+    for last in (1, 0):
+        pfix = np.ones(len(mono.points), np.int32)
+        pfix[-1] = last
+        lin = local_ba_linearizer(mono, stereo, pfix, ctx=gpu_ctx)
+        stats, _ = lin.optimize(5)
+        out.append((stats, lin.get_state()[1]))
+
+        def again():
+            lin.set_state(mono.points, mono.frames, mono.cams)
+            lin.optimize(1)
+
+        names = device_events(again, ["k_pose_optimize" if one_launch and last else "k_schur_assemble"])
+        assert any("k_pose_optimize" in n for n in names) == bool(one_launch and last)
+        lin.close()
+    _, frs, ost, _, _ = oracle.ba_lm(mono, stereo, iterations=5, point_fixed=np.ones(len(mono.points), np.int32))
+    for stats, got in out:
+        assert np.abs(got[0, 4:] - frs[0, 4:]).max() < 1e-5
+        assert np.abs(got[0, :4] - frs[0, :4]).max() < 1e-6
+        assert abs(stats[0, 0] - ost[0, 0]) < 1e-5 * ost[0, 0]
+        assert abs(stats[-1, 1] - ost[-1, 1]) < 1e-5 * ost[-1, 1]

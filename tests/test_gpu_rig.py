@@ -267,3 +267,26 @@ def test_autotune_leaves_the_matcher_alone(gpu_ctx):
     np.testing.assert_array_equal(rows[0], oracle.knn2(q, t))
     rig.close()
     ctx.close()
+
+
+def test_rig_top2_forms_agree_with_popcount(orb_default):
+    """Every top-2 form in the graph and in the plain path against a popcount
+    form (variant 0 is one of the fp4 ones, so it is no reference for them)."""
+    import torch
+    imgs = [torch.from_numpy(im).cuda() for f in range(2) for im in synth.rig_frame(1400 + 10 * f)]
+    ptrs = [im.data_ptr() for im in imgs]
+    rig = RigBatch(orb_default, 2, ratio=0.7, th=50)
+    rig.set_variants(1, 0)
+    rig.run(ptrs, graph=False)
+    want = rig.read()
+    for knn in (0, *range(2, 12)):
+        rig.set_variants(knn, 0)
+        for graph in (True, False):
+            rig.run(ptrs, graph=graph)
+            assert_same_outputs(want, rig.read())
+    rig.close()
+
+
+def test_rig_images_without_keypoints_popcount(orb_default):
+    """The same pairs without queries or trains through a popcount form."""
+    test_rig_images_without_keypoints(orb_default, 1)
