@@ -1076,7 +1076,7 @@ struct BAVariantDesc {
     bool nt;
     const char* name;
 };
-constexpr int kMaxFreeFrames = 7700;  // (6 * 7700)^2 entries of S are the most 31 bits count
+constexpr int kMaxFreeFrames = 7723;  // (6 * 7723)^2 entries of S are the most 31 bits count
 constexpr int kBaVariants = 8;
 static const BAVariantDesc kBaVariant[kBaVariants] = {
     {256, 1024, 1, false, "256x1024 ilp1"},     {256, 1024, 2, false, "256x1024 ilp2"},

@@ -495,3 +495,27 @@ def test_single_pose_route_limits(gpu_ctx, n_edges, n_cams, n_stereo, one_launch
         assert np.abs(got[0, :4] - frs[0, :4]).max() < 1e-6
         assert abs(stats[0, 0] - ost[0, 0]) < 1e-5 * ost[0, 0]
         assert abs(stats[-1, 1] - ost[-1, 1]) < 1e-5 * ost[-1, 1]
+
+
+@pytest.mark.parametrize("free,accepted", [(7723, True), (7724, False)])
+def test_schur_most_free_frames(gpu_ctx, free, accepted):
+    """S of 7723 free keyframes has the most entries that 31 bits count; each
+    keyframe sees a point of its own and one that its neighbours see."""
+    import ctypes
+    from mcvslam_amd import Context
+    from mcvslam_amd._native import lib
+    ctx = Context(0)
+    P = 2 * free
+    pt = np.sort(np.r_[np.arange(P), np.arange(1, P, 2)])
+    fr = np.where(np.r_[True, pt[1:] != pt[:-1]], pt // 2, np.minimum(pt // 2 + 1, free - 1))
+    M = len(pt)
+    lin = BALinearizer(M, P, free, 1, ctx)
+    lin.set_observations(np.full((M, 2), 300.0), pt, fr, np.zeros(M), np.ones(M))
+    lin.set_state(np.tile([0.1, 0.2, 5.0], (P, 1)), np.tile([0, 0, 0, 1.0, 0, 0, 0], (free, 1)),
+                  [[500, 500, 320, 240, 0, 0, 0, 1.0, 0, 0, 0, 2.4]])
+    lin.set_fixed(np.zeros(free))
+    lin.linearize()
+    assert lib().mcv_ba_schur(lin.h, ctypes.c_float(10.0)) == (0 if accepted else -1)
+    ctx.synchronize()
+    lin.close()
+    ctx.close()
