@@ -605,13 +605,27 @@ class BALinearizer:
              np.ascontiguousarray(cams, np.float64)]
         check(self.ctx.h, lib().mcv_ba_set_state(self.h, *[_p(x) for x in a]))
 
+    def increments_fit(self, pose_delta, point_delta) -> bool:
+        """Whether two tensors are what set_state_increments reads: F x 6 and
+        P x 3, float32 or float64, on this device."""
+        return all(d.is_cuda and d.device.index == self.ctx.device and tuple(d.shape) == shape
+                   and str(d.dtype) in ("torch.float32", "torch.float64")
+                   for d, shape in ((pose_delta, (self.F, 6)), (point_delta, (self.P, 3))))
+
     def set_state_increments(self, points, frames, cams, pose_delta, point_delta):
         """The state after the increments pose_delta (F x 6) and point_delta
-        (P x 3): contiguous float32 or float64 tensors on this device."""
+        (P x 3): float32 or float64 tensors on this device."""
+        if not self.increments_fit(pose_delta, point_delta):
+            raise ValueError("increments: F x 6 and P x 3, float32 or float64, on the context's device")
         a = [np.ascontiguousarray(points, np.float64), np.ascontiguousarray(frames, np.float64),
              np.ascontiguousarray(cams, np.float64)]
+        if a[0].shape != (self.P, 3) or a[1].shape != (self.F, 7) or a[2].shape != (self.C, 12):
+            raise ValueError("state: points P x 3, frames F x 7, cams C x 12")
+        # as memory: dense, and without a negation that is still to be done
+        delta = [t.detach().resolve_neg().contiguous() for t in (pose_delta, point_delta)]
+        self.ctx.use_torch_stream()
         d = []
-        for t in (pose_delta, point_delta):
+        for t in delta:
             d += [ctypes.c_void_p(t.data_ptr()), int(t.element_size() == 8)]
         check(self.ctx.h, lib().mcv_ba_set_state_increments(self.h, *[_p(x) for x in a], *d))
 

@@ -77,25 +77,16 @@ def apply_increments(points, frames, pose_delta, point_delta):
     return np.asarray(points, np.float64) + point_delta, fr
 
 
-def _on_device(d, shape, device):
-    return (d.is_cuda and d.device.index == device and tuple(d.shape) == shape
-            and d.dtype in (torch.float32, torch.float64))
-
-
 class Reprojection(torch.autograd.Function):
     @staticmethod
     def forward(ctx, pose_delta: torch.Tensor, point_delta: torch.Tensor, lin: BALinearizer, state):
         points, frames, cams = state
         # increments of other kinds (another type, broadcast rows, another
         # device or the host) are applied on the host
-        native = (_on_device(pose_delta, (lin.F, 6), lin.ctx.device)
-                  and _on_device(point_delta, (lin.P, 3), lin.ctx.device)
-                  and np.shape(points) == (lin.P, 3) and np.shape(frames) == (lin.F, 7))
+        native = (lin.increments_fit(pose_delta, point_delta) and np.shape(points) == (lin.P, 3)
+                  and np.shape(frames) == (lin.F, 7) and np.shape(cams) == (lin.C, 12))
         if native:
-            # as memory: dense, and without a negation that is still to be done
-            dp, dx = (d.detach().resolve_neg().contiguous() for d in (pose_delta, point_delta))
-            lin.ctx.use_torch_stream()
-            lin.set_state_increments(points, frames, cams, dp, dx)
+            lin.set_state_increments(points, frames, cams, pose_delta, point_delta)
             lin.linearize()
             e = torch.empty((lin.M, 2), dtype=torch.float32, device=pose_delta.device)
             lin.copy_residuals_dev(e.data_ptr())

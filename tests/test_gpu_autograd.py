@@ -233,3 +233,29 @@ def test_pose_adjoint_shapes(gpu_ctx, F, M, shape):
         mag = np.bincount(fr, np.abs(J[0, c] * G[0]) + np.abs(J[1, c] * G[1]), F)
         assert (np.abs(got[:, c] - want) <= (n + 2) * 2.0 ** -24 * mag + 1e-30).all()
     lin.close()
+
+
+def test_set_state_increments_checks_its_tensors(gpu_ctx):
+    """What the device would read past or misread is refused before anything
+    is enqueued; strided tensors give what dense ones give."""
+    import torch
+    prob = _problem()
+    lin = BALinearizer.from_problem(prob, ctx=gpu_ctx)
+    F, P = len(prob.frames), len(prob.points)
+    state = (prob.points, prob.frames, prob.cams)
+    dp, dx = torch.full((F, 6), 1e-2, device="cuda"), torch.full((P, 3), 1e-2, device="cuda")
+    before = lin.get_state()
+    for a, b in ((dp[:-1], dx), (dp, dx[:-1]), (dp, dx[:1]), (dp.half(), dx), (dp, dx.int()), (dp.cpu(), dx),
+                 (dp, dx.cpu()), (dp.flatten(), dx), (dp, dx[:, :2])):
+        with pytest.raises(ValueError):
+            lin.set_state_increments(*state, a, b)
+    with pytest.raises(ValueError):
+        lin.set_state_increments(prob.points[:-1], prob.frames, prob.cams, dp, dx)
+    for x, y in zip(before, lin.get_state()):
+        np.testing.assert_array_equal(x, y)
+    lin.set_state_increments(*state, dp, dx)
+    want = lin.get_state()
+    lin.set_state_increments(*state, dp.repeat(1, 2)[:, ::2], dx.t().contiguous().t())
+    for x, y in zip(want, lin.get_state()):
+        np.testing.assert_array_equal(x, y)
+    lin.close()
