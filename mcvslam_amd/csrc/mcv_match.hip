@@ -32,6 +32,25 @@ struct MatchPair {
     int32_t* out;         // nq x (i0, d0, i1, d1)
 };
 
+// The workgroup's pair: its row's entry of a table in device memory, or the one
+// that came as an argument.  The popcount forms know which when compiled (kOne):
+// loaded from a choice of the two addresses the pair is not known to be uniform,
+// and their train rows became vector loads (64 rig frames, S<1,4>: 0.71 ms, 0.38
+// so); with two branches they were scheduled for fewer registers (20000 x 3000,
+// S<2,4>: 86 us, 68 so).  The matrix-core forms take branches (M<2> 124 us compiled
+// apart, 112 so, 300 x 5000).
+__device__ __forceinline__ MatchPair pair_of(const MatchPair* pairs, const MatchPair& one) {
+    MatchPair P = one;
+    if (pairs) P = pairs[blockIdx.y];
+    return P;
+}
+
+template <bool kOne>
+__device__ __forceinline__ MatchPair pair_of(const MatchPair* pairs, const MatchPair& one) {
+    if constexpr (kOne) return one;
+    else return pairs[blockIdx.y];
+}
+
 // keeps the two smallest keys (k0 <= k1): the new second is the median of
 // {k0, k1, key}
 __device__ __forceinline__ uint32_t med3_u32(uint32_t a, uint32_t b, uint32_t c) {
@@ -59,10 +78,10 @@ __device__ __forceinline__ void top2_insert2(uint32_t& k0, uint32_t& k1, uint32_
 // workgroup) and the 4 waves split the train set.  Train rows are
 // wave-uniform and come through scalar loads (SGPR operands of the XORs),
 // UNR rows per iteration; the four waves' top-2 keys merge through LDS.
-template <int QPL, int UNR>
+template <int QPL, int UNR, bool kOne>
 __global__ __launch_bounds__(256) void k_knn2_s(const MatchPair* pairs, MatchPair one) {
     __shared__ uint32_t sk[2][4][64 * QPL];
-    const MatchPair P = pairs ? pairs[blockIdx.y] : one;
+    const MatchPair P = pair_of<kOne>(pairs, one);
     const int nq = P.nq_dev ? min(*P.nq_dev, P.nq) : P.nq;
     const int nt = P.nt_dev ? min(*P.nt_dev, P.nt) : P.nt;
     const int lane = threadIdx.x & 63;
@@ -151,9 +170,10 @@ __global__ __launch_bounds__(256) void k_knn2_s(const MatchPair* pairs, MatchPai
 constexpr int kKnnTile = 128;
 constexpr int kKnnQ = 256;  // queries per workgroup
 
+template <bool kOne>
 __global__ __launch_bounds__(256) void k_knn2_lds(const MatchPair* pairs, MatchPair one) {
     __shared__ uint4 s_t[2][2 * kKnnTile];
-    const MatchPair P = pairs ? pairs[blockIdx.y] : one;
+    const MatchPair P = pair_of<kOne>(pairs, one);
     const int nq = P.nq_dev ? min(*P.nq_dev, P.nq) : P.nq;
     const int nt = P.nt_dev ? min(*P.nt_dev, P.nt) : P.nt;
     const int q0 = blockIdx.x * kKnnQ;
@@ -287,7 +307,7 @@ constexpr int kMSub = 4;  // 32-train sub-tiles per 128-train super-tile
 template <int QT>
 __global__ __launch_bounds__(256) void k_knn2_m(const MatchPair* pairs, MatchPair one) {
     __shared__ mcv_v4i s_b[kMSub][9][64];  // a super-tile as B operands, [sub-tile][step][lane]
-    const MatchPair P = pairs ? pairs[blockIdx.y] : one;
+    const MatchPair P = pair_of(pairs, one);
     const int nq = P.nq_dev ? min(*P.nq_dev, P.nq) : P.nq;
     const int nt = P.nt_dev ? min(*P.nt_dev, P.nt) : P.nt;
     const int q0 = blockIdx.x * 128 * QT;
@@ -756,6 +776,25 @@ struct KnnLaunch {
     uint2* part = nullptr;
 };
 
+// the popcount and int8 forms
+template <bool kOne>
+inline void launch_knn2_exact(int variant, const KnnLaunch& K, hipStream_t s) {
+    auto go = [&](auto kernel, int per) {
+        hipLaunchKernelGGL(kernel, dim3((K.max_nq + per - 1) / per, K.npairs), dim3(256), 0, s, K.pairs, K.one);
+    };
+    switch (variant) {
+    case 1: go(k_knn2_s<1, 4, kOne>, 64); break;
+    case 2: go(k_knn2_s<2, 2, kOne>, 128); break;
+    case 3: go(k_knn2_s<2, 4, kOne>, 128); break;
+    case 4: go(k_knn2_lds<kOne>, kKnnQ); break;
+    case 5: go(k_knn2_s<2, 8, kOne>, 128); break;
+    case 6: go(k_knn2_s<1, 8, kOne>, 64); break;
+    case 7: go(k_knn2_s<4, 2, kOne>, 256); break;
+    case 8: go(k_knn2_m<1>, 128); break;
+    default: go(k_knn2_m<2>, 256); break;
+    }
+}
+
 inline void launch_knn2(int variant, const KnnLaunch& K, hipStream_t s) {
     const int np = K.npairs, nq = K.max_nq;
     auto grid = [&](int per) { return dim3((nq + per - 1) / per, np); };
@@ -776,15 +815,9 @@ inline void launch_knn2(int variant, const KnnLaunch& K, hipStream_t s) {
             hipLaunchKernelGGL(k_knn2_merge, grid(16), dim3(256), 0, s, K.pairs, K.one, part, nq, seg);
         break;
     }
-    case 1: hipLaunchKernelGGL((k_knn2_s<1, 4>), grid(64), dim3(256), 0, s, K.pairs, K.one); break;
-    case 2: hipLaunchKernelGGL((k_knn2_s<2, 2>), grid(128), dim3(256), 0, s, K.pairs, K.one); break;
-    case 3: hipLaunchKernelGGL((k_knn2_s<2, 4>), grid(128), dim3(256), 0, s, K.pairs, K.one); break;
-    case 4: hipLaunchKernelGGL(k_knn2_lds, grid(kKnnQ), dim3(256), 0, s, K.pairs, K.one); break;
-    case 5: hipLaunchKernelGGL((k_knn2_s<2, 8>), grid(128), dim3(256), 0, s, K.pairs, K.one); break;
-    case 6: hipLaunchKernelGGL((k_knn2_s<1, 8>), grid(64), dim3(256), 0, s, K.pairs, K.one); break;
-    case 7: hipLaunchKernelGGL((k_knn2_s<4, 2>), grid(256), dim3(256), 0, s, K.pairs, K.one); break;
-    case 8: hipLaunchKernelGGL((k_knn2_m<1>), grid(128), dim3(256), 0, s, K.pairs, K.one); break;
-    default: hipLaunchKernelGGL((k_knn2_m<2>), grid(256), dim3(256), 0, s, K.pairs, K.one); break;
+    default:
+        if (K.pairs) launch_knn2_exact<false>(variant, K, s);
+        else launch_knn2_exact<true>(variant, K, s);
     }
 }
 
